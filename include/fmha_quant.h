@@ -44,6 +44,26 @@ int FMHAQuantizeI8BF16(hipStream_t stream, const uint16_t* x, long long n, float
                        int8_t* out);
 int FMHADequantizeI8BF16(hipStream_t stream, const int8_t* x, long long n, float amax, uint16_t* out);
 
+/* Abs-max and quantisation of up to three tensors of one type in one call - the Q, K and V of an attention call
+ * (test_fmha_i8.cpp:91-110 does them one after the other) - with the results of the two calls above for each of them.
+ * The maxima of the workgroups go through `workspace` (FMHA_QUANT_WORKSPACE_FLOATS floats of device memory, contents
+ * undefined before and after) instead of an atomic on one address, so a call is two launches, or one where every
+ * tensor fits one workgroup's registers.  amax_out: `count` floats of device memory.
+ * note: NULL, or `count` 8-byte words of pinned host memory that the device can write: word i receives
+ * (ticket << 32) | bits of amax[i] in one store, as soon as that maximum is known and before the int8 values are all
+ * written, so that a host that needs the maxima (FMHAParamI8 takes them by value) can go on while the device does. */
+#define FMHA_QUANT_MAX_TENSORS 3
+#define FMHA_QUANT_WORKSPACE_FLOATS 1024
+#define FMHA_QUANT_F32 0
+#define FMHA_QUANT_BF16 1
+typedef struct FMHAQuantTensor {
+  const void* x;   /* n elements, 16-byte aligned */
+  int8_t* out;     /* n bytes, 16-byte aligned */
+  long long n;
+} FMHAQuantTensor;
+int FMHAMeasureAndQuantizeI8(hipStream_t stream, const FMHAQuantTensor* tensors, int count, int element_type,
+                             float* workspace, float* amax_out, unsigned long long* note, unsigned ticket);
+
 #ifdef __cplusplus
 } /* extern "C" */
 #endif
