@@ -7,18 +7,22 @@ it with ctypes and keeps the reference's names and argument order (inc/fmha_i8.h
 
 ``q, k, v, padding_mask, o`` are device pointers (ints) or objects with ``data_ptr()`` (torch tensors on the GPU);
 ``stream`` is a ``hipStream_t`` value (int), a ``torch.cuda.Stream`` or None for the null stream.  There is no CPU
-fallback: if the library is missing or cannot be loaded, every call raises.
+fallback: if the library is missing or cannot be loaded, every call raises.  The entry points that take torch tensors
+(``fmha_infer_i8`` and the others at the end) run their host path in ``_fmha_torch.so``, built from csrc/fmha_torch.cpp.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libfmha_i8.so")
+TORCH_PATH = os.path.join(_HERE, "_fmha_torch.so")
 
 EXPORTED_SYMBOLS = ("FMHAInferI8", "FMHAInferI8Status", "FMHAInferI8CheckArgs", "FMHAInferI8StatusString",
                     "FMHAInferI8Version", "FMHAInferI8Cross", "FMHAInferI8CrossCheckArgs",
                     "FMHAInferI8CrossFullRangeP", "FMHAAbsMaxF32", "FMHAQuantizeI8", "FMHADequantizeI8",
-                    "FMHAAbsMaxBF16", "FMHAQuantizeI8BF16", "FMHADequantizeI8BF16")
+                    "FMHAAbsMaxBF16", "FMHAQuantizeI8BF16", "FMHADequantizeI8BF16", "FMHAMeasureAndQuantizeI8")
 
 FMHA_I8_OK = 0
 FMHA_I8_ERR_NULL_POINTER = 1
@@ -110,9 +114,38 @@ def load_library(path=None):
     L.FMHAQuantizeI8BF16.restype = C.c_int
     L.FMHADequantizeI8BF16.argtypes = L.FMHADequantizeI8.argtypes
     L.FMHADequantizeI8BF16.restype = C.c_int
+    L.FMHAMeasureAndQuantizeI8.argtypes = [ptr, ptr, C.c_int, C.c_int, ptr, ptr, ptr, C.c_uint]
+    L.FMHAMeasureAndQuantizeI8.restype = C.c_int
     if path is None:
         _lib = L
     return L
+
+
+_native = None
+
+
+def _load_native():
+    """The native host path of the torch entry points.  Raises if it is not built."""
+    global _native
+    load_library()
+    if _native is None:
+        if not os.path.exists(TORCH_PATH):
+            raise FileNotFoundError(
+                "%s is not built; run `python -c 'import __graft_entry__ as g; g.build()'` at the repository root"
+                % TORCH_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_fmha_torch", TORCH_PATH)
+        spec = importlib.util.spec_from_loader("_fmha_torch", loader, origin=TORCH_PATH)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _native = module
+    return _native
+
+
+def _result(r):
+    """What a native entry point returned: its result, or a status that becomes an FMHAError."""
+    if r.__class__ is int:
+        _check(r)
+    return r
 
 
 def _ptr(x):
@@ -211,34 +244,12 @@ def FMHADequantizeI8BF16(stream, x, n, amax, out):
 def quantize_tensor(x, amax=None, stream=None):
     """Convenience for a contiguous float32 or bfloat16 torch tensor on the GPU: returns (int8 tensor, amax as a
     1-element float32 device tensor).  With amax=None the maximum is measured on the GPU and never visits the host."""
-    import torch
-    if not (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16) and x.is_contiguous()):
-        raise ValueError("x must be a contiguous float32 or bfloat16 tensor on the GPU")
-    absmax, quant = (FMHAAbsMaxF32, FMHAQuantizeI8) if x.dtype == torch.float32 else (FMHAAbsMaxBF16, FMHAQuantizeI8BF16)
-    st = stream if stream is not None else torch.cuda.current_stream(x.device)
-    out = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-    if amax is None:
-        a = torch.empty(1, dtype=torch.float32, device=x.device)
-        _check(absmax(st, x, x.numel(), a))
-        _check(quant(st, x, x.numel(), 0.0, a, out))
-    else:
-        a = torch.full((1,), float(amax), dtype=torch.float32, device=x.device)
-        _check(quant(st, x, x.numel(), float(amax), None, out))
-    return out, a
+    return _result((_native or _load_native()).quantize_tensor(x, amax, stream))
 
 
 def dequantize_tensor(x, amax, stream=None, dtype=None):
     """int8 torch tensor on the GPU -> float32 (default) or bfloat16, (float)x / 127 * amax."""
-    import torch
-    if not (x.is_cuda and x.dtype == torch.int8 and x.is_contiguous()):
-        raise ValueError("x must be a contiguous int8 tensor on the GPU")
-    dtype = dtype or torch.float32
-    if dtype not in (torch.float32, torch.bfloat16):
-        raise ValueError("dtype must be float32 or bfloat16")
-    st = stream if stream is not None else torch.cuda.current_stream(x.device)
-    out = torch.empty(x.shape, dtype=dtype, device=x.device)
-    _check((FMHADequantizeI8 if dtype == torch.float32 else FMHADequantizeI8BF16)(st, x, x.numel(), float(amax), out))
-    return out
+    return _result((_native or _load_native()).dequantize_tensor(x, amax, stream, dtype))
 
 
 def fmha_infer_i8(q, k, v, padding_mask, q_amax, k_amax, v_amax, o_amax=1.0, out=None, stream=None,
@@ -249,32 +260,8 @@ def fmha_infer_i8(q, k, v, padding_mask, q_amax, k_amax, v_amax, o_amax=1.0, out
     out (inc/fmha_i8.cuh:189-192).  Returns int8 O [B, H, Sq, d].  Sq == S goes through the reference's entry point
     (FMHAInferI8Status), anything else through FMHAInferI8Cross; full_range_p=True selects
     FMHAInferI8CrossFullRangeP (P on 255 steps instead of 128).  Raises FMHAError on a nonzero status."""
-    import torch
-
-    for name, t in (("q", q), ("k", k), ("v", v), ("padding_mask", padding_mask)):
-        if not (t.is_cuda and t.dtype == torch.int8 and t.is_contiguous()):
-            raise ValueError("%s must be a contiguous int8 tensor on the GPU" % name)
-    B, H, Sq, d = q.shape
-    S = k.shape[2] if k.dim() == 4 else -1
-    if tuple(k.shape) != (B, H, S, d) or v.shape != k.shape or tuple(padding_mask.shape) != (B, S):
-        raise ValueError("shape mismatch: q [B,H,Sq,d], k/v [B,H,S,d] and padding_mask [B,S] expected")
-    if out is None:
-        out = torch.empty_like(q)
-    elif not (out.is_cuda and out.dtype == torch.int8 and out.is_contiguous() and out.shape == q.shape):
-        raise ValueError("out must be a contiguous int8 tensor on the GPU, shaped like q")
-    if stream is None:
-        stream = torch.cuda.current_stream(q.device)
-    param = FMHAParamI8(q_amax, k_amax, v_amax, o_amax, 1.0)
-    if full_range_p:
-        st = FMHAInferI8CrossFullRangeP(stream, param, FMHACrossAttnDescriptor(B, Sq, S, H, d), q, k, v, padding_mask,
-                                        out)
-    elif Sq == S:
-        st = FMHAInferI8Status(stream, param, AttnDataDescriptor(B, S, H, d), q, k, v, padding_mask, out, True)
-    else:
-        st = FMHAInferI8Cross(stream, param, FMHACrossAttnDescriptor(B, Sq, S, H, d), q, k, v, padding_mask, out)
-    if st != FMHA_I8_OK:
-        raise FMHAError(st, status_string(st))
-    return out
+    return _result((_native or _load_native()).infer_i8(q, k, v, padding_mask, q_amax, k_amax, v_amax, o_amax, out,
+                                                        stream, full_range_p))
 
 
 def fmha_infer_from_float(q, k, v, padding_mask, o_amax, out_dtype=None, stream=None, full_range_p=False):
@@ -282,25 +269,13 @@ def fmha_infer_from_float(q, k, v, padding_mask, o_amax, out_dtype=None, stream=
     host by their abs-max, :204-222 launches the kernel, inc/utils.hpp:53 de-quantises O): q [B,H,Sq,d] and k, v
     [B,H,S,d] are contiguous float32 or bfloat16 tensors on the GPU, padding_mask int8 [B,S] (nonzero = masked out),
     o_amax the range the int8 output is scaled to (the driver takes max |O| of its float path).  Returns
-    (O as out_dtype - default: q's dtype -, int8 O, (q_amax, k_amax, v_amax)).  The three maxima are read back in one
-    copy because FMHAParamI8 is passed by value, as in the reference; nothing else leaves the device."""
+    (O as out_dtype - default: q's dtype -, int8 O, (q_amax, k_amax, v_amax)).  The three maxima come back through
+    pinned memory because FMHAParamI8 is passed by value, as in the reference; nothing else leaves the device, and the
+    call waits for nothing but them."""
     import torch
-    if stream is None:
-        st = torch.cuda.current_stream(q.device)
-    elif isinstance(stream, torch.cuda.Stream):
-        st = stream
-    else:
+    if stream is not None and not isinstance(stream, torch.cuda.Stream):
         # Every tensor of the flow is allocated by torch's caching allocator, which orders the reuse of a block by the
         # stream it was allocated under; a raw handle gives it nothing to order by.
         raise TypeError("stream must be a torch.cuda.Stream (or None for the current one), not %r" % type(stream))
-    # The whole flow runs with `st` as torch's current stream: the intermediate and output tensors are then allocated
-    # under the stream that the kernels writing them are queued on.
-    with torch.cuda.stream(st):
-        (qi, qa), (ki, ka), (vi, va) = (quantize_tensor(t, stream=st) for t in (q, k, v))
-        amax = [float(x) for x in torch.cat((qa, ka, va)).cpu()]  # the one synchronisation of the flow
-        if min(amax) <= 0.0:
-            raise ValueError("q, k and v must each hold a nonzero value (abs-max %r)" % (amax,))
-        o_i8 = fmha_infer_i8(qi, ki, vi, padding_mask, amax[0], amax[1], amax[2], o_amax, stream=st,
-                             full_range_p=full_range_p)
-        o = dequantize_tensor(o_i8, o_amax, stream=st, dtype=out_dtype or q.dtype)
-    return o, o_i8, tuple(amax)
+    return _result((_native or _load_native()).infer_from_float(q, k, v, padding_mask, o_amax, out_dtype, stream,
+                                                                full_range_p))

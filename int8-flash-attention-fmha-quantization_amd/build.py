@@ -1,11 +1,15 @@
-"""Build recipe of libfmha_i8.so: one hipcc line, gfx950 only, output in-tree beside this file."""
+"""Build recipe of libfmha_i8.so (one hipcc line, gfx950 only) and of _fmha_torch.so, the host path of the torch entry
+points (one g++ line); outputs in-tree beside this file."""
 import os
 import shutil
 import subprocess
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_PATH = os.path.join(HERE, "libfmha_i8.so")
+TORCH_PATH = os.path.join(HERE, "_fmha_torch.so")
+TORCH_SOURCE = os.path.join(HERE, "csrc", "fmha_torch.cpp")
 SOURCES = [os.path.join(HERE, "csrc", "fmha_i8_api.hip"), os.path.join(HERE, "csrc", "fmha_quant.hip")]
 DEPENDS = SOURCES + [os.path.join(HERE, "csrc", "fmha_i8_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
                      os.path.join(ROOT, "include", "fmha_i8.h"), os.path.join(ROOT, "include", "fmha_param_i8.h"),
@@ -32,12 +36,34 @@ def build_library(verbose=False):
     return LIB_PATH
 
 
+def build_torch(verbose=False):
+    """Compile the native host path of the torch entry points into _fmha_torch.so (host code only; it calls the C ABI of
+    libfmha_i8.so, which must be built first and is found beside it at run time)."""
+    import torch
+    at = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc_path())))
+    include = [sysconfig.get_paths()["include"], os.path.join(at, "include"),
+               os.path.join(at, "include", "torch", "csrc", "api", "include"), os.path.join(rocm, "include")]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    cmd += [x for d in include for x in ("-I", d)]
+    cmd += ["-o", TORCH_PATH, TORCH_SOURCE, LIB_PATH, "-L", os.path.join(at, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
+    if verbose and proc.stdout.strip():
+        print(proc.stdout)
+    return TORCH_PATH
+
+
 def is_stale():
-    if not os.path.exists(LIB_PATH):
+    if not (os.path.exists(LIB_PATH) and os.path.exists(TORCH_PATH)):
         return True
     t = os.path.getmtime(LIB_PATH)
-    return any(os.path.getmtime(p) > t for p in DEPENDS)
+    return any(os.path.getmtime(p) > t for p in DEPENDS) or os.path.getmtime(TORCH_SOURCE) > os.path.getmtime(TORCH_PATH)
 
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_torch(verbose=True))
