@@ -11,13 +11,17 @@ LIB_PATH = os.path.join(HERE, "libfmha_i8.so")
 TORCH_PATH = os.path.join(HERE, "_fmha_torch.so")
 TORCH_SOURCE = os.path.join(HERE, "csrc", "fmha_torch.cpp")
 SOURCES = [os.path.join(HERE, "csrc", "fmha_i8_api.hip"), os.path.join(HERE, "csrc", "fmha_quant.hip")]
-DEPENDS = SOURCES + [os.path.join(HERE, "csrc", "fmha_i8_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
+DEPENDS = SOURCES + [os.path.join(HERE, "csrc", "fmha_i8_kernel.hip"),
+                     os.path.join(HERE, "csrc", "fmha_i8_split_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
                      os.path.join(ROOT, "include", "fmha_i8.h"), os.path.join(ROOT, "include", "fmha_param_i8.h"),
                      os.path.join(ROOT, "include", "fmha_quant.h")]
 # Packed-FP32 instruction selection is switched off for all device code (a flag for hipcc's device pass; the host pass
 # prints a harmless "not a recognized feature" note).
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+               # MFMA results in ordinary registers: a kernel of one wavefront per SIMD otherwise gets them in accumulation
+               # registers and copies every score out of them (a fifth of its instructions)
+               "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 
 def hipcc_path():

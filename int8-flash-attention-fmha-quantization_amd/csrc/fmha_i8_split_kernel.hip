@@ -1,0 +1,581 @@
+// The attention kernel for calls that fill too few compute units with workgroups of 256 query rows: a handful of heads, a
+// chunk of a prefill, one new row per sequence.  Same arithmetic as fmha_i8_fwd_kernel (fmha_i8_kernel.hip) and the same
+// BYTES for every row: which of the two kernels serves a call is a question of speed alone.
+//
+// A workgroup owns R groups of 32 query rows (R = 1 or 2) of one head and works on FOUR key blocks at a time, a "round":
+//   * wavefront (r, c) computes S^T, the block softmax and the quantised P^T of row group r and key block 4 i + c, so the
+//     part that bounds the attention kernel - the vector instructions of the softmax - is spread over four times as many
+//     wavefronts as there are row groups;
+//   * P^T goes through LDS to the four wavefronts of the row group, a quarter of what exchanging O would take, and each
+//     of them runs GEMM 2 and the online merge of all four key blocks, in key order, for ITS 32 output columns.  Every
+//     output element is thus merged by one wavefront, block after block, with the operations of the other kernel in the
+//     same order - which no scheme that merges partial results of separate key ranges can do, since float addition is not
+//     associative.  (At head_dim 64 there are two column tiles: two wavefronts do each.)
+// K and V tiles go HBM -> LDS directly, as in the other kernel and with the same swizzles.  A call has more than one key
+// block (the host sees to it): a single one leaves three quarters of the wavefronts without a softmax.
+#pragma once
+
+namespace fmha_i8_gfx950 {
+
+constexpr int kSplitKeys = 4;  // key blocks of a round
+
+template <int N>
+struct Const {  // a constant as a function argument
+  static constexpr int value = N;
+};
+
+// Division of a non-negative int by a divisor known on the host: a multiplication and two shifts where the division takes
+// some thirty instructions that everything in the prologue waits for (Granlund and Montgomery, 1994).
+struct Divisor {
+  unsigned factor;
+  int shift;  // of a divisor d > 1: ceil(log2 d) - 1; -1 for d = 1
+};
+inline Divisor make_divisor(int d) {
+  int bits = 0;
+  while ((1ll << bits) < d) ++bits;
+  if (bits == 0) return {0u, -1};
+  return {(unsigned)((((1ull << bits) - (unsigned)d) << 32) / (unsigned)d + 1), bits - 1};
+}
+__device__ __forceinline__ int divide(int n, Divisor d) {
+  if (d.shift < 0) return n;
+  const unsigned t = __umulhi(d.factor, (unsigned)n);
+  return (int)((t + (((unsigned)n - t) >> 1)) >> d.shift);
+}
+
+struct SplitKernelArgs : KernelArgs {
+  Divisor q_blocks_divisor, head_num_divisor;
+};
+
+template <int D, int BK, bool BIAS, bool FASTACC, bool FULLP, int R>
+__global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKernelArgs args) {
+  constexpr int kChunks = D / 16;
+  constexpr int kTileBytes = BK * D;
+  constexpr int kRowWaves = 4 * R;
+  constexpr int kRegions = kTileBytes / 1024;
+  constexpr int kLoads = kSplitKeys * kRegions / kRowWaves;  // direct-to-LDS loads per wavefront for four K (or V) tiles
+  constexpr int kRowsPerRegion = 1024 / D;
+  constexpr int kDSteps = D / 32;
+  constexpr int kKeyTiles = BK / 32;
+  // LDS holds 160 KB: tiles of 8 KB and less are double buffered.  Beside 128 KB of tiles there is room for 16 KB of P: all
+  // of a round, or, for two row groups and blocks of 128 keys, half of it, which then goes through in two steps.
+  constexpr int kBuffers = kTileBytes <= 8192 ? 2 : 1;
+  constexpr bool kTwoSteps = BK == 128 && R == 2;
+  constexpr int kPSlots = kTwoSteps ? 2 : 4;
+  // With one row group a K tile has one reader: the wavefront fetches it itself, waits for it itself, and asks for the next
+  // one as soon as it has read this one's operands, without any barrier.
+  constexpr bool kOwnK = kBuffers == 1 && R == 1;
+
+  __shared__ __attribute__((aligned(1024))) int8_t lds[kBuffers][2][kSplitKeys][kTileBytes];  // [buffer][K|V][slot][tile]
+  __shared__ __attribute__((aligned(16))) v4i lds_p[R][kPSlots][kKeyTiles][64];  // P^T as the B operand of GEMM 2
+  __shared__ __attribute__((aligned(16))) float lds_ml[R][kSplitKeys][32][2];    // block maximum and row sum per query
+  __shared__ unsigned lds_class4[kMaxKeyBlocks / 4];  // byte j: bit0 = block has a masked key, bit1 = all its keys are
+  __shared__ unsigned lds_mask[kMaxKeyBlocks * kBlockKSmall / 32];
+  __shared__ int lds_scan[kRowWaves];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5;
+  const int i32 = lane & 31;
+  const int c = wave & 3;   // key block of the round
+  const int r = wave >> 2;  // row group
+  const int u_out = c & (kDSteps - 1);  // output column tile of this wavefront
+
+  int wg;
+  {  // XCD-aware placement, as in the other kernel
+    const int L = blockIdx.x, per = args.total_wgs / kXcds, rem = args.total_wgs % kXcds, x = L % kXcds;
+    wg = x * per + (x < rem ? x : rem) + L / kXcds;
+  }
+  const int bh = divide(wg, args.q_blocks_divisor);
+  const int qb = wg - bh * args.q_blocks;
+  const int b = divide(bh, args.head_num_divisor);
+  const int S = args.seq_kv;
+  const int Sq = args.seq_q;
+  const int8_t* __restrict__ kg = args.k + (long)bh * S * D;
+  const int8_t* __restrict__ vg = args.v + (long)bh * S * D;
+  const int8_t* __restrict__ mg = args.mask + (long)b * S;
+  const long q_head_off = (long)bh * Sq * D;
+  const int n_blocks = (S + BK - 1) / BK;
+  const int S_pad = n_blocks * BK;
+  // A partly filled last block: the tile is fetched so that it ends with the last key (see the other kernel).
+  const int tail_rows = S - (n_blocks - 1) * BK;
+  const bool ragged = tail_rows != BK;
+  const int tail_kb = ragged ? n_blocks - 1 : -1;
+
+  // ---- tile loads --------------------------------------------------------------------------------------------------
+  // A load moves 1 KiB: lane l lands at byte 16 l of a region of the tile and fetches the chunk that the swizzle assigns to
+  // that place.  Addresses are 32-bit offsets inside the head.
+  const int ld_row_in = lane / kChunks;
+  const int region_of_wave = kRegions >= kRowWaves ? wave : wave % kRegions;  // of the loads that the wavefronts share
+  int ld_k, ld_k_odd = 0, ld_v;
+  {
+    const int p = lane % kChunks;
+    const int vrow = (D == 128) ? (ld_row_in | ((wave & 1) << 3)) : ld_row_in;
+    ld_k = ld_row_in * D + ((p ^ k_swizzle<D>(kOwnK ? ld_row_in : vrow)) << 4) + (kOwnK ? 0 : region_of_wave * 1024);
+    if (kOwnK) ld_k_odd = ld_row_in * D + ((p ^ k_swizzle<D>(ld_row_in + kRowsPerRegion)) << 4);
+    ld_v = ld_row_in * D + ((p ^ v_swizzle<D>(vrow)) << 4) + region_of_wave * 1024;
+  }
+  const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t*)&lds[0][0][0][0];
+  const unsigned lds_of_wave = lds_base + (unsigned)(region_of_wave * 1024);
+  // Load number `it` of this wavefront's kLoads for the four K (which = 0) or V (which = 1) tiles of a round.  A block past
+  // the last one (`last`) is replaced by it: the wait counts below are constants.
+  auto issue = [&](int round, int which, int it, int last) __attribute__((always_inline)) {
+    const bool own = kOwnK && which == 0;
+    const int slot = own ? c : kRegions >= kRowWaves ? it * kRowWaves / kRegions : (it * kRowWaves + wave) / kRegions;
+    const int region = own ? it : kRegions >= kRowWaves ? it * kRowWaves % kRegions : 0;  // besides region_of_wave
+    const int kb = min(kSplitKeys * round + slot, last);
+    const int tile = (kb == tail_kb ? (S - BK) * D : kb * kTileBytes) + region * 1024;
+    const unsigned dst = (own ? lds_base : lds_of_wave) +
+                         (unsigned)((((round & (kBuffers - 1)) * 2 + which) * kSplitKeys + slot) * kTileBytes + region * 1024);
+    int src = tile + (which ? ld_v : own && (it & 1) ? ld_k_odd : ld_k);
+    if (!fmha_in_bounds(src >= 0 && src + 16 <= S * D)) src = 0;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(src), "s"(which ? vg : kg) : "memory");
+  };
+  auto barrier = [&]() { asm volatile("s_barrier" ::: "memory"); };
+  auto wait_loads = [&](auto outstanding) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(outstanding)::value) : "memory"); };
+
+  const Const<0> none;
+  const Const<kLoads> one_kind;
+  const Const<kLoads / 2> half_kind;
+
+  // ---- prologue: mask bytes, Q rows and K of round 0, in this order; every load in flight before the first wait ---------
+  const int row0 = (qb * R + r) * 32;
+  const bool active = row0 < Sq;
+  constexpr int kKeysPerLane = 16;
+  constexpr int kKeysPerPass = kKeysPerLane * 64 * kRowWaves;
+  v4i mask_bytes, tail_bytes;
+  {
+    int j = kKeysPerLane * tid + kKeysPerLane <= S ? kKeysPerLane * tid : 0, jt = S - kKeysPerLane;
+    if (!fmha_in_bounds(j >= 0 && j + kKeysPerLane <= S && jt >= 0)) j = jt = 0;
+    asm volatile("global_load_dwordx4 %0, %2, %3\n\tglobal_load_dwordx4 %1, %4, %3"
+                 : "=&v"(mask_bytes), "=v"(tail_bytes) : "v"(j), "s"(mg), "v"(jt) : "memory");
+  }
+  v4i qreg[kDSteps];
+  {
+    int qrow = min(row0 + i32, Sq - 1);  // rows past the end load the last row (unused)
+    if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
+    const int8_t* qp = args.q + q_head_off;
+    const int qoff = qrow * D + 16 * g;
+#pragma unroll
+    for (int kk = 0; kk < kDSteps; ++kk)
+      asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(qreg[kk]) : "v"(qoff + 32 * kk), "s"(qp) : "memory");
+  }
+#pragma unroll
+  for (int it = 0; it < kLoads; ++it) issue(0, 0, it, n_blocks - 1);
+
+  // operand addresses (see the other kernel)
+  int k_read_off[kDSteps];
+#pragma unroll
+  for (int kk = 0; kk < kDSteps; ++kk) k_read_off[kk] = i32 * D + (((2 * kk + g) ^ k_swizzle<D>(i32)) << 4);
+  int v_read_off;
+  {
+    const int jin = lane & 15, hh = (lane >> 4) & 1, kslot = jin >> 1;
+    const int key_lane = 4 * g + (kslot < 4 ? kslot : kslot + 4);
+    v_read_off = key_lane * D + (((2 * u_out + hh) ^ v_swizzle<D>(key_lane)) << 4) + 8 * (jin & 1);
+  }
+
+  // ---- state -------------------------------------------------------------------------------------------------------
+  float o_f[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) o_f[e] = 0.f;
+  float m_ref = args.floor2 - 2.f * kLazyLog2, t_run = 0.f, l_run = 0.f;
+  const float c2 = BIAS ? args.c2 * kBaseScale : args.c2;
+  constexpr int kScoreBaseBits = score_base_bits<D>();
+  const float bias_c2 = BIAS ? __builtin_bit_cast(float, kScoreBaseBits) * c2 : 0.f;
+  v16i base_c, base_s;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    base_c[e] = FULLP ? 0 : kBaseBits;
+    base_s[e] = BIAS ? kScoreBaseBits : 0;
+  }
+  asm volatile("" : "+v"(base_c));
+  if (BIAS) asm volatile("" : "+v"(base_s));
+
+  // ---- classification of the key blocks, by all wavefronts (the bits are those of the other kernel) -----------------
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + kLoads) : "memory");
+  {
+    constexpr int kLanesPerBlock = BK / kKeysPerLane;
+    unsigned char* cls = reinterpret_cast<unsigned char*>(lds_class4);
+    auto nonzero_bytes = [](unsigned w) -> unsigned {
+      const unsigned t = (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
+      return (((t >> 7) * 0x00204081u) >> 21) & 15u;
+    };
+    auto nonzero16 = [&](const v4i& w) -> unsigned {
+      return nonzero_bytes((unsigned)w[0]) | (nonzero_bytes((unsigned)w[1]) << 4) | (nonzero_bytes((unsigned)w[2]) << 8) |
+             (nonzero_bytes((unsigned)w[3]) << 12);
+    };
+    int live_hi = -1;
+    for (int base = 0; base < S_pad; base += kKeysPerPass) {
+      const int j = base + kKeysPerLane * tid;
+      unsigned bits = 0xffffu;  // keys past the end count as masked
+      if (j + kKeysPerLane <= S) {
+        v4i w = mask_bytes;
+        if (base != 0) {
+          const int jj = fmha_in_bounds(j >= 0 && j + kKeysPerLane <= S) ? j : 0;
+          asm volatile("global_load_dwordx4 %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=v"(w) : "v"(jj), "s"(mg) : "memory");
+        }
+        bits = nonzero16(w);
+      } else if (j < S) {  // the one lane that straddles the end of the row
+        bits = ((nonzero16(tail_bytes) >> (kKeysPerLane - (S - j))) | (0xffffu << (S - j))) & 0xffffu;
+      }
+      const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
+      if ((lane & 1) == 0 && j < S_pad) lds_mask[j >> 5] = word;
+      const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
+      if (lane % kLanesPerBlock == 0 && j < S_pad) {
+        constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
+        const bool blk_some = ((some >> lane) & kBlockBits) != 0, blk_all = ((all >> lane) & kBlockBits) == kBlockBits;
+        cls[j / BK] = (unsigned char)((blk_some ? 1 : 0) | (blk_all ? 2 : 0));
+        if (!blk_all) live_hi = j / BK;
+      }
+    }
+    if (tid < kSplitKeys && n_blocks + tid < (n_blocks + kSplitKeys - 1) / kSplitKeys * kSplitKeys) cls[n_blocks + tid] = 3;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) live_hi = max(live_hi, __shfl_xor(live_hi, off));
+    if (lane == 0) lds_scan[wave] = live_hi;
+  }
+  // K of round 0 and the Q rows have landed
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
+  barrier();
+  int n = -1;
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) n = max(n, lds_scan[w]);
+  n = __builtin_amdgcn_readfirstlane(n) + 1;  // one past the last block with an unmasked key
+  const int rounds = (n + kSplitKeys - 1) / kSplitKeys;
+
+  // ---- one key block of one row group: S^T, softmax, P^T --------------------------------------------------------------
+  float m_blk = 0.f, l_blk = 0.f;
+  v4i pk[kKeyTiles];
+  auto scores_and_softmax = [&](int buf, int kb, int cls, auto between, auto in_softmax) __attribute__((always_inline)) {
+    const int8_t* lds_k = &lds[buf][0][c][0];
+    v16i acc[kKeyTiles];
+    int mx[2] = {(int)0x80000000, (int)0x80000000};
+    auto tile_max = [&](const v16i& a, int kk) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 8 * kk / kDSteps; e < 8 * (kk + 1) / kDSteps; e += 2) {
+        mx[0] = max(max(mx[0], a[e]), a[e + 1]);
+        mx[1] = max(max(mx[1], a[8 + e]), a[9 + e]);
+      }
+    };
+    auto gemm1 = [&](auto masked_t) __attribute__((always_inline)) {
+      constexpr bool kMasked = decltype(masked_t)::value;
+      if constexpr (kMasked) {
+        // start values of masked keys: lose every maximum, exponential exactly 0 (see the other kernel)
+        unsigned mw[kKeyTiles];
+        int gone = BIAS ? (int)0xFF000000 : -(1 << 30);
+        asm volatile("" : "+v"(gone));
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) mw[t] = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[kb * kKeyTiles + t]);
+        if (kb == tail_kb) {  // bit j of word t <-> key S - BK + 32 t + j; repeated keys count as masked
+          const int repeated = BK - tail_rows;
+#pragma unroll
+          for (int t = 0; t < kKeyTiles; ++t) {
+            const int start = S - BK + 32 * t, w = start >> 5, sh = start & 31;
+            const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[w]);
+            const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[w + (sh ? 1 : 0)]);
+            unsigned word = sh ? (lo >> sh) | (hi << (32 - sh)) : lo;
+            const int forced = repeated - 32 * t;
+            if (forced >= 32) word = 0xffffffffu;
+            else if (forced > 0) word |= (1u << forced) - 1u;
+            mw[t] = word;
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int key = 8 * (e / 4) + (e % 4);
+            const unsigned lo = (unsigned)(((int)(mw[t] << (31 - key))) >> 31), hi = (unsigned)(((int)(mw[t] << (27 - key))) >> 31);
+            const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
+            int x;
+            asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(base_s[e]), "v"(gone), "s"(lanes));
+            acc[t][e] = x;
+          }
+        asm volatile("s_nop 1" ::: "memory");  // (the compiler does not know that these statements wrote registers an MFMA reads)
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // Operand reads run two key tiles ahead of the MFMAs, held there by the fences: left alone, the compiler reads each
+      // operand right in front of its MFMA and the wavefront waits out the LDS latency sixteen times.
+      v4i ka[3][kDSteps];
+      auto read_k = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kk = 0; kk < kDSteps; ++kk) ka[t % 3][kk] = *reinterpret_cast<const v4i*>(lds_k + k_read_off[kk] + 32 * t * D);
+      };
+      read_k(0);
+      if (kKeyTiles > 1) read_k(1);
+#pragma unroll
+      for (int t = 0; t < kKeyTiles; ++t) {
+        if (t + 2 < kKeyTiles) read_k(t + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < kDSteps; ++kk) {
+          acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[t % 3][kk], qreg[kk], (kk == 0 && !kMasked) ? base_s : acc[t], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          between(t * kDSteps + kk, kKeyTiles * kDSteps);
+          if (t >= 1) tile_max(acc[t - 1], kk);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    if (cls & 1) gemm1(Const<1>{});
+    else gemm1(Const<0>{});
+#pragma unroll
+    for (int kk = 0; kk < kDSteps; ++kk) tile_max(acc[kKeyTiles - 1], kk);
+    int ti = max(mx[0], mx[1]);
+    ti = half_max(ti);
+    if (cls & 1) ti = max(ti, (BIAS ? kScoreBaseBits : 0) - 1000000);  // the reference's sentinel (inc/fmha_i8.cuh:191-193)
+    const float top = BIAS ? __int_as_float(ti) : (float)ti;
+    float off = top * c2;
+    if (!BIAS) off = __builtin_fmaf(fabsf(off), 2.384185791015625e-07f, off);
+    if (!BIAS) off = fmaxf(off, args.floor2);
+    m_blk = off - bias_c2;
+    const float offq = off - (FULLP ? kLog2PscaleFull : kLog2Pscale);
+    // Step q: the exponentials of quad q, the scaling of quad q+1 and the sum of quad q-1 (in the order of additions of the
+    // other kernel), and a place for a tile load.
+    constexpr int kQuads = 4 * kKeyTiles;
+    float x[kQuads][4];
+    auto scale = [&](int qd) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int s = acc[qd / 4][4 * (qd % 4) + j];
+        x[qd][j] = __builtin_fmaf(BIAS ? __int_as_float(s) : (float)s, c2, -offq);
+      }
+    };
+    auto sum = [&](int qd) __attribute__((always_inline)) {
+      float s01 = x[qd][0] + x[qd][1];
+      const float s23 = x[qd][2] + x[qd][3];
+      s01 += s23;
+      l_blk += s01;
+    };
+    l_blk = 0.f;
+    scale(0);
+#pragma unroll
+    for (int qd = 0; qd < kQuads; ++qd) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[qd][j] = __builtin_amdgcn_exp2f(x[qd][j]);
+      if (qd + 1 < kQuads) scale(qd + 1);
+      if (qd >= 1) sum(qd - 1);
+      if (kOwnK) {  // (keeps the step in front of the load)
+        asm volatile("" : "+v"(x[qd][0]), "+v"(x[qd][1]), "+v"(x[qd][2]), "+v"(x[qd][3]));
+        in_softmax(qd, kQuads);
+      }
+    }
+    sum(kQuads - 1);
+    l_blk = half_sum(l_blk);
+#pragma unroll
+    for (int qd = 0; qd < 4 * kKeyTiles; ++qd) {
+      const float(&e)[4] = x[qd];
+      const v2s lo = FULLP ? __builtin_amdgcn_cvt_pknorm_i16(e[0], e[1]) : __builtin_amdgcn_cvt_pknorm_i16(-e[0], -e[1]);
+      const v2s hi = FULLP ? __builtin_amdgcn_cvt_pknorm_i16(e[2], e[3]) : __builtin_amdgcn_cvt_pknorm_i16(-e[2], -e[3]);
+      const int four = __builtin_amdgcn_perm(__builtin_bit_cast(int, hi), __builtin_bit_cast(int, lo), 0x06040200);
+      pk[qd / 4][qd % 4] = FULLP ? four ^ (int)0x80808080 : four;
+    }
+  };
+  auto publish_p = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kKeyTiles; ++t) lds_p[r][c & (kPSlots - 1)][t][lane] = pk[t];
+  };
+  auto publish_ml = [&]() __attribute__((always_inline)) {
+    lds_ml[r][c][i32][0] = m_blk;
+    lds_ml[r][c][i32][1] = l_blk;
+  };
+
+  // ---- GEMM 2 and the merge of key blocks first .. first+COUNT-1 of the round, for this wavefront's columns -----------
+  // A block without an unmasked key enters with weight 0 (its P may be anything: any int8 leaves the accumulators finite).
+  auto gemm2_merge = [&](int buf, int first, auto count_t, unsigned cls4, auto between) __attribute__((always_inline)) {
+    constexpr int kCount = decltype(count_t)::value;
+    typedef v2i __attribute__((address_space(3))) * lds_v2i_ptr;
+    v4i va[2][kKeyTiles], p[2][kKeyTiles];
+    v16i oacc[2];
+    auto read = [&](int j) __attribute__((always_inline)) {
+      const int8_t* lds_v = &lds[buf][1][first + j][0];
+#pragma unroll
+      for (int t = 0; t < kKeyTiles; ++t) {
+        const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(lds_v + v_read_off + 32 * t * D));
+        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(lds_v + v_read_off + 32 * t * D + 16 * D));
+        va[j & 1][t] = v4i{lo[0], lo[1], hi[0], hi[1]};
+        p[j & 1][t] = lds_p[r][(first + j) & (kPSlots - 1)][t][lane];
+      }
+    };
+    float take[kCount], keep[kCount];
+    auto merge_piece = [&](int j, int piece, int pieces, auto moved_t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 16 * piece / pieces; e < 16 * (piece + 1) / pieces; ++e) {
+        const float v = FASTACC ? __int_as_float(oacc[j & 1][e]) : __int_as_float(oacc[j & 1][e]) - (FULLP ? kBaseFull : kBase);
+        o_f[e] = __builtin_fmaf(FULLP ? take[j] : -take[j], v, decltype(moved_t)::value ? o_f[e] * keep[j] : o_f[e]);
+      }
+    };
+    auto start = [&](int j) __attribute__((always_inline)) {
+      oacc[j & 1] = base_c;
+      if (FULLP) {
+        // 128 times the column sums of the tile, in the accumulators' own layout: a product with 64s, doubled
+        const v4i half = {0x40404040, 0x40404040, 0x40404040, 0x40404040};
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t)
+          oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], half, oacc[j & 1], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[j & 1][e] = 2 * oacc[j & 1][e] + kBaseBitsFull;
+      }
+    };
+    auto product = [&](int j, int t) __attribute__((always_inline)) {
+      oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], p[j & 1][t], oacc[j & 1], 0, 0, 0);
+    };
+    // Operand reads one block ahead; the merge of a block stands behind the MFMAs of the next one.
+    float ml[kCount][2];
+#pragma unroll
+    for (int j = 0; j < kCount; ++j) {
+      ml[j][0] = lds_ml[r][first + j][i32][0];
+      ml[j][1] = lds_ml[r][first + j][i32][1];
+    }
+    read(0);
+    read(1);
+    __builtin_amdgcn_sched_barrier(0);
+    start(0);
+#pragma unroll
+    for (int t = 0; t < kKeyTiles; ++t) {
+      product(0, t);
+      between(t, kCount * kKeyTiles);
+    }
+    bool moved = false;  // some row's reference exponent moves (wave-uniform)
+#pragma unroll
+    for (int j = 0; j < kCount; ++j) {
+      const bool dead = (cls4 >> (8 * (first + j))) & 2;
+      const float mb = dead ? -__builtin_inff() : ml[j][0], lb = dead ? 0.f : ml[j][1];
+      const bool moves = __ballot(mb > m_ref + kLazyLog2) != 0;
+      const float m_new = moves ? fmaxf(m_ref, mb) : m_ref;
+      keep[j] = __builtin_amdgcn_exp2f(m_ref - m_new);  // exactly 1 where nothing moves
+      m_ref = m_new;
+      moved |= moves;
+      take[j] = __builtin_amdgcn_exp2f(mb - m_ref);
+      l_run = __builtin_fmaf(take[j], lb, l_run * keep[j]);
+      if (FASTACC) t_run = t_run * keep[j] + take[j];
+    }
+    auto rest = [&](auto moved_t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 1; j < kCount; ++j) {
+        start(j);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) {
+          product(j, t);
+          __builtin_amdgcn_sched_barrier(0);
+          between(j * kKeyTiles + t, kCount * kKeyTiles);
+          merge_piece(j - 1, t, kKeyTiles, moved_t);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (j + 1 < kCount) read(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      merge_piece(kCount - 1, 0, 1, moved_t);
+    };
+    if (moved) rest(Const<1>{});
+    else rest(Const<0>{});
+  };
+
+  // ---- the rounds --------------------------------------------------------------------------------------------------
+  // S: GEMM 1 and softmax of block 4i+c; G: GEMM 2 and merge.  Barrier b1 publishes P and V of the round, b4 frees them and
+  // publishes K of the next round.  The tile loads of a round stand behind the MFMAs, one after each: the CU's vector
+  // memory path takes 64 bytes per cycle, a wavefront that issues its share in one go is held for 1000 cycles per kind.
+  //   two buffers:              S(i) with K(i+1) | b1 | G(i) with V(i+1) | b4
+  //   one buffer, R = 1:        S(i) with V(i) behind GEMM 1 and K(i+1) in the softmax | b1 | G(i) | b4
+  //   one buffer, two steps:    S(i) with V of blocks 2, 3 of i, P of blocks 0, 1 | b1 | G of blocks 0, 1 with K(i+1) | b2 |
+  //                             P of blocks 2, 3 | b3 | G of blocks 2, 3 with V of blocks 0, 1 of i+1 | b4
+  auto written = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  // V of round 0, or the half of it that the rounds themselves do not ask for
+  if (!kOwnK && rounds > 0) {
+#pragma unroll
+    for (int it = 0; it < (kBuffers == 2 ? kLoads : kLoads / 2); ++it) issue(0, 1, it, n - 1);
+  }
+  for (int i = 0; i < rounds; ++i) {
+    const int buf = i & (kBuffers - 1);
+    const bool more = i + 1 < rounds;
+    const unsigned cls4 = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_class4[i]);
+    const int cls = (cls4 >> (8 * c)) & 3;
+    const bool work = active && !(cls & 2);
+    // `loads` tile loads from number `first` on, spread over `slots` places
+    auto spread = [&](bool wanted, int round, int which, int first, int loads, int slot, int slots) __attribute__((always_inline)) {
+#pragma unroll
+      for (int it = slot * loads / slots; it < (slot + 1) * loads / slots; ++it)
+        if (wanted) issue(round, which, first + it, n - 1);
+    };
+    constexpr bool kTwoBuffers = kBuffers == 2;
+    constexpr int kHalf = kLoads / 2;
+    auto loads_in_gemm1 = [&](int slot, int slots) __attribute__((always_inline)) {
+      if (kTwoBuffers) spread(more, i + 1, 0, 0, kLoads, slot, slots);
+      else if (kOwnK) spread(true, i, 1, 0, kLoads, slot, slots);
+      else spread(true, i, 1, kHalf, kHalf, slot, slots);
+    };
+    auto loads_in_softmax = [&](int slot, int slots) __attribute__((always_inline)) {
+      if (kOwnK) spread(more, i + 1, 0, 0, kLoads, slot, slots);
+    };
+    auto loads_in_gemm2 = [&](int slot, int slots) __attribute__((always_inline)) {
+      if (kTwoBuffers) spread(more, i + 1, 1, 0, kTwoSteps ? kHalf : kLoads, slot, slots);
+      else if (!kOwnK) spread(more, i + 1, 0, 0, kLoads, slot, slots);
+    };
+    auto loads_in_second_step = [&](int slot, int slots) __attribute__((always_inline)) {
+      if (kTwoBuffers) spread(more, i + 1, 1, kHalf, kHalf, slot, slots);
+      else spread(more, i + 1, 1, 0, kHalf, slot, slots);
+    };
+    if (work) {
+      scores_and_softmax(buf, kSplitKeys * i + c, cls, loads_in_gemm1, loads_in_softmax);
+      publish_ml();
+      if (!kTwoSteps || c < 2) publish_p();
+    } else {
+      loads_in_gemm1(0, 1);
+      loads_in_softmax(0, 1);
+    }
+    written();
+    // V of this round (of its blocks 0, 1 in the last form); what has been asked for since may be in flight
+    if (!kTwoBuffers && !kOwnK) wait_loads(half_kind);
+    else if (more) wait_loads(one_kind);
+    else wait_loads(none);
+    barrier();  // b1
+    if (active) gemm2_merge(buf, 0, Const<kTwoSteps ? 2 : 4>{}, cls4, loads_in_gemm2);
+    else loads_in_gemm2(0, 1);
+    if constexpr (kTwoSteps) {
+      barrier();  // b2
+      if (work && c >= 2) publish_p();
+      written();
+      if (!kTwoBuffers && more) wait_loads(one_kind);  // V of blocks 2, 3
+      else if (!kTwoBuffers) wait_loads(none);
+      barrier();  // b3
+      if (active) gemm2_merge(buf, 2, Const<2>{}, cls4, loads_in_second_step);
+      else loads_in_second_step(0, 1);
+    }
+    // K of the next round
+    if (kTwoBuffers && more) wait_loads(one_kind);
+    else if (!kTwoBuffers && !kOwnK && more) wait_loads(half_kind);
+    else wait_loads(none);
+    barrier();  // b4
+  }
+  wait_loads(none);  // nothing may still be writing LDS when the wavefront ends (only possible when every key is masked)
+  if (!active || c >= kDSteps) return;
+
+  // ---- epilogue (see the other kernel) -----------------------------------------------------------------------------
+  const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
+  const float corr = FASTACC ? (FULLP ? -kBaseFull * t_run : kBase * t_run) : 0.f;
+  int w[4];  // w[a]: output dims 32 u_out + 8a + 4g .. +3 of query row i32
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    float y[4];
+#pragma unroll
+    for (int bb = 0; bb < 4; ++bb)
+      y[bb] = __builtin_amdgcn_fmed3f(__builtin_fmaf(FASTACC ? o_f[4 * a + bb] + corr : o_f[4 * a + bb], fin, kMagic), kMagic - 127.f, kMagic + 127.f);
+    const int lo = __builtin_amdgcn_perm(__float_as_int(y[1]), __float_as_int(y[0]), 0x0c0c0400);
+    const int hi = __builtin_amdgcn_perm(__float_as_int(y[3]), __float_as_int(y[2]), 0x0c0c0400);
+    w[a] = __builtin_amdgcn_perm(hi, lo, 0x05040100);
+  }
+  if (row0 + i32 >= Sq) return;
+  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D)) return;
+  // words a of lanes l and l+32 are neighbours: the exchange hands lane l the pair of word 0 (2) and lane l+32 that of word 1 (3)
+  int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * u_out + 8 * g;
+#pragma unroll
+  for (int a = 0; a < 4; a += 2) {
+    const auto s = __builtin_amdgcn_permlane32_swap(w[a], w[a + 1], false, false);
+    *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
+  }
+}
+
+}  // namespace fmha_i8_gfx950

@@ -33,6 +33,12 @@
 //                        the loop (the kernel's own choice otherwise): for re-measuring what the placement costs
 #pragma once
 
+// The test builds that change the attention kernel of 256-row workgroups serve every call with it, so that what they are
+// compared or timed for is that kernel at every size (the shipped library writes the same bytes with either kernel).
+#if defined(FMHA_FEW_INSTANTIATIONS) || defined(FMHA_TWO_BARRIERS) || defined(FMHA_LOOP_PAD_A)
+#define FMHA_NO_SPLIT_KERNEL
+#endif
+
 namespace fmha_i8_gfx950 {
 namespace test_build {
 

@@ -1,0 +1,80 @@
+"""The kernel that serves calls of few workgroups (fmha_i8_split_kernel: one or two groups of 32 query rows per workgroup,
+four key blocks at a time) must write the bytes of the kernel of 256-row workgroups for every row: a caller sees no
+difference between a head computed alone and in a batch.  The reference is the test build that has the latter only."""
+import ctypes as C
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import fmha_cases as fc
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+CSRC = os.path.join(ROOT, "int8-flash-attention-fmha-quantization_amd", "csrc")
+
+# (B, H, Sq, S, d): row groups 1 and 2 of the split kernel, one to many rounds of four key blocks, rounds that are not full,
+# rows that do not fill a group, both block sizes, ragged ends, sequences shorter than a block, more than one workgroup
+# per compute unit, mask rows of more than one classification pass
+SHAPES = [
+    (1, 2, 1, 2048, 128), (2, 3, 31, 640, 64), (1, 2, 33, 1100, 128), (1, 3, 512, 512, 64), (1, 4, 777, 777, 128),
+    (2, 8, 320, 320, 128), (1, 16, 777, 777, 64), (1, 32, 300, 1536, 128), (4, 12, 256, 448, 64), (2, 24, 65, 1027, 128),
+    (1, 2, 40, 70, 128), (1, 1, 33, 15, 64), (2, 1, 5, 3, 128), (1, 2, 40, 8300, 64), (24, 16, 3, 300, 128), (1, 1, 2, 65536, 64),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("full_range_p", [False, True], ids=["P_128_steps", "P_255_steps"])
+@pytest.mark.parametrize("B,H,Sq,S,d", SHAPES)
+def test_same_bytes_as_the_kernel_of_256_row_workgroups(pkg, dev, B, H, Sq, S, d, full_range_p):
+    import torch
+    path = os.path.join(HERE, "bin", "libfmha_i8_two_barriers.so")
+    assert os.path.exists(path), "%s is missing: build it with `make -C tests all`" % path
+    wide, shipped = C.CDLL(path), pkg.load_library()
+    name = "FMHAInferI8CrossFullRangeP" if full_range_p else "FMHAInferI8Cross"
+    # normal scores read as floats; a large score scale (converted scores); an output scale that rules out the one-fma merge
+    for n, (dist, scale, o_amax, pad) in enumerate([("normal", 1, 1.0, "scatter"), ("student_t", 8, 1.0, "none"), ("normal", 1, 0.1, "dead")]):
+        c = fc.make_inputs(B, H, (S + 63) // 64 * 64, d, dist=dist, pad="scatter" if pad == "scatter" else "none", seed=900 + n)
+        mask = c["mask"][:, :S].copy()
+        if pad == "dead":  # whole blocks without an unmasked key, at the end and inside; one batch entry with none at all
+            mask[:, S - S // 3:] = 1
+            mask[:, S // 8:S // 8 + 260] = 1
+            if B > 1:
+                mask[1] = 1
+        q = fc.make_inputs(B, H, Sq, d, dist=dist, seed=950 + n)["q"]
+        t = [torch.from_numpy(np.ascontiguousarray(a)).to(dev) for a in (q, c["k"][:, :, :S], c["v"][:, :, :S], mask)]
+        scales = pkg.FMHAParamI8(c["q_amax"] * scale, c["k_amax"], c["v_amax"], o_amax, 1.0)
+        outs = []
+        for lib in (wide, shipped):
+            entry = getattr(lib, name)
+            entry.argtypes = [C.c_void_p, pkg.FMHAParamI8, pkg.FMHACrossAttnDescriptor] + [C.c_void_p] * 5
+            entry.restype = C.c_int
+            o = torch.full((t[0].numel() + 256,), 77, dtype=torch.int8, device=dev)
+            print((B, H, Sq, S, d, dist, pad, full_range_p), flush=True)
+            assert entry(None, scales, pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d), *(x.data_ptr() for x in t), o.data_ptr()) == 0
+            torch.cuda.synchronize()
+            outs.append(o)
+        assert torch.equal(outs[0], outs[1]), (dist, pad, int((outs[0] != outs[1]).sum()))
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(tmp_path):
+    """The same check as for the other kernel (test_kernel_async_loads.py), on the compiled split kernel."""
+    from test_kernel_async_loads import _check_function
+    args = ["<%d, %d, %s, %s, %s, %d>" % (d, bk, bias, fast, full, r)
+            for d, bk, bias, fast, full in ((128, 128, "true", "true", "false"), (64, 64, "false", "false", "true"),
+                                            (128, 64, "false", "true", "false"), (64, 128, "true", "false", "true")) for r in (1, 2)]
+    src = tmp_path / "split.hip"
+    src.write_text('#include "%s/fmha_i8_kernel.hip"\n#include "%s/fmha_i8_split_kernel.hip"\nnamespace fmha_i8_gfx950 {\n' % (CSRC, CSRC) +
+                   "".join("template __global__ void fmha_i8_split_kernel%s(SplitKernelArgs);\n" % a for a in args) + "}\n")
+    out = tmp_path / "split.s"
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-S", "--cuda-device-only", "-o", str(out), str(src)],
+                   check=True, capture_output=True)
+    funcs = re.split(r"\n(?=_ZN14fmha_i8_gfx95020fmha_i8_split_kernel[^\n]*:\s)", out.read_text())[1:]
+    assert len(funcs) == len(args)
+    for f in funcs:
+        assert _check_function(f.split(":")[0], f) >= 4  # mask bytes (twice) and the Q rows
