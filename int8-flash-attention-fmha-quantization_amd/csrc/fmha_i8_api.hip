@@ -10,6 +10,7 @@
 #include "fmha_i8_kernel.hip"
 #ifndef FMHA_NO_SPLIT_KERNEL
 #include "fmha_i8_split_kernel.hip"
+#include "fmha_i8_pair_kernel.hip"
 #endif
 
 namespace {
@@ -92,58 +93,80 @@ hipError_t launch_variant(Variant var, dim3 grid, dim3 block, hipStream_t stream
 
 #ifndef FMHA_NO_SPLIT_KERNEL
 template <int D, int BK, int R>
-hipError_t launch_split2(Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
+const void* split_kernel(Variant var) {
+  using namespace fmha_i8_gfx950;
+#define FMHA_VARIANT(KERNEL, ...)                                                                                    \
+  (var.full_range_p ? (var.bias ? (var.fast ? FMHA_KERNEL(KERNEL, true, true, true) : FMHA_KERNEL(KERNEL, true, false, true))        \
+                                : (var.fast ? FMHA_KERNEL(KERNEL, false, true, true) : FMHA_KERNEL(KERNEL, false, false, true)))     \
+                    : (var.bias ? (var.fast ? FMHA_KERNEL(KERNEL, true, true, false) : FMHA_KERNEL(KERNEL, true, false, false))      \
+                                : (var.fast ? FMHA_KERNEL(KERNEL, false, true, false) : FMHA_KERNEL(KERNEL, false, false, false))))
+  if constexpr (R == 4) {
+#define FMHA_KERNEL(KERNEL, BB, FF, PP) reinterpret_cast<const void*>(&KERNEL<D, BK, BB, FF, PP>)
+    return FMHA_VARIANT(fmha_i8_pair_kernel);
+#undef FMHA_KERNEL
+  } else {
+#define FMHA_KERNEL(KERNEL, BB, FF, PP) reinterpret_cast<const void*>(&KERNEL<D, BK, BB, FF, PP, R>)
+    return FMHA_VARIANT(fmha_i8_split_kernel);
+#undef FMHA_KERNEL
+  }
+#undef FMHA_VARIANT
+}
+template <int D, int BK>
+hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
   using namespace fmha_i8_gfx950;
   SplitKernelArgs args{of_call};
-  const int heads = args.total_wgs / args.q_blocks;
-  args.q_blocks = (args.seq_q + 32 * R - 1) / (32 * R);
+  const int heads = args.total_wgs / args.q_blocks, rows = 32 * row_groups;
+  args.q_blocks = (args.seq_q + rows - 1) / rows;
   args.total_wgs = heads * args.q_blocks;
   args.q_blocks_divisor = make_divisor(args.q_blocks);
   args.head_num_divisor = make_divisor(args.head_num);
   void* kernel_args[] = {&args};
-#define FMHA_KERNEL(BB, FF, PP) reinterpret_cast<const void*>(&fmha_i8_split_kernel<D, BK, BB, FF, PP, R>)
-  const void* kernel = var.full_range_p ? (var.bias ? (var.fast ? FMHA_KERNEL(true, true, true) : FMHA_KERNEL(true, false, true))
-                                                    : (var.fast ? FMHA_KERNEL(false, true, true) : FMHA_KERNEL(false, false, true)))
-                                        : (var.bias ? (var.fast ? FMHA_KERNEL(true, true, false) : FMHA_KERNEL(true, false, false))
-                                                    : (var.fast ? FMHA_KERNEL(false, true, false) : FMHA_KERNEL(false, false, false)));
-#undef FMHA_KERNEL
-  return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(256 * R), kernel_args, 0, stream);
+  const void* kernel = row_groups == 1 ? split_kernel<D, BK, 1>(var) : row_groups == 2 ? split_kernel<D, BK, 2>(var) : split_kernel<D, BK, 4>(var);
+  return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 ? 256 : 512), kernel_args, 0, stream);
 }
-template <int D, int BK>
-hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& args) {
-  return row_groups == 1 ? launch_split2<D, BK, 1>(var, stream, args) : launch_split2<D, BK, 2>(var, stream, args);
-}
-// Row groups per workgroup of the split kernel that serves a call, or 0 for the kernel of 256-row workgroups.
+// Groups of 32 query rows per workgroup of the kernel that serves a call: 1 or 2 (fmha_i8_split_kernel), 4
+// (fmha_i8_pair_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
 // Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (start + step * rounds): a round is
-// one key block for the 256-row kernel and four for the split kernels.  The constants are microseconds * 100 measured on one
-// MI355X at 512 to 4096 keys with one workgroup per CU, rows [head_dim 64, 128][blocks of 64, 128 keys]; what they order is
-// far apart nearly everywhere (H8 Sq2048 S2048 d128: 31.5 us in 256-row workgroups, 18.7 with two row groups; H4: 31.3 and
-// 14.6 with one), so that a few percent of error only shifts the boundary between equals.
-int split_row_groups(const FMHACrossAttnDescriptor& a, int block_keys) {
+// one key block for the last two and four for the split kernel.  The constants are microseconds * 100 measured on one MI355X
+// at 512 to 4096 keys with one workgroup per CU, [head_dim 64, 128][blocks of 64, 128 keys].  What they order is far apart
+// nearly everywhere - d128, S2048: H4 31.3 us in 256-row workgroups, 24.3 in those of four groups, 17.6 of two, 13.5 of one;
+// H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error only shift the
+// boundary between equals.
+int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
 #ifdef FMHA_SPLIT_FORCE
   return a.seq_len_kv > block_keys ? FMHA_SPLIT_FORCE : 0;
 #endif
   if (a.seq_len_kv <= block_keys) return 0;
-  struct Cost { int start, step; };
-  static constexpr Cost kWide[2][2] = {{{0, 95}, {100, 128}}, {{160, 112}, {250, 162}}};
-  static constexpr Cost kSplit[2][2][2] = {{{{60, 130}, {60, 208}}, {{80, 160}, {100, 263}}},    // one row group
-                                           {{{0, 207}, {65, 310}}, {{70, 220}, {150, 348}}}};    // two
+  struct Kernel {
+    int row_groups, keys_per_round;
+    struct { int start, step; } cost[2][2];
+  };
+  static constexpr Kernel kKernels[] = {{0, 1, {{{0, 95}, {95, 128}}, {{160, 112}, {250, 162}}}},
+                                        {4, 1, {{{110, 65}, {170, 97}}, {{180, 89}, {300, 116}}}},
+                                        {2, 4, {{{0, 208}, {45, 312}}, {{60, 220}, {140, 332}}}},
+                                        {1, 4, {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}}}};
   const int d = a.head_dim == 128, k = block_keys == fmha_i8_gfx950::kBlockK;
   const long long heads = (long long)a.batch_num * a.head_num;
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
-  const int rounds = (blocks + fmha_i8_gfx950::kSplitKeys - 1) / fmha_i8_gfx950::kSplitKeys;
-  auto cost = [&](int rows, const Cost& c, int steps) {
+  int best = 0;
+  long long least = -1;
+  for (const Kernel& kernel : kKernels) {
+    // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
+    // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 14.1 with two; d64: 11.7 either way).
+    const bool helper = a.seq_len_q <= 32 && kernel.row_groups == 2;
+    if (helper && !(d && k)) continue;
+    const int rows = kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups;
+    const auto& c = kernel.cost[d][k];
+    const int rounds = (blocks + kernel.keys_per_round - 1) / kernel.keys_per_round;
     const long long per_cu = (heads * ((a.seq_len_q + rows - 1) / rows) + 255) / 256;
-    return per_cu * (c.start + c.step * steps);
-  };
-  const long long wide = cost(fmha_i8_gfx950::kBlockQ, kWide[d][k], blocks);
-  const long long one = cost(32, kSplit[0][d][k], rounds);
-  // With one row group's worth of rows the second group only helps to fetch the tiles: worth it where a round is 128 KB
-  // (B8 H16 Sq1 S2048 d128: 16.0 us with one group, 14.6 with two; d64: 11.7 and 12.0).
-  const long long two = a.seq_len_q > 32 ? cost(64, kSplit[1][d][k], rounds) : d ? one - 1 : one + 1;
-  if (wide <= one && wide <= two) return 0;
-  return one <= two ? 1 : 2;
+    const long long cost = per_cu * (helper ? 95 + 240 * rounds : c.start + c.step * rounds);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = kernel.row_groups;
+    }
+  }
+  return best;
 }
 #endif
 
@@ -191,7 +214,7 @@ int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescript
   const Variant var{bias, fast, full_range_p};
   hipError_t err;
 #ifndef FMHA_NO_SPLIT_KERNEL
-  if (const int row_groups = split_row_groups(a, block_keys)) {
+  if (const int row_groups = row_groups_of(a, block_keys)) {
     if (a.head_dim == 128)
       err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<128, fmha_i8_gfx950::kBlockK>(row_groups, var, stream, args)
                                                   : launch_split<128, fmha_i8_gfx950::kBlockKSmall>(row_groups, var, stream, args);

@@ -46,6 +46,95 @@ struct SplitKernelArgs : KernelArgs {
   Divisor q_blocks_divisor, head_num_divisor;
 };
 
+// Classification of the key blocks of a batch entry by the first WAVES wavefronts of a workgroup, sixteen mask bytes per lane
+// (the bits are those of fmha_i8_fwd_kernel): mask bits to `words`, per block bit0 = some key masked, bit1 = all keys masked to
+// `cls` (blocks that fill up the last four count as the latter).  mask_bytes: the lane's first sixteen bytes, tail_bytes: the
+// row's last sixteen (for the one lane that straddles the end); both have landed.  S >= 16.  Returns this wavefront's last
+// block with an unmasked key, -1 if there is none.
+constexpr int kMaskBytesPerLane = 16;
+template <int BK, int WAVES>
+__device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const v4i& tail_bytes, const int8_t* __restrict__ mg, int S,
+                                                   int tid, unsigned* words, unsigned char* cls) {
+  constexpr int kLanesPerBlock = BK / kMaskBytesPerLane;
+  const int lane = tid & 63, n_blocks = (S + BK - 1) / BK, S_pad = n_blocks * BK;
+  auto nonzero_bytes = [](unsigned w) -> unsigned {
+    const unsigned t = (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
+    return (((t >> 7) * 0x00204081u) >> 21) & 15u;
+  };
+  auto nonzero16 = [&](const v4i& w) -> unsigned {
+    return nonzero_bytes((unsigned)w[0]) | (nonzero_bytes((unsigned)w[1]) << 4) | (nonzero_bytes((unsigned)w[2]) << 8) |
+           (nonzero_bytes((unsigned)w[3]) << 12);
+  };
+  int live_hi = -1;
+  for (int base = 0; base < S_pad; base += kMaskBytesPerLane * 64 * WAVES) {
+    const int j = base + kMaskBytesPerLane * tid;
+    unsigned bits = 0xffffu;  // keys past the end count as masked
+    if (j + kMaskBytesPerLane <= S) {
+      v4i w = mask_bytes;
+      if (base != 0) {
+        const int jj = fmha_in_bounds(j >= 0 && j + kMaskBytesPerLane <= S) ? j : 0;
+        asm volatile("global_load_dwordx4 %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=v"(w) : "v"(jj), "s"(mg) : "memory");
+      }
+      bits = nonzero16(w);
+    } else if (j < S) {  // the one lane that straddles the end of the row
+      bits = ((nonzero16(tail_bytes) >> (kMaskBytesPerLane - (S - j))) | (0xffffu << (S - j))) & 0xffffu;
+    }
+    const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
+    if ((lane & 1) == 0 && j < S_pad) words[j >> 5] = word;
+    const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
+    if (lane % kLanesPerBlock == 0 && j < S_pad) {
+      constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
+      const bool blk_some = ((some >> lane) & kBlockBits) != 0, blk_all = ((all >> lane) & kBlockBits) == kBlockBits;
+      cls[j / BK] = (unsigned char)((blk_some ? 1 : 0) | (blk_all ? 2 : 0));
+      if (!blk_all) live_hi = j / BK;
+    }
+  }
+  if (tid < kSplitKeys && n_blocks + tid < (n_blocks + kSplitKeys - 1) / kSplitKeys * kSplitKeys) cls[n_blocks + tid] = 3;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) live_hi = max(live_hi, __shfl_xor(live_hi, off));
+  return live_hi;
+}
+
+// Start values of the GEMM 1 accumulators of a block with masked keys (see fmha_i8_fwd_kernel): `gone` loses every maximum
+// and its exponential is exactly 0.  mw: the block's mask bits, wave-uniform.
+template <bool BIAS, int KEY_TILES>
+__device__ __forceinline__ void masked_start_values(v16i (&acc)[KEY_TILES], const unsigned (&mw)[KEY_TILES], const v16i& base) {
+  int gone = BIAS ? (int)0xFF000000 : -(1 << 30);
+  asm volatile("" : "+v"(gone));
+#pragma unroll
+  for (int t = 0; t < KEY_TILES; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int key = 8 * (e / 4) + (e % 4);
+      const unsigned lo = (unsigned)(((int)(mw[t] << (31 - key))) >> 31), hi = (unsigned)(((int)(mw[t] << (27 - key))) >> 31);
+      const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
+      int x;
+      asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(base[e]), "v"(gone), "s"(lanes));
+      acc[t][e] = x;
+    }
+  asm volatile("s_nop 1" ::: "memory");  // (the compiler does not know that these statements wrote registers an MFMA reads)
+}
+// The mask bits of block kb; tail_kb: the partly filled last block, whose tile ends with the last key - bit j of word t is key
+// S - BK + 32 t + j, the keys it repeats count as masked.
+template <int BK>
+__device__ __forceinline__ void mask_words_of(unsigned (&mw)[BK / 32], const unsigned* words, int kb, int tail_kb, int S) {
+#pragma unroll
+  for (int t = 0; t < BK / 32; ++t) mw[t] = (unsigned)__builtin_amdgcn_readfirstlane((int)words[kb * (BK / 32) + t]);
+  if (kb != tail_kb) return;
+  const int repeated = (tail_kb + 1) * BK - S;
+#pragma unroll
+  for (int t = 0; t < BK / 32; ++t) {
+    const int start = S - BK + 32 * t, w = start >> 5, sh = start & 31;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)words[w]);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)words[w + (sh ? 1 : 0)]);
+    unsigned word = sh ? (lo >> sh) | (hi << (32 - sh)) : lo;
+    const int forced = repeated - 32 * t;
+    if (forced >= 32) word = 0xffffffffu;
+    else if (forced > 0) word |= (1u << forced) - 1u;
+    mw[t] = word;
+  }
+}
+
 template <int D, int BK, bool BIAS, bool FASTACC, bool FULLP, int R>
 __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKernelArgs args) {
   constexpr int kChunks = D / 16;
@@ -96,11 +185,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const int8_t* __restrict__ mg = args.mask + (long)b * S;
   const long q_head_off = (long)bh * Sq * D;
   const int n_blocks = (S + BK - 1) / BK;
-  const int S_pad = n_blocks * BK;
   // A partly filled last block: the tile is fetched so that it ends with the last key (see the other kernel).
-  const int tail_rows = S - (n_blocks - 1) * BK;
-  const bool ragged = tail_rows != BK;
-  const int tail_kb = ragged ? n_blocks - 1 : -1;
+  const int tail_kb = S % BK != 0 ? n_blocks - 1 : -1;
 
   // ---- tile loads --------------------------------------------------------------------------------------------------
   // A load moves 1 KiB: lane l lands at byte 16 l of a region of the tile and fetches the chunk that the swizzle assigns to
@@ -141,12 +227,10 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   // ---- prologue: mask bytes, Q rows and K of round 0, in this order; every load in flight before the first wait ---------
   const int row0 = (qb * R + r) * 32;
   const bool active = row0 < Sq;
-  constexpr int kKeysPerLane = 16;
-  constexpr int kKeysPerPass = kKeysPerLane * 64 * kRowWaves;
   v4i mask_bytes, tail_bytes;
   {
-    int j = kKeysPerLane * tid + kKeysPerLane <= S ? kKeysPerLane * tid : 0, jt = S - kKeysPerLane;
-    if (!fmha_in_bounds(j >= 0 && j + kKeysPerLane <= S && jt >= 0)) j = jt = 0;
+    int j = kMaskBytesPerLane * tid + kMaskBytesPerLane <= S ? kMaskBytesPerLane * tid : 0, jt = S - kMaskBytesPerLane;
+    if (!fmha_in_bounds(j >= 0 && j + kMaskBytesPerLane <= S && jt >= 0)) j = jt = 0;
     asm volatile("global_load_dwordx4 %0, %2, %3\n\tglobal_load_dwordx4 %1, %4, %3"
                  : "=&v"(mask_bytes), "=v"(tail_bytes) : "v"(j), "s"(mg), "v"(jt) : "memory");
   }
@@ -193,46 +277,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
 
   // ---- classification of the key blocks, by all wavefronts (the bits are those of the other kernel) -----------------
   asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + kLoads) : "memory");
-  {
-    constexpr int kLanesPerBlock = BK / kKeysPerLane;
-    unsigned char* cls = reinterpret_cast<unsigned char*>(lds_class4);
-    auto nonzero_bytes = [](unsigned w) -> unsigned {
-      const unsigned t = (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
-      return (((t >> 7) * 0x00204081u) >> 21) & 15u;
-    };
-    auto nonzero16 = [&](const v4i& w) -> unsigned {
-      return nonzero_bytes((unsigned)w[0]) | (nonzero_bytes((unsigned)w[1]) << 4) | (nonzero_bytes((unsigned)w[2]) << 8) |
-             (nonzero_bytes((unsigned)w[3]) << 12);
-    };
-    int live_hi = -1;
-    for (int base = 0; base < S_pad; base += kKeysPerPass) {
-      const int j = base + kKeysPerLane * tid;
-      unsigned bits = 0xffffu;  // keys past the end count as masked
-      if (j + kKeysPerLane <= S) {
-        v4i w = mask_bytes;
-        if (base != 0) {
-          const int jj = fmha_in_bounds(j >= 0 && j + kKeysPerLane <= S) ? j : 0;
-          asm volatile("global_load_dwordx4 %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=v"(w) : "v"(jj), "s"(mg) : "memory");
-        }
-        bits = nonzero16(w);
-      } else if (j < S) {  // the one lane that straddles the end of the row
-        bits = ((nonzero16(tail_bytes) >> (kKeysPerLane - (S - j))) | (0xffffu << (S - j))) & 0xffffu;
-      }
-      const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
-      if ((lane & 1) == 0 && j < S_pad) lds_mask[j >> 5] = word;
-      const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
-      if (lane % kLanesPerBlock == 0 && j < S_pad) {
-        constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
-        const bool blk_some = ((some >> lane) & kBlockBits) != 0, blk_all = ((all >> lane) & kBlockBits) == kBlockBits;
-        cls[j / BK] = (unsigned char)((blk_some ? 1 : 0) | (blk_all ? 2 : 0));
-        if (!blk_all) live_hi = j / BK;
-      }
-    }
-    if (tid < kSplitKeys && n_blocks + tid < (n_blocks + kSplitKeys - 1) / kSplitKeys * kSplitKeys) cls[n_blocks + tid] = 3;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) live_hi = max(live_hi, __shfl_xor(live_hi, off));
-    if (lane == 0) lds_scan[wave] = live_hi;
-  }
+  const int live_hi = classify_key_blocks<BK, kRowWaves>(mask_bytes, tail_bytes, mg, S, tid, lds_mask, reinterpret_cast<unsigned char*>(lds_class4));
+  if (lane == 0) lds_scan[wave] = live_hi;
   // K of round 0 and the Q rows have landed
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -261,38 +307,9 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     auto gemm1 = [&](auto masked_t) __attribute__((always_inline)) {
       constexpr bool kMasked = decltype(masked_t)::value;
       if constexpr (kMasked) {
-        // start values of masked keys: lose every maximum, exponential exactly 0 (see the other kernel)
         unsigned mw[kKeyTiles];
-        int gone = BIAS ? (int)0xFF000000 : -(1 << 30);
-        asm volatile("" : "+v"(gone));
-#pragma unroll
-        for (int t = 0; t < kKeyTiles; ++t) mw[t] = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[kb * kKeyTiles + t]);
-        if (kb == tail_kb) {  // bit j of word t <-> key S - BK + 32 t + j; repeated keys count as masked
-          const int repeated = BK - tail_rows;
-#pragma unroll
-          for (int t = 0; t < kKeyTiles; ++t) {
-            const int start = S - BK + 32 * t, w = start >> 5, sh = start & 31;
-            const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[w]);
-            const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[w + (sh ? 1 : 0)]);
-            unsigned word = sh ? (lo >> sh) | (hi << (32 - sh)) : lo;
-            const int forced = repeated - 32 * t;
-            if (forced >= 32) word = 0xffffffffu;
-            else if (forced > 0) word |= (1u << forced) - 1u;
-            mw[t] = word;
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < kKeyTiles; ++t)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int key = 8 * (e / 4) + (e % 4);
-            const unsigned lo = (unsigned)(((int)(mw[t] << (31 - key))) >> 31), hi = (unsigned)(((int)(mw[t] << (27 - key))) >> 31);
-            const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
-            int x;
-            asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(base_s[e]), "v"(gone), "s"(lanes));
-            acc[t][e] = x;
-          }
-        asm volatile("s_nop 1" ::: "memory");  // (the compiler does not know that these statements wrote registers an MFMA reads)
+        mask_words_of<BK>(mw, lds_mask, kb, tail_kb, S);
+        masked_start_values<BIAS>(acc, mw, base_s);
         __builtin_amdgcn_sched_barrier(0);
       }
       // Operand reads run two key tiles ahead of the MFMAs, held there by the fences: left alone, the compiler reads each
@@ -400,11 +417,11 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       }
     };
     float take[kCount], keep[kCount];
-    auto merge_piece = [&](int j, int piece, int pieces, auto moved_t) __attribute__((always_inline)) {
+    auto merge_piece = [&](int j, int piece, int pieces) __attribute__((always_inline)) {
 #pragma unroll
       for (int e = 16 * piece / pieces; e < 16 * (piece + 1) / pieces; ++e) {
         const float v = FASTACC ? __int_as_float(oacc[j & 1][e]) : __int_as_float(oacc[j & 1][e]) - (FULLP ? kBaseFull : kBase);
-        o_f[e] = __builtin_fmaf(FULLP ? take[j] : -take[j], v, decltype(moved_t)::value ? o_f[e] * keep[j] : o_f[e]);
+        o_f[e] = __builtin_fmaf(FULLP ? take[j] : -take[j], v, o_f[e]);
       }
     };
     auto start = [&](int j) __attribute__((always_inline)) {
@@ -438,40 +455,43 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       product(0, t);
       between(t, kCount * kKeyTiles);
     }
-    bool moved = false;  // some row's reference exponent moves (wave-uniform)
+    bool moves[kCount];  // some row's reference exponent moves (wave-uniform, rare): O is rescaled in front of that block's merge
 #pragma unroll
     for (int j = 0; j < kCount; ++j) {
       const bool dead = (cls4 >> (8 * (first + j))) & 2;
       const float mb = dead ? -__builtin_inff() : ml[j][0], lb = dead ? 0.f : ml[j][1];
-      const bool moves = __ballot(mb > m_ref + kLazyLog2) != 0;
-      const float m_new = moves ? fmaxf(m_ref, mb) : m_ref;
+      moves[j] = __ballot(mb > m_ref + kLazyLog2) != 0;
+      const float m_new = moves[j] ? fmaxf(m_ref, mb) : m_ref;
       keep[j] = __builtin_amdgcn_exp2f(m_ref - m_new);  // exactly 1 where nothing moves
       m_ref = m_new;
-      moved |= moves;
       take[j] = __builtin_amdgcn_exp2f(mb - m_ref);
       l_run = __builtin_fmaf(take[j], lb, l_run * keep[j]);
       if (FASTACC) t_run = t_run * keep[j] + take[j];
     }
-    auto rest = [&](auto moved_t) __attribute__((always_inline)) {
+    auto rescale = [&](int j) __attribute__((always_inline)) {
+      if (moves[j]) {
 #pragma unroll
-      for (int j = 1; j < kCount; ++j) {
-        start(j);
+        for (int e = 0; e < 16; ++e) o_f[e] *= keep[j];
+      }
+    };
+    rescale(0);
+#pragma unroll
+    for (int j = 1; j < kCount; ++j) {
+      start(j);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < kKeyTiles; ++t) {
+        product(j, t);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = 0; t < kKeyTiles; ++t) {
-          product(j, t);
-          __builtin_amdgcn_sched_barrier(0);
-          between(j * kKeyTiles + t, kCount * kKeyTiles);
-          merge_piece(j - 1, t, kKeyTiles, moved_t);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (j + 1 < kCount) read(j + 1);
+        between(j * kKeyTiles + t, kCount * kKeyTiles);
+        merge_piece(j - 1, t, kKeyTiles);
         __builtin_amdgcn_sched_barrier(0);
       }
-      merge_piece(kCount - 1, 0, 1, moved_t);
-    };
-    if (moved) rest(Const<1>{});
-    else rest(Const<0>{});
+      if (j + 1 < kCount) read(j + 1);
+      rescale(j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    merge_piece(kCount - 1, 0, 1);
   };
 
   // ---- the rounds --------------------------------------------------------------------------------------------------

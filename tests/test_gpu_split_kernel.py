@@ -1,6 +1,7 @@
-"""The kernel that serves calls of few workgroups (fmha_i8_split_kernel: one or two groups of 32 query rows per workgroup,
-four key blocks at a time) must write the bytes of the kernel of 256-row workgroups for every row: a caller sees no
-difference between a head computed alone and in a batch.  The reference is the test build that has the latter only."""
+"""The kernels that serve calls of few workgroups (fmha_i8_split_kernel: one or two groups of 32 query rows per workgroup, four
+key blocks at a time; fmha_i8_pair_kernel: four groups, two key blocks) must write the bytes of the kernel of 256-row
+workgroups for every row: a caller sees no difference between a head computed alone and in a batch.  The reference is the
+test build that has the latter only."""
 import ctypes as C
 import os
 import re
@@ -22,6 +23,7 @@ CSRC = os.path.join(ROOT, "int8-flash-attention-fmha-quantization_amd", "csrc")
 SHAPES = [
     (1, 2, 1, 2048, 128), (2, 3, 31, 640, 64), (1, 2, 33, 1100, 128), (1, 3, 512, 512, 64), (1, 4, 777, 777, 128),
     (2, 8, 320, 320, 128), (1, 16, 777, 777, 64), (1, 32, 300, 1536, 128), (4, 12, 256, 448, 64), (2, 24, 65, 1027, 128),
+    (4, 24, 250, 600, 128), (6, 16, 256, 512, 64), (5, 20, 129, 321, 128), (3, 32, 200, 1400, 64),  # four groups
     (1, 2, 40, 70, 128), (1, 1, 33, 15, 64), (2, 1, 5, 3, 128), (1, 2, 40, 8300, 64), (24, 16, 3, 300, 128), (1, 1, 2, 65536, 64),
 ]
 
@@ -64,17 +66,18 @@ def test_same_bytes_as_the_kernel_of_256_row_workgroups(pkg, dev, B, H, Sq, S, d
 def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(tmp_path):
     """The same check as for the other kernel (test_kernel_async_loads.py), on the compiled split kernel."""
     from test_kernel_async_loads import _check_function
-    args = ["<%d, %d, %s, %s, %s, %d>" % (d, bk, bias, fast, full, r)
+    args = [("pair_kernel<%d, %d, %s, %s, %s>" if r == 4 else "split_kernel<%d, %d, %s, %s, %s, %d>") % (d, bk, bias, fast, full, *([r] if r < 4 else []))
             for d, bk, bias, fast, full in ((128, 128, "true", "true", "false"), (64, 64, "false", "false", "true"),
-                                            (128, 64, "false", "true", "false"), (64, 128, "true", "false", "true")) for r in (1, 2)]
+                                            (128, 64, "false", "true", "false"), (64, 128, "true", "false", "true")) for r in (1, 2, 4)]
     src = tmp_path / "split.hip"
-    src.write_text('#include "%s/fmha_i8_kernel.hip"\n#include "%s/fmha_i8_split_kernel.hip"\nnamespace fmha_i8_gfx950 {\n' % (CSRC, CSRC) +
-                   "".join("template __global__ void fmha_i8_split_kernel%s(SplitKernelArgs);\n" % a for a in args) + "}\n")
+    src.write_text('#include "%s/fmha_i8_kernel.hip"\n#include "%s/fmha_i8_split_kernel.hip"\n' % (CSRC, CSRC) +
+                   '#include "%s/fmha_i8_pair_kernel.hip"\nnamespace fmha_i8_gfx950 {\n' % CSRC +
+                   "".join("template __global__ void fmha_i8_%s(SplitKernelArgs);\n" % a for a in args) + "}\n")
     out = tmp_path / "split.s"
     subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                     "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-S", "--cuda-device-only", "-o", str(out), str(src)],
                    check=True, capture_output=True)
-    funcs = re.split(r"\n(?=_ZN14fmha_i8_gfx95020fmha_i8_split_kernel[^\n]*:\s)", out.read_text())[1:]
+    funcs = re.split(r"\n(?=_ZN14fmha_i8_gfx950\d+fmha_i8_(?:split|pair)_kernel[^\n]*:\s)", out.read_text())[1:]
     assert len(funcs) == len(args)
     for f in funcs:
         assert _check_function(f.split(":")[0], f) >= 4  # mask bytes (twice) and the Q rows
