@@ -242,7 +242,15 @@ PyObject* quantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int status;
     if (a[1] == Py_None) {
       amax = empty({1}, at::kFloat, device);
-      at::Tensor workspace = empty({FMHA_QUANT_WORKSPACE_FLOATS}, at::kFloat, device);
+      // The caller never sees the workspace and it dies with this call: it must belong to the stream that the kernels are
+      // queued on, or the current stream could hand the memory out again while they still use it.
+      at::Tensor workspace;
+      {
+        std::optional<c10::hip::HIPStreamGuard> guard;
+        if (stream != c10::hip::getCurrentHIPStream(device.index()).stream())
+          guard.emplace(c10::hip::getStreamFromExternal(stream, device.index()));
+        workspace = empty({FMHA_QUANT_WORKSPACE_FLOATS}, at::kFloat, device);
+      }
       const FMHAQuantTensor t{x.data_ptr(), static_cast<int8_t*>(out.data_ptr()), (long long)x.numel()};
       Unlocked unlocked;
       status = FMHAMeasureAndQuantizeI8(stream, &t, 1, x.scalar_type() == at::kFloat ? FMHA_QUANT_F32 : FMHA_QUANT_BF16,

@@ -75,3 +75,24 @@ def test_mixed_types_through_the_float_flow(pkg, dev):
     assert torch.equal(o8, pkg.fmha_infer_i8(q8, k8, v8, mask, *amax, 1.0))
     with pytest.raises(ValueError):
         pkg.fmha_infer_from_float(q, torch.zeros_like(q), v, mask, 1.0)
+
+
+@pytest.mark.parametrize("as_handle", [False, True], ids=["stream", "handle"])
+def test_workspace_of_a_call_on_another_stream_is_not_handed_out_early(pkg, dev, as_handle):
+    """quantize_tensor on a stream that is still busy: tensors that the current stream allocates and fills in the meantime must
+    not be the call's workspace (they would put their values among its partial maxima)."""
+    import torch
+    x = torch.randn(1 << 20, device=dev)
+    stream = torch.cuda.Stream()
+    pkg.quantize_tensor(x)  # the current stream's pool has a block of the workspace's size
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            y = torch.randn(4096, 4096, device=dev) @ torch.ones(4096, 4096, device=dev)  # some milliseconds
+    q, amax = pkg.quantize_tensor(x, stream=stream.cuda_stream if as_handle else stream)
+    for _ in range(200):  # between the two kernels of the call, whenever they run
+        fills = [torch.full((1024,), 1e30, device=dev) for _ in range(64)]
+    torch.cuda.synchronize()
+    assert amax.item() == x.abs().max().item()
+    assert torch.equal(q, pkg.quantize_tensor(x)[0])
+    del y, fills
