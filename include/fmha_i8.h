@@ -33,6 +33,7 @@
 #define FMHA_I8_H_
 
 #include <hip/hip_runtime_api.h>
+#include <stddef.h>
 #include "fmha_param_i8.h"
 
 #ifdef __cplusplus
@@ -99,6 +100,17 @@ int FMHAInferI8Cross(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDe
  * adds 128 times the column sums of every V tile. */
 int FMHAInferI8CrossFullRangeP(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
                                const void* k, const void* v, const void* padding_mask, void* o);
+
+/* Either of the two calls above with device memory that it may use while it runs.  A call of few query rows (decoding: at
+ * most 32 per head) over few heads or many keys then works on the key blocks of a head in several workgroups at once (two
+ * kernels are enqueued); the bytes written are the same.  FMHAInferI8CrossWorkspaceBytes says how much it wants, 0 where it
+ * would not use any.  workspace: 16-byte aligned, contents do not matter, the caller's again once the call's work on the
+ * stream has ended; NULL or too small is not an error: the call is then the plain one.  full_range_p: nonzero for
+ * FMHAInferI8CrossFullRangeP. */
+size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc);
+int FMHAInferI8CrossWithWorkspace(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
+                                  const void* k, const void* v, const void* padding_mask, void* o, int full_range_p,
+                                  void* workspace, size_t workspace_bytes);
 
 /* Argument check only, no HIP call: what FMHAInferI8Cross would return before launching. */
 int FMHAInferI8CrossCheckArgs(FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q, const void* k,

@@ -111,6 +111,42 @@ const void* split_kernel(Variant var) {
   }
 #undef FMHA_VARIANT
 }
+// What a call of few query rows needs to share its key blocks out over workgroups (see fmha_i8_merge_kernel).
+struct PartPlan {
+  int rounds_per_part = 0;  // 0: it does not
+  size_t ml_bytes = 0, bytes = 0;
+};
+template <int D, int BK>
+const void* part_kernel(Variant var) {
+  using namespace fmha_i8_gfx950;
+#define FMHA_PART(BB, FF, PP) reinterpret_cast<const void*>(&fmha_i8_split_kernel<D, BK, BB, FF, PP, 1, true>)
+  // (what becomes of the accumulators is up to the merge: FASTACC makes no difference here)
+  if (var.full_range_p) return var.bias ? FMHA_PART(true, true, true) : FMHA_PART(false, true, true);
+  return var.bias ? FMHA_PART(true, true, false) : FMHA_PART(false, true, false);
+#undef FMHA_PART
+}
+template <int D, int BK>
+hipError_t launch_parts(const PartPlan& plan, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call, void* workspace) {
+  using namespace fmha_i8_gfx950;
+  SplitKernelArgs args{of_call};
+  const int heads = args.total_wgs / args.q_blocks, n_blocks = (args.seq_kv + BK - 1) / BK;
+  const int rounds = (n_blocks + kSplitKeys - 1) / kSplitKeys;
+  args.rounds_per_part = plan.rounds_per_part;
+  args.q_blocks = (rounds + plan.rounds_per_part - 1) / plan.rounds_per_part;  // parts per head in the place of query blocks
+  args.total_wgs = heads * args.q_blocks;
+  args.q_blocks_divisor = make_divisor(args.q_blocks);
+  args.head_num_divisor = make_divisor(args.head_num);
+  args.part_ml = static_cast<v2f*>(workspace);
+  args.part_o = reinterpret_cast<int*>(static_cast<char*>(workspace) + plan.ml_bytes);
+  void* kernel_args[] = {&args};
+  const hipError_t err = hipLaunchKernel(part_kernel<D, BK>(var), dim3((unsigned)args.total_wgs), dim3(256), kernel_args, 0, stream);
+  if (err != hipSuccess) return err;
+  int row_lanes = D / 2;
+  while (64 / row_lanes < args.seq_q) row_lanes /= 2;
+  MergeArgs merge{args.part_ml, args.part_o, args.o, n_blocks, args.seq_q, D, row_lanes, args.floor2, args.out_scale, var.fast, var.full_range_p};
+  void* merge_args[] = {&merge};
+  return hipLaunchKernel(n_blocks <= 16 ? reinterpret_cast<const void*>(&fmha_i8_merge_kernel<16>) : reinterpret_cast<const void*>(&fmha_i8_merge_kernel<32>), dim3((unsigned)(D / (2 * row_lanes)), (unsigned)heads), dim3(64), merge_args, 0, stream);
+}
 template <int D, int BK>
 hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
   using namespace fmha_i8_gfx950;
@@ -133,7 +169,7 @@ hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const f
 // nearly everywhere - d128, S2048: H4 31.3 us in 256-row workgroups, 24.3 in those of four groups, 17.6 of two, 13.5 of one;
 // H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error only shift the
 // boundary between equals.
-int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
+int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* cost_of = nullptr) {
 #ifdef FMHA_SPLIT_FORCE
   return a.seq_len_kv > block_keys ? FMHA_SPLIT_FORCE : 0;
 #endif
@@ -166,12 +202,55 @@ int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
       best = kernel.row_groups;
     }
   }
+  if (cost_of != nullptr) *cost_of = least;
   return best;
+}
+// Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for, by the cost
+// table above (start, step of one row group), but no faster than the memory (62 KB in a hundredth of a microsecond, on both
+// sides of the comparison), with the workspace written and read again, and the merge: 2.5 us for the launch and a first batch of
+// key blocks, 0.8 per further batch.  One call, plain -> shared out: B1 H16 Sq1 S2048 d128 12.2 -> 9.2 us, S8192 d64 36.3 -> 11.8,
+// H32 S8192 d128 41.7 -> 19.3, H8 S65536 331 -> 61; H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds
+// already, 14.0 -> 15.9 and hence not.
+PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
+  using namespace fmha_i8_gfx950;
+  PartPlan plan;
+  const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys, rounds = (blocks + kSplitKeys - 1) / kSplitKeys;
+  const long long heads = (long long)a.batch_num * a.head_num;
+  if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
+  const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
+  const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
+  static constexpr struct { int start, step; } kCost[2][2] = {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}};
+  const auto& c = kCost[a.head_dim == 128][block_keys == kBlockK];
+  long long least = 0;
+  row_groups_of(a, block_keys, &least);
+  least = (least > memory ? least : memory) * 20 / 21;
+  long long work = 0;
+  for (int r = 1; r < rounds; ++r) {
+    const long long of_r = (heads * ((rounds + r - 1) / r) + 255) / 256 * (c.start + c.step * r);
+    if (plan.rounds_per_part > 0 && of_r > work) continue;
+    work = of_r;
+    plan.rounds_per_part = r;
+  }
+  if ((work > memory ? work : memory) + merge >= least) plan.rounds_per_part = 0;
+  const size_t rows = (size_t)heads * blocks * a.seq_len_q;
+  plan.ml_bytes = (rows * sizeof(v2f) + 255) / 256 * 256;
+  plan.bytes = plan.ml_bytes + rows * a.head_dim * sizeof(int);
+  return plan;
 }
 #endif
 
+// Blocks of 128 keys, as the reference uses for its multiples of 128; its other lengths (64, 192, 320, 448:
+// src/fmha_i8.cu:41-60) run in blocks of 64 keys, and so does every other odd multiple of 64 here.
+// A key count that is not a multiple of 64 is treated as the next multiple of 64 whose last keys are masked out.
+int padded_keys(int seq_len_kv) {
+  return (seq_len_kv + fmha_i8_gfx950::kBlockKSmall - 1) / fmha_i8_gfx950::kBlockKSmall * fmha_i8_gfx950::kBlockKSmall;
+}
+int block_keys_of(int seq_len_kv) {
+  return padded_keys(seq_len_kv) % fmha_i8_gfx950::kBlockK == 0 ? fmha_i8_gfx950::kBlockK : fmha_i8_gfx950::kBlockKSmall;
+}
+
 int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescriptor& a, const void* q, const void* k,
-           const void* v, const void* mask, void* o, bool full_range_p = false) {
+           const void* v, const void* mask, void* o, bool full_range_p = false, void* workspace = nullptr, size_t workspace_bytes = 0) {
   const int st = check_args(p, a, q, k, v, mask, o);
   if (st != FMHA_I8_OK) return st;
   constexpr float kLog2e = 1.4426950408889634f;
@@ -204,16 +283,25 @@ int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescript
   // Folding the accumulator offset into the running O (see FASTACC in the kernel) costs a rounding of relative size
   // 2^-24 at magnitude kBase * sum(take) per key block; normalised by the row sum (>= sum(take)) and scaled to output
   // LSBs that is at most about 0.0034 * (v_amax/o_amax) * sqrt(key blocks).  Take it while that stays below 0.1 LSB.
-  // Blocks of 128 keys, as the reference uses for its multiples of 128; its other lengths (64, 192, 320, 448:
-  // src/fmha_i8.cu:41-60) run in blocks of 64 keys, and so does every other odd multiple of 64 here.
-  // A key count that is not a multiple of 64 is treated as the next multiple of 64 whose last keys are masked out.
-  const int kv_padded = (a.seq_len_kv + fmha_i8_gfx950::kBlockKSmall - 1) / fmha_i8_gfx950::kBlockKSmall * fmha_i8_gfx950::kBlockKSmall;
-  const int block_keys = kv_padded % fmha_i8_gfx950::kBlockK == 0 ? fmha_i8_gfx950::kBlockK : fmha_i8_gfx950::kBlockKSmall;
+  const int kv_padded = padded_keys(a.seq_len_kv), block_keys = block_keys_of(a.seq_len_kv);
   const float lsb_bound = 0.0034f * fabsf(p.v_amax / p.o_amax) * sqrtf((float)(kv_padded / block_keys));
   const bool fast = lsb_bound < 0.1f;
   const Variant var{bias, fast, full_range_p};
   hipError_t err;
 #ifndef FMHA_NO_SPLIT_KERNEL
+  if (workspace != nullptr) {
+    if ((uintptr_t)workspace & 15u) return FMHA_I8_ERR_ALIGNMENT;
+    const PartPlan plan = part_plan_of(a, block_keys);
+    if (plan.rounds_per_part > 0 && plan.bytes <= workspace_bytes) {
+      if (a.head_dim == 128)
+        err = block_keys == fmha_i8_gfx950::kBlockK ? launch_parts<128, fmha_i8_gfx950::kBlockK>(plan, var, stream, args, workspace)
+                                                    : launch_parts<128, fmha_i8_gfx950::kBlockKSmall>(plan, var, stream, args, workspace);
+      else
+        err = block_keys == fmha_i8_gfx950::kBlockK ? launch_parts<64, fmha_i8_gfx950::kBlockK>(plan, var, stream, args, workspace)
+                                                    : launch_parts<64, fmha_i8_gfx950::kBlockKSmall>(plan, var, stream, args, workspace);
+      return err == hipSuccess ? FMHA_I8_OK : FMHA_I8_ERR_HIP_BASE + (int)err;
+    }
+  }
   if (const int row_groups = row_groups_of(a, block_keys)) {
     if (a.head_dim == 128)
       err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<128, fmha_i8_gfx950::kBlockK>(row_groups, var, stream, args)
@@ -256,6 +344,24 @@ int FMHAInferI8Cross(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDe
 int FMHAInferI8CrossFullRangeP(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
                                const void* k, const void* v, const void* padding_mask, void* o) {
   return launch(stream, fmha_param, desc, q, k, v, padding_mask, o, true);
+}
+
+size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc) {
+#ifndef FMHA_NO_SPLIT_KERNEL
+  if ((desc.head_dim != 64 && desc.head_dim != 128) || desc.seq_len_kv <= 0 || desc.seq_len_kv > 65536 || desc.seq_len_q <= 0 ||
+      desc.batch_num <= 0 || desc.head_num <= 0)
+    return 0;
+  const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv));
+  return plan.rounds_per_part > 0 ? plan.bytes : 0;
+#else
+  return 0;
+#endif
+}
+
+int FMHAInferI8CrossWithWorkspace(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
+                                  const void* k, const void* v, const void* padding_mask, void* o, int full_range_p,
+                                  void* workspace, size_t workspace_bytes) {
+  return launch(stream, fmha_param, desc, q, k, v, padding_mask, o, full_range_p != 0, workspace, workspace_bytes);
 }
 
 int FMHAInferI8CrossCheckArgs(FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q, const void* k,

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
 
   asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + kLoads) : "memory");
   if (h == 0) {  // (for the mask bytes the other half has waited in vain: they are its first loads)
-    const int live_hi = classify_key_blocks<BK, 4>(mask_bytes, tail_bytes, mg, S, tid, lds_mask, lds_class);
+    const int live_hi = classify_key_blocks<BK, 4>(mask_bytes, tail_bytes, mg, S, tid, lds_mask, lds_class, 0, n_blocks * BK);
     if (lane == 0) lds_scan[r] = live_hi;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   }

@@ -17,6 +17,8 @@
 
 namespace fmha_i8_gfx950 {
 
+typedef float v2f __attribute__((ext_vector_type(2)));
+
 constexpr int kSplitKeys = 4;  // key blocks of a round
 
 template <int N>
@@ -44,19 +46,23 @@ __device__ __forceinline__ int divide(int n, Divisor d) {
 
 struct SplitKernelArgs : KernelArgs {
   Divisor q_blocks_divisor, head_num_divisor;
+  // Calls of few query rows whose key blocks are shared out (PARTS): rounds per workgroup, and where its results go.
+  int rounds_per_part;
+  v2f* part_ml;  // [head][key block][row]: block maximum and row sum
+  int* part_o;   // [head][key block][head_dim / 4][row][4]: the accumulators of GEMM 2
 };
 
 // Classification of the key blocks of a batch entry by the first WAVES wavefronts of a workgroup, sixteen mask bytes per lane
 // (the bits are those of fmha_i8_fwd_kernel): mask bits to `words`, per block bit0 = some key masked, bit1 = all keys masked to
 // `cls` (blocks that fill up the last four count as the latter).  mask_bytes: the lane's first sixteen bytes, tail_bytes: the
 // row's last sixteen (for the one lane that straddles the end); both have landed.  S >= 16.  Returns this wavefront's last
-// block with an unmasked key, -1 if there is none.
+// block with an unmasked key, -1 if there is none.  Only keys from .. to-1 are looked at (multiples of BK).
 constexpr int kMaskBytesPerLane = 16;
 template <int BK, int WAVES>
 __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const v4i& tail_bytes, const int8_t* __restrict__ mg, int S,
-                                                   int tid, unsigned* words, unsigned char* cls) {
+                                                   int tid, unsigned* words, unsigned char* cls, int from, int to) {
   constexpr int kLanesPerBlock = BK / kMaskBytesPerLane;
-  const int lane = tid & 63, n_blocks = (S + BK - 1) / BK, S_pad = n_blocks * BK;
+  const int lane = tid & 63, n_blocks = (S + BK - 1) / BK;
   auto nonzero_bytes = [](unsigned w) -> unsigned {
     const unsigned t = (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
     return (((t >> 7) * 0x00204081u) >> 21) & 15u;
@@ -66,12 +72,12 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
            (nonzero_bytes((unsigned)w[3]) << 12);
   };
   int live_hi = -1;
-  for (int base = 0; base < S_pad; base += kMaskBytesPerLane * 64 * WAVES) {
+  for (int base = from; base < to; base += kMaskBytesPerLane * 64 * WAVES) {
     const int j = base + kMaskBytesPerLane * tid;
     unsigned bits = 0xffffu;  // keys past the end count as masked
     if (j + kMaskBytesPerLane <= S) {
       v4i w = mask_bytes;
-      if (base != 0) {
+      if (base != from) {
         const int jj = fmha_in_bounds(j >= 0 && j + kMaskBytesPerLane <= S) ? j : 0;
         asm volatile("global_load_dwordx4 %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=v"(w) : "v"(jj), "s"(mg) : "memory");
       }
@@ -80,9 +86,9 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
       bits = ((nonzero16(tail_bytes) >> (kMaskBytesPerLane - (S - j))) | (0xffffu << (S - j))) & 0xffffu;
     }
     const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
-    if ((lane & 1) == 0 && j < S_pad) words[j >> 5] = word;
+    if ((lane & 1) == 0 && j < to) words[j >> 5] = word;
     const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
-    if (lane % kLanesPerBlock == 0 && j < S_pad) {
+    if (lane % kLanesPerBlock == 0 && j < to) {
       constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
       const bool blk_some = ((some >> lane) & kBlockBits) != 0, blk_all = ((all >> lane) & kBlockBits) == kBlockBits;
       cls[j / BK] = (unsigned char)((blk_some ? 1 : 0) | (blk_all ? 2 : 0));
@@ -135,7 +141,7 @@ __device__ __forceinline__ void mask_words_of(unsigned (&mw)[BK / 32], const uns
   }
 }
 
-template <int D, int BK, bool BIAS, bool FASTACC, bool FULLP, int R>
+template <int D, int BK, bool BIAS, bool FASTACC, bool FULLP, int R, bool PARTS = false>
 __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKernelArgs args) {
   constexpr int kChunks = D / 16;
   constexpr int kTileBytes = BK * D;
@@ -153,6 +159,10 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   // With one row group a K tile has one reader: the wavefront fetches it itself, waits for it itself, and asks for the next
   // one as soon as it has read this one's operands, without any barrier.
   constexpr bool kOwnK = kBuffers == 1 && R == 1;
+  // PARTS: a workgroup does some rounds of a head and leaves what the merge needs of every key block (see the end of the
+  // file).  With one round or two per workgroup the time is that of the first loads, so V is asked for beside K.
+  static_assert(!PARTS || R == 1, "");
+  constexpr bool kEarlyV = PARTS && kOwnK;
 
   __shared__ __attribute__((aligned(1024))) int8_t lds[kBuffers][2][kSplitKeys][kTileBytes];  // [buffer][K|V][slot][tile]
   __shared__ __attribute__((aligned(16))) v4i lds_p[R][kPSlots][kKeyTiles][64];  // P^T as the B operand of GEMM 2
@@ -185,6 +195,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const int8_t* __restrict__ mg = args.mask + (long)b * S;
   const long q_head_off = (long)bh * Sq * D;
   const int n_blocks = (S + BK - 1) / BK;
+  const int first_round = PARTS ? qb * args.rounds_per_part : 0;
   // A partly filled last block: the tile is fetched so that it ends with the last key (see the other kernel).
   const int tail_kb = S % BK != 0 ? n_blocks - 1 : -1;
 
@@ -225,11 +236,16 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const Const<kLoads / 2> half_kind;
 
   // ---- prologue: mask bytes, Q rows and K of round 0, in this order; every load in flight before the first wait ---------
-  const int row0 = (qb * R + r) * 32;
+  const int row0 = PARTS ? 0 : (qb * R + r) * 32;
   const bool active = row0 < Sq;
+  // Keys to classify: all, or those of the rounds of this workgroup and the block in front of them (part of which a partly
+  // filled last block's tile repeats).
+  const int keys_from = PARTS && first_round > 0 ? (kSplitKeys * first_round - 1) * BK : 0;
+  const int keys_to = PARTS ? min(n_blocks, kSplitKeys * (first_round + args.rounds_per_part)) * BK : n_blocks * BK;
   v4i mask_bytes, tail_bytes;
   {
-    int j = kMaskBytesPerLane * tid + kMaskBytesPerLane <= S ? kMaskBytesPerLane * tid : 0, jt = S - kMaskBytesPerLane;
+    const int mine = keys_from + kMaskBytesPerLane * tid;
+    int j = mine + kMaskBytesPerLane <= S ? mine : 0, jt = S - kMaskBytesPerLane;
     if (!fmha_in_bounds(j >= 0 && j + kMaskBytesPerLane <= S && jt >= 0)) j = jt = 0;
     asm volatile("global_load_dwordx4 %0, %2, %3\n\tglobal_load_dwordx4 %1, %4, %3"
                  : "=&v"(mask_bytes), "=v"(tail_bytes) : "v"(j), "s"(mg), "v"(jt) : "memory");
@@ -245,7 +261,11 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(qreg[kk]) : "v"(qoff + 32 * kk), "s"(qp) : "memory");
   }
 #pragma unroll
-  for (int it = 0; it < kLoads; ++it) issue(0, 0, it, n_blocks - 1);
+  for (int it = 0; it < kLoads; ++it) issue(first_round, 0, it, n_blocks - 1);
+  if (kEarlyV) {
+#pragma unroll
+    for (int it = 0; it < kLoads; ++it) issue(first_round, 1, it, n_blocks - 1);
+  }
 
   // operand addresses (see the other kernel)
   int k_read_off[kDSteps];
@@ -276,11 +296,12 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   if (BIAS) asm volatile("" : "+v"(base_s));
 
   // ---- classification of the key blocks, by all wavefronts (the bits are those of the other kernel) -----------------
-  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + kLoads) : "memory");
-  const int live_hi = classify_key_blocks<BK, kRowWaves>(mask_bytes, tail_bytes, mg, S, tid, lds_mask, reinterpret_cast<unsigned char*>(lds_class4));
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + (kEarlyV ? 2 : 1) * kLoads) : "memory");
+  const int live_hi = classify_key_blocks<BK, kRowWaves>(mask_bytes, tail_bytes, mg, S, tid, lds_mask,
+                                                         reinterpret_cast<unsigned char*>(lds_class4), keys_from, keys_to);
   if (lane == 0) lds_scan[wave] = live_hi;
   // K of round 0 and the Q rows have landed
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kEarlyV ? kLoads : 0) : "memory");
 #pragma unroll
   for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
   barrier();
@@ -288,7 +309,13 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
 #pragma unroll
   for (int w = 0; w < kRowWaves; ++w) n = max(n, lds_scan[w]);
   n = __builtin_amdgcn_readfirstlane(n) + 1;  // one past the last block with an unmasked key
-  const int rounds = (n + kSplitKeys - 1) / kSplitKeys;
+  const int rounds = PARTS ? min(first_round + args.rounds_per_part, (n + kSplitKeys - 1) / kSplitKeys) : (n + kSplitKeys - 1) / kSplitKeys;
+  const long part_first = (long)bh * n_blocks;  // PARTS: the head's first key block in part_ml and part_o
+  if constexpr (PARTS) {  // blocks without an unmasked key: a maximum that the merge takes for "nothing here"
+    for (int kb = keys_to / BK - 1 - wave; kb >= kSplitKeys * first_round; kb -= kRowWaves)
+      if ((reinterpret_cast<const unsigned char*>(lds_class4)[kb] & 2) && lane < Sq)
+        args.part_ml[(part_first + kb) * Sq + lane] = v2f{-__builtin_inff(), 0.f};
+  }
 
   // ---- one key block of one row group: S^T, softmax, P^T --------------------------------------------------------------
   float m_blk = 0.f, l_blk = 0.f;
@@ -394,13 +421,18 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
 #pragma unroll
     for (int t = 0; t < kKeyTiles; ++t) lds_p[r][c & (kPSlots - 1)][t][lane] = pk[t];
   };
-  auto publish_ml = [&]() __attribute__((always_inline)) {
+  auto publish_ml = [&](int kb) __attribute__((always_inline)) {
+    if constexpr (PARTS) {
+      if (lane < Sq) args.part_ml[(part_first + kb) * Sq + lane] = v2f{m_blk, l_blk};
+      return;
+    }
     lds_ml[r][c][i32][0] = m_blk;
     lds_ml[r][c][i32][1] = l_blk;
   };
 
   // ---- GEMM 2 and the merge of key blocks first .. first+COUNT-1 of the round, for this wavefront's columns -----------
   // A block without an unmasked key enters with weight 0 (its P may be anything: any int8 leaves the accumulators finite).
+  int part_kb = 0;  // PARTS: the first key block of the round
   auto gemm2_merge = [&](int buf, int first, auto count_t, unsigned cls4, auto between) __attribute__((always_inline)) {
     constexpr int kCount = decltype(count_t)::value;
     typedef v2i __attribute__((address_space(3))) * lds_v2i_ptr;
@@ -416,6 +448,34 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         p[j & 1][t] = lds_p[r][(first + j) & (kPSlots - 1)][t][lane];
       }
     };
+    if constexpr (PARTS) {  // the accumulators of every block to memory
+      read(0);
+#pragma unroll
+      for (int j = 0; j < kCount; ++j) {
+        if (j + 1 < kCount) read(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        oacc[0] = base_c;
+        if (FULLP) {  // (as in start() below)
+          const v4i half = {0x40404040, 0x40404040, 0x40404040, 0x40404040};
+#pragma unroll
+          for (int t = 0; t < kKeyTiles; ++t) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], half, oacc[0], 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) oacc[0][e] = 2 * oacc[0][e] + kBaseBitsFull;
+        }
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) {
+          oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], p[j & 1][t], oacc[0], 0, 0, 0);
+          between(j * kKeyTiles + t, kCount * kKeyTiles);
+        }
+        if (!((cls4 >> (8 * (first + j))) & 2) && c < kDSteps && i32 < Sq) {
+          int* at = args.part_o + (part_first + part_kb + first + j) * Sq * D + ((8 * u_out + g) * Sq + i32) * 4;
+#pragma unroll
+          for (int a = 0; a < 4; ++a)
+            *reinterpret_cast<v4i*>(at + 8 * a * Sq) = v4i{oacc[0][4 * a], oacc[0][4 * a + 1], oacc[0][4 * a + 2], oacc[0][4 * a + 3]};
+        }
+      }
+      return;
+    }
     float take[kCount], keep[kCount];
     auto merge_piece = [&](int j, int piece, int pieces) __attribute__((always_inline)) {
 #pragma unroll
@@ -504,11 +564,12 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   //                             P of blocks 2, 3 | b3 | G of blocks 2, 3 with V of blocks 0, 1 of i+1 | b4
   auto written = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
   // V of round 0, or the half of it that the rounds themselves do not ask for
-  if (!kOwnK && rounds > 0) {
+  if (!kOwnK && rounds > first_round) {
 #pragma unroll
-    for (int it = 0; it < (kBuffers == 2 ? kLoads : kLoads / 2); ++it) issue(0, 1, it, n - 1);
+    for (int it = 0; it < (kBuffers == 2 ? kLoads : kLoads / 2); ++it) issue(first_round, 1, it, n - 1);
   }
-  for (int i = 0; i < rounds; ++i) {
+  for (int i = first_round; i < rounds; ++i) {
+    part_kb = kSplitKeys * i;
     const int buf = i & (kBuffers - 1);
     const bool more = i + 1 < rounds;
     const unsigned cls4 = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_class4[i]);
@@ -524,7 +585,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     constexpr int kHalf = kLoads / 2;
     auto loads_in_gemm1 = [&](int slot, int slots) __attribute__((always_inline)) {
       if (kTwoBuffers) spread(more, i + 1, 0, 0, kLoads, slot, slots);
-      else if (kOwnK) spread(true, i, 1, 0, kLoads, slot, slots);
+      else if (kOwnK) spread(!kEarlyV || i > first_round, i, 1, 0, kLoads, slot, slots);
       else spread(true, i, 1, kHalf, kHalf, slot, slots);
     };
     auto loads_in_softmax = [&](int slot, int slots) __attribute__((always_inline)) {
@@ -540,7 +601,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     };
     if (work) {
       scores_and_softmax(buf, kSplitKeys * i + c, cls, loads_in_gemm1, loads_in_softmax);
-      publish_ml();
+      publish_ml(kSplitKeys * i + c);
       if (!kTwoSteps || c < 2) publish_p();
     } else {
       loads_in_gemm1(0, 1);
@@ -571,7 +632,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     barrier();  // b4
   }
   wait_loads(none);  // nothing may still be writing LDS when the wavefront ends (only possible when every key is masked)
-  if (!active || c >= kDSteps) return;
+  if (PARTS || !active || c >= kDSteps) return;
 
   // ---- epilogue (see the other kernel) -----------------------------------------------------------------------------
   const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
@@ -596,6 +657,97 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     const auto s = __builtin_amdgcn_permlane32_swap(w[a], w[a + 1], false, false);
     *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
   }
+}
+
+// ---- calls of few query rows: key blocks shared out over workgroups ------------------------------------------------------
+// A call of at most kPartRows rows per head has one workgroup per head, which reads all of its K and V: with less than 256
+// heads compute units idle, with a long sequence the time is that of one CU's loads (128 KB in
+// 2.4 us).
+// Partial results of separate key ranges cannot be merged with the same bytes, but those of single key blocks can: PARTS leaves
+// the accumulators of GEMM 2 (whole numbers) and the row's maximum and sum per block, 4 head_dim + 8 bytes per row where the
+// block itself has 2 BK head_dim, and this kernel does the online merge of all blocks in key order.
+constexpr int kPartRows = 32;
+
+struct MergeArgs {
+  const v2f* part_ml;
+  const int* part_o;
+  int8_t* o;
+  int n_blocks, seq_q, head_dim, row_lanes;  // row_lanes: lanes of a wavefront per row, a power of two
+  float floor2, out_scale;
+  bool fast, full_range_p;
+};
+// What bounds it is latency, of its loads and of the chain over the blocks: BATCH blocks are loaded together, all of a short
+// sequence, 32 of a long one, and where no reference exponent moves in a batch (nearly all behind the first) the weights of all
+// of its blocks are independent of each other (B1 H8 Sq1 S65536 d128, 512 blocks: 77 -> 61 us for the call).
+// One wavefront per workgroup: 64 / row_lanes rows (the last repeated) by 2 * row_lanes columns of a head, two columns per lane.
+// All rows of a head are in one wavefront, because a reference exponent that moves in one row moves in all.
+template <int BATCH>
+__global__ __launch_bounds__(64, 1) void fmha_i8_merge_kernel(const MergeArgs args) {
+  const int lane = threadIdx.x;
+  const int Sq = args.seq_q, D = args.head_dim;
+  const long bh = blockIdx.y;
+  const int row = min(lane / args.row_lanes, Sq - 1);
+  const int col = 2 * (blockIdx.x * args.row_lanes + lane % args.row_lanes);
+  const v2f* ml = args.part_ml + bh * args.n_blocks * Sq + row;
+  const int* po = args.part_o + bh * args.n_blocks * Sq * D + (col / 4 * Sq + row) * 4 + col % 4;
+  const float kGone = -__builtin_inff();
+  const float base = args.fast ? 0.f : args.full_range_p ? kBaseFull : kBase;  // (x - 0 is x)
+  const float sign = args.full_range_p ? 1.f : -1.f;
+  float m_ref = args.floor2 - 2.f * kLazyLog2, t_run = 0.f, l_run = 0.f, o[2] = {0.f, 0.f};
+  for (int kb0 = 0; kb0 < args.n_blocks; kb0 += BATCH) {
+    v2f s[BATCH];
+    v2i x[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const long kb = min(kb0 + j, args.n_blocks - 1);
+      s[j] = ml[kb * Sq];
+      x[j] = *reinterpret_cast<const v2i*>(po + kb * Sq * D);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float top = kGone;
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {  // blocks past the end and those without an unmasked key (their accumulators were not written): weight 0
+      if (kb0 + j >= args.n_blocks) s[j] = v2f{kGone, 0.f};
+      if (s[j][0] == kGone) x[j] = v2i{0, 0};
+      top = fmaxf(top, s[j][0]);
+    }
+    if (__ballot(top > m_ref + kLazyLog2) == 0) {
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        const float take = __builtin_amdgcn_exp2f(s[j][0] - m_ref);
+        l_run = __builtin_fmaf(take, s[j][1], l_run);
+        t_run += take;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) o[e] = __builtin_fmaf(sign * take, __int_as_float(x[j][e]) - base, o[e]);
+      }
+      continue;
+    }
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const float mb = s[j][0];
+      if (__ballot(mb > m_ref + kLazyLog2) != 0) {
+        const float m_new = fmaxf(m_ref, mb), keep = __builtin_amdgcn_exp2f(m_ref - m_new);
+        m_ref = m_new;
+        l_run *= keep;
+        t_run *= keep;
+        o[0] *= keep;
+        o[1] *= keep;
+      }
+      const float take = __builtin_amdgcn_exp2f(mb - m_ref);
+      l_run = __builtin_fmaf(take, s[j][1], l_run);
+      t_run += take;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) o[e] = __builtin_fmaf(sign * take, __int_as_float(x[j][e]) - base, o[e]);
+    }
+  }
+  const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
+  const float corr = args.fast ? (args.full_range_p ? -kBaseFull * t_run : kBase * t_run) : 0.f;
+  if (lane / args.row_lanes >= Sq) return;
+  int y[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    y[e] = __float_as_int(__builtin_amdgcn_fmed3f(__builtin_fmaf(args.fast ? o[e] + corr : o[e], fin, kMagic), kMagic - 127.f, kMagic + 127.f)) & 0xff;
+  *reinterpret_cast<unsigned short*>(args.o + (bh * Sq + row) * D + col) = (unsigned short)(y[0] | (y[1] << 8));
 }
 
 }  // namespace fmha_i8_gfx950

@@ -86,11 +86,39 @@ struct Unlocked {
   ~Unlocked() { PyEval_RestoreThread(state); }
 };
 
+// Memory that a call needs while it runs and the caller never sees: it belongs to the stream that the kernels are queued on, or
+// the current stream could hand it out again while they still use it.
+at::Tensor empty_on(hipStream_t stream, int64_t bytes, const at::Device& device) {
+  std::optional<c10::hip::HIPStreamGuard> guard;
+  if (stream != c10::hip::getCurrentHIPStream(device.index()).stream())
+    guard.emplace(c10::hip::getStreamFromExternal(stream, device.index()));
+  return empty({bytes}, at::kChar, device);
+}
+
 struct AttnShape {
   int b, h, sq, s, d;
 };
+// The workspace of an attention call, if it has a use for one (a few query rows per head).  The call does without where memory
+// is short, and where a stream is being captured into an output of the caller's: torch's allocator keeps what it hands out
+// during a capture for the graph only if the capture is torch's own, which a call that allocates its output relies on anyway.
+at::Tensor workspace_of(const AttnShape& n, hipStream_t stream, const at::Device& device, bool own_output) {
+  constexpr int kMostRows = 32;  // no call of more rows wants any: spares the others the question
+  if (n.sq > kMostRows) return {};
+  const size_t bytes = FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor{n.b, n.sq, n.s, n.h, n.d});
+  if (bytes == 0) return {};
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (!own_output && (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)) return {};
+  try {
+    return empty_on(stream, (int64_t)bytes, device);
+  } catch (const c10::OutOfMemoryError&) {
+    return {};
+  }
+}
 int attend(hipStream_t stream, const AttnShape& n, const FMHAParamI8& scales, const void* q, const void* k, const void* v,
-           const void* mask, void* out, bool full_range_p) {
+           const void* mask, void* out, bool full_range_p, const at::Tensor& workspace) {
+  if (workspace.defined())
+    return FMHAInferI8CrossWithWorkspace(stream, scales, FMHACrossAttnDescriptor{n.b, n.sq, n.s, n.h, n.d}, q, k, v, mask, out,
+                                         full_range_p, workspace.data_ptr(), (size_t)workspace.numel());
   if (!full_range_p && n.sq == n.s)
     return FMHAInferI8Status(stream, scales, AttnDataDescriptor{n.b, n.s, n.h, n.d}, q, k, v, mask, out, true);
   const FMHACrossAttnDescriptor desc{n.b, n.sq, n.s, n.h, n.d};
@@ -217,10 +245,11 @@ PyObject* infer_i8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const hipStream_t stream = stream_of(a[9], device);
     const int full = PyObject_IsTrue(a[10]);
     if (full < 0) throw PythonError{};
+    const at::Tensor workspace = workspace_of(shape, stream, device, a[8] == Py_None);
     int status;
     {
       Unlocked unlocked;
-      status = attend(stream, shape, scales, q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), out.data_ptr(), full != 0);
+      status = attend(stream, shape, scales, q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), out.data_ptr(), full != 0, workspace);
     }
     if (status != FMHA_I8_OK) return PyLong_FromLong(status);
     if (a[8] != Py_None) {
@@ -242,19 +271,11 @@ PyObject* quantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int status;
     if (a[1] == Py_None) {
       amax = empty({1}, at::kFloat, device);
-      // The caller never sees the workspace and it dies with this call: it must belong to the stream that the kernels are
-      // queued on, or the current stream could hand the memory out again while they still use it.
-      at::Tensor workspace;
-      {
-        std::optional<c10::hip::HIPStreamGuard> guard;
-        if (stream != c10::hip::getCurrentHIPStream(device.index()).stream())
-          guard.emplace(c10::hip::getStreamFromExternal(stream, device.index()));
-        workspace = empty({FMHA_QUANT_WORKSPACE_FLOATS}, at::kFloat, device);
-      }
+      const at::Tensor workspace = empty_on(stream, 4 * FMHA_QUANT_WORKSPACE_FLOATS, device);
       const FMHAQuantTensor t{x.data_ptr(), static_cast<int8_t*>(out.data_ptr()), (long long)x.numel()};
       Unlocked unlocked;
       status = FMHAMeasureAndQuantizeI8(stream, &t, 1, x.scalar_type() == at::kFloat ? FMHA_QUANT_F32 : FMHA_QUANT_BF16,
-                                        workspace.data_ptr<float>(), amax.data_ptr<float>(), nullptr, 0);
+                                        static_cast<float*>(workspace.data_ptr()), amax.data_ptr<float>(), nullptr, 0);
     } else {
       const float value = number(a[1]);
       amax = at::full({1}, value, out.options().dtype(at::kFloat));
@@ -323,6 +344,7 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor scratch = empty({at_byte[3] + 4 * (FMHA_QUANT_WORKSPACE_FLOATS + 4)}, at::kChar, device);
     int8_t* base = static_cast<int8_t*>(scratch.data_ptr());
     float* workspace = reinterpret_cast<float*>(base + at_byte[3]);
+    const at::Tensor attend_workspace = workspace_of(shape, stream, device, true);
     FMHAQuantTensor t[3];
     int type[3];
     for (int i = 0; i < 3; ++i) {
@@ -351,7 +373,7 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
       const bool all_positive = amax[0] > 0.f && amax[1] > 0.f && amax[2] > 0.f;
       if (status == FMHA_I8_OK && all_positive)
         status = attend(stream, shape, FMHAParamI8{amax[0], amax[1], amax[2], o_amax, 1.0f}, t[0].out, t[1].out, t[2].out,
-                        mask.data_ptr(), o_i8.data_ptr(), full != 0);
+                        mask.data_ptr(), o_i8.data_ptr(), full != 0, attend_workspace);
       if (status == FMHA_I8_OK && all_positive) status = dequantize(stream, static_cast<const int8_t*>(o_i8.data_ptr()), o, o_amax);
     }
     if (status != FMHA_I8_OK) return PyLong_FromLong(status);

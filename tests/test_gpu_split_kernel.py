@@ -62,6 +62,98 @@ def test_same_bytes_as_the_kernel_of_256_row_workgroups(pkg, dev, B, H, Sq, S, d
         assert torch.equal(outs[0], outs[1]), (dist, pad, int((outs[0] != outs[1]).sum()))
 
 
+# (B, H, Sq, S, d) of calls whose key blocks are shared out over workgroups: one round to many per workgroup, rounds that are not
+# full, a partly filled last block that starts a round, both block sizes, 1 to 32 rows, one to many batches of the merge, mask rows
+# of more than one classification pass per workgroup
+PART_SHAPES = [
+    (1, 2, 1, 2048, 128), (8, 16, 1, 2048, 64), (1, 2, 32, 4096, 128), (1, 3, 17, 5000, 64), (1, 1, 8, 1089, 64), (1, 2, 3, 1100, 128), (2, 3, 5, 1030, 64), (1, 1, 1, 513, 128),
+    (3, 4, 2, 1027, 128), (1, 4, 7, 8300, 64), (2, 8, 8, 4032, 128), (1, 1, 1, 65536, 64), (1, 40, 4, 65500, 64), (1, 100, 2, 6200, 64), (1, 40, 1, 12300, 128), (1, 30, 8, 9010, 128), (2, 2, 1, 64 * 517, 128),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("full_range_p", [False, True], ids=["P_128_steps", "P_255_steps"])
+@pytest.mark.parametrize("B,H,Sq,S,d", PART_SHAPES)
+def test_same_bytes_with_a_workspace(pkg, dev, B, H, Sq, S, d, full_range_p):
+    import torch
+    lib = pkg.load_library()
+    desc = pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d)
+    need = lib.FMHAInferI8CrossWorkspaceBytes(desc)
+    assert need >= B * H * ((S + 127) // 128) * Sq * (4 * d + 8)
+    for n, (scale, o_amax, pad) in enumerate([(1, 1.0, "scatter"), (8, 1.0, "none"), (1, 0.1, "dead")]):
+        g = torch.Generator(device=dev)
+        g.manual_seed(70 + n)
+        q, k, v = (torch.randint(-127, 128, (B, H, rows, d), generator=g, device=dev, dtype=torch.int8) for rows in (Sq, S, S))
+        mask = (torch.rand((B, S), generator=g, device=dev) < 0.2).to(torch.int8) if pad == "scatter" else torch.zeros((B, S), dtype=torch.int8, device=dev)
+        if pad == "dead":  # whole blocks without an unmasked key, at the end and inside; one batch entry with none at all
+            mask[:, S - S // 3:] = 1
+            mask[:, S // 8:S // 8 + 260] = 1
+            if B > 1:
+                mask[1] = 1
+        scales = pkg.FMHAParamI8(0.2 * scale, 3.0, 3.0, o_amax, 1.0)
+        plain, parts, short = (torch.full((q.numel() + 256,), 77, dtype=torch.int8, device=dev) for _ in range(3))
+        work = torch.full((need + 256,), 0x7f, dtype=torch.int8, device=dev)  # its contents do not matter: NaN as floats
+        work[need:] = 55
+        t = [x.data_ptr() for x in (q, k, v, mask)]
+        entry = lib.FMHAInferI8CrossFullRangeP if full_range_p else lib.FMHAInferI8Cross
+        print((B, H, Sq, S, d, pad, full_range_p), flush=True)
+        assert entry(None, scales, desc, *t, plain.data_ptr()) == 0
+        assert lib.FMHAInferI8CrossWithWorkspace(None, scales, desc, *t, parts.data_ptr(), full_range_p, work.data_ptr(), need) == 0
+        assert lib.FMHAInferI8CrossWithWorkspace(None, scales, desc, *t, short.data_ptr(), full_range_p, work.data_ptr(), need - 1) == 0
+        assert lib.FMHAInferI8CrossWithWorkspace(None, scales, desc, *t, short.data_ptr(), full_range_p, work.data_ptr() + 4, need) == pkg.FMHA_I8_ERR_ALIGNMENT
+        torch.cuda.synchronize()
+        assert torch.equal(plain, parts), (pad, int((plain != parts).sum()))
+        assert torch.equal(plain, short) and (work[need:] == 55).all()
+
+
+@pytest.mark.gpu
+def test_workspace_of_the_torch_entry_point(pkg, dev):
+    """Replays of a captured graph, with eager calls in between, and calls on a busy stream: the workspace is theirs alone."""
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    q, k, v = (torch.randint(-127, 128, (1, 4, rows, 128), generator=g, device=dev, dtype=torch.int8) for rows in (1, 2048, 2048))
+    mask = torch.zeros((1, 2048), dtype=torch.int8, device=dev)
+    want = torch.empty_like(q)
+    desc = pkg.FMHACrossAttnDescriptor(1, 1, 2048, 4, 128)
+    assert pkg.FMHAInferI8Cross(None, pkg.FMHAParamI8(0.2, 3.0, 3.0, 1.0, 1.0), desc, q, k, v, mask, want) == 0
+    assert pkg.load_library().FMHAInferI8CrossWorkspaceBytes(desc) > 0
+    run = lambda **kw: pkg.fmha_infer_i8(q, k, v, mask, 0.2, 3.0, 3.0, **kw)
+    assert torch.equal(run(), want)
+    given = torch.empty_like(q)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+        run(out=given)
+    for _ in range(3):
+        out.zero_(), given.zero_()
+        junk = [torch.full((n,), 1e30, device=dev) for n in (1 << 12, 1 << 14, 1 << 16)]
+        graph.replay()
+        assert torch.equal(run(), want)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(given, want)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            y = torch.randn(4096, 4096, device=dev) @ torch.ones(4096, 4096, device=dev)
+    got = torch.empty_like(q)
+    run(out=got, stream=side)
+    for _ in range(50):
+        junk = [torch.full((n,), 1e30, device=dev) for n in (1 << 12, 1 << 14, 1 << 16)]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    del y, junk
+
+
+def test_calls_that_want_a_workspace(pkg):
+    """None for more than 32 rows, for a single round of key blocks, for enough heads to fill the card, for shapes that are refused."""
+    need = lambda B, H, Sq, S, d: pkg.load_library().FMHAInferI8CrossWorkspaceBytes(pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d))
+    assert need(1, 16, 1, 4096, 128) > 0 and need(1, 16, 8, 4096, 64) > 0
+    for shape in ((1, 16, 33, 4096, 128), (8, 16, 1, 2048, 128), (1, 16, 1, 512, 128), (64, 32, 1, 4096, 128), (1, 16, 1, 4096, 96), (1, 16, 1, 65537, 64),
+                  (0, 16, 1, 4096, 64), (1, -1, 1, 4096, 64), (1, 16, 0, 4096, 64), (70000, 1, 1, 4096, 64)):
+        assert need(*shape) == 0, shape
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(tmp_path):
     """The same check as for the other kernel (test_kernel_async_loads.py), on the compiled split kernel."""
@@ -69,6 +161,7 @@ def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(tmp_path):
     args = [("pair_kernel<%d, %d, %s, %s, %s>" if r == 4 else "split_kernel<%d, %d, %s, %s, %s, %d>") % (d, bk, bias, fast, full, *([r] if r < 4 else []))
             for d, bk, bias, fast, full in ((128, 128, "true", "true", "false"), (64, 64, "false", "false", "true"),
                                             (128, 64, "false", "true", "false"), (64, 128, "true", "false", "true")) for r in (1, 2, 4)]
+    args += ["split_kernel<128, 128, true, true, false, 1, true>", "split_kernel<64, 64, false, true, true, 1, true>"]
     src = tmp_path / "split.hip"
     src.write_text('#include "%s/fmha_i8_kernel.hip"\n#include "%s/fmha_i8_split_kernel.hip"\n' % (CSRC, CSRC) +
                    '#include "%s/fmha_i8_pair_kernel.hip"\nnamespace fmha_i8_gfx950 {\n' % CSRC +
