@@ -112,6 +112,12 @@ int FMHAInferI8CrossWithWorkspace(hipStream_t stream, FMHAParamI8 fmha_param, FM
                                   const void* k, const void* v, const void* padding_mask, void* o, int full_range_p,
                                   void* workspace, size_t workspace_bytes);
 
+/* Either of the first two calls with the de-quantised output as well: o_float (16-byte aligned, shaped like o; bfloat16 where
+ * o_float_is_bf16 is nonzero, else float) gets (float)o / 127 * o_amax, the bits of FMHADequantizeI8 / BF16 on o. */
+int FMHAInferI8CrossToFloat(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
+                            const void* k, const void* v, const void* padding_mask, void* o, int full_range_p, void* o_float,
+                            int o_float_is_bf16);
+
 /* Argument check only, no HIP call: what FMHAInferI8Cross would return before launching. */
 int FMHAInferI8CrossCheckArgs(FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q, const void* k,
                               const void* v, const void* padding_mask, const void* o);

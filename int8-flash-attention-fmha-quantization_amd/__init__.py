@@ -21,7 +21,7 @@ TORCH_PATH = os.path.join(_HERE, "_fmha_torch.so")
 
 EXPORTED_SYMBOLS = ("FMHAInferI8", "FMHAInferI8Status", "FMHAInferI8CheckArgs", "FMHAInferI8StatusString",
                     "FMHAInferI8Version", "FMHAInferI8Cross", "FMHAInferI8CrossCheckArgs",
-                    "FMHAInferI8CrossFullRangeP", "FMHAInferI8CrossWorkspaceBytes", "FMHAInferI8CrossWithWorkspace", "FMHAAbsMaxF32", "FMHAQuantizeI8", "FMHADequantizeI8",
+                    "FMHAInferI8CrossFullRangeP", "FMHAInferI8CrossWorkspaceBytes", "FMHAInferI8CrossWithWorkspace", "FMHAInferI8CrossToFloat", "FMHAAbsMaxF32", "FMHAQuantizeI8", "FMHADequantizeI8",
                     "FMHAAbsMaxBF16", "FMHAQuantizeI8BF16", "FMHADequantizeI8BF16", "FMHAMeasureAndQuantizeI8")
 
 FMHA_I8_OK = 0
@@ -114,6 +114,8 @@ def load_library(path=None):
     L.FMHAQuantizeI8BF16.restype = C.c_int
     L.FMHADequantizeI8BF16.argtypes = L.FMHADequantizeI8.argtypes
     L.FMHADequantizeI8BF16.restype = C.c_int
+    L.FMHAInferI8CrossToFloat.argtypes = [ptr, FMHAParamI8, FMHACrossAttnDescriptor] + [ptr] * 5 + [C.c_int, ptr, C.c_int]
+    L.FMHAInferI8CrossToFloat.restype = C.c_int
     L.FMHAInferI8CrossWorkspaceBytes.argtypes = [FMHACrossAttnDescriptor]
     L.FMHAInferI8CrossWorkspaceBytes.restype = C.c_size_t
     L.FMHAInferI8CrossWithWorkspace.argtypes = [ptr, FMHAParamI8, FMHACrossAttnDescriptor] + [ptr] * 5 + [C.c_int, ptr, C.c_size_t]

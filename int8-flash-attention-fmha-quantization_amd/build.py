@@ -14,6 +14,7 @@ SOURCES = [os.path.join(HERE, "csrc", "fmha_i8_api.hip"), os.path.join(HERE, "cs
 DEPENDS = SOURCES + [os.path.join(HERE, "csrc", "fmha_i8_kernel.hip"),
                      os.path.join(HERE, "csrc", "fmha_i8_split_kernel.hip"),
                      os.path.join(HERE, "csrc", "fmha_i8_pair_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
+                     os.path.join(HERE, "csrc", "fmha_dequant.h"),
                      os.path.join(ROOT, "include", "fmha_i8.h"), os.path.join(ROOT, "include", "fmha_param_i8.h"),
                      os.path.join(ROOT, "include", "fmha_quant.h")]
 # Packed-FP32 instruction selection is switched off for all device code (a flag for hipcc's device pass; the host pass

@@ -250,7 +250,8 @@ int block_keys_of(int seq_len_kv) {
 }
 
 int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescriptor& a, const void* q, const void* k,
-           const void* v, const void* mask, void* o, bool full_range_p = false, void* workspace = nullptr, size_t workspace_bytes = 0) {
+           const void* v, const void* mask, void* o, bool full_range_p = false, void* workspace = nullptr, size_t workspace_bytes = 0, void* wide = nullptr,
+           bool wide_is_bf16 = false) {
   const int st = check_args(p, a, q, k, v, mask, o);
   if (st != FMHA_I8_OK) return st;
   constexpr float kLog2e = 1.4426950408889634f;
@@ -271,6 +272,9 @@ int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescript
   if (args.c2 < 1e-30f) args.c2 = 1e-30f;
   args.floor2 = -1e6f * kLog2e;
   args.out_scale = output_scale(p);
+  args.wide = wide;
+  args.wide_amax = p.o_amax;
+  args.wide_is_bf16 = wide_is_bf16;
   const dim3 grid((unsigned)args.total_wgs), block(fmha_i8_gfx950::kThreads);
   // The accumulators of Q.K^T can be read as floats without a convert when they start at the bit pattern of a float;
   // the price is that the exponent offset (start value*2^26 + S)*c2 is then rounded on a coarser float grid.  Take that
@@ -344,6 +348,14 @@ int FMHAInferI8Cross(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDe
 int FMHAInferI8CrossFullRangeP(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
                                const void* k, const void* v, const void* padding_mask, void* o) {
   return launch(stream, fmha_param, desc, q, k, v, padding_mask, o, true);
+}
+
+int FMHAInferI8CrossToFloat(hipStream_t stream, FMHAParamI8 fmha_param, FMHACrossAttnDescriptor desc, const void* q,
+                            const void* k, const void* v, const void* padding_mask, void* o, int full_range_p, void* o_float,
+                            int o_float_is_bf16) {
+  if (o_float == nullptr) return FMHA_I8_ERR_NULL_POINTER;
+  if ((uintptr_t)o_float & 15u) return FMHA_I8_ERR_ALIGNMENT;
+  return launch(stream, fmha_param, desc, q, k, v, padding_mask, o, full_range_p != 0, nullptr, 0, o_float, o_float_is_bf16 != 0);
 }
 
 size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc) {

@@ -38,6 +38,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fmha_dequant.h"
+
 // No floating-point contraction by the compiler: every fused multiply-add in this file is written out
 // (__builtin_fmaf), so the bits of the result do not depend on which products the optimiser decides to fuse.
 #pragma clang fp contract(off)
@@ -108,7 +110,37 @@ struct KernelArgs {
   float c2;         // log2(e) * (1/sqrt(d)) * q_amax*k_amax/127^2 : int32 S -> base-2 exponent
   float floor2;     // log2(e) * -1e6 : the reference's initial block maximum (inc/fmha_i8.cuh:116)
   float out_scale;  // v_amax / (o_amax * 128)   (inc/fmha_i8.cuh:318)
+  void* wide;       // the de-quantised output beside o, in the same layout, or null
+  float wide_amax;  // o_amax
+  int wide_is_bf16; // bfloat16, else float
 };
+
+// The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8), where the caller wants it: in
+// place of a launch that passes over o again (B4 H16 S1024 d128, bfloat16: 6.1 us separate, 4.5 here; the host chooses).
+template <int WORDS>
+__device__ __forceinline__ void store_wide(const KernelArgs& args, long at, const int (&w)[WORDS]) {
+  if (args.wide == nullptr) return;
+  auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
+  if (args.wide_is_bf16) {
+    unsigned short* p = static_cast<unsigned short*>(args.wide) + at;
+#pragma unroll
+    for (int k = 0; k < WORDS; k += 2) {
+      v4i r;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = (int)cvt_pk_bf16(value(k + j / 2, 2 * (j % 2)), value(k + j / 2, 2 * (j % 2) + 1));
+      *reinterpret_cast<v4i*>(p + 4 * k) = r;
+    }
+  } else {
+    float* p = static_cast<float*>(args.wide) + at;
+#pragma unroll
+    for (int k = 0; k < WORDS; ++k) {
+      v4i r;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = __float_as_int(value(k, j));
+      *reinterpret_cast<v4i*>(p + 4 * k) = r;
+    }
+  }
+}
 
 // 16-byte-chunk swizzles.  K is read 32 consecutive rows at a time (ds_read_b128); V is read by ds_read_b64_tr_b8
 // whose 16-lane groups touch keys {0,1,2,3,8,9,10,11} (+4, +16, +20) of a 32-key slab.
@@ -1331,6 +1363,8 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
     }
     *reinterpret_cast<v4i*>(op + 32 * u) = v4i{g0[0], g1[0], g0[1], g1[1]};
     *reinterpret_cast<v4i*>(op + 32 * u + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
+    const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
+    store_wide(args, op - args.o + 32 * u, both);
   }
 }
 

@@ -656,6 +656,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   for (int a = 0; a < 4; a += 2) {
     const auto s = __builtin_amdgcn_permlane32_swap(w[a], w[a + 1], false, false);
     *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
+    const int both[2] = {(int)s[0], (int)s[1]};
+    store_wide(args, op - args.o + 8 * a, both);
   }
 }
 

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "../../include/fmha_quant.h"
+#include "fmha_dequant.h"
 
 // Every float operation below must round exactly where the reference's host code rounds: no fused multiply-add that is
 // not written out.
@@ -273,20 +274,6 @@ __global__ __launch_bounds__(kSmallThreads) void quantize_small_kernel(QuantJob 
   if (rest < n) out[rest] = (int8_t)quant1(last, scale);
 }
 
-// inc/utils.hpp:53: (float)v / 127.0f * amax, in that order.  The quotient is formed without the division sequence: with
-// 1/127 as the sum of two floats hi + lo, fma(v, hi, fl(v * lo)) rounds v (hi + lo) once, and for each of the 256 values
-// of v that is the correctly rounded v / 127.0f (checked exhaustively by the tests).
-__device__ __forceinline__ float dequant1(int v, float amax) {
-  constexpr float kHi = 1.0f / 127.0f;
-  constexpr float kLo = (float)(1.0 / 127.0 - (double)kHi);
-  const float fv = (float)v;
-  return __builtin_fmaf(fv, kHi, fv * kLo) * amax;
-}
-__device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {  // to nearest even, NaN stays NaN
-  unsigned r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
 __device__ __forceinline__ void dequant_unit(int w, float amax, v4f& r) {
   r = v4f{dequant1((int8_t)(w & 0xff), amax), dequant1((int8_t)((w >> 8) & 0xff), amax), dequant1((int8_t)((w >> 16) & 0xff), amax),
           dequant1(w >> 24, amax)};

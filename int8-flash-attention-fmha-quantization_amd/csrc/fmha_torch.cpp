@@ -316,7 +316,7 @@ PyObject* dequantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // (q, k, v, padding_mask, o_amax, out_dtype, stream, full_range_p) -> (O, int8 O, (q_amax, k_amax, v_amax)), or the status
 //
-// Launches: abs-max of the three tensors, their quantisation, the attention, the de-quantisation.  The attention's scales
+// Launches: abs-max of the three tensors, their quantisation, the attention, which may de-quantise its output too.  The attention's scales
 // are call arguments, so the host needs the three maxima in between: the quantising kernel writes them to pinned memory
 // as its first act and the host, which polls for them, has the attention queued while the quantisation still runs.
 PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -371,10 +371,21 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
         pool.give_back(note);
       }
       const bool all_positive = amax[0] > 0.f && amax[1] > 0.f && amax[2] > 0.f;
+      const FMHAParamI8 scales{amax[0], amax[1], amax[2], o_amax, 1.0f};
+      // With a small output the attention kernel de-quantises it too, which saves a launch.  A lane owns 32 bytes of a row, 64 or
+      // 128 as floats: with a large output those scattered stores cost what the launch saves.  The flow with a second launch and
+      // fused, us: B1 H2 S128 d64 16.4 and 13.8, B2 H8 S300 d128 21.6 and 17.9, B2 H16 S1024 d64 (2.1 M elements) 27.7 and 25.6 as
+      // bfloat16, 30.3 and 28.8 as float32; B8 H12 S512 d64 (3.1 M) 27.2 and 26.3, 29.8 and 31.2; B1 H16 S2048 d128 (4.2 M) 44.3
+      // and 45.0, 49.2 and 49.2; 8.4 M and more level.  The merge of shared-out key blocks writes int8 only.
+      constexpr int64_t kMostFused = 2 << 20;
+      const bool fused = !attend_workspace.defined() && o.numel() <= kMostFused;
       if (status == FMHA_I8_OK && all_positive)
-        status = attend(stream, shape, FMHAParamI8{amax[0], amax[1], amax[2], o_amax, 1.0f}, t[0].out, t[1].out, t[2].out,
-                        mask.data_ptr(), o_i8.data_ptr(), full != 0, attend_workspace);
-      if (status == FMHA_I8_OK && all_positive) status = dequantize(stream, static_cast<const int8_t*>(o_i8.data_ptr()), o, o_amax);
+        status = fused ? FMHAInferI8CrossToFloat(stream, scales, FMHACrossAttnDescriptor{shape.b, shape.sq, shape.s, shape.h, shape.d},
+                                                 t[0].out, t[1].out, t[2].out, mask.data_ptr(), o_i8.data_ptr(), full != 0, o.data_ptr(),
+                                                 out_type == at::kBFloat16)
+                       : attend(stream, shape, scales, t[0].out, t[1].out, t[2].out, mask.data_ptr(), o_i8.data_ptr(), full != 0,
+                                attend_workspace);
+      if (status == FMHA_I8_OK && all_positive && !fused) status = dequantize(stream, static_cast<const int8_t*>(o_i8.data_ptr()), o, o_amax);
     }
     if (status != FMHA_I8_OK) return PyLong_FromLong(status);
     PyObject* maxima = Py_BuildValue("(ddd)", (double)amax[0], (double)amax[1], (double)amax[2]);

@@ -96,3 +96,32 @@ def test_workspace_of_a_call_on_another_stream_is_not_handed_out_early(pkg, dev,
     assert amax.item() == x.abs().max().item()
     assert torch.equal(q, pkg.quantize_tensor(x)[0])
     del y, fills
+
+
+# one shape per attention kernel and head size: 256, 128, 64 and 32 query rows per workgroup, rows that do not fill the last group,
+# key blocks shared out over workgroups (the last two)
+@pytest.mark.parametrize("out_type", ["float32", "bfloat16"])
+@pytest.mark.parametrize("B,H,Sq,S,d", [(4, 20, 900, 200, 128), (4, 20, 900, 200, 64), (1, 9, 100, 60, 64), (2, 24, 250, 600, 128), (2, 24, 250, 600, 64),
+                                        (1, 32, 300, 1536, 128), (1, 12, 450, 1536, 64), (1, 3, 129, 777, 128), (1, 3, 129, 777, 64),
+                                        (1, 2, 3, 4096, 128), (1, 2, 3, 4096, 64)])
+def test_float_output_is_the_dequantised_int8_output(pkg, dev, B, H, Sq, S, d, out_type):
+    import torch
+    g = torch.Generator(device=dev)
+    g.manual_seed(11)
+    q, k, v = (torch.randn((B, H, rows, d), generator=g, device=dev) for rows in (Sq, S, S))
+    mask = (torch.rand((B, S), generator=g, device=dev) < 0.2).to(torch.int8)
+    dtype = getattr(torch, out_type)
+    print((B, H, Sq, S, d, out_type), flush=True)
+    o, o8, amax = pkg.fmha_infer_from_float(q, k, v, mask, 0.7, out_dtype=dtype)
+    assert o.dtype == dtype and torch.equal(o, pkg.dequantize_tensor(o8, 0.7, dtype=dtype))
+    (q8, _), (k8, _), (v8, _) = (pkg.quantize_tensor(t) for t in (q, k, v))
+    assert torch.equal(o8, pkg.fmha_infer_i8(q8, k8, v8, mask, *amax, 0.7))
+    lib = pkg.load_library()  # nothing behind the last row; what is not a pointer it can store to is refused
+    desc, scales = pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d), pkg.FMHAParamI8(*amax, 0.7, 1.0)
+    wide = torch.full((o.numel() + 256,), 3.0, dtype=dtype, device=dev)
+    again = torch.empty_like(o8)
+    call = lambda p: lib.FMHAInferI8CrossToFloat(None, scales, desc, *(t.data_ptr() for t in (q8, k8, v8, mask, again)), 0, p, out_type == "bfloat16")
+    torch.cuda.synchronize()
+    assert call(wide.data_ptr()) == 0 and call(None) == pkg.FMHA_I8_ERR_NULL_POINTER and call(wide.data_ptr() + 8) == pkg.FMHA_I8_ERR_ALIGNMENT
+    torch.cuda.synchronize()
+    assert torch.equal(wide[:o.numel()].view_as(o), o) and (wide[o.numel():] == 3).all() and torch.equal(again, o8)
