@@ -69,6 +69,8 @@ hipStream_t stream_of(PyObject* o, const at::Device& device) {
   if (p == nullptr && PyErr_Occurred()) throw PythonError{};
   return static_cast<hipStream_t>(p);
 }
+// The null stream is that of the current device: a call makes its tensors' device current, and the caller's again when it ends.
+using OnDevice = c10::hip::HIPGuard;
 // Memory of torch's caching allocator, ordered by the stream that is current on the device.
 at::Tensor empty(c10::IntArrayRef sizes, at::ScalarType type, const at::Device& device) {
   return at::detail::empty_cuda(sizes, type, device, std::nullopt);
@@ -234,6 +236,7 @@ PyObject* infer_i8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const AttnShape shape = shape_of(q, k, v, mask);
     const FMHAParamI8 scales{number(a[4]), number(a[5]), number(a[6]), number(a[7]), 1.0f};
     const at::Device device = q.device();
+    const OnDevice on_device(device.index());
     at::Tensor out;
     if (a[8] == Py_None) {
       out = empty(q.sizes(), at::kChar, device);
@@ -266,6 +269,7 @@ PyObject* quantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     const at::Tensor& x = float_on_gpu(a[0]);
     const at::Device device = x.device();
+    const OnDevice on_device(device.index());
     const hipStream_t stream = stream_of(a[2], device);
     at::Tensor out = empty(x.sizes(), at::kChar, device), amax;
     int status;
@@ -302,6 +306,7 @@ PyObject* dequantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor& x = int8_on_gpu(a[0], "x must be a contiguous int8 tensor on the GPU");
     const at::ScalarType type = float_type(a[3], at::kFloat);
     const float amax = number(a[1]);
+    const OnDevice on_device(x.device().index());
     const hipStream_t stream = stream_of(a[2], x.device());
     at::Tensor out = empty(x.sizes(), type, x.device());
     int status;
@@ -329,6 +334,7 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const float o_amax = number(a[4]);
     const at::ScalarType out_type = float_type(a[5], x[0]->scalar_type());
     const at::Device device = x[0]->device();
+    const OnDevice on_device(device.index());
     const hipStream_t stream = stream_of(a[6], device);
     const int full = PyObject_IsTrue(a[7]);
     if (full < 0) throw PythonError{};

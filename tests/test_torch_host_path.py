@@ -1,0 +1,92 @@
+"""The host path of the torch entry points (csrc/fmha_torch.cpp) on two GPUs that are host memory (fake_hip.cpp): which
+device and stream the work is queued on, and which exceptions leave it.  One GPU cannot show the former, and no test fills a
+real GPU's memory.  Each case runs in a process of its own, whose torch calls the stand-in runtime."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_call.restype = ctypes.c_char_p
+fake.fake_memory_limit.argtypes = [ctypes.c_size_t]
+import torch
+sys.path.insert(0, %r)
+import __graft_entry__ as g
+pkg = g.load_package()
+torch.cuda.init()
+assert torch._C._cuda_getDeviceCount() == 2
+
+def calls():
+    out = []
+    for i in range(fake.fake_calls()):
+        device, stream = ctypes.c_int(), ctypes.c_void_p()
+        name = fake.fake_call(i, ctypes.byref(device), ctypes.byref(stream)).decode()
+        out.append((name, device.value, stream.value or 0))
+    fake.fake_forget_calls()
+    return out
+
+def attention(device, sq=128, s=128, dtype=torch.int8):
+    q = torch.empty((1, 2, sq, 64), dtype=dtype, device=device)
+    k, v = (torch.empty((1, 2, s, 64), dtype=dtype, device=device) for _ in range(2))
+    return q, k, v, torch.empty((1, s), dtype=torch.int8, device=device)
+""" % ROOT
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include", "-o", out,
+                    os.path.join(HERE, "fake_hip.cpp")], check=True)
+    return out
+
+
+def run(fake, code):
+    p = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code), fake], stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert p.returncode == 0, p.stdout[-4000:]
+
+
+def test_work_is_queued_on_the_device_of_the_tensors(fake):
+    """Tensors on GPU 1 while GPU 0 is current: the null stream means GPU 1's, whoever names it, and GPU 0 stays current."""
+    run(fake, """
+    entries = {
+        "attend": lambda s: pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0, stream=s),
+        "full range": lambda s: pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0, stream=s, full_range_p=True),
+        "decode": lambda s: pkg.fmha_infer_i8(*attention("cuda:1", 1, 8192), 1.0, 1.0, 1.0, stream=s),
+        "quantize": lambda s: pkg.quantize_tensor(torch.empty(999, device="cuda:1"), stream=s),
+        "quantize by": lambda s: pkg.quantize_tensor(torch.empty(999, device="cuda:1"), 2.0, stream=s),
+        "dequantize": lambda s: pkg.dequantize_tensor(torch.empty(999, dtype=torch.int8, device="cuda:1"), 1.0, stream=s),
+    }
+    floats = {
+        "float": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", dtype=torch.float32)[:3], attention("cuda:1")[3], 1.0, stream=s),
+        "float, large": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1 << 15, 128, torch.bfloat16)[:3], attention("cuda:1")[3], 1.0, stream=s),
+        "float, decode": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 8192, torch.float32)[:3], attention("cuda:1", 1, 8192)[3], 1.0, stream=s),
+    }
+    side, null = torch.cuda.Stream("cuda:1"), torch.cuda.default_stream(1)
+    seen = set()
+    for name, entry in {**entries, **floats}.items():
+        for stream in (None, null, side) + ((0, side.cuda_stream) if name in entries else ()):
+            entry(stream)
+            got = calls()
+            handle = stream if isinstance(stream, int) else stream.cuda_stream if stream is not None else 0
+            assert got and all(c[1:] == (1, handle) for c in got), (name, stream, got)
+            assert torch.cuda.current_device() == 0 and fake.fake_current_device() == 0, name
+            assert torch.cuda.current_stream(0) == torch.cuda.default_stream(0) and torch.cuda.current_stream(1) == null
+            seen |= {c[0] for c in got}
+    assert {"FMHAInferI8Status", "FMHAInferI8CrossFullRangeP", "FMHAInferI8CrossWithWorkspace", "FMHAInferI8CrossToFloat",
+            "FMHAInferI8Cross", "FMHAMeasureAndQuantizeI8", "FMHAQuantizeI8", "FMHADequantizeI8", "FMHADequantizeI8BF16"} <= seen, seen
+    with torch.cuda.device(1), torch.cuda.stream(side):  # and the other way round, with a current stream of its own
+        pkg.fmha_infer_i8(*attention("cuda:0"), 1.0, 1.0, 1.0)
+        pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0)
+        assert [c[1:] for c in calls()] == [(0, 0), (1, side.cuda_stream)]
+    """)
