@@ -211,12 +211,8 @@ PyObject* guarded(F f) {
   } catch (const PythonError&) {
     return nullptr;
   }
-  catch (const c10::Error& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-    return nullptr;
-  }
-  catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  catch (const std::exception&) {  // (as torch's own functions raise it: torch.OutOfMemoryError and the others by their types)
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

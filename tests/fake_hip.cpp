@@ -19,7 +19,6 @@ constexpr size_t kMemory = 1ull << 30;
 thread_local int current = 0;
 std::mutex mutex;
 std::map<void*, size_t> allocated;
-std::map<void*, int> owner;  // stream -> device
 size_t used = 0, limit = kMemory;
 struct Call {
   const char* name;
@@ -98,7 +97,6 @@ hipError_t hipDeviceGetStreamPriorityRange(int* least, int* greatest) { return *
 hipError_t hipStreamCreateWithPriority(hipStream_t* s, unsigned, int) {
   std::lock_guard<std::mutex> lock(mutex);
   if (n_streams == (int)sizeof streams) return hipErrorOutOfMemory;
-  owner[streams + n_streams] = current;
   return *s = reinterpret_cast<hipStream_t>(streams + n_streams++), hipSuccess;
 }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }

@@ -90,3 +90,41 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
         pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0)
         assert [c[1:] for c in calls()] == [(0, 0), (1, side.cuda_stream)]
     """)
+
+
+def test_memory_that_runs_out_is_an_out_of_memory_error(fake):
+    """A caller that catches torch.OutOfMemoryError and shrinks its batch sees that type, as from torch's own functions; where a
+    call merely works faster with memory (decoding's workspace) it goes on without."""
+    run(fake, """
+    MB = 1 << 20
+    big = dict(sq=32 * MB // 128, s=128)  # 32 MB of int8 output: more than the rest of a cached segment
+    i8, f32 = attention("cuda:0", **big), attention("cuda:0", **big, dtype=torch.float32)
+    decode = attention("cuda:0", 32, 65536)  # (a workspace of 8.7 MB)
+    out = torch.empty_like(decode[0])
+    x, x8 = torch.empty(32 * MB, device="cuda:0"), torch.empty(32 * MB, dtype=torch.int8, device="cuda:0")
+    entries = [
+        lambda: pkg.fmha_infer_i8(*i8, 1.0, 1.0, 1.0),
+        lambda: pkg.fmha_infer_from_float(*f32[:3], i8[3], 1.0),
+        lambda: pkg.quantize_tensor(x),
+        lambda: pkg.quantize_tensor(x, 1.0),
+        lambda: pkg.dequantize_tensor(x8, 1.0),
+    ]
+    torch.cuda.empty_cache()
+    fake.fake_forget_calls()
+    fake.fake_memory_limit(0)
+    for n, entry in enumerate(entries):
+        try:
+            entry()
+        except torch.OutOfMemoryError as e:
+            assert "out of memory" in str(e)
+        else:
+            raise AssertionError(n)
+        assert not calls()
+    pkg.fmha_infer_i8(*decode, 1.0, 1.0, 1.0, out=out)
+    assert calls() == [("FMHAInferI8Cross", 0, 0)]
+    fake.fake_memory_limit(1 << 30)
+    for entry in entries:
+        entry()
+    pkg.fmha_infer_i8(*decode, 1.0, 1.0, 1.0, out=out)
+    assert calls()[-1] == ("FMHAInferI8CrossWithWorkspace", 0, 0)
+    """)
