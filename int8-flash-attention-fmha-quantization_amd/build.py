@@ -53,8 +53,11 @@ def build_torch(verbose=False):
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
     cmd += [x for d in include for x in ("-I", d)]
-    cmd += ["-o", TORCH_PATH, TORCH_SOURCE, LIB_PATH, "-L", os.path.join(at, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
-            "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    # libfmha_i8.so by name and from this file's own folder, before any LD_LIBRARY_PATH (a library given by its path would be
+    # recorded, and looked for, under that path wherever the package goes)
+    cmd += ["-o", TORCH_PATH, TORCH_SOURCE, "-L", HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
+            "-Wl,--disable-new-dtags", "-L", os.path.join(at, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+            "-ltorch_python"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError("g++ failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
