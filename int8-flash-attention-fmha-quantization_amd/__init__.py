@@ -137,8 +137,8 @@ def _load_native():
     if _native is None:
         if not os.path.exists(TORCH_PATH):
             raise FileNotFoundError(
-                "%s is not built; run `python -c 'import __graft_entry__ as g; g.build()'` at the repository root"
-                % TORCH_PATH)
+                "%s is not built (a build without torch leaves it out); run `python -c 'import __graft_entry__ as g; "
+                "g.build()'` at the repository root, or copy it there from the CMake build, with libfmha_i8.so" % TORCH_PATH)
         loader = importlib.machinery.ExtensionFileLoader("_fmha_torch", TORCH_PATH)
         spec = importlib.util.spec_from_loader("_fmha_torch", loader, origin=TORCH_PATH)
         module = importlib.util.module_from_spec(spec)

@@ -5,6 +5,7 @@ the shared library it produces exports every symbol the headers declare.  Cross-
 import os
 import shutil
 import subprocess
+import sys
 
 import pytest
 
@@ -29,3 +30,19 @@ def test_cmake_configures_builds_and_exports_the_c_abi(pkg, tmp_path):
     targets = subprocess.run(["strings", "-n", "8", lib], stdout=subprocess.PIPE, text=True, check=True).stdout
     assert "amdgcn-amd-amdhsa--gfx950" in targets
     assert not any(t in targets for t in ("--gfx90a", "--gfx942", "--gfx1100"))
+    # the package with the two files of this build in place of its own: the torch entry points load and use them
+    at = tmp_path / "package"
+    at.mkdir()
+    for f in (os.path.join(PKG_DIR, "__init__.py"), lib, os.path.join(build, "_fmha_torch.so")):
+        shutil.copy(f, at)
+    code = """
+import importlib.util, sys
+spec = importlib.util.spec_from_file_location("cmake_package", sys.argv[1] + "/__init__.py")
+pkg = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(pkg)
+pkg._load_native()
+used = {line.split()[-1] for line in open("/proc/self/maps") if "fmha" in line}
+assert used == {sys.argv[1] + "/libfmha_i8.so", sys.argv[1] + "/_fmha_torch.so"}, used
+"""
+    p = subprocess.run([sys.executable, "-c", code, str(at)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert p.returncode == 0, p.stdout[-4000:]
