@@ -44,8 +44,13 @@ def build_library(verbose=False):
 
 def build_torch(verbose=False):
     """Compile the native host path of the torch entry points into _fmha_torch.so (host code only; it calls the C ABI of
-    libfmha_i8.so, which must be built first and is found beside it at run time)."""
-    import torch
+    libfmha_i8.so, which must be built first and is found beside it at run time).  None where torch is not installed: the
+    library serves C and C++ callers without it."""
+    try:
+        import torch
+    except ImportError:
+        print("torch is not installed: %s is not built" % os.path.basename(TORCH_PATH))
+        return None
     at = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc_path())))
     include = [sysconfig.get_paths()["include"], os.path.join(at, "include"),

@@ -145,3 +145,23 @@ assert used == {sys.argv[1] + "/libfmha_i8.so", sys.argv[1] + "/_fmha_torch.so"}
 """
     p = subprocess.run([sys.executable, "-c", code, at], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
     assert p.returncode == 0, p.stdout[-4000:]
+
+
+def test_build_without_torch(tmp_path):
+    """C and C++ callers build the library where torch is not installed; the rest of build() goes through, compilers stubbed."""
+    code = """
+import subprocess, sys
+sys.modules["torch"] = None  # import torch raises ModuleNotFoundError
+sys.path.insert(0, sys.argv[1])
+import __graft_entry__ as g
+commands = []
+def run(cmd, **kw):
+    commands.append(cmd)
+    return subprocess.CompletedProcess(cmd, 0, stdout="")
+subprocess.run = run
+g.build()
+assert any("fmha_i8_api.hip" in " ".join(c) for c in commands)
+assert not any("fmha_torch.cpp" in " ".join(c) for c in commands)
+"""
+    p = subprocess.run([sys.executable, "-c", code, ROOT], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert p.returncode == 0, p.stdout[-4000:]
