@@ -160,34 +160,37 @@ hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const f
   const void* kernel = row_groups == 1 ? split_kernel<D, BK, 1>(var) : row_groups == 2 ? split_kernel<D, BK, 2>(var) : split_kernel<D, BK, 4>(var);
   return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 ? 256 : 512), kernel_args, 0, stream);
 }
+// What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
+// split kernel.  The constants are microseconds * 100 measured on one MI355X at 512 to 4096 keys with one workgroup per CU,
+// [head_dim 64, 128][blocks of 64, 128 keys].
+struct KernelCost {
+  int row_groups, keys_per_round;
+  struct { int start, step; } cost[2][2];
+};
+constexpr KernelCost kKernelCosts[] = {{0, 1, {{{0, 95}, {95, 128}}, {{160, 112}, {250, 162}}}},
+                                       {4, 1, {{{110, 65}, {170, 97}}, {{180, 89}, {300, 116}}}},
+                                       {2, 4, {{{0, 208}, {45, 312}}, {{60, 220}, {140, 332}}}},
+                                       {1, 4, {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}}}};
+constexpr KernelCost kOneGroupCost = kKernelCosts[3];
+static_assert(kOneGroupCost.row_groups == 1, "");
 // Groups of 32 query rows per workgroup of the kernel that serves a call: 1 or 2 (fmha_i8_split_kernel), 4
 // (fmha_i8_pair_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
-// Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (start + step * rounds): a round is
-// one key block for the last two and four for the split kernel.  The constants are microseconds * 100 measured on one MI355X
-// at 512 to 4096 keys with one workgroup per CU, [head_dim 64, 128][blocks of 64, 128 keys].  What they order is far apart
-// nearly everywhere - d128, S2048: H4 31.3 us in 256-row workgroups, 24.3 in those of four groups, 17.6 of two, 13.5 of one;
-// H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error only shift the
-// boundary between equals.
+// Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (cost of one).  What the constants
+// order is far apart nearly everywhere - d128, S2048: H4 31.3 us in 256-row workgroups, 24.3 in those of four groups, 17.6 of
+// two, 13.5 of one; H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error
+// only shift the boundary between equals.
 int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* cost_of = nullptr) {
 #ifdef FMHA_SPLIT_FORCE
   return a.seq_len_kv > block_keys ? FMHA_SPLIT_FORCE : 0;
 #endif
   if (a.seq_len_kv <= block_keys) return 0;
-  struct Kernel {
-    int row_groups, keys_per_round;
-    struct { int start, step; } cost[2][2];
-  };
-  static constexpr Kernel kKernels[] = {{0, 1, {{{0, 95}, {95, 128}}, {{160, 112}, {250, 162}}}},
-                                        {4, 1, {{{110, 65}, {170, 97}}, {{180, 89}, {300, 116}}}},
-                                        {2, 4, {{{0, 208}, {45, 312}}, {{60, 220}, {140, 332}}}},
-                                        {1, 4, {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}}}};
   const int d = a.head_dim == 128, k = block_keys == fmha_i8_gfx950::kBlockK;
   const long long heads = (long long)a.batch_num * a.head_num;
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
   int best = 0;
   long long least = -1;
-  for (const Kernel& kernel : kKernels) {
+  for (const KernelCost& kernel : kKernelCosts) {
     // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
     // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 14.1 with two; d64: 11.7 either way).
     const bool helper = a.seq_len_q <= 32 && kernel.row_groups == 2;
@@ -219,8 +222,7 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
-  static constexpr struct { int start, step; } kCost[2][2] = {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}};
-  const auto& c = kCost[a.head_dim == 128][block_keys == kBlockK];
+  const auto& c = kOneGroupCost.cost[a.head_dim == 128][block_keys == kBlockK];
   long long least = 0;
   row_groups_of(a, block_keys, &least);
   least = (least > memory ? least : memory) * 20 / 21;
