@@ -181,10 +181,8 @@ static_assert(kOneGroupCost.row_groups == 1, "");
 // two, 13.5 of one; H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error
 // only shift the boundary between equals.
 int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* cost_of = nullptr) {
-#ifdef FMHA_SPLIT_FORCE
-  return a.seq_len_kv > block_keys ? FMHA_SPLIT_FORCE : 0;
-#endif
   if (a.seq_len_kv <= block_keys) return 0;
+  if (fmha_i8_gfx950::test_build::forced_route() >= 0) return fmha_i8_gfx950::test_build::forced_route();
   const int d = a.head_dim == 128, k = block_keys == fmha_i8_gfx950::kBlockK;
   const long long heads = (long long)a.batch_num * a.head_num;
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
@@ -220,6 +218,7 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys, rounds = (blocks + kSplitKeys - 1) / kSplitKeys;
   const long long heads = (long long)a.batch_num * a.head_num;
   if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
+  if (test_build::forced_route() >= 0) return plan;
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
   const auto& c = kOneGroupCost.cost[a.head_dim == 128][block_keys == kBlockK];
@@ -233,7 +232,7 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
     work = of_r;
     plan.rounds_per_part = r;
   }
-  if ((work > memory ? work : memory) + merge >= least) plan.rounds_per_part = 0;
+  if ((work > memory ? work : memory) + merge >= least && test_build::forced_route() != test_build::kSharedOut) plan.rounds_per_part = 0;
   const size_t rows = (size_t)heads * blocks * a.seq_len_q;
   plan.ml_bytes = (rows * sizeof(v2f) + 255) / 256 * 256;
   plan.bytes = plan.ml_bytes + rows * a.head_dim * sizeof(int);
@@ -417,6 +416,11 @@ int FMHAInferI8DebugOutOfBounds(void) {
   if (hipMemcpyToSymbol(HIP_SYMBOL(fmha_i8_gfx950::g_fmha_oob_count), &zero, sizeof(int)) != hipSuccess) return -1;
   return count;
 }
+#endif
+
+#ifdef FMHA_FORCED_ROUTE
+// Test build only: the kernel that serves the calls from here on (see the flag list of the test builds).
+void FMHAInferI8DebugRoute(int route) { fmha_i8_gfx950::test_build::g_route = route; }
 #endif
 
 #ifdef FMHA_TRACE_TICKS

@@ -29,15 +29,17 @@
 //                        the first byte, so that the run ends normally and the test can read the count.  An
 //                        out-of-bounds READ changes no result and, inside a caching allocator's pool, raises no fault:
 //                        nothing else shows it.
-//   FMHA_SPLIT_FORCE=n   calls of more than one key block are served by the kernel with n groups of 32 rows per workgroup (1,
-//                        2, 4; 0: 256 rows) whatever their size: for re-measuring the costs that the choice rests on
+//   FMHA_FORCED_ROUTE    exports FMHAInferI8DebugRoute(n), after which calls of more than one key block are served by the
+//                        kernel with n groups of 32 rows per workgroup (1, 2, 4; 0: 256 rows) whatever their size, or, with
+//                        n = -2, calls with a workspace share their key blocks out whenever they can (-1: the library's own
+//                        choice): for tests of one kernel at small sizes, and for re-measuring the costs that the choice rests on
 //   FMHA_LOOP_PAD_A=n    n s_nops between the 64-byte boundary in front of the steady-state loop of wavefronts 0..3 and
 //                        the loop (the kernel's own choice otherwise): for re-measuring what the placement costs
 #pragma once
 
 // The test builds that change the attention kernel of 256-row workgroups serve every call with it, so that what they are
 // compared or timed for is that kernel at every size (the shipped library writes the same bytes with either kernel).
-#if (defined(FMHA_FEW_INSTANTIATIONS) && !defined(FMHA_SPLIT_FORCE)) || defined(FMHA_TWO_BARRIERS) || defined(FMHA_LOOP_PAD_A)
+#if defined(FMHA_FEW_INSTANTIATIONS) || defined(FMHA_TWO_BARRIERS) || defined(FMHA_LOOP_PAD_A)
 #define FMHA_NO_SPLIT_KERNEL
 #endif
 
@@ -113,6 +115,15 @@ constexpr bool kTraceTicks = false;
 constexpr int kLoopPadA = FMHA_LOOP_PAD_A;
 #else
 constexpr int kLoopPadA = -1;  // the kernel's own choice
+#endif
+
+// Which kernel serves a call (see FMHA_FORCED_ROUTE)
+constexpr int kOwnChoice = -1, kSharedOut = -2;
+#ifdef FMHA_FORCED_ROUTE
+inline int g_route = kOwnChoice;
+inline int forced_route() { return g_route; }
+#else
+constexpr int forced_route() { return kOwnChoice; }
 #endif
 
 // What a knocked-out producer leaves behind: a register (or a vector of them) whose content is undefined, at no cost.

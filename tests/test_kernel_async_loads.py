@@ -1,8 +1,8 @@
-"""The attention kernel loads the mask word and the Q rows with inline-assembly loads whose results arrive
-asynchronously, and retires them with explicit `s_waitcnt vmcnt(n)` that count the loads still allowed in flight.  The
+"""The attention kernels load the mask bytes and the Q rows with inline-assembly loads whose results arrive
+asynchronously, and retire them with explicit `s_waitcnt vmcnt(n)` that count the loads still allowed in flight.  The
 compiler knows nothing of that protocol: were it to copy or read one of those registers between the load and its wait
 (it did once, when the wait was written into two branches), it would read stale data without any error.  This test
-compiles the kernel to assembly and checks, for every instantiation, that no instruction touches an asynchronously
+compiles the kernels to assembly and checks, for every instantiation, that no instruction touches an asynchronously
 loaded register before a wait that is strict enough to have retired the load.  Host-side: needs hipcc, no GPU."""
 import os
 import re
@@ -24,23 +24,37 @@ def _regs(line):
     return used
 
 
-def _assembly(path, *extra):
-    subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-                    "-packed-fp32-ops", "-S", "--cuda-device-only", *extra, "-o", path, SRC], check=True,
-                   capture_output=True)
-    text = open(path).read()
-    funcs = re.split(r"\n(?=_ZN14fmha_i8_gfx95018fmha_i8_fwd_kernel[^\n]*:\s)", text)[1:]
-    assert len(funcs) == 64
+def _start_assembly(path, *extra):
+    return subprocess.Popen(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                             "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1", "-S", "--cuda-device-only", *extra,
+                             "-o", path, SRC], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+
+
+def _functions(path):
+    funcs = re.split(r"\n(?=_ZN14fmha_i8_gfx950\d+fmha_i8_(?:fwd|split|pair)_kernel[^\n]*:\s)", open(path).read())[1:]
+    # (head size, block size, two arithmetic variants, P range) for each kernel, and ragged ends (256 rows), row groups 1 and 2
+    # (split); the shared-out form has one arithmetic variant less
+    assert [sum(k in f.split(":")[0] for f in funcs) for k in ("fwd", "split", "pair")] == [64, 64 + 16, 32]
     return funcs
 
 
 @pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
-    return _assembly(str(tmp_path_factory.mktemp("asm") / "kernel.s"))
+def assembly(tmp_path_factory):
+    """Every instantiation as shipped, and with contraction switched off on the command line."""
+    at = tmp_path_factory.mktemp("asm")
+    paths = str(at / "kernel.s"), str(at / "kernel_off.s")
+    compilers = [_start_assembly(paths[0]), _start_assembly(paths[1], "-ffp-contract=off")]
+    assert [c.wait() for c in compilers] == [0, 0]
+    return [_functions(p) for p in paths]
+
+
+@pytest.fixture(scope="module")
+def kernels(assembly):
+    return assembly[0]
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-def test_the_compiler_fuses_no_multiply_add_on_its_own(kernels, tmp_path):
+def test_the_compiler_fuses_no_multiply_add_on_its_own(assembly):
     """The source pins floating-point contraction off and writes out every fma it wants, so the result bits do not
     depend on which products an optimiser fuses (hipcc's default is to fuse where it sees fit: two builds of the same
     arithmetic once differed in one output LSB of a few elements per thousand).  Compiled with contraction switched
@@ -54,8 +68,7 @@ def test_the_compiler_fuses_no_multiply_add_on_its_own(kernels, tmp_path):
             if t and not t.startswith(".") and not t.endswith(":"):
                 ops.append(re.sub(r"\.LBB\d+_\d+", "L", re.sub(r"_ZZN\w+", "SYM", t)))
         return ops
-    pinned = _assembly(str(tmp_path / "kernel_off.s"), "-ffp-contract=off")
-    for a, b in zip(kernels, pinned):
+    for a, b in zip(*assembly):
         assert a.split(":")[0] == b.split(":")[0]
         assert stream(a) == stream(b), a.split(":")[0]
 
