@@ -117,9 +117,10 @@ struct KernelArgs {
 
 // The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8), where the caller wants it: in
 // place of a launch that passes over o again (B4 H16 S1024 d128, bfloat16: 6.1 us separate, 4.5 here; the host chooses).
-template <int WORDS>
+template <int D, int WORDS>
 __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, const int (&w)[WORDS]) {
   if (args.wide == nullptr) return;
+  if (kCheckBounds && !fmha_in_bounds(at >= 0 && at + 4 * WORDS <= (long)args.total_wgs / args.q_blocks * args.seq_q * D)) return;
   auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
   if (args.wide_is_bf16) {
     unsigned short* p = static_cast<unsigned short*>(args.wide) + at;
@@ -1364,7 +1365,7 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
     *reinterpret_cast<v4i*>(op + 32 * u) = v4i{g0[0], g1[0], g0[1], g1[1]};
     *reinterpret_cast<v4i*>(op + 32 * u + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
     const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
-    store_wide(args, op - args.o + 32 * u, both);
+    store_wide<D>(args, op - args.o + 32 * u, both);
   }
 }
 

@@ -458,7 +458,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
     *reinterpret_cast<v4i*>(op) = v4i{g0[0], g1[0], g0[1], g1[1]};
     *reinterpret_cast<v4i*>(op + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
     const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
-    store_wide(args, op - args.o, both);
+    store_wide<D>(args, op - args.o, both);
   } else {
     op += 8 * g;
 #pragma unroll
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       const auto s = __builtin_amdgcn_permlane32_swap(w[0][a], w[0][a + 1], false, false);
       *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
       const int both[2] = {(int)s[0], (int)s[1]};
-      store_wide(args, op - args.o + 8 * a, both);
+      store_wide<D>(args, op - args.o + 8 * a, both);
     }
   }
 }

@@ -311,9 +311,13 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   n = __builtin_amdgcn_readfirstlane(n) + 1;  // one past the last block with an unmasked key
   const int rounds = PARTS ? min(first_round + args.rounds_per_part, (n + kSplitKeys - 1) / kSplitKeys) : (n + kSplitKeys - 1) / kSplitKeys;
   const long part_first = (long)bh * n_blocks;  // PARTS: the head's first key block in part_ml and part_o
+  auto in_workspace = [&](int kb, int row) __attribute__((always_inline)) {  // block kb of this head, and what the host made room for
+    const long heads = args.total_wgs / args.q_blocks;
+    return fmha_in_bounds(kb >= 0 && kb < n_blocks && row >= 0 && row < Sq && (part_first + kb) * Sq + row < heads * n_blocks * Sq);
+  };
   if constexpr (PARTS) {  // blocks without an unmasked key: a maximum that the merge takes for "nothing here"
     for (int kb = keys_to / BK - 1 - wave; kb >= kSplitKeys * first_round; kb -= kRowWaves)
-      if ((reinterpret_cast<const unsigned char*>(lds_class4)[kb] & 2) && lane < Sq)
+      if ((reinterpret_cast<const unsigned char*>(lds_class4)[kb] & 2) && lane < Sq && (!kCheckBounds || in_workspace(kb, lane)))
         args.part_ml[(part_first + kb) * Sq + lane] = v2f{-__builtin_inff(), 0.f};
   }
 
@@ -423,7 +427,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   };
   auto publish_ml = [&](int kb) __attribute__((always_inline)) {
     if constexpr (PARTS) {
-      if (lane < Sq) args.part_ml[(part_first + kb) * Sq + lane] = v2f{m_blk, l_blk};
+      if (lane < Sq && (!kCheckBounds || in_workspace(kb, lane))) args.part_ml[(part_first + kb) * Sq + lane] = v2f{m_blk, l_blk};
       return;
     }
     lds_ml[r][c][i32][0] = m_blk;
@@ -467,7 +471,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
           oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], p[j & 1][t], oacc[0], 0, 0, 0);
           between(j * kKeyTiles + t, kCount * kKeyTiles);
         }
-        if (!((cls4 >> (8 * (first + j))) & 2) && c < kDSteps && i32 < Sq) {
+        if (!((cls4 >> (8 * (first + j))) & 2) && c < kDSteps && i32 < Sq &&
+            (!kCheckBounds || (in_workspace(part_kb + first + j, i32) && fmha_in_bounds((8 * u_out + g) * 4 + 8 * 3 + 4 <= D)))) {
           int* at = args.part_o + (part_first + part_kb + first + j) * Sq * D + ((8 * u_out + g) * Sq + i32) * 4;
 #pragma unroll
           for (int a = 0; a < 4; ++a)
@@ -657,7 +662,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     const auto s = __builtin_amdgcn_permlane32_swap(w[a], w[a + 1], false, false);
     *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
     const int both[2] = {(int)s[0], (int)s[1]};
-    store_wide(args, op - args.o + 8 * a, both);
+    store_wide<D>(args, op - args.o + 8 * a, both);
   }
 }
 
@@ -690,6 +695,7 @@ __global__ __launch_bounds__(64, 1) void fmha_i8_merge_kernel(const MergeArgs ar
   const long bh = blockIdx.y;
   const int row = min(lane / args.row_lanes, Sq - 1);
   const int col = 2 * (blockIdx.x * args.row_lanes + lane % args.row_lanes);
+  if (kCheckBounds && !fmha_in_bounds(row >= 0 && row < Sq && col >= 0 && col + 2 <= D)) return;
   const v2f* ml = args.part_ml + bh * args.n_blocks * Sq + row;
   const int* po = args.part_o + bh * args.n_blocks * Sq * D + (col / 4 * Sq + row) * 4 + col % 4;
   const float kGone = -__builtin_inff();
@@ -701,7 +707,8 @@ __global__ __launch_bounds__(64, 1) void fmha_i8_merge_kernel(const MergeArgs ar
     v2i x[BATCH];
 #pragma unroll
     for (int j = 0; j < BATCH; ++j) {
-      const long kb = min(kb0 + j, args.n_blocks - 1);
+      long kb = min(kb0 + j, args.n_blocks - 1);
+      if (kCheckBounds && !fmha_in_bounds(kb >= 0 && kb < args.n_blocks)) kb = 0;
       s[j] = ml[kb * Sq];
       x[j] = *reinterpret_cast<const v2i*>(po + kb * Sq * D);
     }

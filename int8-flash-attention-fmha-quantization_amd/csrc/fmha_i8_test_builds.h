@@ -139,13 +139,16 @@ __device__ __forceinline__ void consume(const T& x) {
 
 }  // namespace test_build
 
+// (`kCheckBounds && !fmha_in_bounds(...)` keeps even the operands of a check out of the shipped code)
 #ifdef FMHA_CHECK_BOUNDS
+constexpr bool kCheckBounds = true;
 __device__ int g_fmha_oob_count;
 __device__ __forceinline__ bool fmha_in_bounds(bool ok) {
   if (!ok) atomicAdd(&g_fmha_oob_count, 1);
   return ok;
 }
 #else
+constexpr bool kCheckBounds = false;
 __device__ __forceinline__ constexpr bool fmha_in_bounds(bool) { return true; }
 #endif
 
