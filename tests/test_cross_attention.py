@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import fmha_cases as fc
+import routes
 
 WITHIN1_MIN = 0.999
 MAX_ABS_LSB = 2
@@ -90,6 +91,7 @@ def _gpu(pkg, dev, q, c, canary=False):
         out = buf[:q.size].view(q.shape)
     o = pkg.fmha_infer_i8(*t, *_scales(c), out=out)
     torch.cuda.synchronize()
+    routes.check_every_route(pkg, t, _scales(c), o)  # whichever kernel served the call, the others agree
     if canary:
         assert (buf[q.size:] == 77).all().item()
     return o.cpu().numpy()
@@ -280,4 +282,5 @@ def test_random_shapes(pkg, orc, dev):
         t = [torch.from_numpy(np.ascontiguousarray(a)).to(dev) for a in (q, k, v, mask)]
         got = pkg.fmha_infer_i8(*t, *scales)
         torch.cuda.synchronize()
+        routes.check_every_route(pkg, t, scales, got)
         _gate(got.cpu().numpy(), want, "random case %d" % it)

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import fmha_cases as fc
+import routes
 import np_model
 
 WITHIN1_MIN = 0.999
@@ -111,6 +112,7 @@ def _gpu(pkg, dev, c, scales=None):
     t = [torch.from_numpy(np.ascontiguousarray(c[n])).to(dev) for n in ("q", "k", "v", "mask")]
     o = pkg.fmha_infer_i8(*t, *(scales or _scales(c)), full_range_p=True)
     torch.cuda.synchronize()
+    routes.check_every_route(pkg, t, scales or _scales(c), o, full_range_p=True)  # whichever kernel served the call, the others agree
     return o.cpu().numpy()
 
 
@@ -153,7 +155,7 @@ def test_full_range_p_any_key_and_query_count(pkg, orc, dev, S, d):
 def test_full_range_p_every_kernel_variant(pkg, orc, dev):
     """Score scales on both sides of the switch between the two ways the scores are read, output scales on both sides
     of the switch between the two ways the running O is kept, blocks of 128 and of 64 keys, full and ragged ends,
-    both head sizes: the sixteen x two full-range instantiations of the kernel."""
+    both head sizes: the sixteen x two full-range instantiations of the 256-row kernel, and those of the others."""
     for d in (64, 128):
         for S in (256, 320, 250, 300):
             c = fc.make_inputs(2, 2, (S + 63) // 64 * 64, d, pad="scatter", seed=81)

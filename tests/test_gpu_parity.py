@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import fmha_cases as fc
+import routes
 
 pytestmark = pytest.mark.gpu
 
@@ -25,8 +26,10 @@ def gpu_run(pkg, dev, c, **scales):
     s = dict(q_amax=c["q_amax"], k_amax=c["k_amax"], v_amax=c["v_amax"], o_amax=c["o_amax"])
     s.update(scales)
     q, k, v, m = to_dev(dev, c["q"], c["k"], c["v"], c["mask"])
-    o = pkg.fmha_infer_i8(q, k, v, m, s["q_amax"], s["k_amax"], s["v_amax"], s["o_amax"])
+    scales = (s["q_amax"], s["k_amax"], s["v_amax"], s["o_amax"])
+    o = pkg.fmha_infer_i8(q, k, v, m, *scales)
     torch.cuda.synchronize()
+    routes.check_every_route(pkg, (q, k, v, m), scales, o)  # whichever kernel served the call, the others agree
     return o.cpu().numpy()
 
 
@@ -252,7 +255,8 @@ def test_every_kernel_variant(pkg, orc, dev, S, d, qk_scale, vo_ratio):
     """The library picks one of four arithmetic variants of the kernel from the scales (accumulators read as floats or
     converted; accumulator offset folded into the running O or not) for each head_dim, softmax block size (128 or 64
     keys) and for lengths with and without a partly filled last block.  A large q_amax*k_amax forces the converting
-    variant, a large v_amax/o_amax the unfolded one: all thirty-two instantiations must meet the same gate."""
+    variant, a large v_amax/o_amax the unfolded one: all thirty-two instantiations of the 256-row kernel must meet the same
+    gate, and those of the kernels of smaller workgroups must write their bytes."""
     c = fc.make_inputs(2, 2, S, d, dist="normal", pad="scatter", seed=91)
     kw = dict(q_amax=c["q_amax"] * qk_scale, v_amax=vo_ratio, o_amax=1.0 if vo_ratio == 1.0 else 2.0)
     s = dict(q_amax=c["q_amax"], k_amax=c["k_amax"], v_amax=c["v_amax"], o_amax=c["o_amax"])
@@ -321,8 +325,10 @@ def test_every_sequence_of_block_kinds(pkg, orc, dev, d, block, full_range_p):
             gone = np.nonzero(mask[b])[0][::7]
             c["k"][b][:, gone, :] = kq[b][:, gone, :]
         q, k, v, m = to_dev(dev, c["q"], c["k"], c["v"], c["mask"])
-        o = pkg.fmha_infer_i8(q, k, v, m, c["q_amax"], c["k_amax"], c["v_amax"], c["o_amax"], full_range_p=full_range_p)
+        scales = (c["q_amax"], c["k_amax"], c["v_amax"], c["o_amax"])
+        o = pkg.fmha_infer_i8(q, k, v, m, *scales, full_range_p=full_range_p)
         torch.cuda.synchronize()
+        routes.check_every_route(pkg, (q, k, v, m), scales, o, full_range_p)
         blk = 128 if S % 128 == 0 else 64
         if full_range_p:
             want = orc.fmha_i8_blockwise_cross(c["q"], c["k"], c["v"], c["mask"], c["q_amax"], c["k_amax"], c["v_amax"],
@@ -403,12 +409,13 @@ def test_one_hot_attention_closed_form_on_gpu(pkg, dev):
 
 
 # ---- API behaviour -----------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("rows", [None, 256, 128, 64, 32])  # None: the shipped library and its own choice
 @pytest.mark.parametrize("B,H,S,d,pad", [(4, 16, 1024, 128, "none"), (2, 4, 2048, 128, "tail256"), (1, 3, 1337, 128, "scatter"),
                                          (2, 2, 2048, 64, "none"), (1, 2, 704, 64, "scatter")])
-def test_back_to_back_launches_write_the_same_bytes(pkg, dev, B, H, S, d, pad):
+def test_back_to_back_launches_write_the_same_bytes(pkg, dev, B, H, S, d, pad, rows):
     # The K/V tiles live in a ring of LDS stages that is refilled while other wavefronts still compute: a stage
     # refilled too early, or read before it is published, would show as launches of one problem that differ.  200
-    # launches back to back into alternating output buffers, every one compared with the first on the GPU.
+    # launches of each kernel back to back into alternating output buffers, every one compared with the first on the GPU.
     import torch
     Sp = (S + 63) // 64 * 64
     c = fc.make_inputs(B, H, Sp, d, pad="scatter" if pad == "scatter" else pad, seed=77)
@@ -418,11 +425,19 @@ def test_back_to_back_launches_write_the_same_bytes(pkg, dev, B, H, S, d, pad):
     tq, tk, tv, tm = to_dev(dev, q, k, v, m)
     outs = [torch.empty_like(tq), torch.empty_like(tq), torch.empty_like(tq)]
     args = (c["q_amax"], c["k_amax"], c["v_amax"], c["o_amax"])
-    pkg.fmha_infer_i8(tq, tk, tv, tm, *args, out=outs[0])
+    lib = routes.library(pkg)
+
+    def run(o):
+        if rows is None:
+            pkg.fmha_infer_i8(tq, tk, tv, tm, *args, out=o)
+        else:
+            routes.attend(pkg, lib, routes.ROUTES[rows], (tq, tk, tv, tm), args, o)
+
+    run(outs[0])
     differing = torch.zeros((), dtype=torch.int64, device=dev)
     for it in range(200):
         o = outs[1 + it % 2]
-        pkg.fmha_infer_i8(tq, tk, tv, tm, *args, out=o)
+        run(o)
         differing += (o != outs[0]).sum()
     torch.cuda.synchronize()
     assert int(differing.item()) == 0
