@@ -25,8 +25,12 @@ constexpr int kQuantUnroll = 4;          // 16-byte units per thread and loop tr
 // Two workgroups of 4 wavefronts per CU: measured best from 8 to 134 MB in each kernel (bf16 de-quantise of 33.5 M elements:
 // 15.9 us with 512 workgroups, 17.9 with 1024; 256 lose as much below 16 MB).
 constexpr int kQuantMaxBlocks = 256 * 2;
-constexpr long long kCacheBytes = 256ll << 20;  // beyond the last-level cache, loads bypass it (non-temporal): +18 %
-                                                // at 1 GiB, -8 % at 128 MiB, hence the switch
+// An input larger than the last-level cache is quantised with loads that bypass it (non-temporal): fp32 62.6 -> 60.0 us at 288
+// MiB, 88.3 -> 81.8 at 384, 243 -> 229 at 1 GiB, bf16 75.8 -> 71.8 at 288, 141.5 -> 129.0 at 512; at 256 MiB they lose (fp32 47.0 ->
+// 53.2, bf16 57.5 -> 63.3).  Nowhere else: behind an abs-max, which has just read the tensor, they lose up to 700 MiB (fp32 92.9 ->
+// 98.2 us at 288, level at 640) and gain 1 to 3 % above; the de-quantisation reads a byte per element (fp32, 268 M elements:
+// 208 -> 243 us).
+constexpr long long kCacheBytes = 256ll << 20;
 // What a kernel writes it never reads again: stores are non-temporal at every size, so that the input - read a second
 // time by the quantisation behind the abs-max - keeps the L2 (fp32, abs-max + quantise: 13.6 -> 12.8 us at 8.4 M elements,
 // 48.2 -> 45.1 at 33.5 M; de-quantise 7.9 -> 6.4 at 8.4 M; level elsewhere).
@@ -159,9 +163,10 @@ __device__ __forceinline__ v2i32 quant_unit(const v8h& v, float scale) {
   auto q = [&](int e) { return quant1(BF16::widen(v[e]), scale); };
   return v2i32{pack4(q(0), q(1), q(2), q(3)), pack4(q(4), q(5), q(6), q(7))};
 }
-template <typename P>
-__device__ __forceinline__ P load_unit(const P* p, bool nt) {
-  return nt ? __builtin_nontemporal_load(p) : *p;
+template <bool NT, typename P>  // (a run-time choice between the two is merged into one plain load, constant or not)
+__device__ __forceinline__ P load_unit(const P* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
 }
 // This thread's share of a tensor.  BACK: from the last trip to the first, behind an abs-max that walked the same share
 // forwards: the end of the tensor is what the L2 still holds (50.3 -> 48.2 us at 134 MB, level below 32 MB).
@@ -177,7 +182,7 @@ __device__ __forceinline__ void quantize_share(const typename T::elem* __restric
   auto trip_at = [&](long long at) {
     typename T::unit v[kQuantUnroll];
 #pragma unroll
-    for (int u = 0; u < kQuantUnroll; ++u) v[u] = load_unit(&xu[at + u * stride], NT);
+    for (int u = 0; u < kQuantUnroll; ++u) v[u] = load_unit<NT>(&xu[at + u * stride]);
 #pragma unroll
     for (int u = 0; u < kQuantUnroll; ++u) __builtin_nontemporal_store(quant_unit(v[u], scale), &ou[at + u * stride]);
   };
@@ -213,7 +218,7 @@ __device__ __forceinline__ void note_amax(unsigned long long* note, int i, float
 // cache) before it starts, which replaces both the atomics and the launch that clears their target.  With the same split
 // into workgroups as the abs-max, what a workgroup reads here its XCD has read before.
 // abs-max + quantise, fp32: 18.8 -> 12.8 us at 8.4 M elements (a clearing kernel, 512 atomics and 9.5 us of abs-max before).
-template <typename T, bool NT>
+template <typename T>
 __global__ __launch_bounds__(kQuantThreads) void quantize_by_parts_kernel(QuantJob job, const float* __restrict__ parts,
                                                                            float* __restrict__ amax_out,
                                                                            unsigned long long* __restrict__ note, unsigned ticket) {
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_by_parts_kernel(QuantJ
     amax_out[i] = amax;
     note_amax(note, i, amax, ticket);
   }
-  quantize_share<T, NT, true>(static_cast<const typename T::elem*>(job.x[i]), job.n[i], 127.0f / amax, job.out[i],
+  quantize_share<T, false, true>(static_cast<const typename T::elem*>(job.x[i]), job.n[i], 127.0f / amax, job.out[i],
                               blockIdx.x - first, blocks);
 }
 
@@ -286,7 +291,7 @@ __device__ __forceinline__ void dequant_unit(const v2i32& w, float amax, v8h& r)
                                     (int)cvt_pk_bf16(b[2], b[3])});
 }
 
-template <typename T, bool NT>
+template <typename T>
 __global__ __launch_bounds__(kQuantThreads) void dequantize_i8_kernel(const int8_t* __restrict__ x, long long n, float amax,
                                                                        typename T::elem* __restrict__ out) {
   const long long units = n / T::kPerUnit;
@@ -297,7 +302,7 @@ __global__ __launch_bounds__(kQuantThreads) void dequantize_i8_kernel(const int8
   for (; j + (kQuantUnroll - 1) * stride < units; j += kQuantUnroll * stride) {
     typename T::packed w[kQuantUnroll];
 #pragma unroll
-    for (int u = 0; u < kQuantUnroll; ++u) w[u] = load_unit(&xu[j + u * stride], NT);
+    for (int u = 0; u < kQuantUnroll; ++u) w[u] = xu[j + u * stride];
 #pragma unroll
     for (int u = 0; u < kQuantUnroll; ++u) {
       typename T::unit r;
@@ -353,7 +358,7 @@ int quantize(hipStream_t stream, const typename T::elem* x, long long n, float a
   if (amax_dev == nullptr && !(amax_host == amax_host)) return FMHA_I8_ERR_SCALE;
   if (n == 0) return FMHA_I8_OK;
   const int blocks = quant_blocks(n / T::kPerUnit, kQuantMaxBlocks);
-  const bool nt = (long long)(sizeof(typename T::elem) + 1) * n > kCacheBytes;
+  const bool nt = (long long)sizeof(typename T::elem) * n > kCacheBytes;
   return status_of(nt ? launch_kernel(quantize_i8_kernel<T, true>, blocks, kQuantThreads, stream, x, n, amax_host, amax_dev, out)
                       : launch_kernel(quantize_i8_kernel<T, false>, blocks, kQuantThreads, stream, x, n, amax_host, amax_dev, out));
 }
@@ -382,9 +387,7 @@ int measure_and_quantize(hipStream_t stream, const FMHAQuantTensor* t, int count
   job.first_block[FMHA_QUANT_MAX_TENSORS] = blocks;
   hipError_t err = launch_kernel(abs_max_parts_kernel<T>, blocks, kQuantThreads, stream, job, workspace);
   if (err != hipSuccess) return status_of(err);
-  const bool nt = (long long)(sizeof(typename T::elem) + 1) * total > kCacheBytes;
-  return status_of(nt ? launch_kernel(quantize_by_parts_kernel<T, true>, blocks, kQuantThreads, stream, job, workspace, amax_out, note, ticket)
-                      : launch_kernel(quantize_by_parts_kernel<T, false>, blocks, kQuantThreads, stream, job, workspace, amax_out, note, ticket));
+  return status_of(launch_kernel(quantize_by_parts_kernel<T>, blocks, kQuantThreads, stream, job, workspace, amax_out, note, ticket));
 }
 
 template <typename T>
@@ -393,9 +396,7 @@ int dequantize(hipStream_t stream, const int8_t* x, long long n, float amax, typ
   if (!aligned16(x) || !aligned16(out)) return FMHA_I8_ERR_ALIGNMENT;
   if (n == 0) return FMHA_I8_OK;
   const int blocks = quant_blocks(n / T::kPerUnit, kQuantMaxBlocks);
-  const bool nt = (long long)(sizeof(typename T::elem) + 1) * n > kCacheBytes;
-  return status_of(nt ? launch_kernel(dequantize_i8_kernel<T, true>, blocks, kQuantThreads, stream, x, n, amax, out)
-                      : launch_kernel(dequantize_i8_kernel<T, false>, blocks, kQuantThreads, stream, x, n, amax, out));
+  return status_of(launch_kernel(dequantize_i8_kernel<T>, blocks, kQuantThreads, stream, x, n, amax, out));
 }
 
 }  // namespace fmha_i8_gfx950

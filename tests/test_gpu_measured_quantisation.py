@@ -43,6 +43,20 @@ def test_measured_quantisation_of_several_tensors(pkg, orc, dev, sizes, dtype_na
         assert (got[n:] == 77).all()
 
 
+@pytest.mark.parametrize("dtype_name,n", [("float32", (1 << 26) + 5), ("bfloat16", (1 << 27) + 9)])
+def test_inputs_larger_than_the_last_level_cache(pkg, dev, dtype_name, n):
+    """256 MiB and a few elements: another variant of both kernels, the bytes of pieces that the ordinary one quantises."""
+    import torch
+    x = torch.randn(n, device=dev).to(getattr(torch, dtype_name))
+    amax = x.abs().max().item()
+    measured, a = pkg.quantize_tensor(x)
+    given, _ = pkg.quantize_tensor(x, amax)
+    assert a.item() == amax
+    for at in range(0, n, 1 << 24):
+        piece = pkg.quantize_tensor(x[at:at + (1 << 24)], amax)[0]
+        assert torch.equal(piece, measured[at:at + (1 << 24)]) and torch.equal(piece, given[at:at + (1 << 24)])
+
+
 def test_measured_quantisation_checks_its_arguments(pkg, dev):
     import torch
     x = torch.zeros(64, device=dev)
