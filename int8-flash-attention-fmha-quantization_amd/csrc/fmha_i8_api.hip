@@ -161,8 +161,10 @@ hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const f
   return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 ? 256 : 512), kernel_args, 0, stream);
 }
 // What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
-// split kernel.  The constants are microseconds * 100 measured on one MI355X at 512 to 4096 keys with one workgroup per CU,
-// [head_dim 64, 128][blocks of 64, 128 keys].
+// split kernel.  Microseconds * 100 beyond the launch (2.8 to 3.1 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
+// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs).  For blocks of 128 keys a new measurement
+// gives them to 4 %; for blocks of 64 they are right to 5 % at 448 keys and up to 19 % high per further block.  With all CUs at work
+// the first two take up to 39 and 16 % longer per block (the shader clock drops), where the choice is clear anyway.
 struct KernelCost {
   int row_groups, keys_per_round;
   struct { int start, step; } cost[2][2];
@@ -177,9 +179,9 @@ static_assert(kOneGroupCost.row_groups == 1, "");
 // (fmha_i8_pair_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
 // Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (cost of one).  What the constants
-// order is far apart nearly everywhere - d128, S2048: H4 31.3 us in 256-row workgroups, 24.3 in those of four groups, 17.6 of
-// two, 13.5 of one; H8 31.5, 24.6, 17.9, 25.9; H16 32.1, 26.4, 35.3, 51.2; H24 33, 52, 53, 77 - so that a few percent of error
-// only shift the boundary between equals.
+// order is far apart nearly everywhere - d128, S2048: H4 31.0 us in 256-row workgroups, 24.4 in those of four groups, 17.6 of
+// two, 13.4 of one; H8 31.3, 24.6, 17.9, 25.8; H16 31.7, 26.2, 34.5, 50.3; H24 33.9, 48.9, 50.7, 74.6 - so that a few percent of
+// error only shift the boundary between equals.
 int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* cost_of = nullptr) {
   if (a.seq_len_kv <= block_keys) return 0;
   if (fmha_i8_gfx950::test_build::forced_route() >= 0) return fmha_i8_gfx950::test_build::forced_route();
@@ -190,7 +192,8 @@ int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* c
   long long least = -1;
   for (const KernelCost& kernel : kKernelCosts) {
     // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
-    // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 14.1 with two; d64: 11.7 either way).
+    // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 13.9 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with
+    // 16 heads 13.1 and 12.6; d64: 11.7 either way).  Its step is one group's less a little, so that it is taken.
     const bool helper = a.seq_len_q <= 32 && kernel.row_groups == 2;
     if (helper && !(d && k)) continue;
     const int rows = kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups;
@@ -209,9 +212,11 @@ int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* c
 // Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for, by the cost
 // table above (start, step of one row group), but no faster than the memory (62 KB in a hundredth of a microsecond, on both
 // sides of the comparison), with the workspace written and read again, and the merge: 2.5 us for the launch and a first batch of
-// key blocks, 0.8 per further batch.  One call, plain -> shared out: B1 H16 Sq1 S2048 d128 12.2 -> 9.2 us, S8192 d64 36.3 -> 11.8,
-// H32 S8192 d128 41.7 -> 19.3, H8 S65536 331 -> 61; H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds
-// already, 14.0 -> 15.9 and hence not.
+// key blocks, 0.8 per further batch.  Within 5 % of each other (the factor 20/21) the plain route is taken, which needs no memory: the
+// model flatters the other one there - of eleven shapes that it puts 0 to 5 % ahead nine are slower shared out, by 2 to 21 % (H32
+// Sq32 S1500 d128 11.1 -> 13.5 us), two faster (H128 Sq4 S2048 d64 11.6 -> 11.0).  One call, plain
+// -> shared out: B1 H16 Sq1 S2048 d128 12.2 -> 9.2 us, S8192 d64 36.3 -> 11.8, H32 S8192 d128 41.7 -> 19.3, H8 S65536 331 -> 61;
+// H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds already, 14.0 -> 15.9 and hence not.
 PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   using namespace fmha_i8_gfx950;
   PartPlan plan;

@@ -2,12 +2,12 @@
 // the time: for calls whose 256-row workgroups leave compute units idle, in their only wave or in their last.  Same
 // arithmetic, same BYTES for every row.
 //
-// Wavefronts w and w + 4 share a SIMD, as in the other kernel, and the same 32 query rows: w computes S^T, softmax and P of
+// Wavefronts w and w + 4 share a SIMD, as in the 256-row kernel, and the same 32 query rows: w computes S^T, softmax and P of
 // the even key blocks, w + 4 of the odd ones, and each runs GEMM 2 and the merge of ALL key blocks, in key order, for half of
 // the output columns.  What they exchange is P, 4 KB of LDS per key block.  The two halves of the workgroup work in
 // anti-phase: in tick T (between two barriers) the half that owns block T runs the matrix phase
 //     M(T) = publish P(T), GEMM 2 + merge of block T-1 (the other half's P) and of block T, GEMM 1 of block T+2
-// and the other half the softmax and packing of block T+1.  An M phase has the 32 MFMAs of the other kernel's: two key blocks times half
+// and the other half the softmax and packing of block T+1.  An M phase has the 32 MFMAs of the 256-row kernel's: two key blocks times half
 // the columns in GEMM 2.  The half in its softmax requests K and V of two ticks later and waits for them one phase on; the rings
 // hold three K and four V tiles.
 #pragma once
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   const int h = wave >> 2;  // half: owns the blocks of its parity
 
   int wg;
-  {  // XCD-aware placement, as in the other kernel
+  {  // XCD-aware placement, as in the 256-row kernel
     const int L = blockIdx.x, per = args.total_wgs / kXcds, rem = args.total_wgs % kXcds, x = L % kXcds;
     wg = x * per + (x < rem ? x : rem) + L / kXcds;
   }
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
     }
   }
 
-  // operand addresses (see the other kernel)
+  // operand addresses (see the 256-row kernel)
   int k_read_off[kDSteps];
 #pragma unroll
   for (int kk = 0; kk < kDSteps; ++kk) k_read_off[kk] = i32 * D + (((2 * kk + g) ^ k_swizzle<D>(i32)) << 4);
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   all_loads_landed();  // nothing may still be writing LDS when the wavefront ends
   if (!active) return;
 
-  // ---- epilogue (see the other kernel) -----------------------------------------------------------------------------
+  // ---- epilogue (see the 256-row kernel) -----------------------------------------------------------------------------
   const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
   const float corr = FASTACC ? (FULLP ? -kBaseFull * t_run : kBase * t_run) : 0.f;
   int w[kColTiles][4];

@@ -1,6 +1,6 @@
 // The attention kernel for calls that fill too few compute units with workgroups of 256 query rows: a handful of heads, a
 // chunk of a prefill, one new row per sequence.  Same arithmetic as fmha_i8_fwd_kernel (fmha_i8_kernel.hip) and the same
-// BYTES for every row: which of the two kernels serves a call is a question of speed alone.
+// BYTES for every row: which kernel serves a call (row_groups_of, part_plan_of) is a question of speed alone.
 //
 // A workgroup owns R groups of 32 query rows (R = 1 or 2) of one head and works on FOUR key blocks at a time, a "round":
 //   * wavefront (r, c) computes S^T, the block softmax and the quantised P^T of row group r and key block 4 i + c, so the
@@ -8,10 +8,10 @@
 //     wavefronts as there are row groups;
 //   * P^T goes through LDS to the four wavefronts of the row group, a quarter of what exchanging O would take, and each
 //     of them runs GEMM 2 and the online merge of all four key blocks, in key order, for ITS 32 output columns.  Every
-//     output element is thus merged by one wavefront, block after block, with the operations of the other kernel in the
+//     output element is thus merged by one wavefront, block after block, with the operations of the 256-row kernel in the
 //     same order - which no scheme that merges partial results of separate key ranges can do, since float addition is not
 //     associative.  (At head_dim 64 there are two column tiles: two wavefronts do each.)
-// K and V tiles go HBM -> LDS directly, as in the other kernel and with the same swizzles.  A call has more than one key
+// K and V tiles go HBM -> LDS directly, as in the 256-row kernel and with the same swizzles.  A call has more than one key
 // block (the host sees to it): a single one leaves three quarters of the wavefronts without a softmax.
 #pragma once
 
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const int u_out = c & (kDSteps - 1);  // output column tile of this wavefront
 
   int wg;
-  {  // XCD-aware placement, as in the other kernel
+  {  // XCD-aware placement, as in the 256-row kernel
     const int L = blockIdx.x, per = args.total_wgs / kXcds, rem = args.total_wgs % kXcds, x = L % kXcds;
     wg = x * per + (x < rem ? x : rem) + L / kXcds;
   }
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const long q_head_off = (long)bh * Sq * D;
   const int n_blocks = (S + BK - 1) / BK;
   const int first_round = PARTS ? qb * args.rounds_per_part : 0;
-  // A partly filled last block: the tile is fetched so that it ends with the last key (see the other kernel).
+  // A partly filled last block: the tile is fetched so that it ends with the last key (see the 256-row kernel).
   const int tail_kb = S % BK != 0 ? n_blocks - 1 : -1;
 
   // ---- tile loads --------------------------------------------------------------------------------------------------
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     for (int it = 0; it < kLoads; ++it) issue(first_round, 1, it, n_blocks - 1);
   }
 
-  // operand addresses (see the other kernel)
+  // operand addresses (see the 256-row kernel)
   int k_read_off[kDSteps];
 #pragma unroll
   for (int kk = 0; kk < kDSteps; ++kk) k_read_off[kk] = i32 * D + (((2 * kk + g) ^ k_swizzle<D>(i32)) << 4);
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   asm volatile("" : "+v"(base_c));
   if (BIAS) asm volatile("" : "+v"(base_s));
 
-  // ---- classification of the key blocks, by all wavefronts (the bits are those of the other kernel) -----------------
+  // ---- classification of the key blocks, by all wavefronts (the bits are those of the 256-row kernel) -----------------
   asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + (kEarlyV ? 2 : 1) * kLoads) : "memory");
   const int live_hi = classify_key_blocks<BK, kRowWaves>(mask_bytes, tail_bytes, mg, S, tid, lds_mask,
                                                          reinterpret_cast<unsigned char*>(lds_class4), keys_from, keys_to);
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   wait_loads(none);  // nothing may still be writing LDS when the wavefront ends (only possible when every key is masked)
   if (PARTS || !active || c >= kDSteps) return;
 
-  // ---- epilogue (see the other kernel) -----------------------------------------------------------------------------
+  // ---- epilogue (see the 256-row kernel) -----------------------------------------------------------------------------
   const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
   const float corr = FASTACC ? (FULLP ? -kBaseFull * t_run : kBase * t_run) : 0.f;
   int w[4];  // w[a]: output dims 32 u_out + 8a + 4g .. +3 of query row i32

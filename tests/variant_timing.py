@@ -10,6 +10,14 @@ no MFMA phase, no LDS operand reads, no tile loads, no LDS swizzle - so that wha
 their results are garbage on purpose, and only the build called `few` (the shipped kernel with fewer instantiations) and
 `no_swizzle` are checked against the shipped library here.  With a `trace_ticks` build the per-wavefront time stamps
 of the barriers are read back and summarised: how long a wavefront works between two barriers and how long it waits.
+
+    python tests/variant_timing.py --kernel-costs
+    python tests/variant_timing.py --shapes "1,16,2048,2048,128 1,16,1,8192,64"
+
+The first measures what the library's choice of kernels rests on, each kernel on half and on all of the CUs with one
+workgroup each, the second times
+(B, H, Sq, S, d) on every kernel that can serve it and on the library's own choice; both print tables and use the build
+called `routed`.
 """
 import argparse
 import ctypes as C
@@ -23,6 +31,88 @@ sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
 
+def events_us(torch, call, calls):
+    """Best of five bursts, at the settled clock."""
+    t0 = time.perf_counter()
+    while time.perf_counter() - t0 < 0.04:
+        for _ in range(20):
+            call()
+        torch.cuda.synchronize()
+    best = 1e30
+    for _ in range(5):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(calls):
+            call()
+        e1.record()
+        torch.cuda.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1e3 / calls)
+    return best
+
+
+def time_route(pkg, lib, routes, route, shape, calls=100):
+    """Microseconds per call, or None where the call does not have that route.  No masked key, uniform random bytes."""
+    import torch
+    B, H, Sq, S, d = shape
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    t = [torch.randint(-127, 128, (B, H, rows, d), generator=g, device="cuda", dtype=torch.int8) for rows in (Sq, S, S)]
+    t.append(torch.zeros((B, S), dtype=torch.int8, device="cuda"))
+    o = torch.empty_like(t[0])
+    desc = pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d)
+    args = [torch.cuda.current_stream().cuda_stream, pkg.FMHAParamI8(0.2, 3.0, 3.0, 1.0, 1.0), desc] + [x.data_ptr() for x in t] + [o.data_ptr(), 0]
+    lib.FMHAInferI8DebugRoute(route)
+    need = lib.FMHAInferI8CrossWorkspaceBytes(desc)
+    work = torch.empty(max(need, 16), dtype=torch.int8, device="cuda")
+    if route == routes.SHARED_OUT and need == 0:
+        return None
+    args += [work.data_ptr(), need]
+
+    def call():
+        if lib.FMHAInferI8CrossWithWorkspace(*args) != 0:
+            raise RuntimeError("call refused")
+
+    us = events_us(torch, call, calls)
+    lib.FMHAInferI8DebugRoute(routes.OWN_CHOICE)
+    return us
+
+
+def time_shapes(shapes):
+    import torch  # noqa: F401
+    import __graft_entry__ as g
+    import routes
+    pkg = g.load_package()
+    lib = routes.library(pkg)
+    names = list(routes.ROUTES)
+    print("| B, H, Sq, S, d | %s | key blocks shared out | the library's choice |" % " | ".join("%d rows" % r for r in names))
+    print("|" + "---|" * (len(names) + 3))
+    for shape in shapes:
+        us = [time_route(pkg, lib, routes, routes.ROUTES[r], shape) for r in names]
+        us += [time_route(pkg, lib, routes, route, shape) for route in (routes.SHARED_OUT, routes.OWN_CHOICE)]
+        print("| %s | %s |" % (", ".join(map(str, shape)), " | ".join("-" if u is None else "%.2f" % u for u in us)), flush=True)
+
+
+def kernel_costs():
+    """Time of a call against its key blocks, with one workgroup on half of the CUs and on each (8 or 16 heads of 16 workgroups)."""
+    import torch  # noqa: F401
+    import __graft_entry__ as g
+    import routes
+    pkg = g.load_package()
+    lib = routes.library(pkg)
+    keys = {64: (448, 960, 1984, 4032), 128: (512, 1024, 2048, 4096)}
+    print("| d | keys per block | query rows | workgroups | us at %s | start + step * rounds, us |" % " / ".join("%d or %d keys" % p for p in zip(keys[64], keys[128])))
+    print("|" + "---|" * 6)
+    for d in (64, 128):
+        for block in (64, 128):
+            for rows, route in routes.ROUTES.items():
+                for heads in (8, 16):
+                    us = [time_route(pkg, lib, routes, route, (1, heads, 16 * rows, s, d)) for s in keys[block]]
+                    rounds = [(s // block + 3) // 4 if rows <= 64 else s // block for s in keys[block]]
+                    step = (us[3] - us[0]) / (rounds[3] - rounds[0])
+                    print("| %d | %d | %d | %d | %s | %.2f + %.3f |" % (d, block, rows, 16 * heads, " / ".join("%.2f" % u for u in us),
+                                                                       us[0] - step * rounds[0], step), flush=True)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--lib", default=None, help="library to time (default: the shipped libfmha_i8.so)")
@@ -30,7 +120,13 @@ def main():
     ap.add_argument("--calls", type=int, default=1000)
     ap.add_argument("--preheat-ms", type=float, default=100.0)
     ap.add_argument("--compare", action="store_true", help="compare the output bytes with the shipped library's")
+    ap.add_argument("--kernel-costs", action="store_true", help="each kernel's time against the number of key blocks")
+    ap.add_argument("--shapes", default=None, help="\"B,H,Sq,S,d B,H,Sq,S,d ...\" on every kernel")
     args = ap.parse_args()
+    if args.kernel_costs:
+        return kernel_costs()
+    if args.shapes:
+        return time_shapes([tuple(int(x) for x in shape.split(",")) for shape in args.shapes.split()])
 
     import numpy as np
     import torch
