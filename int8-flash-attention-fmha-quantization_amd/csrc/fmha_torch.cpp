@@ -70,7 +70,13 @@ hipStream_t stream_of(PyObject* o, const at::Device& device) {
   return static_cast<hipStream_t>(p);
 }
 // The null stream is that of the current device: a call makes its tensors' device current, and the caller's again when it ends.
-using OnDevice = c10::hip::HIPGuard;
+// (Where it is current already the guard, whose end asks the runtime for the device's state, costs a call 0.1 us.)
+struct OnDevice {
+  std::optional<c10::hip::HIPGuard> guard;
+  explicit OnDevice(c10::DeviceIndex index) {
+    if (c10::hip::current_device() != index) guard.emplace(index);
+  }
+};
 // Memory of torch's caching allocator, ordered by the stream that is current on the device.
 at::Tensor empty(c10::IntArrayRef sizes, at::ScalarType type, const at::Device& device) {
   return at::detail::empty_cuda(sizes, type, device, std::nullopt);
