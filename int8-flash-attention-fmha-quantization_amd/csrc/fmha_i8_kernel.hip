@@ -193,8 +193,37 @@ __device__ __forceinline__ float half_sum(float x) {
 // bit flipped) and the missing 128 * sum_j v[j][c] per key block and output column goes in as the START VALUE of the
 // accumulators: wavefronts 4..7 sum the columns of every V tile one phase before its GEMM 2 (v_dot4 on the transposed
 // operand reads), leave kBaseBitsFull + 128 * sum in LDS, and every wavefront reads its C operand from there.
+// The start values of GEMM 1 for a 32-key tile with masked keys (bit j of `word`: key j), by one matrix instruction: the outer
+// product of -1 per masked key and a power of two, on top of the usual start value, read as bits.  Per masked key that is
+// 0xFF000000 (-2^127; with the usual start value beside it nothing changes) or, where the scores are converted, 0xC0000000 (-2.0f,
+// the integer -2^30); the others keep theirs exactly.
+// One v_cndmask per score on lane masks that the scalar unit built from `word` - 64 vector and 128 scalar instructions per wavefront
+// and block where this takes 8 and 4 MFMAs - measured, with a fifth of the keys masked: B4 H16 S1024 d128 24.5 -> 22.8 us (no
+// mask: 21.8), the same with 255 steps and 1000 keys 27.3 -> 26.3, B16 H16 S2048 d64 242 -> 226, converted scores 275 -> 249.
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <bool BIAS>
+struct MaskedUnits {
+  int minus_one = 0xBF80, power = BIAS ? 0x7F00 : 0x4000;  // bfloat16 -1, and 2^127 or 2
+  // (opaque, or the compiler holds them in registers throughout the key loop)
+  __device__ __forceinline__ MaskedUnits() { asm volatile("" : "+v"(minus_one), "+v"(power)); }
+};
+template <bool BIAS>
+__device__ __forceinline__ v16i masked_start(unsigned word, const MaskedUnits<BIAS>& unit, const v16i& base) {
+  const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // (a: -1 in the k-slots of lanes 0..31 alone)
+  const v2i a = {__builtin_amdgcn_inverse_ballot_w64(word) ? unit.minus_one : 0, 0}, b = {unit.power, 0};
+  return __builtin_bit_cast(v16i, __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(v4s, a), __builtin_bit_cast(v4s, b),
+                                                                          BIAS ? __builtin_bit_cast(v16f, base) : zero, 0, 0, 0));
+}
+
+// Wavefronts per SIMD to leave registers for: two of them are this workgroup's.  The converting d = 64 kernel stays below 168
+// registers, with which a wavefront of the next workgroup starts as soon as one of this has ended (B16 H16 S2048: 214 us, 219 with 172).
+template <int D, bool BIAS>
+constexpr int waves_per_simd() { return D == 64 && !BIAS ? 3 : 2; }
+
 template <int D, int BK, bool BIAS, bool FASTACC, bool RAGGED, bool FULLP>
-__global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelArgs args) {
+__global__ __launch_bounds__(kThreads, (waves_per_simd<D, BIAS>())) void fmha_i8_fwd_kernel(const KernelArgs args) {
   constexpr int kChunks = D / 16;                     // 16-byte chunks per row
   constexpr int kTileBytes = BK * D;                  // one K or V tile
   constexpr int kWaves = kThreads / 64;
@@ -367,10 +396,8 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
   // inside a function.  The d = 64 kernel is sensitive to where the MFMAs of GEMM 1 and the row-maximum instructions
   // behind them fall (+12 % when they straddle), so it pins those, the scale fmas and the P packing to aligned
   // addresses; the d = 128 kernel measures the same either way (+-0.3 %) in its loop without masked keys and is left
-  // alone there (pinning everything costs it 0.4 %).  Its loop for blocks WITH masked keys is sensitive (up to 9 % between
-  // two placements, B1 H4 S8192 with a scattered mask), so that loop pins the same groups, and GEMM 1 with start values
-  // pins each tile's run of v_cndmask and its MFMAs at either head size: 1.5 to 3 % faster and 3 % left between
-  // placements.
+  // alone there (pinning everything costs it 0.4 %).  Its loop for blocks WITH masked keys was more sensitive (up to 9 % between
+  // two placements, B1 H4 S8192 with a scattered mask), so that loop pins the same groups at either head size.
   auto align8 = [&](bool also_at_128 = false) { if (D == 64 || also_at_128) asm volatile(".p2align 3" ::: "memory"); };
   // The steady-state loops start at a fixed distance from a 64-byte boundary, so that what is measured for them does
   // not change with the code in front of them: at d = 64 the loop of wavefronts 0..3 runs 12 % slower when it starts
@@ -658,9 +685,7 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
   // the MFMAs add to it - read as a float on the BIAS variant, 0xFF000000 + S is below -2^126 for every |S| < 2^21;
   // where the scores are converted, -2^30 + S times that variant's c2 >= 2.7e-4 is an exponent below -2.9e5 - so that
   // the row maximum taken behind the MFMAs and the whole softmax need no further look at the mask.  The start values
-  // are one v_cndmask per score on wave-uniform lane masks - lanes 0..31 hold key 8a+bb of a tile, lanes 32..63 key
-  // 8a+4+bb, so the scalar unit builds them from the block's mask bits - written into the accumulator registers
-  // themselves, tile by tile, in front of the tile's MFMAs.
+  // of a tile come from one matrix instruction (masked_start).
   auto phase_gemm1 = [&](int kb, v16i (&acc)[kKeyTiles], int (&mx)[2], bool masked = false) __attribute__((always_inline)) {
     if constexpr (test_build::kNoMfma) {
 #pragma unroll
@@ -679,52 +704,16 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
       return operand;
     };
     unsigned mw[kKeyTiles];  // masked: the block's mask bits, bit j of word t <-> key 32 t + j of the block
-    int gone = BIAS ? (int)0xFF000000 : -(1 << 30);
+    auto start = [&](int t) __attribute__((always_inline)) {
+      const MaskedUnits<BIAS> units;
+      acc[t] = masked_start(mw[t], units, base_s);
+    };
     if (masked) {
-      asm volatile("" : "+v"(gone));  // a register operand
 #pragma unroll
       for (int t = 0; t < kKeyTiles; ++t)
         mw[t] = (RAGGED && kb == tail_kb) ? tail_word[t]
                                           : (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[kb * kKeyTiles + t]);
-    }
-    auto start_piece = [&](int t, int first, int count) __attribute__((always_inline)) {  // start values of registers first .. first+count-1 of tile t
-#pragma unroll
-      for (int r = first; r < first + count; ++r) {
-        const int key = 8 * (r / 4) + (r % 4);
-        const unsigned lo = (unsigned)(((int)(mw[t] << (31 - key))) >> 31), hi = (unsigned)(((int)(mw[t] << (27 - key))) >> 31);
-        const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
-        int e;
-        if (BIAS) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(e) : "v"(base_s[0]), "v"(gone), "s"(lanes));
-        else asm volatile("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(e) : "v"(gone), "s"(lanes));
-        acc[t][r] = e;
-      }
-    };
-    if (masked) {
-      // One operand buffer and no read-ahead: the start values of a tile are written while its operand reads are in
-      // flight, and the registers that the read-ahead would take are what the accumulators of the next tile, live one
-      // chain early here, need (with both, the d = 128 kernel spills).
-#pragma unroll
-      for (int t = 0; t < kKeyTiles; ++t) {
-#pragma unroll
-        for (int kk = 0; kk < kDSteps; ++kk) ka[0][kk] = read_k(k_read_off[kk] + 32 * t * D);
-        align8(true);
-        start_piece(t, 0, 16);
-        asm volatile("s_nop 1" ::: "memory");  // (the compiler does not know that the statements above wrote registers an MFMA reads)
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kk = 0; kk < kDSteps; ++kk) {
-          align8(true);
-          acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[0][kk], qreg[kk], acc[t], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          if (t >= 1) {
-#pragma unroll
-            for (int j = kk * 4 / kDSteps; j < (kk + 1) * 4 / kDSteps; ++j) tile_max_piece(acc[t - 1], mx, t == 1, j);
-            asm volatile("" : "+v"(mx[0]), "+v"(mx[1]));
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      }
-      return;
+      start(0);
     }
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk) ka[0][kk] = read_k(k_read_off[kk]);
@@ -738,10 +727,14 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kk = 0; kk < kDSteps; ++kk) {
-        align8();
+        align8(masked);
         acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[t & 1][kk], qreg[kk],
-                                                       kk == 0 ? (BIAS ? base_s : zero_c) : acc[t], 0, 0, 0);
+                                                       kk == 0 && !masked ? (BIAS ? base_s : zero_c) : acc[t], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        if (masked && kk == kDSteps - 2 && t + 1 < kKeyTiles) {  // (one MFMA ahead: nothing waits for it)
+          start(t + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
         if (t >= 1) {
 #pragma unroll
           for (int j = kk * 4 / kDSteps; j < (kk + 1) * 4 / kDSteps; ++j) tile_max_piece(acc[t - 1], mx, t == 1, j);
@@ -780,6 +773,24 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
       // off = top*c2 rounded; p' = exp2(s*c2 - off) = p * 2^(resid) with one row-wide resid below 1 ulp of off, and the
       // block maximum that is consistent with p' is off itself (minus the constant kBase*c2 when BIAS).
       float off = top * c2;
+      if (split && !BIAS) {
+        // All conversions in front of all fmas: they do not wait for the row maximum, and mixed with the fmas, as the compiler
+        // schedules them now and then, they cost 6 to 18 % of the whole kernel (d = 64, B16 H16 S2048: 228 to 257 us against 215).
+        // Making the exponent offset depend on conversions of every tile says so without holding any of them behind a barrier.
+        float some[28] = {};
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const float f = (float)acc[t][r];
+            acc[t][r] = __float_as_int(f);
+            if (r % 2 == 1 && r >= 3) some[7 * t + r / 2 - 1] = f;
+          }
+        asm("" : "+v"(off) : "v"(some[0]), "v"(some[1]), "v"(some[2]), "v"(some[3]), "v"(some[4]), "v"(some[5]), "v"(some[6]), "v"(some[7]),
+            "v"(some[8]), "v"(some[9]), "v"(some[10]), "v"(some[11]), "v"(some[12]), "v"(some[13]), "v"(some[14]), "v"(some[15]), "v"(some[16]),
+            "v"(some[17]), "v"(some[18]), "v"(some[19]), "v"(some[20]), "v"(some[21]), "v"(some[22]), "v"(some[23]), "v"(some[24]), "v"(some[25]),
+            "v"(some[26]), "v"(some[27]));
+      }
       // Where the scores are converted, c2 is large and |off| can reach 10^5 and more: the rounding of this product and
       // of offq below then amounts to a percent of p, and a p above 1 by 0.4 % quantises to -129, whose low byte is
       // +127.  Two units in the last place upwards make off an upper bound of the exact product: every p is at most 1,
@@ -805,7 +816,7 @@ __global__ __launch_bounds__(kThreads, 2) void fmha_i8_fwd_kernel(const KernelAr
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             xs[qd][j] = test_build::kNoScaleRun ? __int_as_float(acc[qd / 4][4 * (qd % 4) + j])
-                                                : __builtin_fmaf(sf(qd / 4, 4 * (qd % 4) + j), c2, -offq);
+                                                : __builtin_fmaf(__int_as_float(acc[qd / 4][4 * (qd % 4) + j]), c2, -offq);
 #pragma unroll
         for (int qd = 0; qd < kQuads; ++qd) asm volatile("" : "+v"(xs[qd][0]), "+v"(xs[qd][1]), "+v"(xs[qd][2]), "+v"(xs[qd][3]));
         __builtin_amdgcn_sched_barrier(0);

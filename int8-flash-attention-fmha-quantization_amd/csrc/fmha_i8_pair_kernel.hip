@@ -183,11 +183,10 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   };
   auto gemm1 = [&](int kb, int stage, auto masked_t) __attribute__((always_inline)) {
     constexpr bool kMasked = decltype(masked_t)::value;
+    unsigned mw[kKeyTiles];
     if constexpr (kMasked) {
-      unsigned mw[kKeyTiles];
       mask_words_of<BK>(mw, lds_mask, kb, tail_kb, S);
-      masked_start_values<BIAS>(acc, mw, base_s);
-      __builtin_amdgcn_sched_barrier(0);
+      acc[0] = masked_start(mw[0], MaskedUnits<BIAS>(), base_s);
     }
     mx[0] = mx[1] = (int)0x80000000;
 #pragma unroll
@@ -198,6 +197,11 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       for (int kk = 0; kk < kDSteps; ++kk) {
         acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[t % 3][kk], qreg[kk], (kk == 0 && !kMasked) ? base_s : acc[t], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kMasked)
+          if (kk == kDSteps - 2 && t + 1 < kKeyTiles) {
+            acc[t + 1] = masked_start(mw[t + 1], MaskedUnits<BIAS>(), base_s);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         if (t >= 1) {
 #pragma unroll
           for (int j = kk * 4 / kDSteps; j < (kk + 1) * 4 / kDSteps; ++j) tile_max_piece(acc[t - 1], j);

@@ -101,25 +101,6 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
   return live_hi;
 }
 
-// Start values of the GEMM 1 accumulators of a block with masked keys (see fmha_i8_fwd_kernel): `gone` loses every maximum
-// and its exponential is exactly 0.  mw: the block's mask bits, wave-uniform.
-template <bool BIAS, int KEY_TILES>
-__device__ __forceinline__ void masked_start_values(v16i (&acc)[KEY_TILES], const unsigned (&mw)[KEY_TILES], const v16i& base) {
-  int gone = BIAS ? (int)0xFF000000 : -(1 << 30);
-  asm volatile("" : "+v"(gone));
-#pragma unroll
-  for (int t = 0; t < KEY_TILES; ++t)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int key = 8 * (e / 4) + (e % 4);
-      const unsigned lo = (unsigned)(((int)(mw[t] << (31 - key))) >> 31), hi = (unsigned)(((int)(mw[t] << (27 - key))) >> 31);
-      const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
-      int x;
-      asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(base[e]), "v"(gone), "s"(lanes));
-      acc[t][e] = x;
-    }
-  asm volatile("s_nop 1" ::: "memory");  // (the compiler does not know that these statements wrote registers an MFMA reads)
-}
 // The mask bits of block kb; tail_kb: the partly filled last block, whose tile ends with the last key - bit j of word t is key
 // S - BK + 32 t + j, the keys it repeats count as masked.
 template <int BK>
@@ -337,11 +318,10 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     };
     auto gemm1 = [&](auto masked_t) __attribute__((always_inline)) {
       constexpr bool kMasked = decltype(masked_t)::value;
+      unsigned mw[kKeyTiles];
       if constexpr (kMasked) {
-        unsigned mw[kKeyTiles];
         mask_words_of<BK>(mw, lds_mask, kb, tail_kb, S);
-        masked_start_values<BIAS>(acc, mw, base_s);
-        __builtin_amdgcn_sched_barrier(0);
+        acc[0] = masked_start(mw[0], MaskedUnits<BIAS>(), base_s);
       }
       // Operand reads run two key tiles ahead of the MFMAs, held there by the fences: left alone, the compiler reads each
       // operand right in front of its MFMA and the wavefront waits out the LDS latency sixteen times.
@@ -360,6 +340,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         for (int kk = 0; kk < kDSteps; ++kk) {
           acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ka[t % 3][kk], qreg[kk], (kk == 0 && !kMasked) ? base_s : acc[t], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
+          if constexpr (kMasked)
+            if (kk == kDSteps - 2 && t + 1 < kKeyTiles) acc[t + 1] = masked_start(mw[t + 1], MaskedUnits<BIAS>(), base_s);
           between(t * kDSteps + kk, kKeyTiles * kDSteps);
           if (t >= 1) tile_max(acc[t - 1], kk);
           __builtin_amdgcn_sched_barrier(0);
