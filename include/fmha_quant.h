@@ -47,8 +47,9 @@ int FMHADequantizeI8BF16(hipStream_t stream, const int8_t* x, long long n, float
 /* Abs-max and quantisation of up to three tensors of one type in one call - the Q, K and V of an attention call
  * (test_fmha_i8.cpp:91-110 does them one after the other) - with the results of the two calls above for each of them.
  * The maxima of the workgroups go through `workspace` (FMHA_QUANT_WORKSPACE_FLOATS floats of device memory, contents
- * undefined before and after) instead of an atomic on one address, so a call is two launches, or one where every
- * tensor fits one workgroup's registers.  amax_out: `count` floats of device memory.
+ * undefined before and after) instead of an atomic on one address.  A call is one launch where the chip's registers and
+ * LDS hold the tensors (104 MB together), the stream is not being captured and the workspace is 8-byte aligned, else two.
+ * amax_out: `count` floats of device memory.
  * note: NULL, or `count` 8-byte words of pinned host memory that the device can write: word i receives
  * (ticket << 32) | bits of amax[i] in one store, as soon as that maximum is known and before the int8 values are all
  * written, so that a host that needs the maxima (FMHAParamI8 takes them by value) can go on while the device does. */
