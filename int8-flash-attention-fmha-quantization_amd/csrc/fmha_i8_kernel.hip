@@ -218,12 +218,13 @@ __device__ __forceinline__ v16i masked_start(unsigned word, const MaskedUnits<BI
 }
 
 // Wavefronts per SIMD to leave registers for: two of them are this workgroup's.  The converting d = 64 kernel stays below 168
-// registers, with which a wavefront of the next workgroup starts as soon as one of this has ended (B16 H16 S2048: 214 us, 219 with 172).
-template <int D, bool BIAS>
-constexpr int waves_per_simd() { return D == 64 && !BIAS ? 3 : 2; }
+// registers, with which a wavefront of the next workgroup starts as soon as one of this has ended (B16 H16 S2048: 214 us, 219 with
+// 172), and with blocks of 64 keys below 128, with which two workgroups share a CU (B4 H64 S960: 59 us, 65 with 132).
+template <int D, int BK, bool BIAS>
+constexpr int waves_per_simd() { return D == 64 && !BIAS ? (BK == kBlockKSmall ? 4 : 3) : 2; }
 
 template <int D, int BK, bool BIAS, bool FASTACC, bool RAGGED, bool FULLP>
-__global__ __launch_bounds__(kThreads, (waves_per_simd<D, BIAS>())) void fmha_i8_fwd_kernel(const KernelArgs args) {
+__global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmha_i8_fwd_kernel(const KernelArgs args) {
   constexpr int kChunks = D / 16;                     // 16-byte chunks per row
   constexpr int kTileBytes = BK * D;                  // one K or V tile
   constexpr int kWaves = kThreads / 64;
