@@ -91,6 +91,15 @@ hipError_t launch_variant(Variant var, dim3 grid, dim3 block, hipStream_t stream
   return launch_variant3<D, BK, false>(var, grid, block, stream, args);
 }
 
+// The kernel of 256-row workgroups: args.total_wgs of them.
+hipError_t launch_wide(int head_dim, int block_keys, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& args) {
+  using fmha_i8_gfx950::kBlockK, fmha_i8_gfx950::kBlockKSmall;
+  const dim3 grid((unsigned)args.total_wgs), block(fmha_i8_gfx950::kThreads);
+  if (head_dim == 128)
+    return block_keys == kBlockK ? launch_variant<128, kBlockK>(var, grid, block, stream, args) : launch_variant<128, kBlockKSmall>(var, grid, block, stream, args);
+  return block_keys == kBlockK ? launch_variant<64, kBlockK>(var, grid, block, stream, args) : launch_variant<64, kBlockKSmall>(var, grid, block, stream, args);
+}
+
 #ifndef FMHA_NO_SPLIT_KERNEL
 template <int D, int BK, int R>
 const void* split_kernel(Variant var) {
@@ -147,13 +156,19 @@ hipError_t launch_parts(const PartPlan& plan, Variant var, hipStream_t stream, c
   void* merge_args[] = {&merge};
   return hipLaunchKernel(n_blocks <= 16 ? reinterpret_cast<const void*>(&fmha_i8_merge_kernel<16>) : reinterpret_cast<const void*>(&fmha_i8_merge_kernel<32>), dim3((unsigned)(D / (2 * row_lanes)), (unsigned)heads), dim3(64), merge_args, 0, stream);
 }
+// A part of a call: rows first_row .. end_row - 1 of `heads` heads from first_head on, by one kernel.
+struct Piece {
+  int row_groups, first_head, heads, first_row, end_row;
+};
 template <int D, int BK>
-hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
+hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
   using namespace fmha_i8_gfx950;
   SplitKernelArgs args{of_call};
-  const int heads = args.total_wgs / args.q_blocks, rows = 32 * row_groups;
-  args.q_blocks = (args.seq_q + rows - 1) / rows;
-  args.total_wgs = heads * args.q_blocks;
+  const int row_groups = piece.row_groups, rows = 32 * row_groups;
+  args.q_blocks = (piece.end_row - piece.first_row + rows - 1) / rows;
+  args.total_wgs = piece.heads * args.q_blocks;
+  args.first_head = piece.first_head;
+  args.first_row = piece.first_row;
   args.q_blocks_divisor = make_divisor(args.q_blocks);
   args.head_num_divisor = make_divisor(args.head_num);
   void* kernel_args[] = {&args};
@@ -161,53 +176,87 @@ hipError_t launch_split(int row_groups, Variant var, hipStream_t stream, const f
   return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 ? 256 : 512), kernel_args, 0, stream);
 }
 // What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
-// split kernel.  Microseconds * 100 beyond the launch (2.8 to 3.1 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
-// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs).  For blocks of 128 keys a new measurement
-// gives them to 4 %; for blocks of 64 they are right to 5 % at 448 keys and up to 19 % high per further block.  With all CUs at work
-// the first two take up to 39 and 16 % longer per block (the shader clock drops), where the choice is clear anyway.
+// split kernel.  Microseconds * 100 beyond the launch (2.9 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
+// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs); measurements differ by 4 %.
+// With all CUs at work the first two take up to 34 and 11 % longer per block (the shader clock drops).
 struct KernelCost {
   int row_groups, keys_per_round;
   struct { int start, step; } cost[2][2];
 };
-constexpr KernelCost kKernelCosts[] = {{0, 1, {{{0, 95}, {95, 128}}, {{160, 112}, {250, 162}}}},
-                                       {4, 1, {{{110, 65}, {170, 97}}, {{180, 89}, {300, 116}}}},
-                                       {2, 4, {{{0, 208}, {45, 312}}, {{60, 220}, {140, 332}}}},
-                                       {1, 4, {{{40, 130}, {30, 213}}, {{65, 160}, {95, 243}}}}};
+constexpr KernelCost kKernelCosts[] = {{0, 1, {{{72, 80}, {95, 128}}, {{200, 99}, {250, 162}}}},
+                                       {4, 1, {{{137, 62}, {170, 97}}, {{225, 83}, {300, 116}}}},
+                                       {2, 4, {{{39, 183}, {45, 312}}, {{108, 199}, {140, 332}}}},
+                                       {1, 4, {{{23, 141}, {30, 213}}, {{73, 159}, {95, 243}}}}};
 constexpr KernelCost kOneGroupCost = kKernelCosts[3];
 static_assert(kOneGroupCost.row_groups == 1, "");
-// Groups of 32 query rows per workgroup of the kernel that serves a call: 1 or 2 (fmha_i8_split_kernel), 4
+// Groups of 32 query rows per workgroup of the kernel that serves `rows` query rows of `heads` heads: 1 or 2 (fmha_i8_split_kernel), 4
 // (fmha_i8_pair_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
 // Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (cost of one).  What the constants
 // order is far apart nearly everywhere - d128, S2048: H4 31.0 us in 256-row workgroups, 24.4 in those of four groups, 17.6 of
 // two, 13.4 of one; H8 31.3, 24.6, 17.9, 25.8; H16 31.7, 26.2, 34.5, 50.3; H24 33.9, 48.9, 50.7, 74.6 - so that a few percent of
 // error only shift the boundary between equals.
-int row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys, long long* cost_of = nullptr) {
-  if (a.seq_len_kv <= block_keys) return 0;
-  if (fmha_i8_gfx950::test_build::forced_route() >= 0) return fmha_i8_gfx950::test_build::forced_route();
-  const int d = a.head_dim == 128, k = block_keys == fmha_i8_gfx950::kBlockK;
-  const long long heads = (long long)a.batch_num * a.head_num;
-  const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
-  int best = 0;
-  long long least = -1;
+struct Choice {
+  int row_groups;
+  long long cost;  // hundredths of a microsecond
+};
+constexpr int kComputeUnits = 256;
+int cost_of_workgroup(const KernelCost& kernel, int head_dim, int blocks, int block_keys) {
+  const auto& c = kernel.cost[head_dim == 128][block_keys == fmha_i8_gfx950::kBlockK];
+  return c.start + c.step * ((blocks + kernel.keys_per_round - 1) / kernel.keys_per_round);
+}
+int rows_of(const KernelCost& kernel) { return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups; }
+Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
+  Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
     // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
     // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 13.9 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with
     // 16 heads 13.1 and 12.6; d64: 11.7 either way).  Its step is one group's less a little, so that it is taken.
-    const bool helper = a.seq_len_q <= 32 && kernel.row_groups == 2;
-    if (helper && !(d && k)) continue;
-    const int rows = kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups;
-    const auto& c = kernel.cost[d][k];
+    const bool helper = rows <= 32 && kernel.row_groups == 2;
+    if (helper && !(head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK)) continue;
     const int rounds = (blocks + kernel.keys_per_round - 1) / kernel.keys_per_round;
-    const long long per_cu = (heads * ((a.seq_len_q + rows - 1) / rows) + 255) / 256;
-    const long long cost = per_cu * (helper ? 95 + 240 * rounds : c.start + c.step * rounds);
-    if (least < 0 || cost < least) {
-      least = cost;
-      best = kernel.row_groups;
-    }
+    const long long per_cu = (heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)) + kComputeUnits - 1) / kComputeUnits;
+    const long long cost = per_cu * (helper ? 95 + 240 * rounds : cost_of_workgroup(kernel, head_dim, blocks, block_keys));
+    if (best.cost < 0 || cost < best.cost) best = {kernel.row_groups, cost};
   }
-  if (cost_of != nullptr) *cost_of = least;
   return best;
+}
+Choice row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
+  if (a.seq_len_kv <= block_keys) return {0, -1};
+  if (fmha_i8_gfx950::test_build::forced_route() >= 0) return {fmha_i8_gfx950::test_build::forced_route(), -1};
+  return cheapest_kernel((long long)a.batch_num * a.head_num, a.seq_len_q, a.head_dim, (a.seq_len_kv + block_keys - 1) / block_keys, block_keys);
+}
+// The launches of a call: one, or two where large workgroups would leave most compute units idle in their last wave, or in the last
+// rows of every head.  The first launch then takes as many heads, or as many rows of every head, as make full waves of workgroups of 256
+// or 128 rows, the second one the rest in smaller ones.  A second launch costs 2.9 us, and 5 % are left to the model's error.
+int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[2]) {
+  const int heads = a.batch_num * a.head_num, rows = a.seq_len_q, blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
+  const Choice whole = row_groups_of(a, block_keys);
+  pieces[0] = {whole.row_groups, 0, heads, 0, rows};
+  if (whole.cost < 0 || rows <= 32) return 1;
+  constexpr long long kLaunch = 290;
+  long long least = whole.cost * 19 / 20;
+  int count = 1;
+  auto consider = [&](const KernelCost& kernel, int first_heads, int first_rows) {
+    const bool by_heads = first_rows == rows;
+    const int rest_heads = by_heads ? heads - first_heads : heads, rest_rows = by_heads ? rows : rows - first_rows;
+    if (first_heads <= 0 || first_rows <= 0 || rest_heads <= 0 || rest_rows <= 0) return;
+    const long long wgs = (long long)first_heads * ((first_rows + rows_of(kernel) - 1) / rows_of(kernel));
+    const Choice rest = cheapest_kernel(rest_heads, rest_rows, a.head_dim, blocks, block_keys);
+    const long long cost = (wgs + kComputeUnits - 1) / kComputeUnits * cost_of_workgroup(kernel, a.head_dim, blocks, block_keys) + kLaunch + rest.cost;
+    if (rest.row_groups == 0 || cost >= least) return;
+    least = cost;
+    count = 2;
+    pieces[0] = {kernel.row_groups, 0, first_heads, 0, first_rows};
+    pieces[1] = {rest.row_groups, heads - rest_heads, rest_heads, rows - rest_rows, rows};
+  };
+  for (const KernelCost& kernel : kKernelCosts) {
+    if (kernel.row_groups != 0 && kernel.row_groups != 4) continue;
+    const long long per_head = (rows + rows_of(kernel) - 1) / rows_of(kernel), full_waves = heads * per_head / kComputeUnits;
+    consider(kernel, (int)(full_waves * kComputeUnits / per_head), rows);
+    consider(kernel, heads, rows / rows_of(kernel) * rows_of(kernel));
+  }
+  return count;
 }
 // Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for, by the cost
 // table above (start, step of one row group), but no faster than the memory (62 KB in a hundredth of a microsecond, on both
@@ -227,8 +276,7 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
   const auto& c = kOneGroupCost.cost[a.head_dim == 128][block_keys == kBlockK];
-  long long least = 0;
-  row_groups_of(a, block_keys, &least);
+  long long least = row_groups_of(a, block_keys).cost;
   least = (least > memory ? least : memory) * 20 / 21;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
@@ -281,7 +329,7 @@ int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescript
   args.wide = wide;
   args.wide_amax = p.o_amax;
   args.wide_is_bf16 = wide_is_bf16;
-  const dim3 grid((unsigned)args.total_wgs), block(fmha_i8_gfx950::kThreads);
+  args.first_head = args.first_row = 0;
   // The accumulators of Q.K^T can be read as floats without a convert when they start at the bit pattern of a float;
   // the price is that the exponent offset (start value*2^26 + S)*c2 is then rounded on a coarser float grid.  Take that
   // path only while the offset stays below 2^12, i.e. while the rounding moves a whole row by less than 2^-13 in log2.
@@ -312,23 +360,25 @@ int launch(hipStream_t stream, const FMHAParamI8& p, const FMHACrossAttnDescript
       return err == hipSuccess ? FMHA_I8_OK : FMHA_I8_ERR_HIP_BASE + (int)err;
     }
   }
-  if (const int row_groups = row_groups_of(a, block_keys)) {
-    if (a.head_dim == 128)
-      err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<128, fmha_i8_gfx950::kBlockK>(row_groups, var, stream, args)
-                                                  : launch_split<128, fmha_i8_gfx950::kBlockKSmall>(row_groups, var, stream, args);
-    else
-      err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<64, fmha_i8_gfx950::kBlockK>(row_groups, var, stream, args)
-                                                  : launch_split<64, fmha_i8_gfx950::kBlockKSmall>(row_groups, var, stream, args);
-    return err == hipSuccess ? FMHA_I8_OK : FMHA_I8_ERR_HIP_BASE + (int)err;
+  Piece pieces[2];
+  const int count = pieces_of(a, block_keys, pieces);
+  err = hipSuccess;
+  for (int i = 0; i < count && err == hipSuccess; ++i) {
+    if (pieces[i].row_groups == 0) {
+      args.q_blocks = (pieces[i].end_row + fmha_i8_gfx950::kBlockQ - 1) / fmha_i8_gfx950::kBlockQ;
+      args.total_wgs = pieces[i].heads * args.q_blocks;
+      err = launch_wide(a.head_dim, block_keys, var, stream, args);
+    } else if (a.head_dim == 128) {
+      err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<128, fmha_i8_gfx950::kBlockK>(pieces[i], var, stream, args)
+                                                  : launch_split<128, fmha_i8_gfx950::kBlockKSmall>(pieces[i], var, stream, args);
+    } else {
+      err = block_keys == fmha_i8_gfx950::kBlockK ? launch_split<64, fmha_i8_gfx950::kBlockK>(pieces[i], var, stream, args)
+                                                  : launch_split<64, fmha_i8_gfx950::kBlockKSmall>(pieces[i], var, stream, args);
+    }
   }
+#else
+  err = launch_wide(a.head_dim, block_keys, var, stream, args);
 #endif
-  if (a.head_dim == 128) {
-    if (block_keys == fmha_i8_gfx950::kBlockK) err = launch_variant<128, fmha_i8_gfx950::kBlockK>(var, grid, block, stream, args);
-    else err = launch_variant<128, fmha_i8_gfx950::kBlockKSmall>(var, grid, block, stream, args);
-  } else {
-    if (block_keys == fmha_i8_gfx950::kBlockK) err = launch_variant<64, fmha_i8_gfx950::kBlockK>(var, grid, block, stream, args);
-    else err = launch_variant<64, fmha_i8_gfx950::kBlockKSmall>(var, grid, block, stream, args);
-  }
   return err == hipSuccess ? FMHA_I8_OK : FMHA_I8_ERR_HIP_BASE + (int)err;
 }
 
@@ -426,6 +476,14 @@ int FMHAInferI8DebugOutOfBounds(void) {
 #ifdef FMHA_FORCED_ROUTE
 // Test build only: the kernel that serves the calls from here on (see the flag list of the test builds).
 void FMHAInferI8DebugRoute(int route) { fmha_i8_gfx950::test_build::g_route = route; }
+// Test build only: how many launches serve a call of this shape, and the heads and the rows of the first one.
+int FMHAInferI8DebugLaunches(FMHACrossAttnDescriptor desc, int* first_heads, int* first_rows) {
+  Piece pieces[2];
+  const int count = pieces_of(desc, block_keys_of(desc.seq_len_kv), pieces);
+  *first_heads = pieces[0].heads;
+  *first_rows = pieces[0].end_row;
+  return count;
+}
 #endif
 
 #ifdef FMHA_TRACE_TICKS

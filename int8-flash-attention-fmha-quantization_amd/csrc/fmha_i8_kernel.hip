@@ -113,6 +113,7 @@ struct KernelArgs {
   void* wide;       // the de-quantised output beside o, in the same layout, or null
   float wide_amax;  // o_amax
   int wide_is_bf16; // bfloat16, else float
+  int first_head, first_row;  // of this launch, for the kernels of smaller workgroups (see pieces_of in the launch code), else 0
 };
 
 // The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8), where the caller wants it: in
@@ -120,7 +121,7 @@ struct KernelArgs {
 template <int D, int WORDS>
 __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, const int (&w)[WORDS]) {
   if (args.wide == nullptr) return;
-  if (kCheckBounds && !fmha_in_bounds(at >= 0 && at + 4 * WORDS <= (long)args.total_wgs / args.q_blocks * args.seq_q * D)) return;
+  if (kCheckBounds && !fmha_in_bounds(at >= 0 && at + 4 * WORDS <= ((long)args.total_wgs / args.q_blocks + args.first_head) * args.seq_q * D)) return;
   auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
   if (args.wide_is_bf16) {
     unsigned short* p = static_cast<unsigned short*>(args.wide) + at;

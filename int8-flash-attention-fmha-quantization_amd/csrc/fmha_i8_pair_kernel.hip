@@ -48,8 +48,8 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
     const int L = blockIdx.x, per = args.total_wgs / kXcds, rem = args.total_wgs % kXcds, x = L % kXcds;
     wg = x * per + (x < rem ? x : rem) + L / kXcds;
   }
-  const int bh = divide(wg, args.q_blocks_divisor);
-  const int qb = wg - bh * args.q_blocks;
+  const int bh_here = divide(wg, args.q_blocks_divisor), bh = bh_here + args.first_head;
+  const int qb = wg - bh_here * args.q_blocks;
   const int b = divide(bh, args.head_num_divisor);
   const int S = args.seq_kv;
   const int Sq = args.seq_q;
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   auto written = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
 
   // ---- prologue: mask bytes (first half), Q rows, K of the first own block; all in flight before the first wait --------
-  const int row0 = (qb * 4 + r) * 32;
+  const int row0 = args.first_row + (qb * 4 + r) * 32;
   const bool active = row0 < Sq;
   v4i mask_bytes, tail_bytes;
   {
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       w[u][a] = __builtin_amdgcn_perm(hi, lo, 0x05040100);
     }
   if (row0 + i32 >= Sq) return;
-  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D)) return;
+  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= ((long)args.total_wgs / args.q_blocks + args.first_head) * Sq * D)) return;
   int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * kColTiles * h;
   if constexpr (kColTiles == 2) {  // 32 contiguous bytes per lane
     op += 32 * g;

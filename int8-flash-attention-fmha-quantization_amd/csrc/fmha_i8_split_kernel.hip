@@ -166,8 +166,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     const int L = blockIdx.x, per = args.total_wgs / kXcds, rem = args.total_wgs % kXcds, x = L % kXcds;
     wg = x * per + (x < rem ? x : rem) + L / kXcds;
   }
-  const int bh = divide(wg, args.q_blocks_divisor);
-  const int qb = wg - bh * args.q_blocks;
+  const int bh_here = divide(wg, args.q_blocks_divisor), bh = bh_here + args.first_head;
+  const int qb = wg - bh_here * args.q_blocks;
   const int b = divide(bh, args.head_num_divisor);
   const int S = args.seq_kv;
   const int Sq = args.seq_q;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   const Const<kLoads / 2> half_kind;
 
   // ---- prologue: mask bytes, Q rows and K of round 0, in this order; every load in flight before the first wait ---------
-  const int row0 = PARTS ? 0 : (qb * R + r) * 32;
+  const int row0 = PARTS ? 0 : args.first_row + (qb * R + r) * 32;
   const bool active = row0 < Sq;
   // Keys to classify: all, or those of the rounds of this workgroup and the block in front of them (part of which a partly
   // filled last block's tile repeats).
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
     w[a] = __builtin_amdgcn_perm(hi, lo, 0x05040100);
   }
   if (row0 + i32 >= Sq) return;
-  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D)) return;
+  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= ((long)args.total_wgs / args.q_blocks + args.first_head) * Sq * D)) return;
   // words a of lanes l and l+32 are neighbours: the exchange hands lane l the pair of word 0 (2) and lane l+32 that of word 1 (3)
   int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * u_out + 8 * g;
 #pragma unroll
