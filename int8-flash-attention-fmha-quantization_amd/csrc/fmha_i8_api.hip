@@ -11,6 +11,7 @@
 #ifndef FMHA_NO_SPLIT_KERNEL
 #include "fmha_i8_split_kernel.hip"
 #include "fmha_i8_pair_kernel.hip"
+#include "fmha_i8_few_kernel.hip"
 #endif
 
 namespace {
@@ -101,6 +102,8 @@ hipError_t launch_wide(int head_dim, int block_keys, Variant var, hipStream_t st
 }
 
 #ifndef FMHA_NO_SPLIT_KERNEL
+// R, and row_groups below: groups of 32 query rows per workgroup, or kFew for fmha_i8_few_kernel.
+constexpr int kFew = 16;
 template <int D, int BK, int R>
 const void* split_kernel(Variant var) {
   using namespace fmha_i8_gfx950;
@@ -113,6 +116,13 @@ const void* split_kernel(Variant var) {
 #define FMHA_KERNEL(KERNEL, BB, FF, PP) reinterpret_cast<const void*>(&KERNEL<D, BK, BB, FF, PP>)
     return FMHA_VARIANT(fmha_i8_pair_kernel);
 #undef FMHA_KERNEL
+  } else if constexpr (R == kFew) {
+    if constexpr (D == 128 && BK == kBlockK) return nullptr;  // (shared-out key blocks alone)
+    else {
+#define FMHA_KERNEL(KERNEL, BB, FF, PP) reinterpret_cast<const void*>(&KERNEL<D, BK, BB, FF, PP, false>)
+      return FMHA_VARIANT(fmha_i8_few_kernel);
+#undef FMHA_KERNEL
+    }
   } else {
 #define FMHA_KERNEL(KERNEL, BB, FF, PP) reinterpret_cast<const void*>(&KERNEL<D, BK, BB, FF, PP, R>)
     return FMHA_VARIANT(fmha_i8_split_kernel);
@@ -126,10 +136,11 @@ struct PartPlan {
   size_t ml_bytes = 0, bytes = 0;
 };
 template <int D, int BK>
-const void* part_kernel(Variant var) {
+const void* part_kernel(Variant var, int rows) {
   using namespace fmha_i8_gfx950;
-#define FMHA_PART(BB, FF, PP) reinterpret_cast<const void*>(&fmha_i8_split_kernel<D, BK, BB, FF, PP, 1, true>)
   // (what becomes of the accumulators is up to the merge: FASTACC makes no difference here)
+#define FMHA_PART(BB, FF, PP) \
+  (rows <= kFewRows ? reinterpret_cast<const void*>(&fmha_i8_few_kernel<D, BK, BB, FF, PP, true>) : reinterpret_cast<const void*>(&fmha_i8_split_kernel<D, BK, BB, FF, PP, 1, true>))
   if (var.full_range_p) return var.bias ? FMHA_PART(true, true, true) : FMHA_PART(false, true, true);
   return var.bias ? FMHA_PART(true, true, false) : FMHA_PART(false, true, false);
 #undef FMHA_PART
@@ -148,7 +159,7 @@ hipError_t launch_parts(const PartPlan& plan, Variant var, hipStream_t stream, c
   args.part_ml = static_cast<v2f*>(workspace);
   args.part_o = reinterpret_cast<int*>(static_cast<char*>(workspace) + plan.ml_bytes);
   void* kernel_args[] = {&args};
-  const hipError_t err = hipLaunchKernel(part_kernel<D, BK>(var), dim3((unsigned)args.total_wgs), dim3(256), kernel_args, 0, stream);
+  const hipError_t err = hipLaunchKernel(part_kernel<D, BK>(var, args.seq_q), dim3((unsigned)args.total_wgs), dim3(256), kernel_args, 0, stream);
   if (err != hipSuccess) return err;
   int row_lanes = D / 2;
   while (64 / row_lanes < args.seq_q) row_lanes /= 2;
@@ -164,7 +175,7 @@ template <int D, int BK>
 hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, const fmha_i8_gfx950::KernelArgs& of_call) {
   using namespace fmha_i8_gfx950;
   SplitKernelArgs args{of_call};
-  const int row_groups = piece.row_groups, rows = 32 * row_groups;
+  const int row_groups = piece.row_groups, rows = row_groups == kFew ? kFewRows : 32 * row_groups;
   args.q_blocks = (piece.end_row - piece.first_row + rows - 1) / rows;
   args.total_wgs = piece.heads * args.q_blocks;
   args.first_head = piece.first_head;
@@ -172,8 +183,8 @@ hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, con
   args.q_blocks_divisor = make_divisor(args.q_blocks);
   args.head_num_divisor = make_divisor(args.head_num);
   void* kernel_args[] = {&args};
-  const void* kernel = row_groups == 1 ? split_kernel<D, BK, 1>(var) : row_groups == 2 ? split_kernel<D, BK, 2>(var) : split_kernel<D, BK, 4>(var);
-  return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 ? 256 : 512), kernel_args, 0, stream);
+  const void* kernel = row_groups == kFew ? split_kernel<D, BK, kFew>(var) : row_groups == 1 ? split_kernel<D, BK, 1>(var) : row_groups == 2 ? split_kernel<D, BK, 2>(var) : split_kernel<D, BK, 4>(var);
+  return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 || row_groups == kFew ? 256 : 512), kernel_args, 0, stream);
 }
 // What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
 // split kernel.  Microseconds * 100 beyond the launch (2.9 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
@@ -186,11 +197,12 @@ struct KernelCost {
 constexpr KernelCost kKernelCosts[] = {{0, 1, {{{72, 80}, {95, 128}}, {{200, 99}, {250, 162}}}},
                                        {4, 1, {{{137, 62}, {170, 97}}, {{225, 83}, {300, 116}}}},
                                        {2, 4, {{{39, 183}, {45, 312}}, {{108, 199}, {140, 332}}}},
-                                       {1, 4, {{{23, 141}, {30, 213}}, {{73, 159}, {95, 243}}}}};
-constexpr KernelCost kOneGroupCost = kKernelCosts[3];
-static_assert(kOneGroupCost.row_groups == 1, "");
+                                       {1, 4, {{{23, 141}, {30, 213}}, {{73, 159}, {95, 243}}}},
+                                       {kFew, 4, {{{0, 97}, {0, 149}}, {{15, 138}, {75, 225}}}}};
+constexpr KernelCost kOneGroupCost = kKernelCosts[3], kFewCost = kKernelCosts[4];
+static_assert(kOneGroupCost.row_groups == 1 && kFewCost.row_groups == kFew, "");
 // Groups of 32 query rows per workgroup of the kernel that serves `rows` query rows of `heads` heads: 1 or 2 (fmha_i8_split_kernel), 4
-// (fmha_i8_pair_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
+// (fmha_i8_pair_kernel), kFew (fmha_i8_few_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
 // Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (cost of one).  What the constants
 // order is far apart nearly everywhere - d128, S2048: H4 31.0 us in 256-row workgroups, 24.4 in those of four groups, 17.6 of
@@ -205,10 +217,17 @@ int cost_of_workgroup(const KernelCost& kernel, int head_dim, int blocks, int bl
   const auto& c = kernel.cost[head_dim == 128][block_keys == fmha_i8_gfx950::kBlockK];
   return c.start + c.step * ((blocks + kernel.keys_per_round - 1) / kernel.keys_per_round);
 }
-int rows_of(const KernelCost& kernel) { return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups; }
-Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
+int rows_of(const KernelCost& kernel) {
+  return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : kernel.row_groups == kFew ? fmha_i8_gfx950::kFewRows : 32 * kernel.row_groups;
+}
+// At most sixteen rows, and not the geometry that the split kernel's second group serves better (see fmha_i8_few_kernel).
+bool few_takes(int rows, int head_dim, int block_keys) {
+  return rows <= fmha_i8_gfx950::kFewRows && !(head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK);
+}
+Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys, bool with_few = true) {
   Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
+    if (kernel.row_groups == kFew && !(with_few && few_takes(rows, head_dim, block_keys))) continue;
     // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
     // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 13.9 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with
     // 16 heads 13.1 and 12.6; d64: 11.7 either way).  Its step is one group's less a little, so that it is taken.
@@ -223,7 +242,8 @@ Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int 
 }
 Choice row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   if (a.seq_len_kv <= block_keys) return {0, -1};
-  if (fmha_i8_gfx950::test_build::forced_route() >= 0) return {fmha_i8_gfx950::test_build::forced_route(), -1};
+  const int forced = fmha_i8_gfx950::test_build::forced_route();
+  if (forced >= 0 && (forced != kFew || few_takes(a.seq_len_q, a.head_dim, block_keys))) return {forced, -1};
   return cheapest_kernel((long long)a.batch_num * a.head_num, a.seq_len_q, a.head_dim, (a.seq_len_kv + block_keys - 1) / block_keys, block_keys);
 }
 // The launches of a call: one, or two where large workgroups would leave most compute units idle in their last wave, or in the last
@@ -264,9 +284,12 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
 // key blocks, 0.8 per further batch.  Within 5 % of each other (the factor 20/21) the plain route is taken, which needs no memory: the
 // model flatters the other one there - of eleven shapes that it puts 0 to 5 % ahead nine are slower shared out, by 2 to 21 % (H32
 // Sq32 S1500 d128 11.1 -> 13.5 us), two faster (H128 Sq4 S2048 d64 11.6 -> 11.0).  One call, plain
-// -> shared out: B1 H16 Sq1 S2048 d128 12.2 -> 9.2 us, S8192 d64 36.3 -> 11.8, H32 S8192 d128 41.7 -> 19.3, H8 S65536 331 -> 61;
-// H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds already, 14.0 -> 15.9 and hence not.
-PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
+// -> shared out: B1 H16 Sq1 S2048 d128 12.6 -> 8.3 us, H32 S4096 22.2 -> 10.1, H32 S8192 42.8 -> 18.7; H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds already, 14.0 -> 15.9 and hence not.
+// Up to sixteen rows both sides are fmha_i8_few_kernel's, or the split kernel's second group's against it; plain -> shared out: d64 B8 H16
+// Sq1 S2048 8.9 -> 9.4 us, S8192 28.9 -> 28.9, H64 S2048 8.7 -> 7.6, H16 S1024 5.8 -> 7.4, H16 S4096 14.7 -> 8.6; d128 B4 H16 Sq4 S1984
+// 14.4 -> 12.0, B8 H16 Sq1 S1984 14.8 -> 16.8.
+// with_few = false: by the split kernel's costs alone, the shapes for which a workspace has always been asked.
+PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys, bool with_few = true) {
   using namespace fmha_i8_gfx950;
   PartPlan plan;
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys, rounds = (blocks + kSplitKeys - 1) / kSplitKeys;
@@ -275,8 +298,9 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   if (test_build::forced_route() >= 0) return plan;
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
-  const auto& c = kOneGroupCost.cost[a.head_dim == 128][block_keys == kBlockK];
-  long long least = row_groups_of(a, block_keys).cost;
+  const KernelCost& kernel = with_few && a.seq_len_q <= kFewRows ? kFewCost : kOneGroupCost;
+  const auto& c = kernel.cost[a.head_dim == 128][block_keys == kBlockK];
+  long long least = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys, with_few).cost;
   least = (least > memory ? least : memory) * 20 / 21;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
@@ -419,8 +443,12 @@ size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc) {
   if ((desc.head_dim != 64 && desc.head_dim != 128) || desc.seq_len_kv <= 0 || desc.seq_len_kv > 65536 || desc.seq_len_q <= 0 ||
       desc.batch_num <= 0 || desc.head_num <= 0)
     return 0;
-  const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv));
-  return plan.rounds_per_part > 0 ? plan.bytes : 0;
+  // What a call may use.  Whether it does is its own choice, which fmha_i8_few_kernel changes for some shapes; a size once told stays.
+  for (const bool with_few : {true, false}) {
+    const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv), with_few);
+    if (plan.rounds_per_part > 0) return plan.bytes;
+  }
+  return 0;
 #else
   return 0;
 #endif

@@ -116,7 +116,7 @@ struct KernelArgs {
   int first_head, first_row;  // of this launch, for the kernels of smaller workgroups (see pieces_of in the launch code), else 0
 };
 
-// The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8), where the caller wants it: in
+// The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8, or of 4 for a single word), where the caller wants it: in
 // place of a launch that passes over o again (B4 H16 S1024 d128, bfloat16: 5.2 us separate, 4.5 here; the host chooses).
 template <int D, int WORDS>
 __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, const int (&w)[WORDS]) {
@@ -125,6 +125,10 @@ __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, cons
   auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
   if (args.wide_is_bf16) {
     unsigned short* p = static_cast<unsigned short*>(args.wide) + at;
+    if constexpr (WORDS == 1) {
+      *reinterpret_cast<v2i*>(p) = v2i{(int)cvt_pk_bf16(value(0, 0), value(0, 1)), (int)cvt_pk_bf16(value(0, 2), value(0, 3))};
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < WORDS; k += 2) {
       v4i r;

@@ -649,9 +649,9 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
 }
 
 // ---- calls of few query rows: key blocks shared out over workgroups ------------------------------------------------------
-// A call of at most kPartRows rows per head has one workgroup per head, which reads all of its K and V: with less than 256
-// heads compute units idle, with a long sequence the time is that of one CU's loads (128 KB in
-// 2.4 us).
+// A call of at most kPartRows rows per head has one workgroup per head, which does all of its key blocks: with less than 256
+// heads compute units idle, with a long sequence the time is that of one CU (2.4 us per 512 keys at d128).  Up to sixteen rows
+// the workgroups are those of fmha_i8_few_kernel.
 // Partial results of separate key ranges cannot be merged with the same bytes, but those of single key blocks can: PARTS leaves
 // the accumulators of GEMM 2 (whole numbers) and the row's maximum and sum per block, 4 head_dim + 8 bytes per row where the
 // block itself has 2 BK head_dim, and this kernel does the online merge of all blocks in key order.
