@@ -132,9 +132,12 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   constexpr int kRowsPerRegion = 1024 / D;
   constexpr int kDSteps = D / 32;
   constexpr int kKeyTiles = BK / 32;
-  // LDS holds 160 KB: tiles of 8 KB and less are double buffered.  Beside 128 KB of tiles there is room for 16 KB of P: all
-  // of a round, or, for two row groups and blocks of 128 keys, half of it, which then goes through in two steps.
-  constexpr int kBuffers = kTileBytes <= 8192 ? 2 : 1;
+  // LDS holds 160 KB: tiles of 8 KB and less are double buffered, unless own K tiles (below) do better: with one row group and
+  // blocks of 64 keys H16 Sq512 S576 d128 8.56 -> 8.37 us, H32 Sq200 S960 10.15 -> 10.02, H16 Sq400 S320 d64 5.96 -> 5.90, and at d64 three
+  // workgroups fit a CU (H16 Sq777 S777 in 400 of them 16.9 -> 10.9); with blocks of 128 keys, d64, H16 Sq256 S1024 7.54 -> 7.70.
+  // Beside 128 KB of tiles there is room for 16 KB of P: all of a round, or, for two row groups and blocks of 128 keys, half of it,
+  // which then goes through in two steps.
+  constexpr int kBuffers = kTileBytes <= 8192 && !(R == 1 && BK == 64 && !PARTS) ? 2 : 1;
   constexpr bool kTwoSteps = BK == 128 && R == 2;
   constexpr int kPSlots = kTwoSteps ? 2 : 4;
   // With one row group a K tile has one reader: the wavefront fetches it itself, waits for it itself, and asks for the next

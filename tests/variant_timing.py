@@ -50,6 +50,13 @@ def events_us(torch, call, calls):
     return best
 
 
+FEW = 16  # the kernel of sixteen rows, as FMHAInferI8DebugRoute's number and as its rows
+
+
+def few_takes(rows, s, d):
+    return rows <= FEW and not (d == 128 and (s + 63) // 64 % 2 == 0)
+
+
 def time_route(pkg, lib, routes, route, shape, calls=100):
     """Microseconds per call, or None where the call does not have that route.  No masked key, uniform random bytes."""
     import torch
@@ -83,11 +90,11 @@ def time_shapes(shapes):
     import routes
     pkg = g.load_package()
     lib = routes.library(pkg)
-    names = list(routes.ROUTES)
+    names = list(routes.ROUTES) + [FEW]
     print("| B, H, Sq, S, d | %s | key blocks shared out | the library's choice |" % " | ".join("%d rows" % r for r in names))
     print("|" + "---|" * (len(names) + 3))
     for shape in shapes:
-        us = [time_route(pkg, lib, routes, routes.ROUTES[r], shape) for r in names]
+        us = [time_route(pkg, lib, routes, routes.ROUTES.get(r, FEW), shape) if r != FEW or few_takes(*shape[2:]) else None for r in names]
         us += [time_route(pkg, lib, routes, route, shape) for route in (routes.SHARED_OUT, routes.OWN_CHOICE)]
         print("| %s | %s |" % (", ".join(map(str, shape)), " | ".join("-" if u is None else "%.2f" % u for u in us)), flush=True)
 
@@ -104,9 +111,11 @@ def kernel_costs():
     print("|" + "---|" * 6)
     for d in (64, 128):
         for block in (64, 128):
-            for rows, route in routes.ROUTES.items():
+            for rows, route in list(routes.ROUTES.items()) + ([(FEW, FEW)] if few_takes(1, block, d) else []):
                 for heads in (8, 16):
-                    us = [time_route(pkg, lib, routes, route, (1, heads, 16 * rows, s, d)) for s in keys[block]]
+                    # (sixteen workgroups per head, or with sixteen rows one workgroup per head)
+                    shape = (1, 16 * heads, 1) if rows == FEW else (1, heads, 16 * rows)
+                    us = [time_route(pkg, lib, routes, route, (*shape, s, d)) for s in keys[block]]
                     rounds = [(s // block + 3) // 4 if rows <= 64 else s // block for s in keys[block]]
                     step = (us[3] - us[0]) / (rounds[3] - rounds[0])
                     print("| %d | %d | %d | %d | %s | %.2f + %.3f |" % (d, block, rows, 16 * heads, " / ".join("%.2f" % u for u in us),
