@@ -281,9 +281,11 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
 // Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for, by the cost
 // table above (start, step of one row group), but no faster than the memory (62 KB in a hundredth of a microsecond, on both
 // sides of the comparison), with the workspace written and read again, and the merge: 2.5 us for the launch and a first batch of
-// key blocks, 0.8 per further batch.  Within 5 % of each other (the factor 20/21) the plain route is taken, which needs no memory: the
-// model flatters the other one there - of eleven shapes that it puts 0 to 5 % ahead nine are slower shared out, by 2 to 21 % (H32
-// Sq32 S1500 d128 11.1 -> 13.5 us), two faster (H128 Sq4 S2048 d64 11.6 -> 11.0).  One call, plain
+// key blocks, 0.8 per further batch; with more than sixteen rows, of which some row moves its reference in nearly every block, 1.2 and 0.06
+// per block on top (plain and shared out: H32 Sq32 S777 d64 8.8 and 9.5, H64 Sq32 S3000 d64 20.4 and 22.6, B2 H16 Sq32 S2048 d128 12.8 and
+// 14.2 us, all of which the model put 6 to 18 % the other way round).  Within 5 % of each other (the factor 20/21) the plain route is taken, which needs no memory: the
+// model flatters the other one there - of eleven shapes that it put 0 to 5 % ahead nine were slower shared out, by 2 to 21 % (H32
+// Sq32 S1500 d128 11.1 -> 13.5 us).  One call, plain
 // -> shared out: B1 H16 Sq1 S2048 d128 12.6 -> 8.3 us, H32 S4096 22.2 -> 10.1, H32 S8192 42.8 -> 18.7; H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds already, 14.0 -> 15.9 and hence not.
 // Up to sixteen rows both sides are fmha_i8_few_kernel's, or the split kernel's second group's against it; plain -> shared out: d64 B8 H16
 // Sq1 S2048 8.9 -> 9.4 us, S8192 28.9 -> 28.9, H64 S2048 8.7 -> 7.6, H16 S1024 5.8 -> 7.4, H16 S4096 14.7 -> 8.6; d128 B4 H16 Sq4 S1984
@@ -297,8 +299,9 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys, bool wit
   if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
   if (test_build::forced_route() >= 0) return plan;
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
-  const long long merge = 250 + 80 * ((blocks - 1) / 32) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
-  const KernelCost& kernel = with_few && a.seq_len_q <= kFewRows ? kFewCost : kOneGroupCost;
+  const bool one_group = a.seq_len_q > kFewRows;
+  const long long merge = 250 + 80 * ((blocks - 1) / 32) + (one_group ? 120 + 6 * blocks : 0) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
+  const KernelCost& kernel = with_few && !one_group ? kFewCost : kOneGroupCost;
   const auto& c = kernel.cost[a.head_dim == 128][block_keys == kBlockK];
   long long least = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys, with_few).cost;
   least = (least > memory ? least : memory) * 20 / 21;
@@ -443,7 +446,7 @@ size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc) {
   if ((desc.head_dim != 64 && desc.head_dim != 128) || desc.seq_len_kv <= 0 || desc.seq_len_kv > 65536 || desc.seq_len_q <= 0 ||
       desc.batch_num <= 0 || desc.head_num <= 0)
     return 0;
-  // What a call may use.  Whether it does is its own choice, which fmha_i8_few_kernel changes for some shapes; a size once told stays.
+  // What a call may use: what its own choice takes, or what the split kernel's costs alone would (see part_plan_of).
   for (const bool with_few : {true, false}) {
     const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv), with_few);
     if (plan.rounds_per_part > 0) return plan.bytes;
