@@ -22,11 +22,13 @@ __device__ __forceinline__ int row_max16(int x) {
   return half_max(max((int)r[0], (int)r[1]));
 }
 
-// V tiles are read by ds_read_b64_tr_b8 whose 16-lane groups touch keys {0, 1, 2, 3, 16, 17, 18, 19} (+4, +8, +12): the chunks of
-// keys 16 apart, which start in the same bank, are swapped by bit 4 of the key.
+// V tiles are read by ds_read_b64_tr_b8.  Thirty-two lanes read one chunk column of keys {0 .. 7, 16 .. 23} (+8): rows that start in the
+// same bank get different chunks by bits 1 (at d128), 2 and 4 of the key.  (By bits 0, 1 and 4, which tell the keys of sixteen lanes
+// apart: 256 cycles of bank conflicts per round; B8 H16 Sq1 S2048 d64 9.12 -> 8.97 us, H16 S4096 14.5 -> 14.3, H16 Sq16 S1984 d128
+// 14.2 -> 14.0.)
 template <int D>
 __device__ __forceinline__ int few_v_swizzle(int key) {
-  return D == 128 ? ((key & 3) | ((key >> 2) & 4)) : (((key >> 1) & 1) | ((key >> 3) & 2));
+  return D == 128 ? (((key >> 1) & 3) | ((key >> 2) & 4)) : (((key >> 2) & 1) | ((key >> 3) & 2));
 }
 
 template <int D, int BK, bool BIAS, bool FASTACC, bool FULLP, bool PARTS>
