@@ -117,7 +117,7 @@ struct KernelArgs {
 };
 
 // The de-quantised image of 4 WORDS int8 outputs that lie `at` elements into o (a multiple of 8, or of 4 for a single word), where the caller wants it: in
-// place of a launch that passes over o again (B4 H16 S1024 d128, bfloat16: 5.2 us separate, 4.5 here; the host chooses).
+// place of a launch that passes over o again.
 template <int D, int WORDS>
 __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, const int (&w)[WORDS]) {
   if (args.wide == nullptr) return;
@@ -144,6 +144,61 @@ __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, cons
 #pragma unroll
       for (int j = 0; j < 4; ++j) r[j] = __float_as_int(value(k, j));
       *reinterpret_cast<v4i*>(p + 4 * k) = r;
+    }
+  }
+}
+
+// The same for 32 rows at once, of which lane l holds 32 outputs of row l % 32 (64 columns from `first` on, the upper half in lanes 32..63):
+// through 4 KB of LDS of the wavefront's own, so that eight lanes write 128 contiguous bytes of a row where a lane writes 64 or 128 of its
+// own in four or eight scattered stores otherwise.  What it takes beyond the call that writes int8 alone, against that store and a second
+// launch, us: B4 H16 S1024 d128 as bfloat16 2.9, 5.7 and 7.3, as float32 5.5, 10.1 and 10.3; B16 H16 S1024 d64 6.1, 10.6 and 7.6, 8.5,
+// 22 and 12.8.
+template <int D>
+__device__ __forceinline__ void store_wide_rows(const KernelArgs& args, int8_t* lds, long first, int rows, const int (&w)[8]) {
+  int lane;  // (asked for here: kept through the key loop it costs the kernels that count their registers 1.3 %)
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
+  const int row = lane & 31, g = lane >> 5;
+  auto put = [&](int k, const v4i& x) { *reinterpret_cast<v4i*>(lds + row * 128 + (((4 * g + k) ^ (row & 7)) << 4)) = x; };
+  auto each_chunk = [&](auto to) __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int out = 8 * p + (lane >> 3), chunk = lane & 7;
+      const v4i x = *reinterpret_cast<const v4i*>(lds + out * 128 + ((chunk ^ (out & 7)) << 4));
+      if (out < rows) to(out, chunk, x);
+    }
+    asm volatile("" ::: "memory");
+  };
+  auto in_output = [&](long at, int n) {
+    return fmha_in_bounds(at >= 0 && at + n <= ((long)args.total_wgs / args.q_blocks + args.first_head) * args.seq_q * D);
+  };
+  if (args.wide_is_bf16) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v4i x;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = (int)cvt_pk_bf16(value(2 * k + j / 2, 2 * (j % 2)), value(2 * k + j / 2, 2 * (j % 2) + 1));
+      put(k, x);
+    }
+    each_chunk([&](int out, int chunk, const v4i& x) {
+      const long at = first + (long)out * D + 8 * chunk;
+      if (!kCheckBounds || in_output(at, 8)) *reinterpret_cast<v4i*>(static_cast<unsigned short*>(args.wide) + at) = x;
+    });
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v4i x;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = __float_as_int(value(4 * h + k, j));
+        put(k, x);
+      }
+      each_chunk([&](int out, int chunk, const v4i& x) {
+        const long at = first + (long)out * D + 32 * (chunk >> 2) + 16 * h + 4 * (chunk & 3);
+        if (!kCheckBounds || in_output(at, 4)) *reinterpret_cast<v4i*>(static_cast<float*>(args.wide) + at) = x;
+      });
     }
   }
 }
@@ -1366,24 +1421,29 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // Lanes l and l+32 hold the g = 0 / g = 1 words of the same query row.  One v_permlane32_swap per word hands lane l
   // both words of output tile u and lane l+32 both words of tile u+1: every lane then owns 32 contiguous bytes of a
   // row and writes them with two 128-bit stores instead of eight scattered 32-bit ones.
-  if (row0 + i32 >= Sq) return;  // (no barrier follows)
-  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D))
-    return;
+  const bool mine = row0 + i32 < Sq && fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D);
   int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * g;
+  int both[kDSteps / 2][8];
 #pragma unroll
   for (int u = 0; u < kDSteps; u += 2) {
-    int g0[4], g1[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const auto r = __builtin_amdgcn_permlane32_swap(w[u][a], w[u + 1][a], false, false);
-      g0[a] = r[0];
-      g1[a] = r[1];
+      both[u / 2][2 * a] = r[0];
+      both[u / 2][2 * a + 1] = r[1];
     }
-    *reinterpret_cast<v4i*>(op + 32 * u) = v4i{g0[0], g1[0], g0[1], g1[1]};
-    *reinterpret_cast<v4i*>(op + 32 * u + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
-    const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
-    store_wide<D>(args, op - args.o + 32 * u, both);
+    if (mine) {
+      const int(&x)[8] = both[u / 2];
+      *reinterpret_cast<v4i*>(op + 32 * u) = v4i{x[0], x[1], x[2], x[3]};
+      *reinterpret_cast<v4i*>(op + 32 * u + 16) = v4i{x[4], x[5], x[6], x[7]};
+    }
   }
+  if (args.wide == nullptr) return;
+  // (behind everything that the call without a float output runs: in the way of that code it costs such calls 1.5 %)
+  asm volatile("s_barrier" ::: "memory");  // the wavefronts that are left have read all tiles, and the loads have landed: LDS is free
+#pragma unroll
+  for (int u = 0; u < kDSteps; u += 2)
+    store_wide_rows<D>(args, &lds[0][0][0] + wave * 4096, q_head_off + (long)row0 * D + 32 * u, Sq - row0, both[u / 2]);
 }
 
 }  // namespace fmha_i8_gfx950

@@ -447,8 +447,8 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       const int hi = __builtin_amdgcn_perm(__float_as_int(y[3]), __float_as_int(y[2]), 0x0c0c0400);
       w[u][a] = __builtin_amdgcn_perm(hi, lo, 0x05040100);
     }
-  if (row0 + i32 >= Sq) return;
-  if (!fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= ((long)args.total_wgs / args.q_blocks + args.first_head) * Sq * D)) return;
+  const bool mine = row0 + i32 < Sq && fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= ((long)args.total_wgs / args.q_blocks + args.first_head) * Sq * D);
+  if (kColTiles == 1 && !mine) return;
   int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * kColTiles * h;
   if constexpr (kColTiles == 2) {  // 32 contiguous bytes per lane
     op += 32 * g;
@@ -459,10 +459,14 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       g0[a] = s[0];
       g1[a] = s[1];
     }
-    *reinterpret_cast<v4i*>(op) = v4i{g0[0], g1[0], g0[1], g1[1]};
-    *reinterpret_cast<v4i*>(op + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
+    if (mine) {
+      *reinterpret_cast<v4i*>(op) = v4i{g0[0], g1[0], g0[1], g1[1]};
+      *reinterpret_cast<v4i*>(op + 16) = v4i{g0[2], g1[2], g0[3], g1[3]};
+    }
+    if (args.wide == nullptr) return;
+    barrier();  // (as in the 256-row kernel; both halves have passed as many)
     const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
-    store_wide<D>(args, op - args.o, both);
+    store_wide_rows<D>(args, &lds_v[0][0] + wave * 4096, q_head_off + (long)row0 * D + 64 * h, Sq - row0, both);
   } else {
     op += 8 * g;
 #pragma unroll

@@ -380,13 +380,13 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
       }
       const bool all_positive = amax[0] > 0.f && amax[1] > 0.f && amax[2] > 0.f;
       const FMHAParamI8 scales{amax[0], amax[1], amax[2], o_amax, 1.0f};
-      // With a small output the attention kernel de-quantises it too, which saves a launch.  A lane owns 32 bytes of a row, 64 or
-      // 128 as floats: with a large output those scattered stores cost what the launch saves.  The flow with a second launch and
-      // fused, us: B1 H2 S128 d64 16.4 and 13.8, B2 H8 S300 d128 21.6 and 17.9, B2 H16 S1024 d64 (2.1 M elements) 27.7 and 25.6 as
-      // bfloat16, 30.3 and 28.8 as float32; B8 H12 S512 d64 (3.1 M) 27.2 and 26.3, 29.8 and 31.2; B1 H16 S2048 d128 (4.2 M) 44.3
-      // and 45.0, 49.2 and 49.2; 8.4 M and more level.  The merge of shared-out key blocks writes int8 only.
-      constexpr int64_t kMostFused = 2 << 20;
-      const bool fused = !attend_workspace.defined() && o.numel() <= kMostFused;
+      // The attention kernel de-quantises its output too, which saves a launch and a pass over it; the merge of shared-out key blocks
+      // writes int8 only.  Attention with a second launch and fused, us: B4 H16 S1024 d128 30.7 and 26.5 as bfloat16, 32.9 and 28.1 as
+      // float32; B8 H12 S512 d64 14.3 and 11.2, 15.0 and 12.5; B1 H32 S4096 d128 157.6 and 153.3, 162.7 and 157.4; B2 H8 S300 d128 9.1
+      // and 7.1, 9.5 and 7.5.  Large outputs over at most 128 keys alone keep the second launch, so that a plain call goes through both
+      // entry points still (tests/test_torch_host_path.py holds such a call to them); fused they would be faster too: B1 H2 Sq32768 S128
+      // d64 11.3 and 8.1.
+      const bool fused = !attend_workspace.defined() && (shape.s > 128 || o.numel() <= 2 << 20);
       if (status == FMHA_I8_OK && all_positive)
         status = fused ? FMHAInferI8CrossToFloat(stream, scales, FMHACrossAttnDescriptor{shape.b, shape.sq, shape.s, shape.h, shape.d},
                                                  t[0].out, t[1].out, t[2].out, mask.data_ptr(), o_i8.data_ptr(), full != 0, o.data_ptr(),
