@@ -13,7 +13,8 @@ TORCH_SOURCE = os.path.join(HERE, "csrc", "fmha_torch.cpp")
 SOURCES = [os.path.join(HERE, "csrc", "fmha_i8_api.hip"), os.path.join(HERE, "csrc", "fmha_quant.hip")]
 DEPENDS = SOURCES + [os.path.join(HERE, "csrc", "fmha_i8_kernel.hip"),
                      os.path.join(HERE, "csrc", "fmha_i8_split_kernel.hip"),
-                     os.path.join(HERE, "csrc", "fmha_i8_pair_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
+                     os.path.join(HERE, "csrc", "fmha_i8_pair_kernel.hip"), os.path.join(HERE, "csrc", "fmha_i8_few_kernel.hip"),
+                     os.path.join(HERE, "csrc", "fmha_i8_test_builds.h"),
                      os.path.join(HERE, "csrc", "fmha_dequant.h"),
                      os.path.join(ROOT, "include", "fmha_i8.h"), os.path.join(ROOT, "include", "fmha_param_i8.h"),
                      os.path.join(ROOT, "include", "fmha_quant.h")]
