@@ -148,6 +148,14 @@ __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, cons
   }
 }
 
+// The lane, asked for anew: what is computed from threadIdx.x and used on both sides of the key loops is kept through them, or spilled
+// (see waves_per_simd).
+__device__ __forceinline__ int lane_again() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  return lane;
+}
+
 // The same for 32 rows at once, of which lane l holds 32 outputs of row l % 32 (64 columns from `first` on, the upper half in lanes 32..63):
 // through 4 KB of LDS of the wavefront's own, so that eight lanes write 128 contiguous bytes of a row where a lane writes 64 or 128 of its
 // own in four or eight scattered stores otherwise.  What it takes beyond the call that writes int8 alone, against that store and a second
@@ -155,8 +163,7 @@ __device__ __forceinline__ void store_wide(const KernelArgs& args, long at, cons
 // 22 and 12.8.
 template <int D>
 __device__ __forceinline__ void store_wide_rows(const KernelArgs& args, int8_t* lds, long first, int rows, const int (&w)[8]) {
-  int lane;  // (asked for here: kept through the key loop it costs the kernels that count their registers 1.3 %)
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  const int lane = lane_again();
   auto value = [&](int word, int byte) { return dequant1((int)((unsigned)w[word] << (24 - 8 * byte)) >> 24, args.wide_amax); };
   const int row = lane & 31, g = lane >> 5;
   auto put = [&](int k, const v4i& x) { *reinterpret_cast<v4i*>(lds + row * 128 + (((4 * g + k) ^ (row & 7)) << 4)) = x; };
@@ -279,7 +286,11 @@ __device__ __forceinline__ v16i masked_start(unsigned word, const MaskedUnits<BI
 
 // Wavefronts per SIMD to leave registers for: two of them are this workgroup's.  The converting d = 64 kernel stays below 168
 // registers, with which a wavefront of the next workgroup starts as soon as one of this has ended (B16 H16 S2048: 214 us, 219 with
-// 172), and with blocks of 64 keys below 128, with which two workgroups share a CU (B4 H64 S960: 59 us, 65 with 132).
+// 172), and with blocks of 64 keys below 128, with which two workgroups share a CU (B4 H64 S960: 59 us, 65 with 132).  It meets both
+// without spilling as long as nothing but what the key loops use lives through them: the lane is asked for anew in front of and behind
+// them (lane_again), and the constants of the output rounding are made there.  (With 2 to 6 registers spilled, which the bounds alone bring, and in
+// one form one of them reloaded in a key loop, behind a wait for every tile in flight: B4 H64 S950 60.3 -> 62.7 us, with a scattered
+// mask 67.2 -> 69.9, B8 H32 S1000 64.7 -> 66.6, B4 H12 S2349 74.7 -> 75.2, B16 H16 S2048 212.2 -> 214.0.)
 template <int D, int BK, bool BIAS>
 constexpr int waves_per_simd() { return D == 64 && !BIAS ? (BK == kBlockKSmall ? 4 : 3) : 2; }
 
@@ -344,9 +355,8 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // direct-to-LDS loads: lane l of a 1 KiB region lands at byte 16*l of the region, so the lane FETCHES the chunk that
   // the swizzle assigns to that slot.
   int ld_goff_k, ld_goff_v;
-  const int ld_row_in = lane / kChunks;
   {
-    const int row_in = ld_row_in, p = lane % kChunks;
+    const int row_in = lane / kChunks, p = lane % kChunks;
     // A 1 KiB region is 8 rows at D = 128 and this wavefront's regions all have the parity of its index: that is the
     // one row bit beyond row_in that the swizzles look at.
     const int vrow = (D == 128) ? (row_in | ((wave & 1) << 3)) : row_in;
@@ -384,7 +394,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // BK - S rows past the end of K and V.
   auto issue_short_region = [&](const int8_t* gbase, int which, int goff, int region) __attribute__((always_inline)) {
     const unsigned dst = lds_base + (unsigned)(which * kTileBytes + region * 1024);
-    const int row = region * kRowsPerRegion + ld_row_in;
+    const int row = region * kRowsPerRegion + lane_again() / kChunks;
     int src = goff + region * 1024 - (row >= S ? (row - (S - 1)) * D : 0);
     if (!fmha_in_bounds(src >= 0 && src + 16 <= S * D)) src = 0;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -515,7 +525,6 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   const float c2 = BIAS ? args.c2 * kBaseScale : args.c2;  // exponent per unit of sf() below
   constexpr int kScoreBaseBits = score_base_bits<D>();  // start value of the GEMM 1 accumulators on the BIAS variant
   const float bias_c2 = BIAS ? __builtin_bit_cast(float, kScoreBaseBits) * c2 : 0.f;
-  float magic;
   int flip_top;
   v16i base_c;             // start value of the GEMM 2 accumulators (and of GEMM 1 at head_dim 128), in sixteen registers
   v16i base_s;             // start value of the GEMM 1 accumulators
@@ -532,8 +541,6 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     m_ref = args.floor2 - 2.f * kLazyLog2;
     t_run = 0.f;
     l_run = 0.f;
-    magic = kMagic;
-    asm volatile("" : "+v"(magic));  // a register operand: as a literal it would double the size of every instruction using it
     flip_top = (int)0x80808080;
     if (FULLP) asm volatile("" : "+s"(flip_top));  // a register operand, for the same reason
     base_c = v16i{kBaseBits, kBaseBits, kBaseBits, kBaseBits, kBaseBits, kBaseBits, kBaseBits, kBaseBits,
@@ -562,9 +569,10 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   auto load_q_rows = [&]() __attribute__((always_inline)) {
     // rows past the end of the sequence load the last row (unused) so that every wavefront has the same loads in flight
     const int8_t* qp = args.q + q_head_off;
-    int qrow = row0 + i32 < Sq ? row0 + i32 : Sq - 1;
+    const int q_lane = lane_again();
+    int qrow = min(row0 + (q_lane & 31), Sq - 1);
     if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
-    const int qoff = qrow * D + 16 * g;
+    const int qoff = qrow * D + 16 * (q_lane >> 5);
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk)
       asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(qreg[kk]) : "v"(qoff + 32 * kk), "s"(qp) : "memory");
@@ -1400,8 +1408,8 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // l_run sums 128 p / 32767 and O sums 128 p v, so mean(v) = O / (32767 l_run); a row with no unmasked key yields 0
   const float fin = (l_run > 0.f) ? args.out_scale * (128.f / kSnorm) * kBaseScale / l_run : 0.f;
   const float corr = FASTACC ? (FULLP ? -kBaseFull * t_run : kBase * t_run) : 0.f;
-  float magic_lo = kMagic - 127.f, magic_hi = kMagic + 127.f;
-  asm volatile("" : "+v"(magic_lo), "+v"(magic_hi));  // register operands, like magic
+  float magic = kMagic, magic_lo = kMagic - 127.f, magic_hi = kMagic + 127.f;
+  asm volatile("" : "+v"(magic), "+v"(magic_lo), "+v"(magic_hi));  // register operands: a literal would double the size of every instruction using it
   int w[kDSteps][4];  // w[u][a]: the four int8 of output dims 32u + 8a + 4g .. +3 of query row i32
 #pragma unroll
   for (int u = 0; u < kDSteps; ++u)
@@ -1421,8 +1429,9 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // Lanes l and l+32 hold the g = 0 / g = 1 words of the same query row.  One v_permlane32_swap per word hands lane l
   // both words of output tile u and lane l+32 both words of tile u+1: every lane then owns 32 contiguous bytes of a
   // row and writes them with two 128-bit stores instead of eight scattered 32-bit ones.
-  const bool mine = row0 + i32 < Sq && fmha_in_bounds(row0 + i32 >= 0 && q_head_off + (long)(row0 + i32 + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D);
-  int8_t* op = args.o + q_head_off + (long)(row0 + i32) * D + 32 * g;
+  const int out_lane = lane_again(), out_row = row0 + (out_lane & 31);
+  const bool mine = out_row < Sq && fmha_in_bounds(out_row >= 0 && q_head_off + (long)(out_row + 1) * D <= (long)args.total_wgs / args.q_blocks * Sq * D);
+  int8_t* op = args.o + q_head_off + (long)out_row * D + 32 * (out_lane >> 5);
   int both[kDSteps / 2][8];
 #pragma unroll
   for (int u = 0; u < kDSteps; u += 2) {

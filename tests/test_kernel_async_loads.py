@@ -39,13 +39,18 @@ def _functions(path):
 
 
 @pytest.fixture(scope="module")
-def assembly(tmp_path_factory):
+def assembly_files(tmp_path_factory):
     """Every instantiation as shipped, and with contraction switched off on the command line."""
     at = tmp_path_factory.mktemp("asm")
     paths = str(at / "kernel.s"), str(at / "kernel_off.s")
     compilers = [_start_assembly(paths[0]), _start_assembly(paths[1], "-ffp-contract=off")]
     assert [c.wait() for c in compilers] == [0, 0]
-    return [_functions(p) for p in paths]
+    return paths
+
+
+@pytest.fixture(scope="module")
+def assembly(assembly_files):
+    return [_functions(p) for p in assembly_files]
 
 
 @pytest.fixture(scope="module")
@@ -183,3 +188,13 @@ def test_the_checker_itself_finds_a_missing_wait():
                "\tv_mov_b32 v9, v2\n\ts_endpgm\n")
     with pytest.raises(AssertionError):
         _check_function("skipped", skipped)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_no_kernel_keeps_anything_in_scratch(assembly_files):
+    """A launch bound that the register count does not meet is met by spilling, without a word: the reload of a spilled
+    register in a key loop waits for every tile in flight (`s_waitcnt vmcnt(0)`), and the prefetch is gone."""
+    scratch = dict(re.findall(r"\.amdhsa_kernel (\S+)\n(?:\s+\.amdhsa_(?!private)\S+ .*\n)*\s+\.amdhsa_private_segment_fixed_size (\d+)",
+                              open(assembly_files[0]).read()))
+    assert sum("_fwd_kernel" in name for name in scratch) == 64 and sum("_few_kernel" in name for name in scratch) > 0
+    assert {name: size for name, size in scratch.items() if size != "0"} == {}
