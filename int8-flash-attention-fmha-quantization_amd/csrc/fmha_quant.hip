@@ -366,16 +366,22 @@ __global__ __launch_bounds__(kSmallThreads) void quantize_small_kernel(QuantJob 
 //
 // A slot is two 8-byte words, each 48 bits of the call's tag and half of the maximum; the tags of no two calls are alike (TagSource),
 // so that what a slot held before is never taken for its maximum and nothing has to be cleared first.
-// No workgroup depends on another one's progress: one whose slot has not come after `patience` (ticks of 10 ns) - because
-// other work holds its compute unit - is not waited for any longer, and whoever misses it reads its share for itself.
+// No workgroup depends on another one's progress: one whose slot has not come after `patience` (ticks of 10 ns) - because other work
+// holds its compute unit - is not waited for any longer.  Whoever misses it reads one of the shares that have not come, leaves its
+// maximum in its slot, where the others find it, and looks again: what all of them read comes to one pass over those shares or two.
+// (Every one reading every missing share for itself: 170, 453 and 810 us for fp32 16.8 M elements beside a kernel of another stream that
+// held 16, 64 and 128 compute units; this 44, 54 and 66, two launches 36, 44 and 49.  25 M: 226, 649, 1185; 58, 72, 88; 51, 62, 68.
+// Up to 52 MB, where two workgroups fit on a compute unit, at most the two launches' time.  With 240 compute units held by attention the
+// call ends with that kernel, 0.6 ms, while the two launches' workgroups fit beside it: 27 to 130 us.)  The patience is what such a call
+// loses first; with less than 10 us, calls that nothing disturbs run out of it (25 M with 5 us: 23.3 -> 23.9), on cold inputs too.
 struct SlotTag {
   unsigned long long word[2];  // 48 bits each, in the upper ones
 };
 constexpr int kHeldBlocks = 256;  // one per CU; of 512 threads while they hold the call, so that two such calls fit beside each other
 #ifdef FMHA_FORCED_ROUTE
-std::atomic<unsigned> kPatience{5000};  // test build only: FMHAQuantDebugPatience
+std::atomic<unsigned> kPatience{1000};  // test build only: FMHAQuantDebugPatience
 #else
-constexpr unsigned kPatience = 5000;
+constexpr unsigned kPatience = 1000;
 #endif
 static_assert(kHeldBlocks * sizeof(SlotTag) <= FMHA_QUANT_WORKSPACE_FLOATS * sizeof(float), "one slot per workgroup");
 
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(THREADS, 4) void quantize_held_kernel(QuantJob job,
                                                                      SlotTag tag, unsigned patience, unsigned long long* __restrict__ note,
                                                                      unsigned ticket) {
   __shared__ float part[THREADS / 64];
-  __shared__ unsigned char missing[kHeldBlocks];
+  __shared__ unsigned long long absent[kHeldBlocks / 64];
   __shared__ __attribute__((aligned(1024))) typename T::unit more[IN_LDS > 0 ? IN_LDS : 1][THREADS];  // a thread's own units only
   int i = 0;
 #pragma unroll
@@ -430,36 +436,53 @@ __global__ __launch_bounds__(THREADS, 4) void quantize_held_kernel(QuantJob job,
   }
   take_abs(m, last);
   m = block_max<THREADS>(m, part);
-  if (tid < 2) {
-    const unsigned bits = __float_as_uint(m);
-    __hip_atomic_store(slots + 2 * blockIdx.x + tid, (tid == 0 ? tag.word[0] : tag.word[1]) | (tid == 0 ? bits >> 16 : bits & 0xffffu),
+  auto leave = [&](int share, float largest_of_share) {
+    if (tid >= 2) return;
+    const unsigned bits = __float_as_uint(largest_of_share);
+    __hip_atomic_store(slots + 2 * (first + share) + tid, (tid == 0 ? tag.word[0] : tag.word[1]) | (tid == 0 ? bits >> 16 : bits & 0xffffu),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  bool here = true;
-  if (tid < kHeldBlocks) {  // whole wavefronts
-    here = tid >= blocks || tid == block;
-    const unsigned long long since = __builtin_amdgcn_s_memrealtime();
-    for (;;) {
-      if (!here) {
-        const unsigned long long* slot = slots + 2 * (first + tid);
-        const unsigned long long w0 = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long w1 = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (((w0 ^ tag.word[0]) | (w1 ^ tag.word[1])) >> 16 == 0) {
-          m = fmaxf(m, __uint_as_float((unsigned)(w0 & 0xffffu) << 16 | (unsigned)(w1 & 0xffffu)));
-          here = true;
+  };
+  leave(block, m);
+  bool here = tid >= blocks || tid == block;  // thread t < kHeldBlocks: the maximum of share t is in m, or there is no such share
+  for (unsigned until = patience;; until = 0) {  // (at most `blocks` times: every time around a share's maximum is added)
+    if (tid < kHeldBlocks) {  // whole wavefronts
+      const unsigned long long since = __builtin_amdgcn_s_memrealtime();
+      for (;;) {
+        if (!here) {
+          const unsigned long long* slot = slots + 2 * (first + tid);
+          const unsigned long long w0 = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const unsigned long long w1 = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (((w0 ^ tag.word[0]) | (w1 ^ tag.word[1])) >> 16 == 0) {
+            m = fmaxf(m, __uint_as_float((unsigned)(w0 & 0xffffu) << 16 | (unsigned)(w1 & 0xffffu)));
+            here = true;
+          }
         }
+        if (__all(here) || __builtin_amdgcn_s_memrealtime() - since >= until) break;
+        __builtin_amdgcn_s_sleep(1);
       }
-      if (__all(here) || __builtin_amdgcn_s_memrealtime() - since > patience) break;
-      __builtin_amdgcn_s_sleep(1);
+      const unsigned long long of_wave = __ballot(!here);
+      if ((tid & 63) == 0) absent[tid >> 6] = of_wave;
     }
-    missing[tid] = !here;
-  }
-  if (__syncthreads_or(!here)) {
-    for (int other = 0; other < blocks; ++other) {
-      if (!missing[other]) continue;
-      for (int j = other * THREADS + tid; j < units; j += stride) take_abs_unit<T>(m, xu[j]);
-      if (other == 0 && rest < n) take_abs(m, T::widen(x[rest]));
-    }
+    if (!__syncthreads_or(tid < kHeldBlocks && !here)) break;
+    // One of the absent shares, as far as they go another one in every workgroup, its maximum left in its slot; then the slots again.
+    int count = 0, word = 0;
+#pragma unroll
+    for (int w = 0; w < kHeldBlocks / 64; ++w) count += __popcll(absent[w]);
+    int nth = block % count;
+    while (nth >= __popcll(absent[word])) nth -= __popcll(absent[word++]);
+    unsigned long long left = absent[word];
+    while (nth-- > 0) left &= left - 1;
+    const int other = 64 * word + __builtin_ctzll(left);
+    // (the very units that its own workgroup takes, the last one again past the end: two workgroups that leave a maximum in one slot
+    // must leave the same bits, since a reader may find one word of each)
+    float of_share = 0.f;
+#pragma unroll 4
+    for (int u = 0; u < UNITS + IN_LDS; ++u) take_abs_unit<T>(of_share, xu[min(other * THREADS + tid + u * stride, units - 1)]);
+    if (other == 0 && rest < n) take_abs(of_share, T::widen(x[rest]));
+    of_share = block_max<THREADS>(of_share, part);
+    leave(other, of_share);
+    m = fmaxf(m, of_share);
+    here |= tid == other;
   }
   const float amax = block_max<THREADS>(m, part);
   if (block == 0 && tid == 0) {
@@ -629,7 +652,7 @@ bool held_blocks(const long long* units_of, int count, int per, QuantJob& job) {
   job.first_block[FMHA_QUANT_MAX_TENSORS] = at;
   return true;
 }
-// Forms of quantize_held_kernel: threads per workgroup, units per thread in registers (16 take 96 to 104 of them) and in LDS (9: 72 KB
+// Forms of quantize_held_kernel: threads per workgroup, units per thread in registers (16 take 106 to 124 of them) and in LDS (9: 72 KB
 // of 512 threads).  The first that holds a call serves it: the fewer units, the more of the compute units share the work.
 template <int THREADS, int UNITS, int IN_LDS = 0>
 struct Held {

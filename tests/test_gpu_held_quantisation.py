@@ -115,3 +115,89 @@ def test_calls_on_several_streams_at_once(pkg, dev):
     torch.cuda.synchronize()
     for i, (q, amax) in enumerate(got):
         assert amax.item() == xs[i % 4].abs().max().item() and torch.equal(q, want[i % 4])
+
+
+@pytest.fixture
+def patience(pkg):
+    """Sets how long workgroups of the test build wait for each other, in ticks of 10 ns."""
+    lib = routes.library(pkg)
+    lib.FMHAQuantDebugPatience.argtypes = [C.c_uint]
+    yield lib.FMHAQuantDebugPatience
+    lib.FMHAQuantDebugPatience(1000)
+
+
+@pytest.mark.parametrize("dtype_name", ["float32", "bfloat16"])
+def test_whoever_measures_a_share_leaves_the_same_bits(pkg, dev, patience, dtype_name):
+    """With little patience a share is measured by its own workgroup and by others, which all write the two words of its slot: were
+    the maxima not the same bits, a reader could put halves of two together.  The largest value is in the last unit, which
+    workgroups read again where their share ends before their threads do."""
+    import torch
+    lib, per = routes.library(pkg), UNIT[dtype_name]
+    for e in EDGES:
+        for n in (per * e - 1, per * (e - 7777)):
+            x = torch.randn(n, device=dev).to(getattr(torch, dtype_name))
+            x[n - per] = -9.517
+            for ticks in (0, 60, 150, 400):
+                patience(ticks)
+                print(dtype_name, n, ticks, flush=True)
+                check(pkg, lib, [x])
+
+
+def call_us(pkg, lib, x, calls):
+    import torch
+    out = torch.empty(x.numel(), dtype=torch.int8, device=x.device)
+    work, amax = torch.empty(1100, device=x.device), torch.empty(1, device=x.device)
+    item = Tensor(x.data_ptr(), out.data_ptr(), x.numel())
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    e0.record()
+    for _ in range(calls):
+        assert lib.FMHAMeasureAndQuantizeI8(torch.cuda.current_stream().cuda_stream, C.addressof(item), 1, 0, work.data_ptr(), amax.data_ptr(), None, 0) == 0
+    e1.record()
+    torch.cuda.synchronize()
+    assert amax.item() == x.abs().max().item()
+    return e0.elapsed_time(e1) * 1e3 / calls
+
+
+def test_workgroups_without_patience_share_the_reading(pkg, dev, patience):
+    """Where every workgroup finds most of the others missing, they read the input about once more between them (2.4 times the
+    call's time), not once each (over a hundred times)."""
+    import torch
+    lib, x = routes.library(pkg), torch.randn(8 << 20, device=dev)
+    patience(1000)
+    waits = min(call_us(pkg, lib, x, 20) for _ in range(3))
+    patience(0)
+    reads = min(call_us(pkg, lib, x, 20) for _ in range(3))
+    print(waits, reads, flush=True)
+    assert reads <= 10 * waits, (waits, reads)
+
+
+def test_beside_a_kernel_that_holds_half_of_the_compute_units(pkg, dev, patience):
+    """A kernel of another stream on 128 compute units for half a millisecond: the call goes through beside it (66 us; 810 when every
+    workgroup read the share of every one that was missing)."""
+    import time
+
+    import torch
+    lib = routes.library(pkg)
+    patience(1000)
+    t = [torch.randint(-127, 128, (1, 128, rows, 128), device=dev, dtype=torch.int8) for rows in (256, 32768, 32768)]
+    t += [torch.zeros((1, 32768), dtype=torch.int8, device=dev), torch.empty((1, 128, 256, 128), dtype=torch.int8, device=dev)]
+    x, other = torch.randn(16 << 20, device=dev), torch.cuda.Stream()
+    beside, alone = [], []
+    lib.FMHAInferI8DebugRoute(routes.ROUTES[256])
+    try:
+        for _ in range(6):
+            torch.cuda.synchronize()
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record(other)
+            assert lib.FMHAInferI8Cross(other.cuda_stream, pkg.FMHAParamI8(0.2, 3.0, 3.0, 1.0, 1.0), pkg.FMHACrossAttnDescriptor(1, 256, 32768, 128, 128),
+                                        *[y.data_ptr() for y in t]) == 0
+            e1.record(other)
+            since = time.perf_counter()
+            while time.perf_counter() - since < 60e-6:  # it has begun
+                pass
+            beside.append(call_us(pkg, lib, x, 1))
+            alone.append(e0.elapsed_time(e1) * 1e3)
+    finally:
+        lib.FMHAInferI8DebugRoute(routes.OWN_CHOICE)
+    print(beside, alone, flush=True)
+    assert sorted(beside)[3] <= 250, (beside, alone)
