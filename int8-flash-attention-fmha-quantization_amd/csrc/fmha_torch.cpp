@@ -383,10 +383,11 @@ PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
       // The attention kernel de-quantises its output too, which saves a launch and a pass over it; the merge of shared-out key blocks
       // writes int8 only.  Attention with a second launch and fused, us: B4 H16 S1024 d128 30.7 and 26.5 as bfloat16, 32.9 and 28.1 as
       // float32; B8 H12 S512 d64 14.3 and 11.2, 15.0 and 12.5; B1 H32 S4096 d128 157.6 and 153.3, 162.7 and 157.4; B2 H8 S300 d128 9.1
-      // and 7.1, 9.5 and 7.5.  Large outputs over at most 128 keys alone keep the second launch, so that a plain call goes through both
-      // entry points still (tests/test_torch_host_path.py holds such a call to them); fused they would be faster too: B1 H2 Sq32768 S128
-      // d64 11.3 and 8.1.
-      const bool fused = !attend_workspace.defined() && (shape.s > 128 || o.numel() <= 2 << 20);
+      // and 7.1, 9.5 and 7.5; over at most 128 keys B1 H2 Sq32768 S128 d64 11.3 and 8.2, 11.5 and 9.2, B16 H16 Sq2048 S128 d64 54.4 and
+      // 46.4, 63.7 and 52.2, B256 H16 S128 d64 75.5 and 70.4, 84.9 and 82.9.  Over so few keys the call is all memory, and beyond 32 M
+      // elements its tensors outgrow the last-level cache, where fused calls take from 13 % less to 8 % more (B512 H16 S128 d128 233 and
+      // 217, 290 and 251; B192 79.6 and 85.4, 94.1 and 98.6): those stay with two launches.
+      const bool fused = !attend_workspace.defined() && (shape.s > 128 || o.numel() <= 32 << 20);
       if (status == FMHA_I8_OK && all_positive)
         status = fused ? FMHAInferI8CrossToFloat(stream, scales, FMHACrossAttnDescriptor{shape.b, shape.sq, shape.s, shape.h, shape.d},
                                                  t[0].out, t[1].out, t[2].out, mask.data_ptr(), o_i8.data_ptr(), full != 0, o.data_ptr(),

@@ -37,3 +37,18 @@ def test_float_rows_are_the_dequantised_int8_rows(pkg, dev, shape, dtype):
                 assert torch.equal(o[:n].view_as(want), want) and (o[n:] == 77).all(), (name, rows)
                 assert torch.equal(wide[:n].view_as(want), pkg.dequantize_tensor(want, 0.7, dtype=kind)) and (wide[n:] == 3).all(), (name, rows)
         assert lib.FMHAInferI8DebugOutOfBounds() == 0
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("shape", [(1, 2, 32768, 128, 64), (3, 5, 4099, 31, 128), (16, 16, 2048, 100, 64), (16, 16, 2049, 100, 64)], ids=lambda s: "B%d_H%d_Sq%d_S%d_d%d" % s)
+def test_float_flow_over_few_keys(pkg, dev, shape, dtype):
+    """Over at most 128 keys the last of these is the first output of more than 32 M elements, which a second launch de-quantises."""
+    import torch
+    B, H, Sq, S, d = shape
+    kind = getattr(torch, dtype)
+    q, k, v = (torch.randn((B, H, n, d), device=dev).to(kind) for n in (Sq, S, S))
+    mask = (torch.rand((B, S), device=dev) < 0.2).to(torch.int8)
+    print(shape, dtype, flush=True)
+    wide, o, amax = pkg.fmha_infer_from_float(q, k, v, mask, 0.7)
+    want = pkg.fmha_infer_i8(*(pkg.quantize_tensor(x, a)[0] for x, a in zip((q, k, v), amax)), mask, *amax, o_amax=0.7)
+    assert torch.equal(o, want) and wide.dtype == kind and torch.equal(wide, pkg.dequantize_tensor(o, 0.7, dtype=kind))

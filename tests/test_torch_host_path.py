@@ -63,6 +63,7 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
         "attend": lambda s: pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0, stream=s),
         "full range": lambda s: pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0, stream=s, full_range_p=True),
         "decode": lambda s: pkg.fmha_infer_i8(*attention("cuda:1", 1, 8192), 1.0, 1.0, 1.0, stream=s),
+        "cross": lambda s: pkg.fmha_infer_i8(*attention("cuda:1", 256, 128), 1.0, 1.0, 1.0, stream=s),
         "quantize": lambda s: pkg.quantize_tensor(torch.empty(999, device="cuda:1"), stream=s),
         "quantize by": lambda s: pkg.quantize_tensor(torch.empty(999, device="cuda:1"), 2.0, stream=s),
         "dequantize": lambda s: pkg.dequantize_tensor(torch.empty(999, dtype=torch.int8, device="cuda:1"), 1.0, stream=s),
@@ -71,9 +72,10 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
         "float": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", dtype=torch.float32)[:3], attention("cuda:1")[3], 1.0, stream=s),
         "float, large": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1 << 15, 128, torch.bfloat16)[:3], attention("cuda:1")[3], 1.0, stream=s),
         "float, decode": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 8192, torch.float32)[:3], attention("cuda:1", 1, 8192)[3], 1.0, stream=s),
+        "float, decode as bfloat16": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 8192, torch.bfloat16)[:3], attention("cuda:1", 1, 8192)[3], 1.0, stream=s),
     }
     side, null = torch.cuda.Stream("cuda:1"), torch.cuda.default_stream(1)
-    seen = set()
+    seen, of_entry = set(), {}
     for name, entry in {**entries, **floats}.items():
         for stream in (None, null, side) + ((0, side.cuda_stream) if name in entries else ()):
             entry(stream)
@@ -83,8 +85,11 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
             assert torch.cuda.current_device() == 0 and fake.fake_current_device() == 0, name
             assert torch.cuda.current_stream(0) == torch.cuda.default_stream(0) and torch.cuda.current_stream(1) == null
             seen |= {c[0] for c in got}
+            of_entry[name] = [c[0] for c in got]
     assert {"FMHAInferI8Status", "FMHAInferI8CrossFullRangeP", "FMHAInferI8CrossWithWorkspace", "FMHAInferI8CrossToFloat",
             "FMHAInferI8Cross", "FMHAMeasureAndQuantizeI8", "FMHAQuantizeI8", "FMHADequantizeI8", "FMHADequantizeI8BF16"} <= seen, seen
+    # the attention de-quantises its output itself wherever no key blocks are shared out, over few keys too
+    assert of_entry["float"] == of_entry["float, large"] == ["FMHAMeasureAndQuantizeI8", "FMHAInferI8CrossToFloat"], of_entry
     with torch.cuda.device(1), torch.cuda.stream(side):  # and the other way round, with a current stream of its own
         pkg.fmha_infer_i8(*attention("cuda:0"), 1.0, 1.0, 1.0)
         pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0)
