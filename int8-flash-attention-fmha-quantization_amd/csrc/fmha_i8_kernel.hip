@@ -755,7 +755,17 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // where the scores are converted, -2^30 + S times that variant's c2 >= 2.7e-4 is an exponent below -2.9e5 - so that
   // the row maximum taken behind the MFMAs and the whole softmax need no further look at the mask.  The start values
   // of a tile come from one matrix instruction (masked_start).
-  auto phase_gemm1 = [&](int kb, v16i (&acc)[kKeyTiles], int (&mx)[2], bool masked = false) __attribute__((always_inline)) {
+  // first_read: the operands of tiles 0 and 1, where they have been read already.
+  typedef v4i KOperands[2][kDSteps];  // reads run one key tile ahead of the MFMAs that consume them
+  auto read_k_tile = [&](int kb, int t, KOperands& ka) __attribute__((always_inline)) {
+    const int8_t* lds_k = &lds[kb & (kStages - 1)][0][0];
+#pragma unroll
+    for (int kk = 0; kk < kDSteps; ++kk) {
+      if constexpr (test_build::kNoLdsReads) test_build::undefined(ka[t & 1][kk]);
+      else ka[t & 1][kk] = *reinterpret_cast<const v4i*>(lds_k + k_read_off[kk] + 32 * t * D);
+    }
+  };
+  auto phase_gemm1 = [&](int kb, v16i (&acc)[kKeyTiles], int (&mx)[2], bool masked = false, KOperands* first_read = nullptr) __attribute__((always_inline)) {
     if constexpr (test_build::kNoMfma) {
 #pragma unroll
       for (int t = 0; t < kKeyTiles; ++t) test_build::undefined(acc[t]);
@@ -763,15 +773,9 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
       test_build::undefined(mx[1]);
       return;
     }
-    const int8_t* lds_k = &lds[kb & (kStages - 1)][0][0];
     const v16i zero_c = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    v4i ka[2][kDSteps];  // operand reads run one key tile ahead of the MFMAs that consume them
-    auto read_k = [&](int off) {
-      v4i operand;
-      if constexpr (test_build::kNoLdsReads) test_build::undefined(operand);
-      else operand = *reinterpret_cast<const v4i*>(lds_k + off);
-      return operand;
-    };
+    v4i own[2][kDSteps];
+    auto& ka = first_read != nullptr ? *first_read : own;
     unsigned mw[kKeyTiles];  // masked: the block's mask bits, bit j of word t <-> key 32 t + j of the block
     auto start = [&](int t) __attribute__((always_inline)) {
       const MaskedUnits<BIAS> units;
@@ -784,15 +788,10 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
                                           : (unsigned)__builtin_amdgcn_readfirstlane((int)lds_mask[kb * kKeyTiles + t]);
       start(0);
     }
-#pragma unroll
-    for (int kk = 0; kk < kDSteps; ++kk) ka[0][kk] = read_k(k_read_off[kk]);
+    if (first_read == nullptr) read_k_tile(kb, 0, ka);
 #pragma unroll
     for (int t = 0; t < kKeyTiles; ++t) {
-      if (t + 1 < kKeyTiles) {
-#pragma unroll
-        for (int kk = 0; kk < kDSteps; ++kk)
-          ka[(t + 1) & 1][kk] = read_k(k_read_off[kk] + 32 * (t + 1) * D);
-      }
+      if (t + 1 < kKeyTiles && !(t == 0 && first_read != nullptr)) read_k_tile(kb, t + 1, ka);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kk = 0; kk < kDSteps; ++kk) {
@@ -1031,7 +1030,14 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // registers, which needs the loads of a key block in one place.
   constexpr bool kLoadsInMfmaPhase = !test_build::kStagedLoads || D == 64;
   static_assert(!kLoadsInMfmaPhase || 2 * kRegionsPerWave <= kDSteps, "one tile load per output tile of GEMM 2");
-  auto phase_gemm2_merge = [&](int kb, const v4i (&pk)[kKeyTiles], int k_next, int v_next, bool steady = false) __attribute__((always_inline)) {
+  // first_k: where the operands of tiles 0 and 1 of the GEMM 1 that follows are to be left.  They are read in front of the last tile's
+  // merge, whose sixteen fmas then cover the reads.  The compiler put ten to sixteen of them behind the reads by itself until the loop for
+  // masked keys changed, and two to four in all loops since (the reads got registers that the merge was still using).  Fixed, against
+  // those four, us: B4 H64 S960 d64 with converted scores 70.8 -> 70.1, B8 H32 S1000 d64 71.7 -> 71.1, B16 H16 S2048 d64 238.2 -> 237.9, B4 H16 S1024
+  // d128 24.53 -> 24.49.  At d = 128 partly filled ends and blocks of 64 keys are 0.3 and 0.6 % slower for it (B4 H16 S1000 25.75 -> 25.83,
+  // B2 H16 S1088 24.71 -> 24.85) and keep the compiler's order.
+  constexpr bool kReadsBeforeMerge = D == 64 || (BK == kBlockK && !RAGGED);
+  auto phase_gemm2_merge = [&](int kb, const v4i (&pk)[kKeyTiles], int k_next, int v_next, bool steady = false, KOperands* first_k = nullptr) __attribute__((always_inline)) {
     if constexpr (test_build::kNoMfma) {
       if (kLoadsInMfmaPhase) {
         issue_k(k_next);
@@ -1127,6 +1133,11 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
         else if (u < 2 * kRegionsPerWave) issue_region(vg, v_next, 1, ld_goff_v, u - kRegionsPerWave, steady);
         __builtin_amdgcn_sched_barrier(0);
       }
+    }
+    if (first_k != nullptr) {
+      read_k_tile(kb + 1, 0, *first_k);
+      read_k_tile(kb + 1, 1, *first_k);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) merge_piece(oacc[ob(kDSteps - 1)], kDSteps - 1, j);
@@ -1282,9 +1293,11 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
         pin_scores(acc);
         phase_pack(acc, pk, next_masked);
       }
-      phase_gemm2_merge(i, pk, min(i + 3, last), min(i + kVAhead, last), true);
+      KOperands ka;
+      const bool reads_k = kReadsBeforeMerge && !next_masked;
+      phase_gemm2_merge(i, pk, min(i + 3, last), min(i + kVAhead, last), true, reads_k ? &ka : nullptr);
       if (next_masked) phase_gemm1(i + 1, acc, mx, true);
-      else phase_gemm1(i + 1, acc, mx, false);
+      else phase_gemm1(i + 1, acc, mx, false, reads_k ? &ka : nullptr);
       drop_priority();
     };
     if (active) {
@@ -1352,10 +1365,12 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
         pin_scores(acc);
         phase_pack(acc, pk, next_masked);
       }
-      phase_gemm2_merge(i, pk, min(i + 3, last), min(i + kVAhead, last), true);
+      KOperands ka;
+      const bool reads_k = kReadsBeforeMerge && !next_masked && !FULLP;  // (FULLP: the column sums stand between)
+      phase_gemm2_merge(i, pk, min(i + 3, last), min(i + kVAhead, last), true, reads_k ? &ka : nullptr);
       if (FULLP) phase_colsum(i + 1);
       if (next_masked) phase_gemm1(i + 1, acc, mx, true);
-      else phase_gemm1(i + 1, acc, mx, false);
+      else phase_gemm1(i + 1, acc, mx, false, reads_k ? &ka : nullptr);
       if (FULLP) colsum_written();
       drop_priority();
       staged_writes_done();

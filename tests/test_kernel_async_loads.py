@@ -198,3 +198,41 @@ def test_no_kernel_keeps_anything_in_scratch(assembly_files):
                               open(assembly_files[0]).read()))
     assert sum("_fwd_kernel" in name for name in scratch) == 64 and sum("_few_kernel" in name for name in scratch) > 0
     assert {name: size for name, size in scratch.items() if size != "0"} == {}
+
+
+def _fmas_behind_operand_reads(func_text):
+    """For every loop of a kernel: the fmas between four or more 128-bit LDS reads in a row and the matrix instruction behind
+    them, where there are any."""
+    at, ins, found = {}, [], []
+    for line in func_text.split("\n")[1:]:
+        label, t = re.match(r"^(\.LBB\d+_\d+):", line), line.split(";")[0].strip()
+        if label:
+            at[label.group(1)] = len(ins)
+        elif t and not t.startswith(".") and not t.endswith(":"):
+            ins.append(t)
+            back = re.match(r"s_c?branch\w*\s+(\.LBB\d+_\d+)", t)
+            if back and at.get(back.group(1), len(ins)) < len(ins) - 200:
+                reads = fmas = most = 0
+                for x in ins[at[back.group(1)]:]:
+                    if "mfma" in x:
+                        most, reads, fmas = max(most, fmas if reads >= 4 else 0), 0, 0
+                    elif x.startswith("ds_read_b128"):
+                        reads, fmas = reads + 1, 0
+                    elif x.startswith("v_fma"):
+                        fmas += 1
+                found.append(most)
+    return found
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_the_last_merge_covers_the_first_operand_reads_of_the_next_block(kernels):
+    """Steady-state loops of the 256-row kernel without masked keys: the first K operands are asked for in front of the sixteen fmas of the last
+    output tile.  Where the compiler chose by itself, what changed elsewhere in the kernel could put them behind twelve of those.  (At d = 128
+    partly filled ends and blocks of 64 keys leave it to the compiler.)"""
+    for f in kernels:
+        name = f.split(":")[0]
+        d, block, ragged, full = re.search(r"fwd_kernelILi(\d+)ELi(\d+)ELb.ELb.ELb(.)ELb(.)E", name).groups() if "fwd_kernel" in name else (0,) * 4
+        if d == "64" or (block, ragged) == ("128", "0"):
+            # both halves of the workgroup; with 255 steps (the last template argument) the column sums stand there in the second
+            loops = [n for n in _fmas_behind_operand_reads(f) if n >= 16]
+            assert len(loops) >= (1 if full == "1" else 2), (name, _fmas_behind_operand_reads(f))
