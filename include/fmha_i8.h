@@ -103,7 +103,7 @@ int FMHAInferI8CrossFullRangeP(hipStream_t stream, FMHAParamI8 fmha_param, FMHAC
 
 /* Either of the two calls above with device memory that it may use while it runs.  A call of few query rows (decoding: at
  * most 32 per head) over few heads or many keys then works on the key blocks of a head in several workgroups at once (two
- * kernels are enqueued); the bytes written are the same.  FMHAInferI8CrossWorkspaceBytes says how much it may use, 0 where it
+ * kernels are enqueued); the bytes written are the same.  FMHAInferI8CrossWorkspaceBytes says how much it wants, 0 where it
  * would not use any.  workspace: 16-byte aligned, contents do not matter, the caller's again once the call's work on the
  * stream has ended; NULL or too small is not an error: the call is then the plain one.  full_range_p: nonzero for
  * FMHAInferI8CrossFullRangeP. */

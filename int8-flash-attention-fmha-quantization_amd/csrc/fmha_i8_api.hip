@@ -224,10 +224,10 @@ int rows_of(const KernelCost& kernel) {
 bool few_takes(int rows, int head_dim, int block_keys) {
   return rows <= fmha_i8_gfx950::kFewRows && !(head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK);
 }
-Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys, bool with_few = true) {
+Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
   Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
-    if (kernel.row_groups == kFew && !(with_few && few_takes(rows, head_dim, block_keys))) continue;
+    if (kernel.row_groups == kFew && !few_takes(rows, head_dim, block_keys)) continue;
     // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
     // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 13.9 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with
     // 16 heads 13.1 and 12.6; d64: 11.7 either way).  Its step is one group's less a little, so that it is taken.
@@ -290,8 +290,7 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
 // Up to sixteen rows both sides are fmha_i8_few_kernel's, or the split kernel's second group's against it; plain -> shared out: d64 B8 H16
 // Sq1 S2048 8.9 -> 9.4 us, S8192 28.9 -> 28.9, H64 S2048 8.7 -> 7.6, H16 S1024 5.8 -> 7.4, H16 S4096 14.7 -> 8.6; d128 B4 H16 Sq4 S1984
 // 14.4 -> 12.0, B8 H16 Sq1 S1984 14.8 -> 16.8.
-// with_few = false: by the split kernel's costs alone, the shapes for which a workspace has always been asked.
-PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys, bool with_few = true) {
+PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   using namespace fmha_i8_gfx950;
   PartPlan plan;
   const int blocks = (a.seq_len_kv + block_keys - 1) / block_keys, rounds = (blocks + kSplitKeys - 1) / kSplitKeys;
@@ -301,9 +300,9 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys, bool wit
   const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const bool one_group = a.seq_len_q > kFewRows;
   const long long merge = 250 + 80 * ((blocks - 1) / 32) + (one_group ? 120 + 6 * blocks : 0) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
-  const KernelCost& kernel = with_few && !one_group ? kFewCost : kOneGroupCost;
+  const KernelCost& kernel = !one_group ? kFewCost : kOneGroupCost;
   const auto& c = kernel.cost[a.head_dim == 128][block_keys == kBlockK];
-  long long least = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys, with_few).cost;
+  long long least = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys).cost;
   least = (least > memory ? least : memory) * 20 / 21;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
@@ -446,12 +445,8 @@ size_t FMHAInferI8CrossWorkspaceBytes(FMHACrossAttnDescriptor desc) {
   if ((desc.head_dim != 64 && desc.head_dim != 128) || desc.seq_len_kv <= 0 || desc.seq_len_kv > 65536 || desc.seq_len_q <= 0 ||
       desc.batch_num <= 0 || desc.head_num <= 0)
     return 0;
-  // What a call may use: what its own choice takes, or what the split kernel's costs alone would (see part_plan_of).
-  for (const bool with_few : {true, false}) {
-    const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv), with_few);
-    if (plan.rounds_per_part > 0) return plan.bytes;
-  }
-  return 0;
+  const PartPlan plan = part_plan_of(desc, block_keys_of(desc.seq_len_kv));
+  return plan.rounds_per_part > 0 ? plan.bytes : 0;
 #else
   return 0;
 #endif

@@ -72,6 +72,7 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
         "float": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", dtype=torch.float32)[:3], attention("cuda:1")[3], 1.0, stream=s),
         "float, large": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1 << 15, 128, torch.bfloat16)[:3], attention("cuda:1")[3], 1.0, stream=s),
         "float, decode": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 8192, torch.float32)[:3], attention("cuda:1", 1, 8192)[3], 1.0, stream=s),
+        "float, decode over fewer keys": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 656, torch.float32)[:3], attention("cuda:1", 1, 656)[3], 1.0, stream=s),
         "float, decode as bfloat16": lambda s: pkg.fmha_infer_from_float(*attention("cuda:1", 1, 8192, torch.bfloat16)[:3], attention("cuda:1", 1, 8192)[3], 1.0, stream=s),
     }
     side, null = torch.cuda.Stream("cuda:1"), torch.cuda.default_stream(1)
@@ -88,8 +89,8 @@ def test_work_is_queued_on_the_device_of_the_tensors(fake):
             of_entry[name] = [c[0] for c in got]
     assert {"FMHAInferI8Status", "FMHAInferI8CrossFullRangeP", "FMHAInferI8CrossWithWorkspace", "FMHAInferI8CrossToFloat",
             "FMHAInferI8Cross", "FMHAMeasureAndQuantizeI8", "FMHAQuantizeI8", "FMHADequantizeI8", "FMHADequantizeI8BF16"} <= seen, seen
-    # the attention de-quantises its output itself wherever no key blocks are shared out, over few keys too
-    assert of_entry["float"] == of_entry["float, large"] == ["FMHAMeasureAndQuantizeI8", "FMHAInferI8CrossToFloat"], of_entry
+    # the attention de-quantises its output itself wherever no key blocks are shared out, over few keys and in decoding too
+    assert of_entry["float"] == of_entry["float, large"] == of_entry["float, decode over fewer keys"] == ["FMHAMeasureAndQuantizeI8", "FMHAInferI8CrossToFloat"], of_entry
     with torch.cuda.device(1), torch.cuda.stream(side):  # and the other way round, with a current stream of its own
         pkg.fmha_infer_i8(*attention("cuda:0"), 1.0, 1.0, 1.0)
         pkg.fmha_infer_i8(*attention("cuda:1"), 1.0, 1.0, 1.0)
