@@ -253,7 +253,7 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
   const int heads = a.batch_num * a.head_num, rows = a.seq_len_q, blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
   const Choice whole = row_groups_of(a, block_keys);
   pieces[0] = {whole.row_groups, 0, heads, 0, rows};
-  if (whole.cost < 0 || rows <= 32) return 1;
+  if (whole.cost < 0 || rows <= 32 || fmha_i8_gfx950::test_build::forced_route() == fmha_i8_gfx950::test_build::kOneLaunch) return 1;
   constexpr long long kLaunch = 290;
   long long least = whole.cost * 19 / 20;
   int count = 1;
@@ -509,6 +509,11 @@ int FMHAInferI8DebugLaunches(FMHACrossAttnDescriptor desc, int* first_heads, int
   *first_heads = pieces[0].heads;
   *first_rows = pieces[0].end_row;
   return count;
+}
+// Test build only: the kernel of the second launch, as FMHAInferI8DebugRoute names it, or -1.
+int FMHAInferI8DebugSecondKernel(FMHACrossAttnDescriptor desc) {
+  Piece pieces[2];
+  return pieces_of(desc, block_keys_of(desc.seq_len_kv), pieces) == 2 ? pieces[1].row_groups : -1;
 }
 #endif
 

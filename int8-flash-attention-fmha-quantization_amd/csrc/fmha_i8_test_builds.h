@@ -31,8 +31,8 @@
 //                        nothing else shows it.
 //   FMHA_FORCED_ROUTE    exports FMHAInferI8DebugRoute(n), after which calls of more than one key block are served by the
 //                        kernel with n groups of 32 rows per workgroup (1, 2, 4; 0: 256 rows) whatever their size, with n = 16
-//                        by the one of sixteen rows where it takes them, or, with n = -2, calls with a workspace share their key blocks out whenever they can (-1: the library's own
-//                        choice): for tests of one kernel at small sizes, and for re-measuring the costs that the choice rests on
+//                        by the one of sixteen rows where it takes them, or, with n = -2, calls with a workspace share their key blocks out whenever they can, with n = -3, no
+//                        call takes two launches (-1: the library's own choice): for tests of one kernel at small sizes, and for re-measuring the costs that the choice rests on
 //   FMHA_LOOP_PAD_A=n    n s_nops between the 64-byte boundary in front of the steady-state loop of wavefronts 0..3 and
 //                        the loop (the kernel's own choice otherwise): for re-measuring what the placement costs
 #pragma once
@@ -118,7 +118,7 @@ constexpr int kLoopPadA = -1;  // the kernel's own choice
 #endif
 
 // Which kernel serves a call (see FMHA_FORCED_ROUTE)
-constexpr int kOwnChoice = -1, kSharedOut = -2;
+constexpr int kOwnChoice = -1, kSharedOut = -2, kOneLaunch = -3;
 #ifdef FMHA_FORCED_ROUTE
 inline int g_route = kOwnChoice;
 inline int forced_route() { return g_route; }

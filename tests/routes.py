@@ -5,8 +5,9 @@ import ctypes as C
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-OWN_CHOICE, SHARED_OUT = -1, -2
+OWN_CHOICE, SHARED_OUT, ONE_LAUNCH = -1, -2, -3
 ROUTES = {256: 0, 128: 4, 64: 2, 32: 1}  # query rows per workgroup -> FMHAInferI8DebugRoute
+FEW = 16  # the kernel of sixteen rows: its rows, and its number there
 _loaded = {}
 
 
@@ -51,7 +52,13 @@ def routes_of(q, k):
     """Those that a call has: a single key block is the 256-row kernel's."""
     if k.shape[2] <= (128 if (k.shape[2] + 63) // 64 % 2 == 0 else 64):
         return [("rows 256", ROUTES[256])]
-    return [("rows %d" % rows, route) for rows, route in ROUTES.items()] + ([("shared out", SHARED_OUT)] if q.shape[2] <= 32 else [])
+    return ([("rows %d" % rows, route) for rows, route in ROUTES.items()] + ([("rows 16", FEW)] if few_takes(q.shape[2], k.shape[2], k.shape[3]) else []) +
+            ([("shared out", SHARED_OUT)] if q.shape[2] <= 32 else []))
+
+
+def few_takes(rows, keys, d):
+    """Whether fmha_i8_few_kernel serves such a call: not at d = 128 in blocks of 128 keys."""
+    return rows <= FEW and not (d == 128 and (keys + 63) // 64 % 2 == 0)
 
 
 def check_every_route(pkg, t, scales, want, full_range_p=False):

@@ -30,7 +30,7 @@ def checked(pkg):
 def test_checked_build_counts_nothing_on_any_shape(pkg, orc, checked, dev):
     """Every kernel on every shape it can serve, shared-out key blocks and their merge among them."""
     import torch
-    served = {name: 0 for name in ["rows %d" % r for r in routes.ROUTES] + ["shared out"]}
+    served = {name: 0 for name in ["rows %d" % r for r in [*routes.ROUTES, routes.FEW]] + ["shared out"]}
     assert checked.FMHAInferI8DebugOutOfBounds() == 0  # (also clears the counter)
     rng = np.random.default_rng(77)
     shapes = [(3, 3, 319, 3, 64), (1, 1, 1, 1, 128), (2, 2, 70, 70, 128), (2, 1, 300, 129, 64), (1, 2, 64, 64, 64),
@@ -38,7 +38,9 @@ def test_checked_build_counts_nothing_on_any_shape(pkg, orc, checked, dev):
               (2, 1, 40, 15, 64), (2, 1, 40, 16, 128), (2, 1, 40, 17, 64), (2, 1, 40, 31, 128), (1, 1, 40, 4100, 64),
               # few query rows, whose key blocks can be shared out: whole and partly filled blocks and rounds, one to 32 rows
               (1, 2, 1, 2048, 128), (2, 3, 5, 1030, 64), (1, 1, 8, 1089, 64), (3, 4, 2, 1027, 128), (1, 2, 32, 4096, 128),
-              (1, 3, 17, 5000, 64), (1, 2, 3, 1100, 128), (1, 1, 31, 513, 128), (1, 4, 7, 8300, 64), (2, 2, 1, 640, 128), (1, 1, 1, 320, 64)]
+              (1, 3, 17, 5000, 64), (1, 2, 3, 1100, 128), (1, 1, 31, 513, 128), (1, 4, 7, 8300, 64), (2, 2, 1, 640, 128), (1, 1, 1, 320, 64),
+              # at most sixteen, on the kernel for those
+              (2, 2, 16, 129, 64), (1, 3, 15, 256, 64), (2, 1, 1, 1000, 64), (1, 2, 16, 3000, 64), (2, 2, 1, 65, 128), (1, 2, 16, 577, 128), (1, 3, 9, 1984, 128)]
     for _ in range(40):
         S = int(rng.choice([rng.integers(1, 130), rng.integers(1, 700), rng.integers(500, 2600), 64 * rng.integers(1, 40)]))
         Sq = S if rng.random() < 0.4 else int(rng.choice([rng.integers(1, 70), rng.integers(1, 600), rng.integers(200, 1500)]))

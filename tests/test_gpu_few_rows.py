@@ -9,12 +9,10 @@ import pytest
 import routes
 from test_gpu_split_kernel import CSRC
 
-FEW = 16  # FMHAInferI8DebugRoute
-
 # (B, H, Sq, S, d): one round of four key blocks to many, rounds that are not full, both block sizes, ragged ends, 1 to 16 rows, mask
 # rows of more than one classification pass; d128 in blocks of 128 keys is served with shared-out blocks alone
 SHAPES = [
-    (2, 3, 1, 129, 64), (1, 2, 16, 256, 64), (2, 2, 15, 1100, 64), (1, 3, 5, 8300, 64), (3, 2, 2, 65, 64), (2, 3, 16, 1000, 64), (40, 8, 3, 448, 64),
+    (2, 3, 1, 129, 64), (1, 2, 16, 256, 64), (2, 2, 15, 1100, 64), (1, 3, 5, 8300, 64), (3, 2, 2, 65, 64), (2, 3, 16, 1000, 64), (40, 8, 3, 448, 64), (8, 16, 1, 2048, 64),
     (2, 3, 1, 65, 128), (1, 2, 16, 320, 128), (2, 2, 7, 1984, 128), (1, 3, 16, 8240, 128), (40, 8, 1, 700, 128),
     (2, 2, 1, 513, 128), (1, 3, 16, 2048, 128), (2, 1, 9, 8190, 128),
 ]
@@ -51,14 +49,14 @@ def test_same_bytes_as_the_kernel_of_256_row_workgroups(pkg, dev, shape, full_ra
         size = want.numel()
         for name in ("routed", "checked"):
             lib = routes.library(pkg, name)
-            for route in (FEW, routes.SHARED_OUT):
+            for route in (routes.FEW, routes.SHARED_OUT):
                 o = torch.full((size + 256,), 77, dtype=torch.int8, device=dev)
                 if routes.attend(pkg, lib, route, t, scales, o, full_range_p):
                     assert torch.equal(o[:size].view_as(want), want) and (o[size:] == 77).all(), (name, route, pad)
             for dtype in (torch.bfloat16, torch.float32):  # beside the de-quantised output
                 o = torch.full((size + 256,), 77, dtype=torch.int8, device=dev)
                 wide = torch.full((size + 256,), 3.0, dtype=dtype, device=dev)
-                routes.attend(pkg, lib, FEW, t, scales, o, full_range_p, wide)
+                routes.attend(pkg, lib, routes.FEW, t, scales, o, full_range_p, wide)
                 assert torch.equal(o[:size].view_as(want), want) and (o[size:] == 77).all(), (name, dtype, pad)
                 assert torch.equal(wide[:size].view_as(want), pkg.dequantize_tensor(want, o_amax, dtype=dtype)) and (wide[size:] == 3).all(), (name, pad)
         assert lib.FMHAInferI8DebugOutOfBounds() == 0

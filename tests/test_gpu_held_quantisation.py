@@ -56,10 +56,10 @@ def test_edges_of_the_forms(pkg, dev, dtype_name, patience):
 
 
 @pytest.mark.parametrize("dtype_name", ["float32", "bfloat16"])
-@pytest.mark.parametrize("kind", ["nan", "many_nan", "inf", "minus_inf_and_nan", "zero", "denormal", "large", "most_negative"])
+@pytest.mark.parametrize("kind", ["nan", "many_nan", "inf", "minus_inf_and_nan", "zero", "denormal", "large", "most_negative", "nan_but_one"])
 def test_special_values(pkg, dev, kind, dtype_name):
     import torch
-    for n in (40003, 1000003, 27 << 20):  # the last: two launches
+    for n in (40003, 1000003, (27 if dtype_name == "float32" else 53) << 20):  # the last: two launches
         x = torch.randn(n, device=dev) * {"denormal": 1e-39, "large": 5e37, "zero": 0.0}.get(kind, 1.0)
         if kind == "nan":
             x[n // 3], x[n // 3 + 1] = float("nan"), -9.0
@@ -71,6 +71,9 @@ def test_special_values(pkg, dev, kind, dtype_name):
             x[n // 2], x[7] = float("-inf"), float("nan")
         elif kind == "most_negative":
             x[n - 2] = -77.0
+        elif kind == "nan_but_one":  # all shares but one have nothing else
+            x.fill_(float("nan"))
+            x[n // 2] = -3.0
         print(kind, dtype_name, n, flush=True)
         check(pkg, pkg.load_library(), [x.to(getattr(torch, dtype_name))])
 

@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("full_range_p", [False, True], ids=["P_128_steps", "P_255_steps"])
 @pytest.mark.parametrize("scale", [0.05, 30.0], ids=["scores_as_floats", "scores_converted"])
 @pytest.mark.parametrize("S,d", [(256, 128), (256, 64), (320, 128), (320, 64), (300, 128), (429, 64)])  # blocks of 128 and 64 keys, ragged ends
-def test_the_only_unmasked_key_is_the_output(pkg, dev, S, d, scale, full_range_p):
+@pytest.mark.parametrize("Sq", [33, 16])  # (the kernel of sixteen rows serves no more)
+def test_the_only_unmasked_key_is_the_output(pkg, dev, Sq, S, d, scale, full_range_p):
     import torch
     # edges of quads, of the 32-key tiles of a matrix instruction and of the blocks
     keys = sorted({k for k in (0, 3, 4, 7, 8, 31, 32, 36, 63, 64, 95, 96, 127, 128, 191, 192, 255, 256, 287, S - 32, S - 2, S - 1) if k < S})
-    B, H, Sq = len(keys), 2, 33
+    B, H = len(keys), 2
     g = torch.Generator(device=dev)
     g.manual_seed(S + d)
     q = torch.full((B, H, Sq, d), 127, dtype=torch.int8, device=dev)
@@ -26,5 +27,5 @@ def test_the_only_unmasked_key_is_the_output(pkg, dev, S, d, scale, full_range_p
         k[b, :, key] = -1  # (a masked key enters the row maximum as the integer -1000000: this score is above it)
         mask[b, key] = 0
     want = torch.stack([v[b, :, key] for b, key in enumerate(keys)])[:, :, None, :].expand(B, H, Sq, d).contiguous()
-    print(S, d, scale, full_range_p, flush=True)
+    print(Sq, S, d, scale, full_range_p, flush=True)
     routes.check_every_route(pkg, (q, k, v, mask), (scale, 1.0, 1.0, 1.0), want, full_range_p)

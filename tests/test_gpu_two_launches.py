@@ -16,10 +16,12 @@ SHAPES = [
     (2, 48, 700, 1000, 128, "heads"), (4, 16, 2108, 2108, 64, "rows"), (7, 16, 537, 1500, 64, "rows"), (3, 32, 1472, 1472, 128, "heads"),
     (4, 20, 790, 1100, 128, "rows"),
 ]
+# (B, H, Sq, S, d): 1 to 16 rows are left over, for the kernel of sixteen rows (d = 64, and d = 128 in blocks of 64 keys), with ragged ends too
+FEW_LEFT = [(4, 16, 2049, 2049, 64), (2, 32, 2064, 2048, 64), (8, 8, 2056, 2500, 64), (4, 16, 2049, 1984, 128), (4, 16, 1040, 2111, 128), (8, 16, 513, 1030, 128)]
 
 
 def launches(pkg, lib, shape):
-    B, H, Sq, S, d, _ = shape
+    B, H, Sq, S, d = shape[:5]
     heads, rows = C.c_int(), C.c_int()
     lib.FMHAInferI8DebugLaunches.argtypes = [pkg.FMHACrossAttnDescriptor, C.c_void_p, C.c_void_p]
     count = lib.FMHAInferI8DebugLaunches(pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d), C.addressof(heads), C.addressof(rows))
@@ -29,11 +31,27 @@ def launches(pkg, lib, shape):
 @pytest.mark.parametrize("full_range_p", [False, True], ids=["P_128_steps", "P_255_steps"])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "B%d_H%d_Sq%d_S%d_d%d_by_%s" % s)
 def test_two_launches_write_what_one_writes(pkg, dev, shape, full_range_p):
-    import torch
     B, H, Sq, S, d, by = shape
-    lib = routes.library(pkg)
-    count, heads, rows = launches(pkg, lib, shape)
+    count, heads, rows = launches(pkg, routes.library(pkg), shape)
     assert count == 2 and (heads < B * H, rows < Sq) == (by == "heads", by == "rows"), (count, heads, rows)
+    check(pkg, dev, shape, full_range_p)
+
+
+@pytest.mark.parametrize("full_range_p", [False, True], ids=["P_128_steps", "P_255_steps"])
+@pytest.mark.parametrize("shape", FEW_LEFT, ids=lambda s: "B%d_H%d_Sq%d_S%d_d%d" % s)
+def test_few_rows_left_over(pkg, dev, shape, full_range_p):
+    B, H, Sq, S, d = shape
+    lib = routes.library(pkg)
+    lib.FMHAInferI8DebugSecondKernel.argtypes = [pkg.FMHACrossAttnDescriptor]
+    count, heads, rows = launches(pkg, lib, shape)
+    assert count == 2 and heads == B * H and 1 <= Sq - rows <= 16 and lib.FMHAInferI8DebugSecondKernel(pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d)) == routes.FEW
+    check(pkg, dev, shape, full_range_p)
+
+
+def check(pkg, dev, shape, full_range_p):
+    import torch
+    B, H, Sq, S, d = shape[:5]
+    lib = routes.library(pkg)
     g = torch.Generator(device=dev)
     g.manual_seed(Sq)
     t = [torch.randint(-127, 128, (B, H, n, d), generator=g, device=dev, dtype=torch.int8) for n in (Sq, S, S)]

@@ -50,13 +50,6 @@ def events_us(torch, call, calls):
     return best
 
 
-FEW = 16  # the kernel of sixteen rows, as FMHAInferI8DebugRoute's number and as its rows
-
-
-def few_takes(rows, s, d):
-    return rows <= FEW and not (d == 128 and (s + 63) // 64 % 2 == 0)
-
-
 def time_route(pkg, lib, routes, route, shape, calls=100):
     """Microseconds per call, or None where the call does not have that route.  No masked key, uniform random bytes."""
     import torch
@@ -90,13 +83,47 @@ def time_shapes(shapes):
     import routes
     pkg = g.load_package()
     lib = routes.library(pkg)
-    names = list(routes.ROUTES) + [FEW]
+    names = list(routes.ROUTES) + [routes.FEW]
     print("| B, H, Sq, S, d | %s | key blocks shared out | the library's choice |" % " | ".join("%d rows" % r for r in names))
     print("|" + "---|" * (len(names) + 3))
     for shape in shapes:
-        us = [time_route(pkg, lib, routes, routes.ROUTES.get(r, FEW), shape) if r != FEW or few_takes(*shape[2:]) else None for r in names]
+        us = [time_route(pkg, lib, routes, routes.ROUTES.get(r, routes.FEW), shape) if r != routes.FEW or routes.few_takes(*shape[2:]) else None for r in names]
         us += [time_route(pkg, lib, routes, route, shape) for route in (routes.SHARED_OUT, routes.OWN_CHOICE)]
         print("| %s | %s |" % (", ".join(map(str, shape)), " | ".join("-" if u is None else "%.2f" % u for u in us)), flush=True)
+
+
+def two_launches(count):
+    """Random shapes that the library serves by two launches: one launch by the kernel it would choose then, and the two."""
+    import ctypes as C
+    import math
+    import random
+
+    import torch  # noqa: F401
+    import __graft_entry__ as g
+    import routes
+    pkg = g.load_package()
+    lib = routes.library(pkg)
+    lib.FMHAInferI8DebugLaunches.argtypes = [pkg.FMHACrossAttnDescriptor, C.c_void_p, C.c_void_p]
+    rng, ratios, looked_at = random.Random(7), [], 0
+    print("| B, H, Sq, S, d | first launch | one launch | two launches | two / one |")
+    print("|" + "---|" * 5)
+    while len(ratios) < count:
+        B, H, S, d = rng.randint(1, 8), rng.choice((4, 8, 12, 16, 20, 24, 32, 48)), int(2 ** rng.uniform(8, 12)), rng.choice((64, 128))
+        Sq = S if rng.random() < 0.6 else int(2 ** rng.uniform(8, 12))
+        if B * H * ((Sq + 255) // 256) < 100 or B * H * Sq * S * d > 1 << 36:
+            continue
+        looked_at += 1
+        heads, rows = C.c_int(), C.c_int()
+        if lib.FMHAInferI8DebugLaunches(pkg.FMHACrossAttnDescriptor(B, Sq, S, H, d), C.addressof(heads), C.addressof(rows)) != 2:
+            continue
+        one, two = (time_route(pkg, lib, routes, route, (B, H, Sq, S, d), calls=40) for route in (routes.ONE_LAUNCH, routes.OWN_CHOICE))
+        ratios.append(two / one)
+        first = "%d of %d heads" % (heads.value, B * H) if heads.value < B * H else "%d rows" % rows.value
+        print("| %d, %d, %d, %d, %d | %s | %.2f | %.2f | %.3f |" % (B, H, Sq, S, d, first, one, two, two / one), flush=True)
+    ratios.sort()
+    mean = math.exp(sum(math.log(r) for r in ratios) / len(ratios))
+    print("\n%d of %d shapes take two launches; two / one: geometric mean %.3f, least %.3f, median %.3f, most %.3f" %
+          (len(ratios), looked_at, mean, ratios[0], ratios[len(ratios) // 2], ratios[-1]))
 
 
 def kernel_costs():
@@ -111,10 +138,10 @@ def kernel_costs():
     print("|" + "---|" * 6)
     for d in (64, 128):
         for block in (64, 128):
-            for rows, route in list(routes.ROUTES.items()) + ([(FEW, FEW)] if few_takes(1, block, d) else []):
+            for rows, route in list(routes.ROUTES.items()) + ([(routes.FEW, routes.FEW)] if routes.few_takes(1, block, d) else []):
                 for heads in (8, 16):
                     # (sixteen workgroups per head, or with sixteen rows one workgroup per head)
-                    shape = (1, 16 * heads, 1) if rows == FEW else (1, heads, 16 * rows)
+                    shape = (1, 16 * heads, 1) if rows == routes.FEW else (1, heads, 16 * rows)
                     us = [time_route(pkg, lib, routes, route, (*shape, s, d)) for s in keys[block]]
                     rounds = [(s // block + 3) // 4 if rows <= 64 else s // block for s in keys[block]]
                     step = (us[3] - us[0]) / (rounds[3] - rounds[0])
@@ -130,10 +157,13 @@ def main():
     ap.add_argument("--preheat-ms", type=float, default=100.0)
     ap.add_argument("--compare", action="store_true", help="compare the output bytes with the shipped library's")
     ap.add_argument("--kernel-costs", action="store_true", help="each kernel's time against the number of key blocks")
+    ap.add_argument("--two-launches", type=int, default=0, help="this many random shapes that take two launches, against one launch")
     ap.add_argument("--shapes", default=None, help="\"B,H,Sq,S,d B,H,Sq,S,d ...\" on every kernel")
     args = ap.parse_args()
     if args.kernel_costs:
         return kernel_costs()
+    if args.two_launches:
+        return two_launches(args.two_launches)
     if args.shapes:
         return time_shapes([tuple(int(x) for x in shape.split(",")) for shape in args.shapes.split()])
 
