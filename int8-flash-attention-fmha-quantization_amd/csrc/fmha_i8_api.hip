@@ -188,8 +188,9 @@ hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, con
 }
 // What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
 // split kernel.  Microseconds * 100 beyond the launch (2.9 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
-// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs); measurements differ by 4 %.
-// With all CUs at work the first two take up to 34 and 11 % longer per block (the shader clock drops).
+// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs); measurements differ by 4 %.  The last kernel's
+// entries at d = 64 are its line up to 2048 keys: at 4096 a call of 128 heads, each with its own keys, takes 6 % longer (the memory).
+// With all CUs at work the first two take up to 36 and 14 % longer per block (the shader clock drops).
 struct KernelCost {
   int row_groups, keys_per_round;
   struct { int start, step; } cost[2][2];
@@ -224,18 +225,22 @@ int rows_of(const KernelCost& kernel) {
 bool few_takes(int rows, int head_dim, int block_keys) {
   return rows <= fmha_i8_gfx950::kFewRows && !(head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK);
 }
+// With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a round is 128 KB
+// (B8 H16 Sq1 S2048 d128: 15.9 us with one group, 14.1 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with 16 heads 13.1 and
+// 12.6; at d64 11.7 either way): there it takes one group's place.  128 heads measure 0.5 + 2.6 us a round, the memory's share in it;
+// the price is one group's, 1 % lower: without that, calls of two rounds would share their key blocks out (H16 Sq1 S1024 8.2 us plain,
+// 8.5 shared out).
+bool second_group_fetches(int rows, int head_dim, int block_keys) { return rows <= 32 && head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK; }
+constexpr KernelCost kFetchingCost{2, 4, {{}, {{}, {95, 240}}}};
 Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
   Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
     if (kernel.row_groups == kFew && !few_takes(rows, head_dim, block_keys)) continue;
-    // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a
-    // round is 128 KB (B8 H16 Sq1 S2048 d128: 15.8 us with one group, 13.9 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with
-    // 16 heads 13.1 and 12.6; d64: 11.7 either way).  Its step is one group's less a little, so that it is taken.
-    const bool helper = rows <= 32 && kernel.row_groups == 2;
-    if (helper && !(head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK)) continue;
-    const int rounds = (blocks + kernel.keys_per_round - 1) / kernel.keys_per_round;
+    const bool fetching = second_group_fetches(rows, head_dim, block_keys);
+    if (rows <= 32 && kernel.row_groups == (fetching ? 1 : 2)) continue;
+    const KernelCost& price = fetching && kernel.row_groups == 2 ? kFetchingCost : kernel;
     const long long per_cu = (heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)) + kComputeUnits - 1) / kComputeUnits;
-    const long long cost = per_cu * (helper ? 95 + 240 * rounds : cost_of_workgroup(kernel, head_dim, blocks, block_keys));
+    const long long cost = per_cu * cost_of_workgroup(price, head_dim, blocks, block_keys);
     if (best.cost < 0 || cost < best.cost) best = {kernel.row_groups, cost};
   }
   return best;
