@@ -236,3 +236,20 @@ def test_the_last_merge_covers_the_first_operand_reads_of_the_next_block(kernels
             # both halves of the workgroup; with 255 steps (the last template argument) the column sums stand there in the second
             loops = [n for n in _fmas_behind_operand_reads(f) if n >= 16]
             assert len(loops) >= (1 if full == "1" else 2), (name, _fmas_behind_operand_reads(f))
+
+
+def _jumps_behind_the_end(func_text):
+    """Blocks behind the last `s_endpgm` of a kernel that do nothing but jump back."""
+    tail, alone = func_text.split("s_endpgm")[-1].split(".section")[0], []
+    for block in re.split(r"\n(?=\.LBB\d+_\d+:)", tail)[1:]:
+        ins = [t for t in (line.split(";")[0].strip() for line in block.split("\n")[1:]) if t and not t.startswith(".")]
+        if len(ins) == 1 and ins[0].startswith("s_branch"):
+            alone.append(block.split(":")[0])
+    return alone
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_the_first_block_without_masked_keys_is_not_reached_by_way_of_the_end(kernels):
+    """GEMM 1 of the first key block has two forms; the usual one, without masked keys, is reached without a jump to the end of the kernel and
+    back, whose instruction fetch the smallest calls wait for."""
+    assert {f.split(":")[0]: _jumps_behind_the_end(f) for f in kernels if "fwd_kernel" in f.split(":")[0] and _jumps_behind_the_end(f)} == {}
