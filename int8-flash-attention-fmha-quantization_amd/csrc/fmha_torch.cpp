@@ -323,9 +323,9 @@ PyObject* dequantize_tensor(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // (q, k, v, padding_mask, o_amax, out_dtype, stream, full_range_p) -> (O, int8 O, (q_amax, k_amax, v_amax)), or the status
 //
-// Launches: abs-max of the three tensors, their quantisation, the attention, which may de-quantise its output too.  The attention's scales
-// are call arguments, so the host needs the three maxima in between: the quantising kernel writes them to pinned memory
-// as its first act and the host, which polls for them, has the attention queued while the quantisation still runs.
+// Launches: abs-max of the three tensors and their quantisation, in one or two, and the attention, which may de-quantise its output too.  The
+// attention's scales are call arguments, so the host needs the three maxima in between: the quantising kernel writes them to pinned memory
+// as soon as it has them, and the host, which polls for them, has the attention queued while the int8 values are still being written.
 PyObject* infer_from_float(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!count_is(n, 8)) return nullptr;
   return guarded([&]() -> PyObject* {
