@@ -1244,6 +1244,13 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     for (int t = 0; t < kKeyTiles; ++t) asm volatile("" : "=v"(acc[t]));
     asm volatile("" : "=v"(mx[0]), "=v"(mx[1]));
   };
+  // Likewise P, where the softmax is skipped: otherwise the general loop, which every call takes for its last key block, starts with sixteen
+  // registers of zeros and carries them (us: B1 H2 S128 d64 4.25 -> 4.17, B2 H4 S256 6.33 -> 6.21, B8 H12 S512 10.61 -> 10.50, with masked keys
+  // 11.50 -> 11.34, B4 H16 S1024 d128 24.59 -> 24.51; its registers 228 -> 212).
+  auto forget_p = [&](v4i (&pk)[kKeyTiles]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kKeyTiles; ++t) asm volatile("" : "=v"(pk[t]));
+  };
   auto gemm1_of = [&](int kb) __attribute__((always_inline)) {  // GEMM 1 of block 0, which may or may not have masked keys
     // (The form without masked keys falls through.  Left alone, the compiler reaches it by a jump to the end of the kernel and back, and in
     // the smallest calls that fetch is seen: B1 H2 S128 d64 4.27 us, 4.24 so; with masked keys 4.34 and 4.36.)
@@ -1328,6 +1335,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
       wait_v_for_colsum_a();
       barrier_odd();                           // barrier 2i+1
       if (work) phase_softmax(i, cls, acc, pk, mx);
+      else forget_p(pk);
       issue_after_softmax_a(i);
       wait_tiles(true);
       barrier();                               // barrier 2i+2
@@ -1402,6 +1410,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
       wait_tiles(false);
       barrier();                               // barrier 2i+2
       if (work) phase_softmax(i, cls, acc, pk, mx);
+      else forget_p(pk);
       issue_after_softmax(i);
       wait_v_for_colsum_b();
       barrier_odd();                           // barrier 2i+3

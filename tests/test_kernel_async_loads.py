@@ -253,3 +253,25 @@ def test_the_first_block_without_masked_keys_is_not_reached_by_way_of_the_end(ke
     """GEMM 1 of the first key block has two forms; the usual one, without masked keys, is reached without a jump to the end of the kernel and
     back, whose instruction fetch the smallest calls wait for."""
     assert {f.split(":")[0]: _jumps_behind_the_end(f) for f in kernels if "fwd_kernel" in f.split(":")[0] and _jumps_behind_the_end(f)} == {}
+
+
+def _runs_of_moves(func_text):
+    """Lengths of the runs of eight and more register moves (of a register or 0) in a kernel, address arithmetic between them not counted."""
+    runs, n = [], 0
+    for line in func_text.split("\n")[1:]:
+        t = line.split(";")[0].strip()
+        if re.match(r"v_mov_b(32|64)(_e32)? v(\d+|\[\d+:\d+\]), (v(\d+|\[\d+:\d+\])|0)$", t):
+            n += 1
+        elif t and not t.startswith(".p2align") and not re.match(r"s_(?!c?branch|barrier)|v_or_b32", t):
+            runs += [n] if n >= 8 else []
+            n = 0
+    return runs
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_the_general_loop_carries_no_p_of_blocks_that_have_none(kernels):
+    """P of a key block without an unmasked key is never used; where the general loop does not say so, the compiler starts it at zero, 14 to 24
+    moves in front of the loop that every call takes for its last key block.  The last run of moves is then that one, and not the start of O (some
+    32 registers or more)."""
+    late = {f.split(":")[0]: _runs_of_moves(f) for f in kernels if "fwd_kernel" in f.split(":")[0]}
+    assert late and {name: runs for name, runs in late.items() if runs[-1] < 30} == {}
