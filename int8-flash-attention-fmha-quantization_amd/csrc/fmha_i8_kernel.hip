@@ -1038,9 +1038,9 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // merge, whose sixteen fmas then cover the reads.  The compiler put ten to sixteen of them behind the reads by itself until the loop for
   // masked keys changed, and two to four in all loops since (the reads got registers that the merge was still using).  Fixed, against
   // those four, us: B4 H64 S960 d64 with converted scores 70.8 -> 70.1, B8 H32 S1000 d64 71.7 -> 71.1, B16 H16 S2048 d64 238.2 -> 237.9, B4 H16 S1024
-  // d128 24.53 -> 24.49.  At d = 128 partly filled ends and blocks of 64 keys are 0.3 and 0.6 % slower for it (B4 H16 S1000 25.75 -> 25.83,
-  // B2 H16 S1088 24.71 -> 24.85) and keep the compiler's order.
-  constexpr bool kReadsBeforeMerge = D == 64 || (BK == kBlockK && !RAGGED);
+  // d128 24.53 -> 24.49, partly filled ends H8 S1000 20.38 -> 20.25, with 255 steps 22.20 -> 22.04.  At d = 128 blocks of 64 keys are 0.6 % slower
+  // for it (B2 H16 S1088 24.71 -> 24.85) and keep the compiler's order.
+  constexpr bool kReadsBeforeMerge = D == 64 || BK == kBlockK;
   auto phase_gemm2_merge = [&](int kb, const v4i (&pk)[kKeyTiles], int k_next, int v_next, bool steady = false, KOperands* first_k = nullptr) __attribute__((always_inline)) {
     if constexpr (test_build::kNoMfma) {
       if (kLoadsInMfmaPhase) {
@@ -1250,16 +1250,24 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   };
   // Likewise P, where the softmax is skipped: otherwise the general loop, which every call takes for its last key block, starts with sixteen
   // registers of zeros and carries them (us: B1 H2 S128 d64 4.25 -> 4.17, B2 H4 S256 6.33 -> 6.21, B8 H12 S512 10.61 -> 10.50, with masked keys
-  // 11.50 -> 11.34, B4 H16 S1024 d128 24.59 -> 24.51; its registers 228 -> 212).
+  // 11.50 -> 11.34, B4 H16 S1024 d128 24.59 -> 24.51; its registers 228 -> 212).  At d = 128 not with partly filled ends (H8 S500 13.36 -> 13.54)
+  // nor with 255 steps and blocks of 64 keys (H8 S192 7.83 -> 7.98).
+  constexpr bool kForgetP = D == 64 || (!RAGGED && !(FULLP && BK == kBlockKSmall));
   auto forget_p = [&](v4i (&pk)[kKeyTiles]) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < kKeyTiles; ++t) asm volatile("" : "=v"(pk[t]));
   };
   auto gemm1_of = [&](int kb) __attribute__((always_inline)) {  // GEMM 1 of block 0, which may or may not have masked keys
     // (The form without masked keys falls through.  Left alone, the compiler reaches it by a jump to the end of the kernel and back, and in
-    // the smallest calls that fetch is seen: B1 H2 S128 d64 4.27 us, 4.24 so; with masked keys 4.34 and 4.36.)
-    if (__builtin_expect(cls_of(kb) == 0, 1)) phase_gemm1(kb, acc, mx, false);
-    else phase_gemm1(kb, acc, mx, true);
+    // the smallest calls that fetch is seen: B1 H2 S128 d64 4.27 us, 4.24 so, with masked keys 4.34 and 4.36; d128 5.07 and 5.04, 5.19 both.  Not
+    // where blocks may be partly filled: a lone one has masked keys always.)
+    if constexpr (!RAGGED) {
+      if (__builtin_expect(cls_of(kb) == 0, 1)) phase_gemm1(kb, acc, mx, false);
+      else phase_gemm1(kb, acc, mx, true);
+    } else {
+      if (cls_of(kb) != 0) phase_gemm1(kb, acc, mx, true);
+      else phase_gemm1(kb, acc, mx, false);
+    }
   };
   // The wavefront in its MFMA phase gets the issue slots it asks for: an MFMA, an operand read or a merge instruction
   // that waits behind the other wavefront's softmax stream leaves the MFMA pipe idle, the reverse costs nothing.
@@ -1339,7 +1347,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
       wait_v_for_colsum_a();
       barrier_odd();                           // barrier 2i+1
       if (work) phase_softmax(i, cls, acc, pk, mx);
-      else forget_p(pk);
+      else if constexpr (kForgetP) forget_p(pk);
       issue_after_softmax_a(i);
       wait_tiles(true);
       barrier();                               // barrier 2i+2
@@ -1414,7 +1422,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
       wait_tiles(false);
       barrier();                               // barrier 2i+2
       if (work) phase_softmax(i, cls, acc, pk, mx);
-      else forget_p(pk);
+      else if constexpr (kForgetP) forget_p(pk);
       issue_after_softmax(i);
       wait_v_for_colsum_b();
       barrier_odd();                           // barrier 2i+3

@@ -228,11 +228,11 @@ def _fmas_behind_operand_reads(func_text):
 def test_the_last_merge_covers_the_first_operand_reads_of_the_next_block(kernels):
     """Steady-state loops of the 256-row kernel without masked keys: the first K operands are asked for in front of the sixteen fmas of the last
     output tile.  Where the compiler chose by itself, what changed elsewhere in the kernel could put them behind twelve of those.  (At d = 128
-    partly filled ends and blocks of 64 keys leave it to the compiler.)"""
+    blocks of 64 keys leave it to the compiler.)"""
     for f in kernels:
         name = f.split(":")[0]
-        d, block, ragged, full = re.search(r"fwd_kernelILi(\d+)ELi(\d+)ELb.ELb.ELb(.)ELb(.)E", name).groups() if "fwd_kernel" in name else (0,) * 4
-        if d == "64" or (block, ragged) == ("128", "0"):
+        d, block, full = re.search(r"fwd_kernelILi(\d+)ELi(\d+)ELb.ELb.ELb.ELb(.)E", name).groups() if "fwd_kernel" in name else (0,) * 3
+        if d == "64" or block == "128":
             # both halves of the workgroup; with 255 steps (the last template argument) the column sums stand there in the second
             loops = [n for n in _fmas_behind_operand_reads(f) if n >= 16]
             assert len(loops) >= (1 if full == "1" else 2), (name, _fmas_behind_operand_reads(f))
@@ -251,8 +251,9 @@ def _jumps_behind_the_end(func_text):
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_the_first_block_without_masked_keys_is_not_reached_by_way_of_the_end(kernels):
     """GEMM 1 of the first key block has two forms; the usual one, without masked keys, is reached without a jump to the end of the kernel and
-    back, whose instruction fetch the smallest calls wait for."""
-    assert {f.split(":")[0]: _jumps_behind_the_end(f) for f in kernels if "fwd_kernel" in f.split(":")[0] and _jumps_behind_the_end(f)} == {}
+    back, whose instruction fetch the smallest calls wait for (whole blocks)."""
+    found = {f.split(":")[0]: _jumps_behind_the_end(f) for f in kernels if re.search(r"fwd_kernelILi\d+ELi\d+ELb.ELb.ELb0E", f.split(":")[0])}
+    assert len(found) == 32 and {name: jumps for name, jumps in found.items() if jumps} == {}
 
 
 def _runs_of_moves(func_text):
@@ -272,9 +273,14 @@ def _runs_of_moves(func_text):
 def test_the_general_loop_carries_no_p_of_blocks_that_have_none(kernels):
     """P of a key block without an unmasked key is never used; where the general loop does not say so, the compiler starts it at zero, 14 to 24
     moves in front of the loop that every call takes for its last key block.  The last run of moves is then that one, and not the start of O (some
-    32 registers or more)."""
-    late = {f.split(":")[0]: _runs_of_moves(f) for f in kernels if "fwd_kernel" in f.split(":")[0]}
-    assert late and {name: runs for name, runs in late.items() if runs[-1] < 30} == {}
+    32 registers or more).  Not at d = 128 with partly filled ends, or with 255 steps and blocks of 64 keys."""
+    late = {}
+    for f in kernels:
+        name = f.split(":")[0]
+        d, block, ragged, full = re.search(r"fwd_kernelILi(\d+)ELi(\d+)ELb.ELb.ELb(.)ELb(.)E", name).groups() if "fwd_kernel" in name else (0,) * 4
+        if d == "64" or (d == "128" and ragged == "0" and (block, full) != ("64", "1")):
+            late[name] = _runs_of_moves(f)
+    assert len(late) == 32 + 12 and {name: runs for name, runs in late.items() if runs[-1] < 30} == {}
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
