@@ -57,6 +57,10 @@ struct SplitKernelArgs : KernelArgs {
 // `cls` (blocks that fill up the last four count as the latter).  mask_bytes: the lane's first sixteen bytes, tail_bytes: the
 // row's last sixteen (for the one lane that straddles the end); both have landed.  S >= 16.  Returns this wavefront's last
 // block with an unmasked key, -1 if there is none.  Only keys from .. to-1 are looked at (multiples of BK).
+// What bounds it is a chain of latencies in front of the first barrier: wavefronts whose sixteen bytes per lane lie behind the last key
+// have nothing to do here, the neighbour's bits come by a lane permutation of the vector unit and the last live block from a ballot.
+// With LDS permutations (seven in a row) and all wavefronts at it: B2 H8 S300 d128 6.76 -> 7.20 us, H16 Sq512 S640 8.92 -> 9.33, d64 B2 H12
+// S1024 (pair kernel) 13.14 -> 13.44, B8 H16 Sq1 S2048 (sixteen rows) 8.99 -> 9.34.
 constexpr int kMaskBytesPerLane = 16;
 template <int BK, int WAVES>
 __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const v4i& tail_bytes, const int8_t* __restrict__ mg, int S,
@@ -71,8 +75,9 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
     return nonzero_bytes((unsigned)w[0]) | (nonzero_bytes((unsigned)w[1]) << 4) | (nonzero_bytes((unsigned)w[2]) << 8) |
            (nonzero_bytes((unsigned)w[3]) << 12);
   };
+  const int first_lane = __builtin_amdgcn_readfirstlane(tid - lane);
   int live_hi = -1;
-  for (int base = from; base < to; base += kMaskBytesPerLane * 64 * WAVES) {
+  for (int base = from; base + kMaskBytesPerLane * first_lane < to; base += kMaskBytesPerLane * 64 * WAVES) {
     const int j = base + kMaskBytesPerLane * tid;
     unsigned bits = 0xffffu;  // keys past the end count as masked
     if (j + kMaskBytesPerLane <= S) {
@@ -85,19 +90,21 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
     } else if (j < S) {  // the one lane that straddles the end of the row
       bits = ((nonzero16(tail_bytes) >> (kMaskBytesPerLane - (S - j))) | (0xffffu << (S - j))) & 0xffffu;
     }
-    const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
+    // (the neighbour's sixteen bits by a lane permutation of the vector unit)
+    const unsigned word = bits | ((unsigned)__builtin_amdgcn_mov_dpp((int)bits, 0xB1, 0xf, 0xf, true) << 16);
     if ((lane & 1) == 0 && j < to) words[j >> 5] = word;
     const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
+    bool lives = false;
     if (lane % kLanesPerBlock == 0 && j < to) {
       constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
       const bool blk_some = ((some >> lane) & kBlockBits) != 0, blk_all = ((all >> lane) & kBlockBits) == kBlockBits;
       cls[j / BK] = (unsigned char)((blk_some ? 1 : 0) | (blk_all ? 2 : 0));
-      if (!blk_all) live_hi = j / BK;
+      lives = !blk_all;
     }
+    const unsigned long long live = __ballot(lives);
+    if (live != 0) live_hi = (base + kMaskBytesPerLane * (first_lane + 63 - __builtin_clzll(live))) / BK;
   }
   if (tid < kSplitKeys && n_blocks + tid < (n_blocks + kSplitKeys - 1) / kSplitKeys * kSplitKeys) cls[n_blocks + tid] = 3;
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) live_hi = max(live_hi, __shfl_xor(live_hi, off));
   return live_hi;
 }
 
