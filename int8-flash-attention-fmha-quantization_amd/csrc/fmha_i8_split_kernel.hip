@@ -154,6 +154,14 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   // file).  With one round or two per workgroup the time is that of the first loads, so V is asked for beside K.
   static_assert(!PARTS || R == 1, "");
   constexpr bool kEarlyV = PARTS && kOwnK;
+  // Q: the operands of GEMM 1 straight from memory touch 32 rows with every load, and the four wavefronts of a row group load the same
+  // ones: the first barrier waits for the CU's address path.  Through LDS eight lanes fetch a row's 128 contiguous bytes: with two
+  // buffers a quarter of the rows per wavefront, into what holds V of round 1 from the second barrier on; otherwise each wavefront all
+  // of them, into a place that it has read again before the first barrier.  d128 H16 S777 12.12 -> 11.50 us (11.71 with each wavefront
+  // fetching all of its rows), H32 Sq512 S1152 13.34 -> 12.82, S4096 32.1 -> 31.5, B2 H16 Sq32 S2048 12.6 -> 12.3; with one row group and
+  // blocks of 64 keys B2 H8 S300 6.41 -> 6.47, at d64, where 128 bytes hold two rows, 8.46 -> 8.49 (H16 Sq512 S960): those stay.
+  constexpr bool kQInRegs = D == 64 || (R == 1 && BK == 64), kQShared = !kQInRegs && kBuffers == 2;
+  constexpr int kQLoads = kQShared ? 1 : D / 32;
 
   __shared__ __attribute__((aligned(1024))) int8_t lds[kBuffers][2][kSplitKeys][kTileBytes];  // [buffer][K|V][slot][tile]
   __shared__ __attribute__((aligned(16))) v4i lds_p[R][kPSlots][kKeyTiles][64];  // P^T as the B operand of GEMM 2
@@ -242,14 +250,27 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
                  : "=&v"(mask_bytes), "=v"(tail_bytes) : "v"(j), "s"(mg), "v"(jt) : "memory");
   }
   v4i qreg[kDSteps];
-  {
+  const int8_t* qp = args.q + q_head_off;
+  const int8_t* lds_q = nullptr;
+  if constexpr (kQInRegs) {
     int qrow = min(row0 + i32, Sq - 1);  // rows past the end load the last row (unused)
     if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
-    const int8_t* qp = args.q + q_head_off;
     const int qoff = qrow * D + 16 * g;
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk)
       asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(qreg[kk]) : "v"(qoff + 32 * kk), "s"(qp) : "memory");
+  } else {
+    lds_q = kQShared ? &lds[kBuffers - 1][1][0][0] + r * (32 * D) : kEarlyV ? reinterpret_cast<const int8_t*>(&lds_p[r][c][0][0]) : &lds[0][1][0][0] + wave * (32 * D);
+    static_assert(kEarlyV ? 32 * D <= kKeyTiles * 1024 : kRowWaves * 32 * D <= kSplitKeys * kTileBytes, "");
+    const unsigned dst = (unsigned)(uintptr_t)(__attribute__((address_space(3))) const int8_t*)lds_q;
+#pragma unroll
+    for (int it = 0; it < kQLoads; ++it) {
+      const int region = kQShared ? c : it, row = region * kRowsPerRegion + ld_row_in;
+      int qrow = min(row0 + row, Sq - 1);
+      if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
+      const int src = qrow * D + (((lane % kChunks) ^ k_swizzle<D>(row)) << 4);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * region), "v"(src), "s"(qp) : "memory");
+    }
   }
 #pragma unroll
   for (int it = 0; it < kLoads; ++it) issue(first_round, 0, it, n_blocks - 1);
@@ -287,15 +308,26 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   if (BIAS) asm volatile("" : "+v"(base_s));
 
   // ---- classification of the key blocks, by all wavefronts (the bits are those of the 256-row kernel) -----------------
-  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + (kEarlyV ? 2 : 1) * kLoads) : "memory");
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kQLoads + (kEarlyV ? 2 : 1) * kLoads) : "memory");
   const int live_hi = classify_key_blocks<BK, kRowWaves>(mask_bytes, tail_bytes, mg, S, tid, lds_mask,
                                                          reinterpret_cast<unsigned char*>(lds_class4), keys_from, keys_to);
   if (lane == 0) lds_scan[wave] = live_hi;
+  auto read_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < kDSteps; ++kk) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q + k_read_off[kk]);
+  };
+  if constexpr (!kQInRegs && !kQShared) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kEarlyV ? 2 : 1) * kLoads) : "memory");
+    read_q();
+  }
   // K of round 0 and the Q rows have landed
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kEarlyV ? kLoads : 0) : "memory");
+  if constexpr (!kQShared) {
 #pragma unroll
-  for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
+    for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
+  }
   barrier();
+  if constexpr (kQShared) read_q();
   int n = -1;
 #pragma unroll
   for (int w = 0; w < kRowWaves; ++w) n = max(n, lds_scan[w]);
