@@ -310,6 +310,11 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   __shared__ unsigned char lds_class[kMaxKeyBlocks];  // per key block: bit0 = some key masked, bit1 = all keys masked
   __shared__ unsigned lds_mask[kMaxKeyBlocks * kBlockKSmall / 32];  // bit j%32 of word j/32: key j of this batch entry is masked
   __shared__ __attribute__((aligned(16))) int lds_colsum[FULLP ? 2 * D : 4];  // FULLP: [key block & 1][output column]
+  // Q passes through LDS at head_dim 128 (see load_q_rows).  There is room for the rows of half the wavefronts beside tiles of 128 keys;
+  // those of the others lie in the ring (see q_place).
+  constexpr bool kQThroughLds = D == 128;
+  constexpr int kQSlots = BK == kBlockK ? 4 : 8;
+  __shared__ __attribute__((aligned(16))) int8_t lds_q[kQThroughLds ? kQSlots : 1][kQThroughLds ? 32 * D : 16];
   __shared__ __attribute__((aligned(16))) int lds_scan[8];  // per classifying wavefront: last block with an unmasked key, first block with a masked one
 
   const int tid = threadIdx.x;
@@ -570,10 +575,34 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // it waits for nothing that wavefronts 4..7, which start several hundred cycles later, have asked for.  Each half of
   // the workgroup runs its own prologue and its own schedule behind ONE branch on the wavefront index, so that a load
   // and the wait that retires it always lie on the same path.
+  // FULLP with one barrier per key block: wavefronts 4..7 ask for V0 in front of the first barrier and sum its columns right behind it.
+  constexpr bool kV0BeforeFirstBarrier = FULLP && kOneBarrier;
+  // At head_dim 128 the rows pass through LDS: eight lanes fetch a row's 128 contiguous bytes, where operands fetched straight into
+  // registers touch 32 rows with every load and the CU's address path, which the first barrier waits for, takes twice as long (B4 H16
+  // S1024 21.3 -> 21.0 us, B16 H16 S256 9.54 -> 9.27; at head_dim 64, two rows to 128 bytes, no gain).  Each wavefront reads back what it
+  // has fetched itself, behind its own wait: where a tile will land only if that load is issued behind a later barrier than the read -
+  // V of stage 3 is asked for in the phases of block 1, behind the second barrier; stage 1 right behind the first one.
+  auto q_place = [&]() __attribute__((always_inline)) -> const int8_t* {
+    if (kQSlots == 8) return &lds_q[wave][0];
+    if (kV0BeforeFirstBarrier) return wave < 4 ? &lds_q[wave][0] : &lds[1][0][0] + (wave - 4) * (32 * D);
+    return wave < 4 ? &lds[3][1][0] + wave * (32 * D) : &lds_q[wave - 4][0];
+  };
   auto load_q_rows = [&]() __attribute__((always_inline)) {
     // rows past the end of the sequence load the last row (unused) so that every wavefront has the same loads in flight
     const int8_t* qp = args.q + q_head_off;
     const int q_lane = lane_again();
+    if constexpr (kQThroughLds) {
+      const unsigned dst = (unsigned)(uintptr_t)(__attribute__((address_space(3))) const int8_t*)q_place();
+#pragma unroll
+      for (int it = 0; it < kDSteps; ++it) {
+        const int row = it * kRowsPerRegion + q_lane / kChunks;
+        int qrow = min(row0 + row, Sq - 1);
+        if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
+        const int src = qrow * D + (((q_lane % kChunks) ^ k_swizzle<D>(row)) << 4);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * it), "v"(src), "s"(qp) : "memory");
+      }
+      return;
+    }
     int qrow = min(row0 + (q_lane & 31), Sq - 1);
     if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
     const int qoff = qrow * D + 16 * (q_lane >> 5);
@@ -584,8 +613,16 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // The Q registers are redefined after the wait that retires their loads, so that no use of them can be scheduled
   // above it.
   auto pin_q_rows = [&]() __attribute__((always_inline)) {
+    if constexpr (kQThroughLds) return;
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
+  };
+  auto read_q_rows = [&]() __attribute__((always_inline)) {  // behind the wait that retires their loads
+    if constexpr (kQThroughLds) {
+      const int8_t* lds_q_rows = q_place();
+#pragma unroll
+      for (int kk = 0; kk < kDSteps; ++kk) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q_rows + k_read_off[kk]);
+    }
   };
   // Wavefronts 0..3 also classify the key blocks of this batch entry, sixteen mask bytes per lane and BK/16 lanes per
   // block: their loads are the first to be served.  Per key block: lds_class (bit0 = some key masked, bit1 = all keys
@@ -679,14 +716,16 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   // Wavefronts 4..7 ask for their Q rows only and wait for nothing in front of the first barrier; right behind it they
   // wait for the Q rows (their first GEMM 1 comes one phase later anyway) and then ask for V0, which is first needed
   // behind the second barrier.  Every wait of the prologue is a vmcnt(0): it holds on whatever path leads to it.
-  // (FULLP with one barrier per key block: V0 in front of the first barrier - they sum its columns right behind it.)
-  constexpr bool kV0BeforeFirstBarrier = FULLP && kOneBarrier;
   auto prologue_waves_4_to_7 = [&]() __attribute__((always_inline)) {
     load_q_rows();
     if (kV0BeforeFirstBarrier) issue_tile0_by_half(vg, 1, ld_goff_v);
     init_state();
     if (kV0BeforeFirstBarrier) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (kQThroughLds) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPrologueRegions) : "memory");
+        read_q_rows();
+      }
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       pin_q_rows();
     }
   };
@@ -694,6 +733,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     if (!kV0BeforeFirstBarrier) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       pin_q_rows();
+      read_q_rows();
       issue_tile0_by_half(vg, 1, ld_goff_v);
     }
   };
@@ -702,6 +742,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   auto first_barrier = [&]() __attribute__((always_inline)) {
     prologue_done = true;
     barrier();
+    if (wave < 4) read_q_rows();
     {
       const v4i s0 = *reinterpret_cast<const v4i*>(&lds_scan[0]), s1 = *reinterpret_cast<const v4i*>(&lds_scan[4]);
       kb_end = __builtin_amdgcn_readfirstlane(max(max(s0[0], s0[2]), max(s1[0], s1[2]))) + 1;

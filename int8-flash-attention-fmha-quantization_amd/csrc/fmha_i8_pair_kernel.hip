@@ -96,7 +96,24 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
                  : "=&v"(mask_bytes), "=v"(tail_bytes) : "v"(j), "s"(mg), "v"(jt) : "memory");
   }
   v4i qreg[kDSteps];
-  {
+  // Q: at head_dim 128 through LDS, by whole rows (see the 256-row kernel; B1 H16 S2048 25.39 -> 24.82 us); the two wavefronts of a row group
+  // fetch half of its rows each, into what holds P of the first half from tick 0 on.
+  constexpr bool kQThroughLds = D == 128;
+  constexpr int kQLoads = kQThroughLds ? kDSteps / 2 : kDSteps;
+  const int8_t* lds_q = reinterpret_cast<const int8_t*>(&lds_p[0][0][0][0]) + r * (32 * D);
+  static_assert(!kQThroughLds || 4 * 32 * D <= (int)sizeof(lds_p), "");
+  if constexpr (kQThroughLds) {
+    const unsigned dst = (unsigned)(uintptr_t)(__attribute__((address_space(3))) const int8_t*)lds_q;
+    const int8_t* qp = args.q + q_head_off;
+#pragma unroll
+    for (int it = 0; it < kQLoads; ++it) {
+      const int region = kQLoads * h + it, row = region * (1024 / D) + ld_row_in;
+      int qrow = min(row0 + row, Sq - 1);  // rows past the end load the last row (unused)
+      if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
+      const int src = qrow * D + (((lane % kChunks) ^ k_swizzle<D>(row)) << 4);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * region), "v"(src), "s"(qp) : "memory");
+    }
+  } else {
     int qrow = min(row0 + i32, Sq - 1);  // rows past the end load the last row (unused)
     if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
     const int8_t* qp = args.q + q_head_off;
@@ -149,8 +166,10 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   if (BIAS && !FULLP && kScoreBaseBits == kBaseBits) base_s = base_c;
   else if (BIAS) asm volatile("" : "+v"(base_s));
 
-  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kDSteps + kLoads) : "memory");
-  if (h == 0) {  // (for the mask bytes the other half has waited in vain: they are its first loads)
+  // (the second half, which has 2 kLoads more in flight, waits for its Q rows here, and for the mask bytes in vain)
+  static_assert(kQLoads <= 2 * kLoads, "");
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(mask_bytes), "+v"(tail_bytes) : "n"(kQLoads + kLoads) : "memory");
+  if (h == 0) {
     const int live_hi = classify_key_blocks<BK, 4>(mask_bytes, tail_bytes, mg, S, tid, lds_mask, lds_class, 0, n_blocks * BK);
     if (lane == 0) lds_scan[r] = live_hi;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -158,7 +177,10 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   barrier();
   all_loads_landed();
 #pragma unroll
-  for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
+  for (int kk = 0; kk < kDSteps; ++kk) {
+    if constexpr (kQThroughLds) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q + k_read_off[kk]);
+    else asm volatile("" : "+v"(qreg[kk]));
+  }
   const v4i scan = *reinterpret_cast<const v4i*>(lds_scan);
   const int n = __builtin_amdgcn_readfirstlane(max(max(scan[0], scan[1]), max(scan[2], scan[3]))) + 1;  // one past the last block with an unmasked key
 
