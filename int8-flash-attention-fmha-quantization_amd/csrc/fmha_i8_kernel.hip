@@ -652,8 +652,6 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     asm volatile("s_waitcnt vmcnt(%1)" : "+v"(mask_bytes) : "n"(kDSteps) : "memory");
     asm volatile("" : "+v"(tail_bytes));
     constexpr int kLanesPerBlock = BK / kKeysPerLane;
-    constexpr int kBlocksPerWave = 64 / kLanesPerBlock;
-    constexpr unsigned long long kGroupBits = kLanesPerBlock == 8 ? 0x0101010101010101ull : 0x1111111111111111ull;
     int live_hi = -1, pad_lo = 0x7fffffff;
     // one bit per byte of a dword: set where the byte is not zero
     auto nonzero_bytes = [](unsigned w) -> unsigned {
@@ -682,27 +680,21 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
         }
       }
       // two lanes hold the 32 mask bits of one word
-      const unsigned word = bits | ((unsigned)__shfl_xor((int)bits, 1) << 16);
+      const unsigned word = bits | ((unsigned)__builtin_amdgcn_mov_dpp((int)bits, 0xB1, 0xf, 0xf, true) << 16);
       if ((lane & 1) == 0 && j < S_pad) lds_mask[j >> 5] = word;
       const unsigned long long some = __ballot(bits != 0), all = __ballot(bits == 0xffffu);
+      bool lives = false, pads = false;
       if (lane % kLanesPerBlock == 0 && j < S_pad) {
         constexpr unsigned long long kBlockBits = (1ull << kLanesPerBlock) - 1;
         const unsigned long long blk_some = (some >> lane) & kBlockBits, blk_all = (all >> lane) & kBlockBits;
-        lds_class[j / BK] = (unsigned char)((blk_some != 0 ? 1 : 0) | (blk_all == kBlockBits ? 2 : 0));
+        pads = blk_some != 0;
+        lives = blk_all != kBlockBits;
+        lds_class[j / BK] = (unsigned char)((pads ? 1 : 0) | (lives ? 0 : 2));
       }
-      // the same two facts per block of this wavefront, folded onto the lowest lane of each block (wave-uniform)
-      unsigned long long any = some, every = all;
-#pragma unroll
-      for (int sh = 1; sh < kLanesPerBlock; sh *= 2) {
-        any |= any >> sh;
-        every &= every >> sh;
-      }
-      const int blk0 = (base + kKeysPerLane * 64 * wave) / BK;  // first block of this wavefront in this pass
-      const int n_here = min(max(n_blocks - blk0, 0), kBlocksPerWave);
-      const unsigned long long valid = (n_here == kBlocksPerWave ? ~0ull : ((1ull << (n_here * kLanesPerBlock)) - 1ull)) & kGroupBits;
-      const unsigned long long live = ~every & valid, padded = any & valid;
-      if (live != 0) live_hi = blk0 + (63 - __builtin_clzll(live)) / kLanesPerBlock;
-      if (padded != 0) pad_lo = min(pad_lo, blk0 + __builtin_ctzll(padded) / kLanesPerBlock);
+      const unsigned long long live = __ballot(lives), padded = __ballot(pads);
+      const int first_key = base + kKeysPerLane * 64 * wave;
+      if (live != 0) live_hi = (first_key + kKeysPerLane * (63 - __builtin_clzll(live))) / BK;
+      if (padded != 0) pad_lo = min(pad_lo, (first_key + kKeysPerLane * __builtin_ctzll(padded)) / BK);
     }
     if (lane == 0) {
       lds_scan[2 * wave] = live_hi;
