@@ -490,14 +490,11 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
     const int both[8] = {g0[0], g1[0], g0[1], g1[1], g0[2], g1[2], g0[3], g1[3]};
     store_wide_rows<D>(args, &lds_v[0][0] + wave * 4096, q_head_off + (long)row0 * D + 64 * h, Sq - row0, both);
   } else {
-    op += 8 * g;
-#pragma unroll
-    for (int a = 0; a < 4; a += 2) {
-      const auto s = __builtin_amdgcn_permlane32_swap(w[0][a], w[0][a + 1], false, false);
-      *reinterpret_cast<v2i*>(op + 8 * a) = v2i{(int)s[0], (int)s[1]};
-      const int both[2] = {(int)s[0], (int)s[1]};
-      store_wide<D>(args, op - args.o + 8 * a, both);
-    }
+    op += 16 * g;  // (one store of sixteen bytes per lane, as in the split kernel)
+    const auto s0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[0][2], false, false), s1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[0][3], false, false);
+    const int both[4] = {(int)s0[0], (int)s0[1], (int)s1[0], (int)s1[1]};
+    *reinterpret_cast<v4i*>(op) = v4i{both[0], both[1], both[2], both[3]};
+    store_wide<D>(args, op - args.o, both);
   }
 }
 
