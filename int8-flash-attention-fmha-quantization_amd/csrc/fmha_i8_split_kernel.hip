@@ -162,6 +162,10 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   // file).  With one round or two per workgroup the time is that of the first loads, so V is asked for beside K.
   static_assert(!PARTS || R == 1, "");
   constexpr bool kEarlyV = PARTS && kOwnK;
+  // P of a wavefront's own key block, an operand of its own GEMM 2 too, need not come back from LDS: H16 Sq512 S960 d64 8.41 -> 8.19 us, B4 H8
+  // Sq200 S400 5.77 -> 5.66.  The other forms lose more by the branch in the middle of their operand reads than the reads cost (H16 S777 d128
+  // 11.30 -> 11.50, H32 Sq512 S4096 31.3 -> 31.8, d64 S2048 11.47 -> 11.79).
+  constexpr bool kOwnP = R == 1 && BK == 64 && !PARTS;
   // Q: the operands of GEMM 1 straight from memory touch 32 rows with every load, and the four wavefronts of a row group load the same
   // ones: the first barrier waits for the CU's address path.  Through LDS eight lanes fetch a row's 128 contiguous bytes: with two
   // buffers a quarter of the rows per wavefront, into what holds V of round 1 from the second barrier on; otherwise each wavefront all
@@ -472,7 +476,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   auto gemm2_merge = [&](int buf, int first, auto count_t, unsigned cls4, auto between) __attribute__((always_inline)) {
     constexpr int kCount = decltype(count_t)::value;
     typedef v2i __attribute__((address_space(3))) * lds_v2i_ptr;
-    v4i va[2][kKeyTiles], p[2][kKeyTiles];
+    constexpr int kHeld = kOwnP && !FULLP ? kCount : 2;  // key blocks whose operands are in registers
+    v4i va[kHeld][kKeyTiles], p[kHeld][kKeyTiles];
     v16i oacc[2];
     auto read = [&](int j) __attribute__((always_inline)) {
       const int8_t* lds_v = &lds[buf][1][first + j][0];
@@ -480,8 +485,14 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       for (int t = 0; t < kKeyTiles; ++t) {
         const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(lds_v + v_read_off + 32 * t * D));
         const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(lds_v + v_read_off + 32 * t * D + 16 * D));
-        va[j & 1][t] = v4i{lo[0], lo[1], hi[0], hi[1]};
-        p[j & 1][t] = lds_p[r][(first + j) & (kPSlots - 1)][t][lane];
+        va[j % kHeld][t] = v4i{lo[0], lo[1], hi[0], hi[1]};
+      }
+      if (kOwnP && c == first + j) {
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) p[j % kHeld][t] = pk[t];
+      } else {
+#pragma unroll
+        for (int t = 0; t < kKeyTiles; ++t) p[j % kHeld][t] = lds_p[r][(first + j) & (kPSlots - 1)][t][lane];
       }
     };
     if constexpr (PARTS) {  // the accumulators of every block to memory
@@ -494,13 +505,13 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         if (FULLP) {  // (as in start() below)
           const v4i half = {0x40404040, 0x40404040, 0x40404040, 0x40404040};
 #pragma unroll
-          for (int t = 0; t < kKeyTiles; ++t) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], half, oacc[0], 0, 0, 0);
+          for (int t = 0; t < kKeyTiles; ++t) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j % kHeld][t], half, oacc[0], 0, 0, 0);
 #pragma unroll
           for (int e = 0; e < 16; ++e) oacc[0][e] = 2 * oacc[0][e] + kBaseBitsFull;
         }
 #pragma unroll
         for (int t = 0; t < kKeyTiles; ++t) {
-          oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], p[j & 1][t], oacc[0], 0, 0, 0);
+          oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j % kHeld][t], p[j % kHeld][t], oacc[0], 0, 0, 0);
           between(j * kKeyTiles + t, kCount * kKeyTiles);
         }
         if (!((cls4 >> (8 * (first + j))) & 2) && c < kDSteps && i32 < Sq &&
@@ -528,13 +539,13 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         const v4i half = {0x40404040, 0x40404040, 0x40404040, 0x40404040};
 #pragma unroll
         for (int t = 0; t < kKeyTiles; ++t)
-          oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], half, oacc[j & 1], 0, 0, 0);
+          oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j % kHeld][t], half, oacc[j & 1], 0, 0, 0);
 #pragma unroll
         for (int e = 0; e < 16; ++e) oacc[j & 1][e] = 2 * oacc[j & 1][e] + kBaseBitsFull;
       }
     };
     auto product = [&](int j, int t) __attribute__((always_inline)) {
-      oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j & 1][t], p[j & 1][t], oacc[j & 1], 0, 0, 0);
+      oacc[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(va[j % kHeld][t], p[j % kHeld][t], oacc[j & 1], 0, 0, 0);
     };
     // Operand reads one block ahead; the merge of a block stands behind the MFMAs of the next one.
     float ml[kCount][2];
@@ -543,14 +554,16 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       ml[j][0] = lds_ml[r][first + j][i32][0];
       ml[j][1] = lds_ml[r][first + j][i32][1];
     }
-    read(0);
-    read(1);
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) read(j);
     __builtin_amdgcn_sched_barrier(0);
+    if (kHeld < kCount) {
     start(0);
 #pragma unroll
     for (int t = 0; t < kKeyTiles; ++t) {
       product(0, t);
       between(t, kCount * kKeyTiles);
+    }
     }
     bool moves[kCount];  // some row's reference exponent moves (wave-uniform, rare): O is rescaled in front of that block's merge
 #pragma unroll
@@ -571,6 +584,15 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         for (int e = 0; e < 16; ++e) o_f[e] *= keep[j];
       }
     };
+    if (kHeld == kCount) {
+      __builtin_amdgcn_sched_barrier(0);
+    start(0);
+#pragma unroll
+    for (int t = 0; t < kKeyTiles; ++t) {
+      product(0, t);
+      between(t, kCount * kKeyTiles);
+    }
+    }
     rescale(0);
 #pragma unroll
     for (int j = 1; j < kCount; ++j) {
@@ -584,7 +606,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         merge_piece(j - 1, t, kKeyTiles);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (j + 1 < kCount) read(j + 1);
+      if (kHeld < kCount && j + 1 < kCount) read(j + 1);
       rescale(j);
       __builtin_amdgcn_sched_barrier(0);
     }
