@@ -187,19 +187,23 @@ hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, con
   return hipLaunchKernel(kernel, dim3((unsigned)args.total_wgs), dim3(row_groups == 1 || row_groups == kFew ? 256 : 512), kernel_args, 0, stream);
 }
 // What a workgroup of each kernel costs: (start + step * rounds), a round being one key block for the first two and four for the
-// split kernel.  Microseconds * 100 beyond the launch (2.9 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one
-// MI355X with one workgroup on half of the CUs (tests/variant_timing.py --kernel-costs); measurements differ by 4 %.  The last kernel's
+// split kernel, and `again` for each further one on the same CU, whose prologue nothing covers (the first one's is part of the launch).
+// Microseconds * 100 beyond the launch (2.8 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one MI355X with one
+// workgroup on half of the CUs (tests/variant_timing.py --kernel-costs), `again` with two to eight on every CU (--shapes); measurements differ
+// by 4 %.  With starts measured before Q went through LDS and no `again`, calls of 130 to 256 keys at d64 took the 256-row kernel
+// that smaller workgroups serve faster (B5 H8 S256 6.40 -> 5.41 us, B8 H12 S144 6.62 -> 5.01).  The last kernel's
 // entries at d = 64 are its line up to 2048 keys: at 4096 a call of 128 heads, each with its own keys, takes 6 % longer (the memory).
 // With all CUs at work the first two take up to 36 and 14 % longer per block (the shader clock drops).
+constexpr int kComputeUnits = 256;
 struct KernelCost {
   int row_groups, keys_per_round;
-  struct { int start, step; } cost[2][2];
+  struct { int start, step, again; } cost[2][2];
 };
-constexpr KernelCost kKernelCosts[] = {{0, 1, {{{72, 80}, {95, 128}}, {{200, 99}, {250, 162}}}},
-                                       {4, 1, {{{137, 62}, {170, 97}}, {{225, 83}, {300, 116}}}},
-                                       {2, 4, {{{39, 183}, {45, 312}}, {{108, 199}, {140, 332}}}},
-                                       {1, 4, {{{23, 141}, {30, 213}}, {{73, 159}, {95, 243}}}},
-                                       {kFew, 4, {{{0, 97}, {0, 149}}, {{15, 138}, {75, 225}}}}};
+constexpr KernelCost kKernelCosts[] = {{0, 1, {{{70, 80, 120}, {105, 129, 120}}, {{160, 99, 220}, {235, 162, 220}}}},
+                                       {4, 1, {{{107, 62, 130}, {142, 96, 140}}, {{171, 82, 190}, {252, 117, 200}}}},
+                                       {2, 4, {{{0, 186, 150}, {20, 300, 150}}, {{20, 200, 190}, {61, 332, 260}}}},
+                                       {1, 4, {{{0, 136, 20}, {6, 211, 150}}, {{25, 153, 180}, {36, 247, 180}}}},
+                                       {kFew, 4, {{{0, 97, 0}, {0, 149, 0}}, {{15, 138, 0}, {75, 225, 0}}}}};
 constexpr KernelCost kOneGroupCost = kKernelCosts[3], kFewCost = kKernelCosts[4];
 static_assert(kOneGroupCost.row_groups == 1 && kFewCost.row_groups == kFew, "");
 // Groups of 32 query rows per workgroup of the kernel that serves `rows` query rows of `heads` heads: 1 or 2 (fmha_i8_split_kernel), 4
@@ -213,10 +217,10 @@ struct Choice {
   int row_groups;
   long long cost;  // hundredths of a microsecond
 };
-constexpr int kComputeUnits = 256;
-int cost_of_workgroup(const KernelCost& kernel, int head_dim, int blocks, int block_keys) {
+long long cost_of_workgroups(const KernelCost& kernel, long long wgs, int head_dim, int blocks, int block_keys) {
   const auto& c = kernel.cost[head_dim == 128][block_keys == fmha_i8_gfx950::kBlockK];
-  return c.start + c.step * ((blocks + kernel.keys_per_round - 1) / kernel.keys_per_round);
+  const long long per_cu = (wgs + kComputeUnits - 1) / kComputeUnits;
+  return per_cu * (c.start + c.step * ((blocks + kernel.keys_per_round - 1) / kernel.keys_per_round)) + (per_cu - 1) * c.again;
 }
 int rows_of(const KernelCost& kernel) {
   return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : kernel.row_groups == kFew ? fmha_i8_gfx950::kFewRows : 32 * kernel.row_groups;
@@ -231,7 +235,7 @@ bool few_takes(int rows, int head_dim, int block_keys) {
 // the price is one group's, 1 % lower: without that, calls of two rounds would share their key blocks out (H16 Sq1 S1024 8.2 us plain,
 // 8.5 shared out).
 bool second_group_fetches(int rows, int head_dim, int block_keys) { return rows <= 32 && head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK; }
-constexpr KernelCost kFetchingCost{2, 4, {{}, {{}, {95, 240}}}};
+constexpr KernelCost kFetchingCost{2, 4, {{}, {{}, {95, 240, 260}}}};
 Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
   Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
@@ -239,8 +243,7 @@ Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int 
     const bool fetching = second_group_fetches(rows, head_dim, block_keys);
     if (rows <= 32 && kernel.row_groups == (fetching ? 1 : 2)) continue;
     const KernelCost& price = fetching && kernel.row_groups == 2 ? kFetchingCost : kernel;
-    const long long per_cu = (heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)) + kComputeUnits - 1) / kComputeUnits;
-    const long long cost = per_cu * cost_of_workgroup(price, head_dim, blocks, block_keys);
+    const long long cost = cost_of_workgroups(price, heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)), head_dim, blocks, block_keys);
     if (best.cost < 0 || cost < best.cost) best = {kernel.row_groups, cost};
   }
   return best;
@@ -268,7 +271,7 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
     if (first_heads <= 0 || first_rows <= 0 || rest_heads <= 0 || rest_rows <= 0) return;
     const long long wgs = (long long)first_heads * ((first_rows + rows_of(kernel) - 1) / rows_of(kernel));
     const Choice rest = cheapest_kernel(rest_heads, rest_rows, a.head_dim, blocks, block_keys);
-    const long long cost = (wgs + kComputeUnits - 1) / kComputeUnits * cost_of_workgroup(kernel, a.head_dim, blocks, block_keys) + kLaunch + rest.cost;
+    const long long cost = cost_of_workgroups(kernel, wgs, a.head_dim, blocks, block_keys) + kLaunch + rest.cost;
     if (rest.row_groups == 0 || cost >= least) return;
     least = cost;
     count = 2;
@@ -311,7 +314,7 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   least = (least > memory ? least : memory) * 20 / 21;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
-    const long long of_r = (heads * ((rounds + r - 1) / r) + 255) / 256 * (c.start + c.step * r);
+    const long long of_r = cost_of_workgroups(kernel, heads * ((rounds + r - 1) / r), a.head_dim, kSplitKeys * r, block_keys);
     if (plan.rounds_per_part > 0 && of_r > work) continue;
     work = of_r;
     plan.rounds_per_part = r;
