@@ -476,7 +476,11 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   auto gemm2_merge = [&](int buf, int first, auto count_t, unsigned cls4, auto between) __attribute__((always_inline)) {
     constexpr int kCount = decltype(count_t)::value;
     typedef v2i __attribute__((address_space(3))) * lds_v2i_ptr;
-    constexpr int kHeld = kOwnP && !FULLP ? kCount : 2;  // key blocks whose operands are in registers
+    // The operands of all key blocks of a round in registers, or of two.  With all of them the weights of the blocks are computed in front of
+    // the first product, over the latency of the reads; with two behind it: H32 Sq512 S4096 d128 31.1 us (31.6 with the weights in front),
+    // B2 H16 Sq32 S2048 12.20 (12.31), B8 H16 Sq1 S2048 13.88 (13.99), d64 H16 Sq512 S896 7.11 (7.23), H24 S640 8.42 (8.31).
+    constexpr bool kAllHeld = kOwnP && !FULLP;
+    constexpr int kHeld = kAllHeld ? kCount : 2;
     v4i va[kHeld][kKeyTiles], p[kHeld][kKeyTiles];
     v16i oacc[2];
     auto read = [&](int j) __attribute__((always_inline)) {
@@ -557,14 +561,15 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
 #pragma unroll
     for (int j = 0; j < kHeld; ++j) read(j);
     __builtin_amdgcn_sched_barrier(0);
-    if (kHeld < kCount) {
-    start(0);
+    auto first_products = [&]() __attribute__((always_inline)) {
+      start(0);
 #pragma unroll
-    for (int t = 0; t < kKeyTiles; ++t) {
-      product(0, t);
-      between(t, kCount * kKeyTiles);
-    }
-    }
+      for (int t = 0; t < kKeyTiles; ++t) {
+        product(0, t);
+        between(t, kCount * kKeyTiles);
+      }
+    };
+    if constexpr (!kAllHeld) first_products();
     bool moves[kCount];  // some row's reference exponent moves (wave-uniform, rare): O is rescaled in front of that block's merge
 #pragma unroll
     for (int j = 0; j < kCount; ++j) {
@@ -584,14 +589,9 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         for (int e = 0; e < 16; ++e) o_f[e] *= keep[j];
       }
     };
-    if (kHeld == kCount) {
+    if constexpr (kAllHeld) {
       __builtin_amdgcn_sched_barrier(0);
-    start(0);
-#pragma unroll
-    for (int t = 0; t < kKeyTiles; ++t) {
-      product(0, t);
-      between(t, kCount * kKeyTiles);
-    }
+      first_products();
     }
     rescale(0);
 #pragma unroll
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
         merge_piece(j - 1, t, kKeyTiles);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (kHeld < kCount && j + 1 < kCount) read(j + 1);
+      if (!kAllHeld && j + 1 < kCount) read(j + 1);
       rescale(j);
       __builtin_amdgcn_sched_barrier(0);
     }

@@ -289,3 +289,31 @@ def test_the_tile_of_a_short_sequence_asks_for_no_lane(kernels):
     partly filled ends ask for the lane as often as those without (eight times more often cost such a call 0.1 us)."""
     asked = {re.search(r"fwd_kernelI(\S+?EL)b(.)(ELb.E)EEvNS", f.split(":")[0]).groups(): f.count("v_mbcnt_lo") for f in kernels if "fwd_kernel" in f.split(":")[0]}
     assert len(asked) == 64 and {k: n for k, n in asked.items() if n > asked[k[0], "0", k[2]]} == {}
+
+
+def _maxima_behind_operand_reads(func_text):
+    """Float maxima between the transposing reads of V (and what stands between those) and the next matrix instruction, for each run of them."""
+    found, reads, maxima = [], 0, 0
+    for line in func_text.split("s_endpgm")[0].split("\n")[1:]:
+        t = line.strip()
+        if t.startswith("ds_read_b64_tr"):
+            reads, maxima = reads + 1, 0
+        elif t.startswith("v_mfma"):
+            found += [maxima] if reads else []
+            reads = 0
+        elif t.startswith("v_max_f32"):
+            maxima += 1
+    return found
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_the_first_product_of_a_merge_does_not_wait_for_the_weights(kernels):
+    """Split kernel: the weights of a round's key blocks, a chain of maxima and exponentials, are computed behind the first product, which needs none of
+    them - but where the operands of all blocks are asked for together (one row group, blocks of 64 keys, 128 steps), over whose latency they are."""
+    late = {}
+    for f in kernels:
+        m = re.search(r"split_kernelILi\d+ELi(\d+)ELb.ELb.ELb(.)ELi(\d)ELb0E", f.split(":")[0])
+        if m:
+            all_held = m.groups() == ("64", "0", "1")
+            late[f.split(":")[0]] = (_maxima_behind_operand_reads(f)[0] > 0) == all_held
+    assert len(late) == 64 and [name for name, as_meant in late.items() if not as_meant] == []
