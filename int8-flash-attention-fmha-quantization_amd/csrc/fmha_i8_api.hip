@@ -191,10 +191,9 @@ hipError_t launch_split(const Piece& piece, Variant var, hipStream_t stream, con
 // Microseconds * 100 beyond the launch (2.8 us), [head_dim 64, 128][blocks of 64, 128 keys], measured on one MI355X with one
 // workgroup on half of the CUs (tests/variant_timing.py --kernel-costs), `again` with two to eight on every CU (--shapes); measurements differ
 // by 4 %.  With starts measured before Q went through LDS and no `again`, calls of 130 to 256 keys at d64 took the 256-row kernel
-// that smaller workgroups serve faster (B5 H8 S256 6.40 -> 5.41 us, B8 H12 S144 6.62 -> 5.01).  The last kernel's
-// entries at d = 64 are its line up to 2048 keys: at 4096 a call of 128 heads, each with its own keys, takes 6 % longer (the memory).
+// that smaller workgroups serve faster (B5 H8 S256 6.40 -> 5.41 us, B8 H12 S144 6.62 -> 5.01).
 // With all CUs at work the first two take up to 36 and 14 % longer per block (the shader clock drops).
-constexpr int kComputeUnits = 256;
+constexpr int kComputeUnits = 256, kLaunch = 280;
 struct KernelCost {
   int row_groups, keys_per_round;
   struct { int start, step, again; } cost[2][2];
@@ -202,17 +201,35 @@ struct KernelCost {
 constexpr KernelCost kKernelCosts[] = {{0, 1, {{{70, 80, 120}, {105, 129, 120}}, {{160, 99, 220}, {235, 162, 220}}}},
                                        {4, 1, {{{107, 62, 130}, {142, 96, 140}}, {{171, 82, 190}, {252, 117, 200}}}},
                                        {2, 4, {{{0, 186, 150}, {20, 300, 150}}, {{20, 200, 190}, {61, 332, 260}}}},
-                                       {1, 4, {{{0, 136, 20}, {6, 211, 150}}, {{25, 153, 180}, {36, 247, 180}}}},
-                                       {kFew, 4, {{{0, 97, 0}, {0, 149, 0}}, {{15, 138, 0}, {75, 225, 0}}}}};
-constexpr KernelCost kOneGroupCost = kKernelCosts[3], kFewCost = kKernelCosts[4];
-static_assert(kOneGroupCost.row_groups == 1 && kFewCost.row_groups == kFew, "");
+                                       {1, 4, {{{0, 136, 20}, {6, 211, 150}}, {{25, 153, 180}, {36, 247, 180}}}}};
+// At most 32 query rows: every workgroup, one to a head or to a part of one, fetches keys of its own, and calls of more heads than there
+// are compute units run into the memory.  So these have prices of their own, the same way for a head by one workgroup as for key blocks
+// shared out ([at most sixteen rows, more][head_dim][block]): the workgroups that run at a time take max(start + step * rounds + again,
+// their keys at 67 KB in a hundredth of a microsecond), `again` from the second time on; `together` is how many a CU holds, of which the
+// second adds half of the first one's time.  Fitted to 1,347 calls of 4 to 1024 heads timed on both routes; see part_plan_of.
+struct HeadCost {
+  int start, step, again, together;
+};
+constexpr HeadCost kHeadCosts[2][2][2] = {{{{-60, 103, 140, 2}, {-25, 145, 150, 1}}, {{-20, 131, 150, 1}, {20, 230, 200, 1}}},
+                                          {{{-15, 135, 150, 2}, {0, 213, 240, 1}}, {{20, 152, 230, 1}, {20, 230, 200, 1}}}};
+constexpr HeadCost kPartCosts[2][2][2] = {{{{60, 106, 0, 2}, {20, 200, 80, 1}}, {{20, 165, 130, 1}, {70, 210, 130, 1}}},
+                                          {{{35, 90, 70, 1}, {20, 187, 120, 1}}, {{25, 155, 70, 1}, {10, 285, 260, 1}}}};
+long long cost_of_head_workgroups(const HeadCost& c, long long wgs, int rounds, long long key_bytes) {
+  const long long at_a_time = (long long)kComputeUnits * c.together, full = wgs / at_a_time, rest = wgs % at_a_time;
+  auto one_time = [&](long long n, bool first) -> long long {
+    const long long alone = c.start + c.step * rounds, work = (n > kComputeUnits ? alone * 3 / 2 : alone) + (first ? 0 : c.again);
+    const long long memory = n * key_bytes / (wgs * 67000);
+    return work > memory ? work : memory;
+  };
+  return (full > 0 ? one_time(at_a_time, true) + (full - 1) * one_time(at_a_time, false) : 0) + (rest > 0 ? one_time(rest, full == 0) : 0);
+}
 // Groups of 32 query rows per workgroup of the kernel that serves `rows` query rows of `heads` heads: 1 or 2 (fmha_i8_split_kernel), 4
 // (fmha_i8_pair_kernel), kFew (fmha_i8_few_kernel), or 0 for the kernel of 256-row workgroups.  All write the same bytes.
 //
-// Each kernel's time beyond the dispatch is modelled as (workgroups per CU, rounded up) * (cost of one).  What the constants
-// order is far apart nearly everywhere - d128, S2048: H4 31.0 us in 256-row workgroups, 24.4 in those of four groups, 17.6 of
-// two, 13.4 of one; H8 31.3, 24.6, 17.9, 25.8; H16 31.7, 26.2, 34.5, 50.3; H24 33.9, 48.9, 50.7, 74.6 - so that a few percent of
-// error only shift the boundary between equals.
+// Each kernel's time beyond the launch is modelled as (workgroups per CU, rounded up) * (cost of one), and `again` for all but the
+// first; at most 32 query rows as above.  What the constants order is far apart nearly everywhere - d128, S2048: H4 31.0 us in 256-row
+// workgroups, 24.4 in those of four groups, 17.6 of two, 13.4 of one; H8 31.3, 24.6, 17.9, 25.8; H16 31.7, 26.2, 34.5, 50.3; H24 33.9,
+// 48.9, 50.7, 74.6 - so that a few percent of error only shift the boundary between equals.
 struct Choice {
   int row_groups;
   long long cost;  // hundredths of a microsecond
@@ -223,7 +240,7 @@ long long cost_of_workgroups(const KernelCost& kernel, long long wgs, int head_d
   return per_cu * (c.start + c.step * ((blocks + kernel.keys_per_round - 1) / kernel.keys_per_round)) + (per_cu - 1) * c.again;
 }
 int rows_of(const KernelCost& kernel) {
-  return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : kernel.row_groups == kFew ? fmha_i8_gfx950::kFewRows : 32 * kernel.row_groups;
+  return kernel.row_groups == 0 ? fmha_i8_gfx950::kBlockQ : 32 * kernel.row_groups;
 }
 // At most sixteen rows, and not the geometry that the split kernel's second group serves better (see fmha_i8_few_kernel).
 bool few_takes(int rows, int head_dim, int block_keys) {
@@ -231,19 +248,20 @@ bool few_takes(int rows, int head_dim, int block_keys) {
 }
 // With one group's worth of rows the second group of the split kernel only helps to fetch the tiles, which pays where a round is 128 KB
 // (B8 H16 Sq1 S2048 d128: 15.9 us with one group, 14.1 with two; H96 S2048 14.9 and 13.7, S16384 116 and 99; with 16 heads 13.1 and
-// 12.6; at d64 11.7 either way): there it takes one group's place.  128 heads measure 0.5 + 2.6 us a round, the memory's share in it;
-// the price is one group's, 1 % lower: without that, calls of two rounds would share their key blocks out (H16 Sq1 S1024 8.2 us plain,
-// 8.5 shared out).
+// 12.6; at d64 11.7 either way): there it takes one group's place.
 bool second_group_fetches(int rows, int head_dim, int block_keys) { return rows <= 32 && head_dim == 128 && block_keys == fmha_i8_gfx950::kBlockK; }
-constexpr KernelCost kFetchingCost{2, 4, {{}, {{}, {95, 240, 260}}}};
 Choice cheapest_kernel(long long heads, int rows, int head_dim, int blocks, int block_keys) {
+  if (rows <= 32) {
+    const bool few = few_takes(rows, head_dim, block_keys), fetching = second_group_fetches(rows, head_dim, block_keys);
+    // (a last round of one or two key blocks: the two-step form stops behind its first step, half a microsecond sooner)
+    const int left_out = fetching && (blocks & 3) != 0 && (blocks & 3) <= 2 ? 50 : 0;
+    const HeadCost& price = kHeadCosts[rows > fmha_i8_gfx950::kFewRows][head_dim == 128][block_keys == fmha_i8_gfx950::kBlockK];
+    const HeadCost here{price.start - left_out, price.step, price.again, price.together};
+    return {few ? kFew : fetching ? 2 : 1, cost_of_head_workgroups(here, heads, (blocks + 3) / 4, 2 * heads * blocks * block_keys * head_dim)};
+  }
   Choice best{0, -1};
   for (const KernelCost& kernel : kKernelCosts) {
-    if (kernel.row_groups == kFew && !few_takes(rows, head_dim, block_keys)) continue;
-    const bool fetching = second_group_fetches(rows, head_dim, block_keys);
-    if (rows <= 32 && kernel.row_groups == (fetching ? 1 : 2)) continue;
-    const KernelCost& price = fetching && kernel.row_groups == 2 ? kFetchingCost : kernel;
-    const long long cost = cost_of_workgroups(price, heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)), head_dim, blocks, block_keys);
+    const long long cost = cost_of_workgroups(kernel, heads * ((rows + rows_of(kernel) - 1) / rows_of(kernel)), head_dim, blocks, block_keys);
     if (best.cost < 0 || cost < best.cost) best = {kernel.row_groups, cost};
   }
   return best;
@@ -256,13 +274,12 @@ Choice row_groups_of(const FMHACrossAttnDescriptor& a, int block_keys) {
 }
 // The launches of a call: one, or two where large workgroups would leave most compute units idle in their last wave, or in the last
 // rows of every head.  The first launch then takes as many heads, or as many rows of every head, as make full waves of workgroups of 256
-// or 128 rows, the second one the rest in smaller ones.  A second launch costs 2.9 us, and 5 % are left to the model's error.
+// or 128 rows, the second one the rest in smaller ones.  A second launch costs 2.8 us, and 5 % are left to the model's error.
 int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[2]) {
   const int heads = a.batch_num * a.head_num, rows = a.seq_len_q, blocks = (a.seq_len_kv + block_keys - 1) / block_keys;
   const Choice whole = row_groups_of(a, block_keys);
   pieces[0] = {whole.row_groups, 0, heads, 0, rows};
   if (whole.cost < 0 || rows <= 32 || fmha_i8_gfx950::test_build::forced_route() == fmha_i8_gfx950::test_build::kOneLaunch) return 1;
-  constexpr long long kLaunch = 290;
   long long least = whole.cost * 19 / 20;
   int count = 1;
   auto consider = [&](const KernelCost& kernel, int first_heads, int first_rows) {
@@ -286,18 +303,18 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
   }
   return count;
 }
-// Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for, by the cost
-// table above (start, step of one row group), but no faster than the memory (62 KB in a hundredth of a microsecond, on both
-// sides of the comparison), with the workspace written and read again, and the merge: 2.5 us for the launch and a first batch of
-// key blocks, 0.8 per further batch; with more than sixteen rows, of which some row moves its reference in nearly every block, 1.2 and 0.06
-// per block on top (plain and shared out: H32 Sq32 S777 d64 8.8 and 9.5, H64 Sq32 S3000 d64 20.4 and 22.6, B2 H16 Sq32 S2048 d128 12.8 and
-// 14.2 us, all of which the model put 6 to 18 % the other way round).  Within 5 % of each other (the factor 20/21) the plain route is taken, which needs no memory: the
-// model flatters the other one there - of eleven shapes that it put 0 to 5 % ahead nine were slower shared out, by 2 to 21 % (H32
-// Sq32 S1500 d128 11.1 -> 13.5 us).  One call, plain
-// -> shared out: B1 H16 Sq1 S2048 d128 12.6 -> 8.3 us, H32 S4096 22.2 -> 10.1, H32 S8192 42.8 -> 18.7; H16 Sq32 S4096 21.6 -> 15.1; B8 H16 Sq1 S2048 d128, which the memory bounds already, 14.0 -> 15.9 and hence not.
-// Up to sixteen rows both sides are fmha_i8_few_kernel's, or the split kernel's second group's against it; plain -> shared out: d64 B8 H16
-// Sq1 S2048 8.9 -> 9.4 us, S8192 28.9 -> 28.9, H64 S2048 8.7 -> 7.6, H16 S1024 5.8 -> 7.4, H16 S4096 14.7 -> 8.6; d128 B4 H16 Sq4 S1984
-// 14.4 -> 12.0, B8 H16 Sq1 S1984 14.8 -> 16.8.
+// Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for (kPartCosts), with the
+// workspace written and read again (45 KB in a hundredth of a microsecond, 42 above sixteen rows) and the merge: 2.1 us for the launch and
+// the first batch of key blocks, 1.1 more for batches of 32 instead of 16, 0.8 per further batch; 0.9 on top with more than sixteen rows,
+// of which some row moves its reference in nearly every block.  (One head and up to eight heads are put 0.4 and 0.5 us too low: calls whose
+// two routes are that close stay shared out, as they have been - H1 Sq8 S1089 d64 7.2 us either way, H6 Sq5 S1030 d64 7.4 and 8.0.)  Within 5 %
+// of each other (the factor 20/21) the plain route is taken, which needs no memory and can write a float output besides.
+// One call, plain and shared out, us: d128 B1 H16 Sq1 S2048 12.1 and 8.0, H32 S4096 21.6 and 9.6, H16 Sq32 S4096 21.2 and 14.6, B2 H16 Sq32
+// S1664 11.6 and 12.8, S2048 12.1 and 13.7, H16 Sq17 S1152 9.3 and 9.8, H264 Sq1 S640 15.4 and 18.1, S1152 22.3 and 20.3, B8 H16 Sq1 S2048,
+// which the memory bounds already, 13.8 and 14.7; d64 H64 Sq1 S2048 8.5 and 7.6, H264 Sq1 S1088 9.3 and 14.2.
+// Of 2,115 such calls timed on both routes, 1 to 1024 heads, the choice is more than 2 % slower than the other one in 47, more than 10 % in
+// 6, at most by 17 % (H40 Sq24 S2076 d64).  It was in 208 and 62 with a table that priced the two sides apart and took each further workgroup on
+// a CU for as dear as the first, the memory for a bound on the whole call alone.
 PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   using namespace fmha_i8_gfx950;
   PartPlan plan;
@@ -305,21 +322,20 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   const long long heads = (long long)a.batch_num * a.head_num;
   if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
   if (test_build::forced_route() >= 0) return plan;
-  const long long memory = 2 * heads * a.seq_len_kv * a.head_dim / 62000;
   const bool one_group = a.seq_len_q > kFewRows;
-  const long long merge = 250 + 80 * ((blocks - 1) / 32) + (one_group ? 120 + 6 * blocks : 0) + heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / 62000;
-  const KernelCost& kernel = !one_group ? kFewCost : kOneGroupCost;
-  const auto& c = kernel.cost[a.head_dim == 128][block_keys == kBlockK];
-  long long least = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys).cost;
-  least = (least > memory ? least : memory) * 20 / 21;
+  const long long merge = 210 - 42 / heads + (blocks <= 16 ? 0 : heads > 8 ? 110 : 55) + 80 * ((blocks - 1) / 32) + (one_group ? 90 : 0) +
+                          heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / (one_group ? 42000 : 45000);
+  const HeadCost& price = kPartCosts[one_group][a.head_dim == 128][block_keys == kBlockK];
+  const long long plain = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys).cost * 20 / 21;
+  const long long key_bytes = 2 * heads * blocks * block_keys * a.head_dim;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
-    const long long of_r = cost_of_workgroups(kernel, heads * ((rounds + r - 1) / r), a.head_dim, kSplitKeys * r, block_keys);
+    const long long of_r = cost_of_head_workgroups(price, heads * ((rounds + r - 1) / r), r, key_bytes);
     if (plan.rounds_per_part > 0 && of_r > work) continue;
     work = of_r;
     plan.rounds_per_part = r;
   }
-  if ((work > memory ? work : memory) + merge >= least && test_build::forced_route() != test_build::kSharedOut) plan.rounds_per_part = 0;
+  if (work + merge >= plain && test_build::forced_route() != test_build::kSharedOut) plan.rounds_per_part = 0;
   const size_t rows = (size_t)heads * blocks * a.seq_len_q;
   plan.ml_bytes = (rows * sizeof(v2f) + 255) / 256 * 256;
   plan.bytes = plan.ml_bytes + rows * a.head_dim * sizeof(int);

@@ -156,6 +156,25 @@ def test_calls_that_want_a_workspace(pkg):
         assert need(*shape) == 0, shape
 
 
+# (heads, Sq, S, d) of calls on either side of the line, timed on both routes (plain, shared out, us, on one MI355X)
+PLAIN_OR_SHARED = [
+    # 17 to 32 rows in blocks of 128 keys at d = 128, where the second row group of the plain kernel only fetches
+    (32, 32, 1664, 128, 11.64, 12.71), (32, 32, 1792, 128, 11.66, 12.99), (32, 32, 1920, 128, 12.18, 13.37), (32, 32, 2048, 128, 12.20, 13.65), (16, 17, 1152, 128, 9.29, 9.83),
+    (32, 32, 1152, 128, 9.38, 11.77), (8, 32, 1408, 128, 9.87, 9.47), (16, 32, 2048, 128, 12.15, 11.00), (32, 32, 4096, 128, 21.97, 19.86),
+    # a few heads more than there are compute units
+    (264, 1, 640, 128, 15.28, 18.15), (264, 1, 1152, 128, 22.20, 20.29), (264, 1, 2176, 128, 35.53, 31.22), (384, 1, 640, 128, 16.09, 20.62), (264, 4, 640, 128, 15.43, 19.28),
+    (320, 4, 640, 128, 15.83, 20.07), (264, 1, 1088, 64, 9.36, 14.19), (264, 1, 1600, 64, 13.21, 17.08), (264, 1, 2112, 64, 16.20, 22.35), (264, 1, 3136, 64, 21.85, 27.65),
+    # the sixteen-row kernel
+    (64, 1, 1088, 64, 7.33, 8.90), (52, 16, 2437, 64, 12.80, 16.93), (128, 1, 2048, 64, 8.90, 9.43), (16, 1, 4096, 64, 14.70, 8.60),
+]
+
+
+@pytest.mark.parametrize("heads,rows,keys,d,plain,shared", PLAIN_OR_SHARED)
+def test_the_faster_of_plain_and_shared_out_is_chosen(pkg, heads, rows, keys, d, plain, shared):
+    wants = pkg.load_library().FMHAInferI8CrossWorkspaceBytes(pkg.FMHACrossAttnDescriptor(1, rows, keys, heads, d)) > 0
+    assert wants == (shared < plain)
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(tmp_path):
     """The same check as for the other kernel (test_kernel_async_loads.py), on the compiled split kernel."""
