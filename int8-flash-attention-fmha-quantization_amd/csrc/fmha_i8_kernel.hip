@@ -599,7 +599,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
         int qrow = min(row0 + row, Sq - 1);
         if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
         const int src = qrow * D + (((q_lane % kChunks) ^ k_swizzle<D>(row)) << 4);
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * it), "v"(src), "s"(qp) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 ; Q, shared 0" ::"s"(dst + 1024u * it), "v"(src), "s"(qp) : "memory");
       }
       return;
     }
@@ -617,8 +617,10 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk) asm volatile("" : "+v"(qreg[kk]));
   };
-  auto read_q_rows = [&]() __attribute__((always_inline)) {  // behind the wait that retires their loads
+  auto read_q_rows = [&](bool place_reused) __attribute__((always_inline)) {  // behind the wait that retires their loads
     if constexpr (kQThroughLds) {
+      if (place_reused) asm volatile("; Q from LDS, place reused" ::: "memory");
+      else asm volatile("; Q from LDS" ::: "memory");
       const int8_t* lds_q_rows = q_place();
 #pragma unroll
       for (int kk = 0; kk < kDSteps; ++kk) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q_rows + k_read_off[kk]);
@@ -715,7 +717,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     if (kV0BeforeFirstBarrier) {
       if (kQThroughLds) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPrologueRegions) : "memory");
-        read_q_rows();
+        read_q_rows(kQSlots < 8);
       }
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       pin_q_rows();
@@ -725,7 +727,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
     if (!kV0BeforeFirstBarrier) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       pin_q_rows();
-      read_q_rows();
+      read_q_rows(false);
       issue_tile0_by_half(vg, 1, ld_goff_v);
     }
   };
@@ -734,7 +736,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   auto first_barrier = [&]() __attribute__((always_inline)) {
     prologue_done = true;
     barrier();
-    if (wave < 4) read_q_rows();
+    if (wave < 4) read_q_rows(kQSlots < 8 && !kV0BeforeFirstBarrier);
     {
       const v4i s0 = *reinterpret_cast<const v4i*>(&lds_scan[0]), s1 = *reinterpret_cast<const v4i*>(&lds_scan[4]);
       kb_end = __builtin_amdgcn_readfirstlane(max(max(s0[0], s0[2]), max(s1[0], s1[2]))) + 1;
@@ -1319,8 +1321,12 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   if (wave < kClassWaves) {
     prologue_waves_0_to_3();
     first_barrier();
-    if (n > 0 && works(0)) gemm1_of(0);
-    else forget_scores();
+    if (n > 0 && works(0)) {
+      gemm1_of(0);
+    } else {
+      forget_scores();
+      if (kQThroughLds) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the Q rows, which GEMM 1 has waited for otherwise)
+    }
     issue_first();
     int i = 0;
     // Steady state, as long as blocks i and i+1 exist and have no masked key: the same phases as the general loop

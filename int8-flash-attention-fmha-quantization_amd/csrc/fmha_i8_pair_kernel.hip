@@ -97,7 +97,8 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   }
   v4i qreg[kDSteps];
   // Q: at head_dim 128 through LDS, by whole rows (see the 256-row kernel; B1 H16 S2048 25.39 -> 24.82 us); the two wavefronts of a row group
-  // fetch half of its rows each, into what holds P of the first half from tick 0 on.
+  // fetch half of its rows each, into what holds P from tick 0 on: of the first half in blocks of 128 keys, of both halves and of other row
+  // groups in blocks of 64.  So every wavefront has its operands before it arrives at its next barrier, two in front of the first P (q_rows_read).
   constexpr bool kQThroughLds = D == 128;
   constexpr int kQLoads = kQThroughLds ? kDSteps / 2 : kDSteps;
   const int8_t* lds_q = reinterpret_cast<const int8_t*>(&lds_p[0][0][0][0]) + r * (32 * D);
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       int qrow = min(row0 + row, Sq - 1);  // rows past the end load the last row (unused)
       if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
       const int src = qrow * D + (((lane % kChunks) ^ k_swizzle<D>(row)) << 4);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * region), "v"(src), "s"(qp) : "memory");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 ; Q, shared 1" ::"s"(dst + 1024u * region), "v"(src), "s"(qp) : "memory");
     }
   } else {
     int qrow = min(row0 + i32, Sq - 1);  // rows past the end load the last row (unused)
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
   }
   barrier();
   all_loads_landed();
+  if (kQThroughLds) asm volatile("; Q from LDS, place reused" ::: "memory");
 #pragma unroll
   for (int kk = 0; kk < kDSteps; ++kk) {
     if constexpr (kQThroughLds) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q + k_read_off[kk]);
@@ -424,10 +426,17 @@ __global__ __launch_bounds__(512, 2) void fmha_i8_pair_kernel(const SplitKernelA
       }
     }
   };
+  // (the compiler puts the reads of Q behind the one of the scan: nothing else waits for them in front of these barriers)
+  auto q_rows_read = [&]() { if (kQThroughLds) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
   if (n > 0) {
-    if (h != 0) barrier();  // tick -2 is the first half's: GEMM 1 of block 0
+    if (h != 0) {
+      q_rows_read();
+      barrier();  // tick -2 is the first half's: GEMM 1 of block 0
+    }
     read_first(stage_k);
-    int cls = gemm1_of(h, active ? cls_of(h) : 2);  // of the own block whose scores are in acc
+    int cls = active ? cls_of(h) : 2;  // of the own block whose scores are in acc
+    q_rows_read();
+    gemm1_of(h, cls);
     int T = h;
     for (; T <= n; T += 2) {
       barrier();  // tick T-1

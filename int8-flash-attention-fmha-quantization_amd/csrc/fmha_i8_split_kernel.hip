@@ -281,7 +281,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
       int qrow = min(row0 + row, Sq - 1);
       if (!fmha_in_bounds(qrow >= 0 && qrow < Sq)) qrow = 0;
       const int src = qrow * D + (((lane % kChunks) ^ k_swizzle<D>(row)) << 4);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + 1024u * region), "v"(src), "s"(qp) : "memory");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 ; Q, shared %3"
+                   ::"s"(dst + 1024u * region), "v"(src), "s"(qp), "n"(kQShared) : "memory");
     }
   }
 #pragma unroll
@@ -325,6 +326,7 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
                                                          reinterpret_cast<unsigned char*>(lds_class4), keys_from, keys_to);
   if (lane == 0) lds_scan[wave] = live_hi;
   auto read_q = [&]() __attribute__((always_inline)) {
+    asm volatile("; Q from LDS, place reused" ::: "memory");
 #pragma unroll
     for (int kk = 0; kk < kDSteps; ++kk) qreg[kk] = *reinterpret_cast<const v4i*>(lds_q + k_read_off[kk]);
   };

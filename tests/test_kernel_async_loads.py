@@ -173,7 +173,7 @@ def test_no_read_of_an_asynchronously_loaded_register_before_its_wait(kernels):
     checked = 0
     for f in kernels:
         checked += _check_function(f.split(":")[0], f)
-    # at least the mask bytes and the Q rows (two or four loads) of every kernel
+    # at least the two loads of mask bytes of every kernel and the Q rows of those that load them into registers
     assert checked >= 3 * len(kernels)
 
 
@@ -317,3 +317,104 @@ def test_the_first_product_of_a_merge_does_not_wait_for_the_weights(kernels):
             all_held = m.groups() == ("64", "0", "1")
             late[f.split(":")[0]] = (_maxima_behind_operand_reads(f)[0] > 0) == all_held
     assert len(late) == 64 and [name for name, as_meant in late.items() if not as_meant] == []
+
+
+def _whole_function(func_text):
+    """Basic blocks and successors as in _blocks, those behind the first `s_endpgm` with them; comments stay."""
+    blocks, order, cur = {"entry": []}, ["entry"], "entry"
+    for line in func_text.split(".Lfunc_end")[0].split("\n")[1:]:
+        m, t = re.match(r"^(\.LBB\d+_\d+):", line), line.strip()
+        if m:
+            cur = m.group(1)
+            blocks[cur] = []
+            order.append(cur)
+        elif t and (t.startswith("; Q from LDS") or not re.match(r"[.;]|[^;]*:$", t)):
+            blocks[cur].append(t)
+            if re.match(r"s_c?branch|s_endpgm", t):
+                cur = "%s+%d" % (cur, len(blocks[cur]))
+                blocks[cur] = []
+                order.append(cur)
+    succ = {}
+    for i, name in enumerate(order):
+        last = blocks[name][-1] if blocks[name] else ""
+        to = re.match(r"s_c?branch\w*\s+(\.LBB\d+_\d+)", last)
+        falls = not re.match(r"s_branch|s_endpgm", last) and i + 1 < len(order)
+        succ[name] = ([to.group(1)] if to else []) + ([order[i + 1]] if falls else [])
+    return blocks, succ
+
+
+def _paths(blocks, succ, block, start, state, step):
+    """Runs step(state, instruction) along every path from there; a state is a tuple of numbers, step returns None where a path is done with."""
+    seen, work = set(), [(block, start, state)]
+    while work:
+        b, i, s = work.pop()
+        for t in blocks[b][i:]:
+            s = step(s, t)
+            if s is None:
+                break
+        else:
+            work += [x for x in ((to, 0, s) for to in succ[b]) if x not in seen]
+            seen.update((to, 0, s) for to in succ[b])
+
+
+def _check_q_through_lds(func_text, waits=True):
+    """How many loads ask for Q rows through LDS.  On every path (a) from such a load the place where the rows are read again (the reads cannot be
+    moved in front of it) stands behind the wait that retires the load, and, where other wavefronts fetch some of the rows, behind a barrier after that
+    wait; (b) from there, where the rows' place is written again later, no 128-bit LDS read is in flight at the next barrier."""
+    blocks, succ = _whole_function(func_text)
+
+    def landed(shared):
+        def step(s, t):
+            issued, waited = s
+            w = WAIT.match("\t" + t)
+            waited |= bool(w and int(w.group(1)) <= issued)
+            if waited and (not shared or t.startswith("s_barrier")):
+                return None
+            assert not t.startswith("; Q from LDS"), "read too early"
+            return min(issued + bool(VMEM.match(t)), 63), waited
+        return step
+
+    def arrived(s, t):
+        behind, = s  # LDS and scalar memory instructions behind the last 128-bit read; -1: none in flight
+        w = re.match(r"s_waitcnt\b.*lgkmcnt\((\d+)\)", t)
+        if w and int(w.group(1)) <= behind:
+            behind = -1
+        if t.startswith("s_barrier"):
+            assert behind < 0, "read in flight at a barrier"
+            return None
+        if t.startswith("ds_read_b128"):
+            return 0,
+        return min(behind + (behind >= 0 and bool(re.match(r"ds_|s_load", t))), 15),
+
+    loads = 0
+    for b in blocks:
+        for i, t in enumerate(blocks[b]):
+            m = re.search(r"global_load_lds_dwordx4.*; Q, shared (\d)", t)
+            loads += bool(m)
+            if m and waits:
+                _paths(blocks, succ, b, i + 1, (0, False), landed(m.group(1) == "1"))
+            if t == "; Q from LDS, place reused":
+                _paths(blocks, succ, b, i + 1, (-1,), arrived)
+    return loads
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_q_rows_through_lds_are_waited_for(kernels):
+    """The kernels of head size 128 whose Q rows pass through LDS: all but the split kernel's forms of one row group and blocks of 64 keys.  (No counting of
+    waits in the pair kernel and for partly filled ends in the 256-row one: two branches on one condition there, whose paths this would mix.)"""
+    counted = lambda name: not re.search(r"pair_kernel|fwd_kernelILi128ELi\d+ELb.ELb.ELb1E", name)
+    through = {f.split(":")[0]: _check_q_through_lds(f, counted(f.split(":")[0])) for f in kernels}
+    for name, loads in through.items():
+        kind, d, block = re.search(r"(fwd|split|pair)_kernelILi(\d+)ELi(\d+)", name).groups()
+        own_k = re.search(r"split_kernelILi\d+ELi64ELb.ELb.ELb.ELi1E", name)
+        assert (loads > 0) == (d == "128" and not own_k), (name, loads)
+
+
+def test_the_q_checker_itself_finds_what_it_looks_for():
+    ok = ("f:\n\tglobal_load_lds_dwordx4 v1, s[2:3] ; Q, shared 1\n\ts_waitcnt vmcnt(0)\n\ts_barrier\n\t; Q from LDS, place reused\n\tds_read_b128 v[2:5], v1\n\ts_waitcnt lgkmcnt(0)\n"
+          "\ts_barrier\n\ts_endpgm\n.Lfunc_end0:\n")
+    assert _check_q_through_lds(ok) == 1
+    late = ok.replace("\ts_waitcnt lgkmcnt(0)\n\ts_barrier", "\ts_cbranch_scc1 .LBB0_9\n\ts_waitcnt lgkmcnt(0)\n.LBB0_9:\n\ts_barrier")
+    for wrong in (ok.replace("vmcnt(0)", "vmcnt(1)"), ok.replace("vmcnt(0)\n\ts_barrier", "vmcnt(0)"), ok.replace("lgkmcnt(0)", "lgkmcnt(1)"), late):
+        with pytest.raises(AssertionError):
+            _check_q_through_lds(wrong)
