@@ -312,8 +312,8 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
 // One call, plain and shared out, us: d128 B1 H16 Sq1 S2048 12.1 and 8.0, H32 S4096 21.6 and 9.6, H16 Sq32 S4096 21.2 and 14.6, B2 H16 Sq32
 // S1664 11.6 and 12.8, S2048 12.1 and 13.7, H16 Sq17 S1152 9.3 and 9.8, H264 Sq1 S640 15.4 and 18.1, S1152 22.3 and 20.3, B8 H16 Sq1 S2048,
 // which the memory bounds already, 13.8 and 14.7; d64 H64 Sq1 S2048 8.5 and 7.6, H264 Sq1 S1088 9.3 and 14.2.
-// Of 2,115 such calls timed on both routes, 1 to 1024 heads, the choice is more than 2 % slower than the other one in 47, more than 10 % in
-// 6, at most by 17 % (H40 Sq24 S2076 d64).  It was in 208 and 62 with a table that priced the two sides apart and took each further workgroup on
+// Of 1,923 such calls timed on both routes, 1 to 1024 heads, the choice is more than 2 % slower than the other one in 51, more than 10 % in
+// 6, at most by 18 % (H40 Sq24 S2076 d64).  It was in 193 and 57 with a table that priced the two sides apart and took each further workgroup on
 // a CU for as dear as the first, the memory for a bound on the whole call alone.
 PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   using namespace fmha_i8_gfx950;
@@ -327,14 +327,16 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
                           heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / (one_group ? 42000 : 45000);
   const HeadCost& price = kPartCosts[one_group][a.head_dim == 128][block_keys == kBlockK];
   const long long plain = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys).cost * 20 / 21;
-  const long long key_bytes = 2 * heads * blocks * block_keys * a.head_dim;
   long long work = 0;
   for (int r = 1; r < rounds; ++r) {
-    const long long of_r = cost_of_head_workgroups(price, heads * ((rounds + r - 1) / r), r, key_bytes);
+    // (without the memory, which makes equals of splits that are not: H32 Sq1 S8192 d128 18.6 us in 256 workgroups, 22.0 in 512)
+    const long long of_r = cost_of_head_workgroups(price, heads * ((rounds + r - 1) / r), r, 0);
     if (plan.rounds_per_part > 0 && of_r > work) continue;
     work = of_r;
     plan.rounds_per_part = r;
   }
+  const int r = plan.rounds_per_part;
+  work = cost_of_head_workgroups(price, heads * ((rounds + r - 1) / r), r, 2 * heads * blocks * block_keys * a.head_dim);
   if (work + merge >= plain && test_build::forced_route() != test_build::kSharedOut) plan.rounds_per_part = 0;
   const size_t rows = (size_t)heads * blocks * a.seq_len_q;
   plan.ml_bytes = (rows * sizeof(v2f) + 255) / 256 * 256;
@@ -534,6 +536,8 @@ int FMHAInferI8DebugLaunches(FMHACrossAttnDescriptor desc, int* first_heads, int
   *first_rows = pieces[0].end_row;
   return count;
 }
+// Test build only: the rounds of a workgroup of a call that shares its key blocks out, 0 for others.
+int FMHAInferI8DebugRoundsPerPart(FMHACrossAttnDescriptor desc) { return part_plan_of(desc, block_keys_of(desc.seq_len_kv)).rounds_per_part; }
 // Test build only: the kernel of the second launch, as FMHAInferI8DebugRoute names it, or -1.
 int FMHAInferI8DebugSecondKernel(FMHACrossAttnDescriptor desc) {
   Piece pieces[2];

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import fmha_cases as fc
+import routes
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -173,6 +174,17 @@ PLAIN_OR_SHARED = [
 def test_the_faster_of_plain_and_shared_out_is_chosen(pkg, heads, rows, keys, d, plain, shared):
     wants = pkg.load_library().FMHAInferI8CrossWorkspaceBytes(pkg.FMHACrossAttnDescriptor(1, rows, keys, heads, d)) > 0
     assert wants == (shared < plain)
+
+
+# (us on one MI355X, with the workgroups that the memory's share alone would not tell apart: 512, 1024, 448)
+@pytest.mark.parametrize("heads,keys,d,rounds", [(32, 8192, 128, 2),   # 18.6, 22.0
+                                                (8, 65536, 128, 4),   # 60.0, 64.7
+                                                (64, 3584, 128, 2),   # 15.1, 16.9
+                                                (16, 8192, 64, 1), (16, 2048, 128, 1)])
+def test_shared_out_key_blocks_make_one_wave_of_workgroups(pkg, heads, keys, d, rounds):
+    lib = routes.library(pkg)
+    lib.FMHAInferI8DebugRoundsPerPart.argtypes = [pkg.FMHACrossAttnDescriptor]
+    assert lib.FMHAInferI8DebugRoundsPerPart(pkg.FMHACrossAttnDescriptor(1, 1, keys, heads, d)) == rounds
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
