@@ -161,6 +161,7 @@ def test_calls_that_want_a_workspace(pkg):
 PLAIN_OR_SHARED = [
     # 17 to 32 rows in blocks of 128 keys at d = 128, where the second row group of the plain kernel only fetches
     (32, 32, 1664, 128, 11.64, 12.71), (32, 32, 1792, 128, 11.66, 12.99), (32, 32, 1920, 128, 12.18, 13.37), (32, 32, 2048, 128, 12.20, 13.65), (16, 17, 1152, 128, 9.29, 9.83),
+    (96, 1, 8192, 128, 42.13, 37.58), (80, 4, 4072, 128, 23.16, 20.08), (40, 24, 2076, 64, 15.07, 17.90),
     (32, 32, 1152, 128, 9.38, 11.77), (8, 32, 1408, 128, 9.87, 9.47), (16, 32, 2048, 128, 12.15, 11.00), (32, 32, 4096, 128, 21.97, 19.86),
     # a few heads more than there are compute units
     (264, 1, 640, 128, 15.28, 18.15), (264, 1, 1152, 128, 22.20, 20.29), (264, 1, 2176, 128, 35.53, 31.22), (384, 1, 640, 128, 16.09, 20.62), (264, 4, 640, 128, 15.43, 19.28),
