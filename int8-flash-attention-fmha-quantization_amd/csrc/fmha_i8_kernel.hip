@@ -579,7 +579,7 @@ __global__ __launch_bounds__(kThreads, (waves_per_simd<D, BK, BIAS>())) void fmh
   constexpr bool kV0BeforeFirstBarrier = FULLP && kOneBarrier;
   // At head_dim 128 the rows pass through LDS: eight lanes fetch a row's 128 contiguous bytes, where operands fetched straight into
   // registers touch 32 rows with every load and the CU's address path, which the first barrier waits for, takes twice as long (B4 H16
-  // S1024 21.3 -> 21.0 us, B16 H16 S256 9.54 -> 9.27; at head_dim 64, two rows to 128 bytes, no gain).  Each wavefront reads back what it
+  // S1024 22.6 -> 22.2 us, B16 H16 S256 9.76 -> 9.42, with 255 steps B4 H16 S1024 24.6 -> 24.0; at head_dim 64, two rows to 128 bytes, no gain).  Each wavefront reads back what it
   // has fetched itself, behind its own wait: where a tile will land only if that load is issued behind a later barrier than the read -
   // V of stage 3 is asked for in the phases of block 1, behind the second barrier; stage 1 right behind the first one.
   auto q_place = [&]() __attribute__((always_inline)) -> const int8_t* {

@@ -99,8 +99,8 @@ __device__ __forceinline__ int classify_key_blocks(const v4i& mask_bytes, const 
     if (live != 0) live_hi = (base + kMaskBytesPerLane * (first_lane + 63 - __builtin_clzll(live))) / BK;
   };
   if (from + kMaskBytesPerLane * first_lane < to) pass(from, mask_bytes);
-  // Longer rows, out of the way of the others (B8 H16 Sq1 S2048 d128 14.07 -> 13.87 us, H16 Sq512 S512 5.83 -> 5.73 against one loop for
-  // all, elsewhere within 1 % either way): two passes at a time, two loads behind one wait (H4 Sq512 S16300 scattered 115.9 -> 114.9).
+  // Longer rows, out of the way of the others (B8 H16 Sq1 S2048 d128 14.10 -> 14.00 us, H16 Sq512 S512 5.90 -> 5.82 against one loop for
+  // all, elsewhere within 1 % either way): two passes at a time, two loads behind one wait (H4 Sq512 S16300 scattered 114.8 -> 113.8).
   constexpr int kKeysPerPass = kMaskBytesPerLane * 64 * WAVES;
   for (int base = from + kKeysPerPass; base + kMaskBytesPerLane * first_lane < to; base += 2 * kKeysPerPass) {
     const int j = base + kMaskBytesPerLane * tid;
@@ -162,8 +162,8 @@ __global__ __launch_bounds__(256 * R, R) void fmha_i8_split_kernel(const SplitKe
   // file).  With one round or two per workgroup the time is that of the first loads, so V is asked for beside K.
   static_assert(!PARTS || R == 1, "");
   constexpr bool kEarlyV = PARTS && kOwnK;
-  // P of a wavefront's own key block, an operand of its own GEMM 2 too, need not come back from LDS: H16 Sq512 S960 d64 8.41 -> 8.19 us, B4 H8
-  // Sq200 S400 5.77 -> 5.66.  The other forms lose more by the branch in the middle of their operand reads than the reads cost (H16 S777 d128
+  // P of a wavefront's own key block, an operand of its own GEMM 2 too, need not come back from LDS: H16 Sq512 S960 d64 8.50 -> 8.39 us, B2 H16
+  // Sq100 S576 d128 7.86 -> 7.65, with 255 steps H16 Sq512 S960 d64 9.68 -> 9.38, Sq256 S1984 16.6 -> 16.1, short ones level.  The other forms lose more by the branch in the middle of their operand reads than the reads cost (H16 S777 d128
   // 11.30 -> 11.50, H32 Sq512 S4096 31.3 -> 31.8, d64 S2048 11.47 -> 11.79).
   constexpr bool kOwnP = R == 1 && BK == 64 && !PARTS;
   // Q: the operands of GEMM 1 straight from memory touch 32 rows with every load, and the four wavefronts of a row group load the same
