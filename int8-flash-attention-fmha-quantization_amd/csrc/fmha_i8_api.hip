@@ -206,14 +206,14 @@ constexpr KernelCost kKernelCosts[] = {{0, 1, {{{70, 80, 120}, {105, 129, 120}},
 // are compute units run into the memory.  So these have prices of their own, the same way for a head by one workgroup as for key blocks
 // shared out ([at most sixteen rows, more][head_dim][block]): the workgroups that run at a time take max(start + step * rounds + again,
 // their keys at 67 KB in a hundredth of a microsecond), `again` from the second time on; `together` is how many a CU holds, of which the
-// second adds half of the first one's time; `slowed`: percent of the memory's time on top (d128, S4096: H16 21.2 us, H64 22.9, H96 23.2).  Fitted to 1,347 calls of 4 to 1024 heads timed on both routes; see part_plan_of.
+// second adds half of the first one's time; `slowed`: percent of the memory's time on top (d128, S4096: H16 21.2 us, H64 22.9, H96 23.2).  Fitted to calls of 1 to 1024 heads timed on both routes; see part_plan_of.
 struct HeadCost {
   int start, step, again, together, slowed;
 };
 constexpr HeadCost kHeadCosts[2][2][2] = {{{{-60, 103, 140, 2}, {-25, 145, 150, 1}}, {{-20, 131, 150, 1}, {10, 230, 200, 1, 12}}},
                                           {{{-15, 135, 150, 2}, {0, 213, 240, 1}}, {{20, 152, 230, 1}, {10, 230, 200, 1, 12}}}};
 constexpr HeadCost kPartCosts[2][2][2] = {{{{60, 106, 0, 2}, {20, 200, 80, 1}}, {{20, 165, 130, 1}, {70, 210, 130, 1}}},
-                                          {{{35, 90, 70, 1}, {20, 187, 120, 1}}, {{25, 155, 70, 1}, {10, 285, 260, 1}}}};
+                                          {{{35, 90, 70, 1}, {20, 187, 120, 1}}, {{25, 155, 70, 1}, {0, 280, 260, 1}}}};
 long long cost_of_head_workgroups(const HeadCost& c, long long wgs, int rounds, long long key_bytes) {
   const long long at_a_time = (long long)kComputeUnits * c.together, full = wgs / at_a_time, rest = wgs % at_a_time;
   auto one_time = [&](long long n, bool first) -> long long {
@@ -303,18 +303,26 @@ int pieces_of(const FMHACrossAttnDescriptor& a, int block_keys, Piece (&pieces)[
   }
   return count;
 }
-// Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for (kPartCosts), with the
-// workspace written and read again (45 KB in a hundredth of a microsecond, 42 above sixteen rows) and the merge: 2.1 us for the launch and
-// the first batch of key blocks, 1.1 more for batches of 32 instead of 16, 0.8 per further batch; 0.9 on top, and 0.5 per further batch, with more
-// than sixteen rows, of which some row moves its reference in nearly every block.  (One head and up to eight heads are put 0.4 and 0.5 us too low: calls whose
-// two routes are that close stay shared out, as they have been - H1 Sq8 S1089 d64 7.2 us either way, H6 Sq5 S1030 d64 7.4 and 8.0.)  Within 5 %
-// of each other (the factor 20/21) the plain route is taken, which needs no memory and can write a float output besides.
+// What follows the workgroups of shared-out key blocks ([at most sixteen rows, more], hundredths of a microsecond): the merge's launch and its
+// first batch of key blocks, more for batches of 32 instead of 16, for a second batch, for each further one (with more than sixteen rows some row
+// moves its reference in nearly every block), and the workspace written and read, bytes in a hundredth of a microsecond, those of its first
+// 20 MB on top: with one rate for all (42 KB) calls of 17 to 32 rows over more than 8000 keys lost up to 47 % (H32 Sq32 S14400 d128 100.7 us plain,
+// 68.4 shared out).
+struct MergeCost {
+  int launch, wide, second, further, rate, first_rate;
+};
+constexpr MergeCost kMergeCosts[2] = {{208, 88, 160, 30, 75000, 174000}, {315, 80, 245, 340, 118000, 55500}};
+// Whether a call shares its key blocks out, and how: as few rounds per workgroup as there are compute units for (kPartCosts), and what follows
+// them.  (One head and up to eight heads are put 0.4 us too low: calls whose two routes are that close stay shared out, as they have been - H1
+// Sq8 S1089 d64 7.2 us either way, H6 Sq5 S1030 d64 7.4 and 8.0.)  Within 5 % of each other (the factor 20/21) the plain route is taken, which
+// needs no memory and can write a float output besides.
 // One call, plain and shared out, us: d128 B1 H16 Sq1 S2048 12.1 and 8.0, H32 S4096 21.6 and 9.6, H16 Sq32 S4096 21.2 and 14.6, B2 H16 Sq32
 // S1664 11.6 and 12.8, S2048 12.1 and 13.7, H16 Sq17 S1152 9.3 and 9.8, H264 Sq1 S640 15.4 and 18.1, S1152 22.3 and 20.3, B8 H16 Sq1 S2048,
 // which the memory bounds already, 13.8 and 14.7; d64 H64 Sq1 S2048 8.5 and 7.6, H264 Sq1 S1088 9.3 and 14.2.
-// Of 1,986 such calls timed on both routes, 1 to 1024 heads, the choice is more than 2 % slower than the other one in 53, more than 10 % in 4, at
-// most by 12 % (H31 Sq17 S2478 d128).  It was in 208 and 67 with a table that priced the two sides apart and took each further workgroup on a CU
-// for as dear as the first, the memory for a bound on the whole call alone.
+// Of 2,316 such calls timed on both routes, 1 to 1024 heads and up to 65536 keys, the choice is more than 2 % slower than the other one in 80,
+// more than 10 % in 5; of 500 others, drawn where the two are close, in 28 and 8, at most by 17 % (H140 Sq1 S18624 d64, more than the last cache
+// holds).  It was in 398 and 141, and 71 and 21, with a table that priced the two sides apart, took each further workgroup on a CU for as dear as
+// the first and the memory for a bound on the whole call alone.
 PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   using namespace fmha_i8_gfx950;
   PartPlan plan;
@@ -323,8 +331,10 @@ PartPlan part_plan_of(const FMHACrossAttnDescriptor& a, int block_keys) {
   if (a.seq_len_q > kPartRows || rounds < 2 || heads > 65535) return plan;  // (heads: the y extent of the merge's grid)
   if (test_build::forced_route() >= 0) return plan;
   const bool one_group = a.seq_len_q > kFewRows;
-  const long long merge = 210 - 42 / heads + (blocks <= 16 ? 0 : heads > 8 ? 110 : 55) + (one_group ? 130 : 80) * ((blocks - 1) / 32) + (one_group ? 90 : 0) +
-                          heads * blocks * a.seq_len_q * (8 * a.head_dim + 16) / (one_group ? 42000 : 45000);
+  const MergeCost& c = kMergeCosts[one_group];
+  const long long bytes = heads * blocks * a.seq_len_q * (8 * a.head_dim + 16), first_bytes = bytes < 20000000 ? bytes : 20000000;
+  const long long merge = c.launch - 42 / heads + (blocks <= 16 ? 0 : heads > 8 ? c.wide : c.wide / 2) + (blocks <= 32 ? 0 : c.second + c.further * ((blocks - 33) / 32)) +
+                          bytes / c.rate + first_bytes / c.first_rate;
   const HeadCost& price = kPartCosts[one_group][a.head_dim == 128][block_keys == kBlockK];
   const long long plain = cheapest_kernel(heads, a.seq_len_q, a.head_dim, blocks, block_keys).cost * 20 / 21;
   long long work = 0;

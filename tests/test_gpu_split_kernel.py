@@ -163,6 +163,8 @@ PLAIN_OR_SHARED = [
     (32, 32, 1664, 128, 11.64, 12.71), (32, 32, 1792, 128, 11.66, 12.99), (32, 32, 1920, 128, 12.18, 13.37), (32, 32, 2048, 128, 12.20, 13.65), (16, 17, 1152, 128, 9.29, 9.83),
     (96, 1, 8192, 128, 42.13, 37.58), (80, 4, 4072, 128, 23.16, 20.08), (40, 24, 2076, 64, 15.07, 17.90),
     (32, 32, 1152, 128, 9.38, 11.77), (8, 32, 1408, 128, 9.87, 9.47), (16, 32, 2048, 128, 12.15, 11.00), (32, 32, 4096, 128, 21.97, 19.86),
+    # a workspace of many megabytes
+    (32, 32, 14400, 128, 100.74, 68.40), (64, 24, 14144, 64, 88.30, 60.67), (48, 24, 15488, 128, 82.31, 59.63), (64, 32, 7168, 64, 32.86, 27.64),
     # a few heads more than there are compute units
     (264, 1, 640, 128, 15.28, 18.15), (264, 1, 1152, 128, 22.20, 20.29), (264, 1, 2176, 128, 35.53, 31.22), (384, 1, 640, 128, 16.09, 20.62), (264, 4, 640, 128, 15.43, 19.28),
     (320, 4, 640, 128, 15.83, 20.07), (264, 1, 1088, 64, 9.36, 14.19), (264, 1, 1600, 64, 13.21, 17.08), (264, 1, 2112, 64, 16.20, 22.35), (264, 1, 3136, 64, 21.85, 27.65),
